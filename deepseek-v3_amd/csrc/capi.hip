@@ -337,4 +337,45 @@ int dsv3_wkv_b_absorb(const void* x, int64_t x_token_stride, int64_t x_head_stri
                                nope_dim, v_dim, kv_rank, (hipStream_t)stream);
 }
 
+size_t dsv3_mla_prefill_workspace_bytes(int64_t batch, int64_t rows, int64_t positions, int heads) {
+    if (batch <= 0 || rows <= 0 || positions <= 0 || heads <= 0) return 0;
+    return mla_prefill_workspace_bytes(batch, rows, positions, heads);
+}
+
+// Checks that the two attention entry points share (no GPU call); 0 rows or heads are not looked at further.
+static int mla_validate(const void* q, const float* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
+                        const void* mask, int mask_dtype, const void* y, int64_t batch, int64_t rows, int64_t positions,
+                        int heads, int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale) {
+    if (mask && mask_dtype != DSV3_BF16 && mask_dtype != DSV3_F32) return DSV3_ERR_BAD_DTYPE;
+    if (nope_dim != 128 || rope_dim != 64 || v_dim != 128 || kv_rank != 512) return DSV3_ERR_BAD_SHAPE;
+    if (batch < 0 || rows < 0 || heads < 0 || heads > 65535 || batch > 65535 || rows > 0x7fffff || positions < 1 ||
+        positions > 0x7fffff || !(softmax_scale > 0.f))
+        return DSV3_ERR_BAD_SHAPE;
+    if (batch > 1 && (kv_bs < positions * kv_rank || pe_bs < positions * rope_dim || kv_bs % 8 != 0 || pe_bs % 8 != 0))
+        return DSV3_ERR_BAD_SHAPE;
+    if (batch == 0 || rows == 0 || heads == 0) return DSV3_OK;
+    if (!q || !freqs || !kv || !pe || !y) return DSV3_ERR_NULL_POINTER;
+    if (!aligned(q, 16) || !aligned(freqs, 8) || !aligned(kv, 16) || !aligned(pe, 16) || !aligned(y, 16) ||
+        !aligned(mask, mask_dtype == DSV3_F32 ? 4 : 2))
+        return DSV3_ERR_MISALIGNED;
+    return DSV3_OK;
+}
+
+int dsv3_mla_prefill(const void* q, const float* freqs, const void* kv_cache, int64_t kv_batch_stride,
+                     const void* pe_cache, int64_t pe_batch_stride, const void* wkv_b, const float* wkv_b_scale,
+                     const void* mask, int mask_dtype, void* y, float* s, int64_t batch, int64_t rows, int64_t positions,
+                     int heads, int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale,
+                     void* workspace, size_t workspace_bytes, void* stream) {
+    const int rc = mla_validate(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, mask, mask_dtype, y, batch,
+                                rows, positions, heads, nope_dim, rope_dim, v_dim, kv_rank, softmax_scale);
+    if (rc != DSV3_OK || batch == 0 || rows == 0 || heads == 0) return rc;
+    if (!wkv_b || !wkv_b_scale || !s) return DSV3_ERR_NULL_POINTER;
+    if (!aligned(wkv_b, 16) || !aligned(wkv_b_scale, 4) || !aligned(s, 4)) return DSV3_ERR_MISALIGNED;
+    if (!workspace || !aligned(workspace, 256) || workspace_bytes < mla_prefill_workspace_bytes(batch, rows, positions, heads))
+        return DSV3_ERR_WORKSPACE;
+    return launch_mla_prefill(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, wkv_b, wkv_b_scale, mask,
+                              mask_dtype == DSV3_F32, y, s, batch, rows, positions, heads, softmax_scale, workspace,
+                              (hipStream_t)stream);
+}
+
 }  // extern "C"

@@ -1,0 +1,425 @@
+// Attention of MLA.forward for many new tokens per sequence (reference: inference/model.py:470-497), from the query
+// projection and the latent cache to the FP8 input of the output projection, without a score matrix in memory.
+//
+// The latent cache holds one 512-wide latent and one 64-wide rotary key per position; the key of head h is
+// [W_k[h] latent | rotary key] (128 + 64 wide), its value W_v[h] latent (128 wide), W = wkv_b.  The absorbed form
+// folds W_k into the query and W_v into the output, which costs nothing per position but makes every query-key pair
+// a 576-wide and every weighted sum a 512-wide product; here the keys and values are formed first (2 * 512 * 256
+// operations per head and position) and a pair costs 192 + 128.  With as many new tokens as positions that is 3.4 x
+// less work in front of the matrix cores; where few tokens meet many positions the absorbed form wins (mla_decode.hip).
+// Roundings: keys and values to bf16 (the absorbed form rounds the folded query and the latent sum instead), exponentials
+// to bf16 in front of the value product, scores and sums in binary32, the result to bf16 and then quantised.
+//
+// Three launches: expand (keys and values, and the rotary keys, in the order in which the attention kernel's wavefronts
+// read their operands), flags (which tiles of the mask are all zero or all -inf; only with a mask), attend.
+// At 4096 tokens, 128 heads, causal mask: expand 226 us, flags 23 us, attend 915 us (0.75 PFLOP/s of the pairs the mask
+// leaves); the whole layer 1.77 ms where the absorbed form as tensor operations took 20.2 ms (2 x 2.5 ms score products,
+// 1.6 ms value product and 12 ms of passes over the 4.3 GB score matrix).
+#include "common.hpp"
+
+namespace dsv3 {
+namespace {
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) void* lptr_t;
+
+constexpr int kC = 512, kRope = 64, kNope = 128, kV = 128, kQd = kNope + kRope;
+constexpr int kTile = 64;                       // positions per tile
+// One tile's operands, bytes.  Keys: [position half][16-wide K step][lane][16]; the same for the rotary keys; values:
+// [32 features][16 positions][lane][16].  A wavefront's operand of one MFMA is 1 KiB, lane l's piece at 16 l.
+constexpr int kKeyBytes = kTile * kNope * 2, kValBytes = kTile * kV * 2, kRopeBytes = kTile * kRope * 2;
+constexpr int kHeadTile = kKeyBytes + kValBytes;
+constexpr int kQTile = 256;                     // query rows per workgroup: 8 wavefronts x 32
+
+__device__ __forceinline__ v16f mfma32(v4u a, v4u b, v16f c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t lds_addr_of(const void* p) { return (uint32_t)(uintptr_t)(lptr_t)p; }
+// 1 KiB global -> LDS: lane l's 16 bytes at base + lane_off land at lds_addr + 16 l
+__device__ __forceinline__ void copy16(const void* base, uint32_t lane_off, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(lane_off), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+__device__ __forceinline__ void barrier_no_fence() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// ---------------------------------------------------------------------------------------------------------- expand
+
+struct ExpandArgs {
+    const uint16_t* kv; int64_t kv_bs;          // latents [batch][positions][512], batch stride in elements
+    const uint16_t* pe; int64_t pe_bs;          // rotary keys [batch][positions][64]
+    const uint8_t* w; const float* ws;          // wkv_b fp8 [heads * 256, 512] and its block scales
+    uint8_t* img;                               // [batch][heads][tiles][kHeadTile]
+    uint8_t* rope;                              // [batch][tiles][kRopeBytes]
+    int batch, heads, positions, tiles;
+};
+
+// A workgroup owns one head: wavefronts 0-3 hold 32 key features each, 4-7 32 value features, as bf16 MFMA operands
+// (32 features x 512 = 128 registers, dequantised once), and stream 32-position sub-tiles of the latents past them
+// (32 KiB each, through LDS, one sub-tile ahead).  Key features are issued as the A operand and positions as B, value
+// features the other way round, so that in both cases a lane ends up with 16-byte pieces of the attention kernel's
+// operand order and a store instruction writes 1 KiB of consecutive bytes: MFMA row 8j + 4g + r of a key wavefront is
+// feature 16 (j / 2) + 8 g + 4 (j % 2) + r; a value lane's accumulator registers 8u .. 8u + 7 are, in order, the
+// eight positions that the attention kernel's K step u has in that lane.
+// Bound by the LDS reads of the latents (every wavefront reads the whole sub-tile: 1 KiB per 32-cycle MFMA and SIMD pair,
+// ~0.6 of what the LDS delivers) and the 268 MB of results at 4096 positions.
+__global__ __launch_bounds__(512, 2) void mla_expand_kernel(ExpandArgs p) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * 32 * 1024];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = lane & 31, g = lane >> 5;
+    const int h = blockIdx.x;
+    const int subs = p.batch * p.tiles * 2;                 // 32-position sub-tiles, batch-major
+    const int per = (subs + gridDim.y - 1) / gridDim.y;
+    const int s0 = blockIdx.y * per, s1 = min(subs, s0 + per);
+    if (s0 >= s1) return;
+
+    if (h == p.heads) {                                     // the rotary keys, shared by all heads: only re-ordered
+        for (int sub = s0 + wave; sub < s1; sub += 8) {
+            const int b = sub / (p.tiles * 2), sb = sub - b * p.tiles * 2;
+            const int pos = min(sb * 32 + i, p.positions - 1);
+            const uint16_t* src = p.pe + b * p.pe_bs + (int64_t)pos * kRope + g * 8;
+            v4u* dst = (v4u*)(p.rope + (int64_t)sub * (kRopeBytes / 2)) + lane;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) dst[s * 64] = *(const v4u*)(src + s * 16);
+        }
+        return;
+    }
+
+    // sub-tile rows: 1 KiB each, 16-byte chunk c stored at c ^ (row & 15): 16 rows read at the same c hit 16 distinct
+    // 16-byte columns
+    const uint32_t lds0 = lds_addr_of(lds);
+    auto issue = [&](int sub, int st) {
+        sub = min(sub, s1 - 1);
+        const int b = sub / (p.tiles * 2), sb = sub - b * p.tiles * 2;
+        const uint16_t* base = p.kv + b * p.kv_bs;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int row = wave * 4 + n;
+            const int pos = min(sb * 32 + row, p.positions - 1);
+            copy16(base + (int64_t)pos * kC, (uint32_t)((lane ^ (row & 15)) << 4), lds0 + st * 32768 + row * 1024);
+        }
+    };
+    issue(s0, 0);
+
+    const bool keys = wave < 4;
+    v4u W[32];
+    {
+        const int j = i >> 3, g2 = (i >> 2) & 1, r = i & 3;
+        const int f = keys ? 16 * (j >> 1) + 8 * g2 + 4 * (j & 1) + r : i;
+        const int64_t row = (int64_t)h * (kNope + kV) + (keys ? 0 : kNope) + 32 * (wave & 3) + f;
+        const uint8_t* src = p.w + row * kC + 8 * g;
+        const float* sc = p.ws + (row >> 7) * (kC / 128);
+#pragma unroll
+        for (int s = 0; s < 32; ++s) {
+            const v2u raw = *(const v2u*)(src + 16 * s);
+            const float k = sc[s / 8];
+            const v2f a = fp8x2_lo_to_f32(raw[0]), b = fp8x2_hi_to_f32(raw[0]), c = fp8x2_lo_to_f32(raw[1]), d = fp8x2_hi_to_f32(raw[1]);
+            W[s] = v4u{ pack_bf16(a.x * k, a.y * k), pack_bf16(b.x * k, b.y * k), pack_bf16(c.x * k, c.y * k), pack_bf16(d.x * k, d.y * k) };
+        }
+    }
+    const uint32_t frag = i * 1024;
+    int st = 0;
+    for (int sub = s0; sub < s1; ++sub, st ^= 1) {
+        if (sub == s0) __builtin_amdgcn_s_waitcnt(0x0f70);          // vmcnt(0)
+        else           __builtin_amdgcn_s_waitcnt(0x0f70 | 2);      // vmcnt(2): the two stores of the sub-tile before are younger
+        barrier_no_fence();
+        issue(sub + 1, st ^ 1);
+        v16f acc = {};
+        const uint8_t* t = lds + st * 32768 + frag;
+#pragma unroll
+        for (int s = 0; s < 32; ++s) {
+            const v4u x = *(const v4u*)(t + (((2 * s + g) ^ (i & 15)) << 4));
+            acc = keys ? mfma32(W[s], x, acc) : mfma32(x, W[s], acc);
+        }
+        const int b = sub / (p.tiles * 2), sb = sub - b * p.tiles * 2;
+        uint8_t* tile = p.img + (((int64_t)b * p.heads + h) * p.tiles + (sb >> 1)) * kHeadTile;
+        v4u o[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[u][q] = pack_bf16(acc[8 * u + 2 * q], acc[8 * u + 2 * q + 1]);
+        // keys: K steps 2 wave + u of position half sb & 1; values: positions 16 (2 (sb & 1) + u) of features 32 (wave - 4)
+        v4u* dst = keys ? (v4u*)(tile + ((sb & 1) * 8 + 2 * wave) * 1024) : (v4u*)(tile + kKeyBytes + ((wave & 3) * 4 + 2 * (sb & 1)) * 1024);
+        dst[lane] = o[0];
+        dst[64 + lane] = o[1];
+    }
+    __builtin_amdgcn_s_waitcnt(0x0f70);         // the repeated copies of the last iteration still write LDS
+}
+
+// ----------------------------------------------------------------------------------------------------------- flags
+
+enum : uint8_t { kClear = 0, kMixed = 1, kSkip = 2 };
+
+template <bool F32> __device__ __forceinline__ float mask_at(const void* m, int64_t i) {
+    return F32 ? ((const float*)m)[i] : u32_as_f32((uint32_t)((const uint16_t*)m)[i] << 16);
+}
+
+// flags[tile][q / 32]: what the mask does to 32 query rows x 64 positions (all zero, anything, all -inf or no row)
+template <bool F32>
+__global__ __launch_bounds__(512) void mla_mask_flags_kernel(const void* mask, uint8_t* flags, int rows, int positions, int groups) {
+    const int lane = threadIdx.x & 63, q32 = blockIdx.y * 8 + (threadIdx.x >> 6);
+    const int pos = blockIdx.x * kTile + lane;
+    bool zero = true, ninf = true;
+    if (pos < positions)
+#pragma unroll 8
+        for (int r = 0; r < 32; ++r) {
+            const int q = q32 * 32 + r;
+            if (q < rows) {
+                const float v = mask_at<F32>(mask, (int64_t)q * positions + pos);
+                zero = zero && v == 0.f;
+                ninf = ninf && v == -__builtin_inff();
+            }
+        }
+    const uint8_t f = __all(ninf) ? kSkip : __all(zero) ? kClear : kMixed;
+    if (lane == 0) flags[(int64_t)blockIdx.x * groups + q32] = f;
+}
+
+// ---------------------------------------------------------------------------------------------------------- attend
+
+struct AttendArgs {
+    const uint16_t* q;                          // [batch][rows][heads][192], rotary part not yet rotated
+    const v2f* freqs;                           // [rows][32] (cos, sin)
+    const uint8_t* img; const uint8_t* rope;
+    const void* mask; const uint8_t* flags;     // [rows][positions] / [tiles][groups], or null
+    uint8_t* y; float* ys;                      // fp8 [batch][rows][heads * 128], scales [batch][rows][heads]
+    int batch, heads, rows, positions, tiles, qtiles, groups;
+    float scale, inv_scale;                     // softmax scale and its reciprocal
+};
+
+__device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32); }
+
+// One workgroup: 256 query rows of one head; wavefront w rows 32 w .. 32 w + 31.  Per tile of 64 positions (40 KiB of
+// operands, double-buffered in LDS, copied while the tile before is computed) a wavefront forms S^T = K Q^T (24 MFMAs),
+// exponentials in registers, and O^T += V^T P^T (16 MFMAs).  The transposed products leave a query row in one lane
+// (and the lane 32 further), so maxima and sums need one exchange, the rescale factor is one value per lane, and the
+// accumulator layout of S^T already is the B operand of the second product: position 16 u + 8 a + 4 g + r of a tile sits
+// in register 8 u' + 4 a + r of lane half g, which is slot 4 a + r of K step u, and the values were written in that
+// order.  The running maximum is only raised when it grows by more than 2^8 (exponentials then stay below 2^8, and most
+// tiles skip the 64 multiplications of the rescale).
+// Wavefronts 4-7 run at raised priority: each SIMD holds one wavefront of either group, the two would otherwise do
+// their MFMAs at the same time and their exponentials at the same time.
+template <bool MF32>
+__global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    constexpr int kStage = kHeadTile + kRopeBytes;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = lane & 31, g = lane >> 5;
+    // heads are dealt over the XCDs (whose L2 then holds a head's keys and values for all its query tiles), the query
+    // tiles of a head run last to first: with a causal mask the long ones start first
+    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+    const int bh = xcd + 8 * (idx / p.qtiles), qt = p.qtiles - 1 - idx % p.qtiles;
+    if (bh >= p.batch * p.heads) return;
+    const int b = bh / p.heads, h = bh - b * p.heads;
+    const int q0 = qt * kQTile + wave * 32;
+    const int row = min(q0 + i, p.rows - 1);
+
+    // query operands: lane (row i, half g) holds elements 16 s + 8 g .. + 7; the last four steps are rotated here
+    v4u Q[12];
+    {
+        const uint16_t* src = p.q + (((int64_t)b * p.rows + row) * p.heads + h) * kQd + 8 * g;
+#pragma unroll
+        for (int s = 0; s < 12; ++s) Q[s] = *(const v4u*)(src + 16 * s);
+        const v2f* fr = p.freqs + (int64_t)row * (kRope / 2) + 4 * g;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const v2f cs = fr[8 * s + e];
+                const float re = bf16lo_to_f32(Q[8 + s][e]), im = bf16hi_to_f32(Q[8 + s][e]);
+                Q[8 + s][e] = pack_bf16(re * cs.x - im * cs.y, re * cs.y + im * cs.x);
+            }
+    }
+
+    const uint8_t* himg = p.img + (int64_t)bh * p.tiles * kHeadTile;
+    const uint8_t* rimg = p.rope + (int64_t)b * p.tiles * kRopeBytes;
+    const uint32_t lds0 = lds_addr_of(lds), lane16 = lane * 16;
+    auto issue = [&](int t, int st) {
+        const uint8_t* src = himg + (int64_t)t * kHeadTile;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) copy16(src + (n * 8 + wave) * 1024, lane16, lds0 + st * kStage + (n * 8 + wave) * 1024);
+        copy16(rimg + (int64_t)t * kRopeBytes + wave * 1024, lane16, lds0 + st * kStage + kHeadTile + wave * 1024);
+    };
+    // the workgroup's flags of a tile: one byte per wavefront, 2 everywhere = nobody needs the tile
+    auto tile_flags = [&](int t) -> uint64_t {
+        return p.flags ? *(const uint64_t*)(p.flags + (int64_t)t * p.groups + qt * 8) : 0ull;
+    };
+    constexpr uint64_t kAllSkip = 0x0202020202020202ull;
+    auto next_tile = [&](int t) {
+        while (t < p.tiles && tile_flags(t) == kAllSkip) ++t;
+        return t;
+    };
+
+    v16f O[4] = {};
+    float m = -__builtin_inff(), l = 0.f;           // running maximum (raw scores), this lane's share of the sum
+    const float scale2 = p.scale * 1.44269504088896340736f;
+    int t = next_tile(0), st = 0;
+    if (t < p.tiles) issue(t, 0);
+    if (wave >= 4) __builtin_amdgcn_s_setprio(1);
+    while (t < p.tiles) {
+        const uint8_t flag = (uint8_t)(tile_flags(t) >> (8 * wave));
+        const int tn = next_tile(t + 1);
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        barrier_no_fence();
+        if (tn < p.tiles) issue(tn, st ^ 1);
+        if (flag != kSkip) {
+            const uint8_t* base = lds + st * kStage + lane16;
+            v16f S[2] = {};
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) S[k] = mfma32(*(const v4u*)(base + (k * 8 + s) * 1024), Q[s], S[k]);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) S[k] = mfma32(*(const v4u*)(base + kHeadTile + (k * 4 + s) * 1024), Q[8 + s], S[k]);
+            if (flag == kMixed) {
+                const int64_t mrow = (int64_t)row * p.positions;
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int pos = t * kTile + 32 * k + 8 * (e >> 2) + 4 * g + (e & 3);
+                        S[k][e] += mask_at<MF32>(p.mask, mrow + min(pos, p.positions - 1)) * p.inv_scale;
+                    }
+            }
+            if ((t + 1) * kTile > p.positions) {            // the last tile may reach past the end
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int pos = t * kTile + 32 * k + 8 * (e >> 2) + 4 * g + (e & 3);
+                        if (pos >= p.positions) S[k][e] = -__builtin_inff();
+                    }
+            }
+            float mx = S[0][0];
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, S[k][e]);
+            mx = fmaxf(mx, xor32(mx));
+            const bool raise = (mx - m) * scale2 > 8.f || (m == -__builtin_inff() && mx > m);
+            if (__any(raise)) {
+                const float mn = fmaxf(m, mx);
+                const float a = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f((m - mn) * scale2);
+                l *= a;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) O[d][e] *= a;
+                m = mn;
+            }
+            const float off = m == -__builtin_inff() ? 0.f : m * scale2;
+            float sum = 0.f;
+            v4u P[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int e = 8 * (u & 1) + 2 * q;
+                    const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(S[u >> 1][e], scale2, -off));
+                    const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(S[u >> 1][e + 1], scale2, -off));
+                    sum += x + y;
+                    P[u][q] = pack_bf16(x, y);
+                }
+            l += sum;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int d = 0; d < 4; ++d) O[d] = mfma32(*(const v4u*)(base + kKeyBytes + (d * 4 + u) * 1024), P[u], O[d]);
+        }
+        st ^= 1;
+        t = tn;
+    }
+    __builtin_amdgcn_s_setprio(0);
+
+    // O / l to bf16, then the 128 values of a (token, head) as one quantisation block of the output projection's input
+    l += xor32(l);
+    const float rl = 1.0f / l;
+    uint32_t abits = 0u;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            O[d][e] = round_bf16(O[d][e] * rl);
+            abits = umax_u32(abits, abs_bits(O[d][e]));
+        }
+    abits = umax_u32(abits, (uint32_t)__shfl_xor((int)abits, 32));
+    const float sc = block_scale(abits, false), rs = 1.0f / sc;
+    const bool fast = block_is_finite(abits);
+    const bool live = q0 + i < p.rows;
+    const int64_t out = (((int64_t)b * p.rows + row) * p.heads + h);
+    uint8_t* dst = p.y + out * kV;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            uint32_t by[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                float v[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = block_quotient(O[d][8 * a + 4 * k + r], sc, rs, fast);
+                by[k] = pack_fp8x4(v[0], v[1], v[2], v[3]);
+            }
+            // by[k]: features 32 d + 16 a + 8 k + 4 g ..; after the exchange lane half g holds 16 a + 8 g .. + 7
+            const uint32_t give = g ? by[0] : by[1];
+            const uint32_t got = (uint32_t)__shfl_xor((int)give, 32);
+            const v2u o = g ? v2u{ got, by[1] } : v2u{ by[0], got };
+            if (live) *(v2u*)(dst + 32 * d + 16 * a + 8 * g) = o;
+        }
+    if (live && g == 0) p.ys[out] = sc;
+}
+
+inline int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
+
+}  // namespace
+
+size_t mla_prefill_workspace_bytes(int64_t batch, int64_t rows, int64_t positions, int heads) {
+    const int64_t tiles = (positions + kTile - 1) / kTile, groups = (rows + kQTile - 1) / kQTile * 8;
+    return (size_t)(align256(batch * heads * tiles * kHeadTile) + align256(batch * tiles * kRopeBytes) + align256(tiles * groups));
+}
+
+int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
+                       const void* w, const float* ws, const void* mask, bool mask_f32, void* y, float* ys, int64_t batch,
+                       int64_t rows, int64_t positions, int heads, float scale, void* workspace, hipStream_t st) {
+    const int64_t tiles = (positions + kTile - 1) / kTile, qtiles = (rows + kQTile - 1) / kQTile;
+    const int64_t wgs = (batch * heads + 7) / 8 * 8 * qtiles;
+    if (wgs > 0x7fffffff || batch * tiles * 2 > 0x7fffffff || qtiles > 65535) return DSV3_ERR_BAD_SHAPE;
+    ExpandArgs e;
+    e.kv = (const uint16_t*)kv; e.kv_bs = kv_bs; e.pe = (const uint16_t*)pe; e.pe_bs = pe_bs;
+    e.w = (const uint8_t*)w; e.ws = ws;
+    e.img = (uint8_t*)workspace;
+    e.rope = e.img + align256(batch * heads * tiles * kHeadTile);
+    e.batch = (int)batch; e.heads = heads; e.positions = (int)positions; e.tiles = (int)tiles;
+    uint8_t* flags = e.rope + align256(batch * tiles * kRopeBytes);
+    // two workgroups' worth of position ranges per compute unit at 128 heads; each wants a few sub-tiles behind its
+    // weight conversion
+    const int64_t subs = batch * tiles * 2;
+    int64_t gy = (512 + heads - 1) / heads;
+    gy = gy > (subs + 3) / 4 ? (subs + 3) / 4 : gy;
+    hipLaunchKernelGGL(mla_expand_kernel, dim3(heads + 1, (unsigned)gy), dim3(512), 0, st, e);
+
+    AttendArgs a;
+    a.q = (const uint16_t*)q; a.freqs = (const v2f*)freqs; a.img = e.img; a.rope = e.rope;
+    a.mask = mask; a.flags = mask ? flags : nullptr;
+    a.y = (uint8_t*)y; a.ys = ys;
+    a.batch = (int)batch; a.heads = heads; a.rows = (int)rows; a.positions = (int)positions;
+    a.tiles = (int)tiles; a.qtiles = (int)qtiles; a.groups = (int)(qtiles * 8);
+    a.scale = scale; a.inv_scale = 1.0f / scale;
+    if (mask) {
+        const dim3 grid((unsigned)tiles, (unsigned)qtiles);
+        if (mask_f32) hipLaunchKernelGGL(mla_mask_flags_kernel<true>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions, a.groups);
+        else hipLaunchKernelGGL(mla_mask_flags_kernel<false>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions, a.groups);
+    }
+    constexpr int bytes = 2 * (kHeadTile + kRopeBytes);
+    static LdsGrant grant[2];
+    if (mask && mask_f32) {
+        if (!grant[1].ensure((const void*)mla_attend_kernel<true>, bytes)) return DSV3_ERR_LAUNCH;
+        hipLaunchKernelGGL(mla_attend_kernel<true>, dim3((unsigned)wgs), dim3(512), bytes, st, a);
+    } else {
+        if (!grant[0].ensure((const void*)mla_attend_kernel<false>, bytes)) return DSV3_ERR_LAUNCH;
+        hipLaunchKernelGGL(mla_attend_kernel<false>, dim3((unsigned)wgs), dim3(512), bytes, st, a);
+    }
+    return launch_status();
+}
+
+}  // namespace dsv3

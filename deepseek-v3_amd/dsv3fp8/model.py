@@ -235,6 +235,9 @@ class MLA(nn.Module):
 
     fused: bool = True
     stacked_a: bool = True
+    # from this many new tokens per sequence on, keys and values are formed per head instead of being folded into the
+    # query and the output (csrc/mla_prefill.hip)
+    explicit_min_tokens: int = 32
 
     def __init__(self, args: ModelArgs):
         super().__init__()
@@ -315,6 +318,22 @@ class MLA(nn.Module):
             w = weight_dequant(w, self.wkv_b.scale, block_size)
         return w.view(self.n_local_heads, -1, self.kv_lora_rank)
 
+    def _attention_kernels_ok(self, x, q, positions: int, freqs_cis, mask) -> bool:
+        """Whether the attention between the query projection and ``wo`` can run on the fused kernels: their head
+        dimensions, FP8 weights on both sides, no gradients (the kernels have no backward), a mask of one value per
+        (query, position) pair as the reference builds it (model.py:738-740)."""
+        b, s = x.size(0), x.size(1)
+        return (not torch.is_grad_enabled() and gemm_impl == "fp8" and block_size == 128 and world_size == 1
+                and torch.get_default_dtype() == torch.bfloat16 and q.dtype == torch.bfloat16 and q.is_contiguous()
+                and (self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim, self.kv_lora_rank) == (128, 64, 128, 512)
+                and self.kv_cache.dtype == torch.bfloat16 and self.kv_cache.is_contiguous() and self.pe_cache.is_contiguous()
+                and b <= self.kv_cache.size(0) and s >= 1 and positions <= self.kv_cache.size(1)
+                and self.wo.weight.element_size() == 1 and self.wo.bias is None and self.wkv_b.bias is None
+                and freqs_cis.is_cuda and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous()
+                and freqs_cis.shape == (s, self.qk_rope_head_dim // 2)
+                and (mask is None or (mask.is_cuda and mask.shape == (s, positions) and mask.is_contiguous()
+                                      and mask.dtype in (torch.bfloat16, torch.float32))))
+
     def forward(self, x: torch.Tensor, start_pos: int, freqs_cis: torch.Tensor, mask: Optional[torch.Tensor]):
         b, s = x.size(0), x.size(1)
         t = start_pos + s
@@ -325,6 +344,10 @@ class MLA(nn.Module):
         # this step's rows of the two caches
         self.kv_cache[:b, start_pos:t] = self.kv_norm(kva[..., :self.kv_lora_rank])
         self.pe_cache[:b, start_pos:t] = apply_rotary_emb(kva[..., self.kv_lora_rank:].unsqueeze(2), freqs_cis).squeeze(2)
+        if wkv_b is None and s >= self.explicit_min_tokens and self._attention_kernels_ok(x, q, t, freqs_cis, mask):
+            y = torch.ops.dsv3fp8.mla_prefill(q, freqs_cis, self.kv_cache, self.pe_cache, self.wkv_b.weight, self.wkv_b.scale,
+                                              mask, t, self.softmax_scale)
+            return fp8_gemm(*y, self.wo.weight, self.wo.weight.scale)
         latent, rope_keys = self.kv_cache[:b, :t], self.pe_cache[:b, :t]
         # scores over the latent (query folded through wkv_b) plus the rotary part; softmax in binary32
         q_latent = self._absorb(q[..., :self.qk_nope_head_dim], ops._lib.ABSORB_Q, wkv_b)

@@ -38,6 +38,8 @@ _libdef.define("swiglu_quant(Tensor h, int block_size, int scale_fmt) -> (Tensor
 _libdef.define("moe_combine(Tensor expert_out, Tensor rows, Tensor weights, Tensor? shared) -> Tensor")
 _libdef.define("gate_route(Tensor logits, Tensor? bias, int topk, int n_groups, int topk_groups, int score_func, "
                "float route_scale) -> (Tensor, Tensor)")
+_libdef.define("mla_prefill(Tensor q, Tensor freqs, Tensor kv_cache, Tensor pe_cache, Tensor wkv_b, Tensor scale, "
+               "Tensor? mask, int positions, float softmax_scale) -> (Tensor, Tensor)")
 _libdef.define("wkv_b_absorb(Tensor x, Tensor wkv_b, Tensor scale, int side, int nope_dim, int v_dim) -> Tensor")
 
 
@@ -367,8 +369,51 @@ def _wkv_b_absorb_meta(x, wkv_b, scale, side, nope_dim, v_dim):
     return x.new_empty(*x.size()[:-1], _absorb_out_dim(wkv_b, side, v_dim))
 
 
+def _mla_check(q, freqs, kv_cache, pe_cache, mask, positions: int):
+    """q [b, s, h, nope + rope] bf16; freqs [s, rope / 2] complex64; caches [>= b, >= positions, width] bf16."""
+    b, s = q.size(0), q.size(1)
+    assert q.dim() == 4 and q.is_contiguous() and q.dtype == torch.bfloat16
+    assert freqs.dtype == torch.complex64 and freqs.is_contiguous() and freqs.shape == (s, pe_cache.size(-1) // 2)
+    for c in (kv_cache, pe_cache):
+        assert c.dim() == 3 and c.dtype == torch.bfloat16 and c.stride(2) == 1 and c.stride(1) == c.size(2)
+        assert c.size(0) >= b and c.size(1) >= positions
+    assert mask is None or (mask.shape == (s, positions) and mask.is_contiguous()
+                            and mask.dtype in (torch.bfloat16, torch.float32))
+
+
+def _mla_prefill_dev(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions: int, softmax_scale: float):
+    """The attention of q over the first `positions` rows of the caches, quantised for the output projection:
+    (y [b, s, h * v] e4m3, scales [b, s, h]); see dsv3_mla_prefill in include/dsv3_fp8.h."""
+    _mla_check(q, freqs, kv_cache, pe_cache, mask, positions)
+    assert wkv_b.is_contiguous() and scale.is_contiguous() and wkv_b.element_size() == 1
+    b, s, h, qd = q.shape
+    rope = pe_cache.size(2)
+    nope = qd - rope
+    v = wkv_b.size(0) // h - nope
+    y = torch.empty(b, s, h * v, dtype=FP8, device=q.device)
+    ys = torch.empty(b, s, h, dtype=torch.float32, device=q.device)
+    with torch.cuda.device(q.device):
+        need = _lib.lib.dsv3_mla_prefill_workspace_bytes(b, s, positions, h)
+        ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+        rc = _lib.lib.dsv3_mla_prefill(q.data_ptr(), freqs.data_ptr(), kv_cache.data_ptr(), kv_cache.stride(0),
+                                       pe_cache.data_ptr(), pe_cache.stride(0), wkv_b.data_ptr(), scale.data_ptr(),
+                                       mask.data_ptr() if mask is not None else None,
+                                       dtype_code(mask.dtype) if mask is not None else 0, y.data_ptr(), ys.data_ptr(),
+                                       b, s, positions, h, nope, rope, v, kv_cache.size(2), softmax_scale, ws.data_ptr(),
+                                       need, _stream(q))
+    _lib.check(rc, "dsv3_mla_prefill")
+    return y, ys
+
+
+def _mla_prefill_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale):
+    b, s, h, qd = q.shape
+    v = wkv_b.size(0) // h - (qd - pe_cache.size(2))
+    return q.new_empty(b, s, h * v, dtype=FP8), q.new_empty(b, s, h, dtype=torch.float32)
+
+
 _libimpl = torch.library.Library("dsv3fp8", "IMPL")
-for _name, _dev, _meta in (("wkv_b_absorb", _wkv_b_absorb_dev, _wkv_b_absorb_meta),
+for _name, _dev, _meta in (("mla_prefill", _mla_prefill_dev, _mla_prefill_meta),
+                           ("wkv_b_absorb", _wkv_b_absorb_dev, _wkv_b_absorb_meta),
                            ("linear_fp8", _linear_fp8_dev, _linear_fp8_meta),
                            ("gate_route", _gate_route_dev, _gate_route_meta),
                            ("group_tiles", _group_tiles_dev, _group_tiles_meta),

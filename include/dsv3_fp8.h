@@ -340,6 +340,25 @@ int dsv3_wkv_b_absorb(const void* x, int64_t x_token_stride, int64_t x_head_stri
                       int64_t tokens, int heads, int nope_dim, int v_dim, int64_t kv_rank, int block_size,
                       void* stream);
 
+/*
+ * Attention of MLA.forward for many new tokens (inference/model.py:470-497: scores, softmax, weighted sum and the
+ * wkv_b products around them), in the form that forms every head's keys and values from the latent cache first:
+ *     k[j, h] = [ sum_c W[h*256 + d, c] * kv[j, c] | pe[j] ],  v[j, h] = sum_c W[h*256 + 128 + d, c] * kv[j, c],
+ *     W = bf16( f32(wkv_b) * scale ),  o[i, h] = sum_j softmax_j( k[j, h] . rot(q[i, h]) * softmax_scale + mask[i, j] ) v[j, h]
+ * and quantises o, rounded to bf16, per (token, head) -- the 1 x 128 blocks of the output projection's input.
+ * q: bf16 [batch, rows, heads, 192], contiguous, its last 64 elements not yet rotated; freqs: binary32 (cos, sin) pairs
+ * [rows, 32]; kv_cache / pe_cache: bf16 [batch, >= positions, 512] / [.., 64] with the given batch strides (in elements);
+ * wkv_b: e4m3 [heads*256, 512], wkv_b_scale [heads*2, 4]; mask: [rows, positions] of mask_dtype (DSV3_BF16 or DSV3_F32) or
+ * NULL; y: e4m3 [batch, rows, heads*128]; s: [batch, rows, heads].  Only nope 128, rope 64, v 128, kv_rank 512
+ * (DSV3_ERR_BAD_SHAPE otherwise).  workspace: 256-byte aligned, dsv3_mla_prefill_workspace_bytes() bytes.
+ */
+size_t dsv3_mla_prefill_workspace_bytes(int64_t batch, int64_t rows, int64_t positions, int heads);
+int dsv3_mla_prefill(const void* q, const float* freqs, const void* kv_cache, int64_t kv_batch_stride,
+                     const void* pe_cache, int64_t pe_batch_stride, const void* wkv_b, const float* wkv_b_scale,
+                     const void* mask, int mask_dtype, void* y, float* s, int64_t batch, int64_t rows, int64_t positions,
+                     int heads, int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

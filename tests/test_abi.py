@@ -288,3 +288,22 @@ def test_linear_fp8_validation(L):
     assert call(0, A16 + 2) == 4
     assert call(11, None) == 6 and call(12, 16) == 6         # the split-K workspace is required and checked
     assert call(6, 0) == 0
+
+
+def test_mla_prefill_validation(L):
+    def call(q=A16, kv=A16, pe=A16, w=A16, y=A16, s=A16, mask=None, md=0, b=2, rows=64, pos=64, heads=4, nope=128, rope=64,
+             v=128, c=512, kvs=64 * 512, pes=64 * 64, scale=0.1, ws=0x1000, wsb=1 << 40, freqs=A16):
+        return L.lib.dsv3_mla_prefill(q, freqs, kv, kvs, pe, pes, w, A16, mask, md, y, s, b, rows, pos, heads, nope, rope, v, c,
+                                      scale, ws, wsb, None)
+    for name in ("q", "kv", "pe", "w", "y", "s", "freqs"):
+        assert call(**{name: None}) == 1
+    for bad in ({"nope": 64}, {"rope": 32}, {"v": 64}, {"c": 256}, {"b": -1}, {"rows": -1}, {"pos": 0}, {"heads": 65536},
+                {"kvs": 64 * 512 - 8}, {"pes": 64 * 64 + 4}, {"scale": 0.0}, {"scale": float("nan")}):
+        assert call(**bad) == 2, bad
+    for name in ("q", "kv", "pe", "w", "y"):
+        assert call(**{name: A16 + 8}) == 4
+    assert call(mask=A16, md=L.F16) == 5 and call(mask=A16 + 1) == 4
+    need = L.lib.dsv3_mla_prefill_workspace_bytes(2, 64, 64, 4)
+    assert need > 0 and call(ws=None) == 6 and call(wsb=need - 1) == 6 and call(ws=0x1080) == 6
+    assert call(b=0, q=None) == 0 and call(rows=0, q=None) == 0
+    assert L.lib.dsv3_mla_prefill_workspace_bytes(0, 64, 64, 4) == 0

@@ -1,0 +1,140 @@
+"""The attention kernels of MLA.forward (torch.ops.dsv3fp8.mla_prefill) against a binary64 evaluation of
+inference/model.py:470-497 on the same bf16 inputs, at the edges of their tiles, and MLA.forward on them against the
+torch-CPU oracle."""
+import pytest
+import torch
+
+from oracle import oracle
+from test_gpu_mla import M  # noqa: F401  (fixture)
+from test_oracle_mla import _freqs, small_mla_params
+
+pytestmark = pytest.mark.gpu
+
+FP8 = torch.float8_e4m3fn
+NOPE, ROPE, V, C = 128, 64, 128, 512
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _ops():
+    from dsv3fp8 import ops  # noqa: F401  (registers torch.ops.dsv3fp8)
+
+
+def _inputs(b, s, t, h, seed):
+    """Queries, rotary phases, caches (NaN behind position t: it must not be read), wkv_b and its scales, on the GPU."""
+    g = torch.Generator().manual_seed(seed)
+    q = (torch.randn(b, s, h, NOPE + ROPE, generator=g) * 2).bfloat16()
+    kv = torch.full((b, t + 3, C), float("nan")).bfloat16()
+    pe = torch.full((b, t + 3, ROPE), float("nan")).bfloat16()
+    kv[:, :t] = torch.randn(b, t, C, generator=g).bfloat16()
+    pe[:, :t] = torch.randn(b, t, ROPE, generator=g).bfloat16()
+    ang = torch.rand(s, ROPE // 2, generator=g) * 6.28
+    w8 = torch.randn(h * (NOPE + V), C, generator=g).to(FP8)
+    ws = torch.rand(h * 2, C // 128, generator=g) * 0.03 + 0.01
+    return [x.cuda() for x in (q, torch.polar(torch.ones_like(ang), ang), kv, pe, w8, ws)]
+
+
+def _mask(kind, s, t, seed):
+    if kind is None:
+        return None
+    if kind.startswith("causal"):
+        m = torch.full((s, t), float("-inf")).triu_(1 + t - s)
+        return m.cuda() if kind == "causal_f32" else m.bfloat16().cuda()
+    g = torch.Generator().manual_seed(seed)             # finite values and holes; row 1 sees nothing
+    m = torch.where(torch.rand(s, t, generator=g) < 0.3, float("-inf"), torch.randn(s, t, generator=g))
+    m[1] = float("-inf")
+    return m.bfloat16().cuda()
+
+
+def _reference(q, freqs, kv, pe, w8, ws, mask, t, scale):
+    """Binary64, with the roundings to bf16 that the kernel has in its inputs: weights, keys, values, rotated query."""
+    b, s, h, _ = q.shape
+    w = (w8.float() * ws.repeat_interleave(128, 0).repeat_interleave(128, 1)).bfloat16().double().view(h, NOPE + V, C)
+    pairs = q[..., NOPE:].float().unflatten(-1, (-1, 2))
+    re, im = pairs[..., 0], pairs[..., 1]
+    cos, sin = freqs.real.view(1, s, 1, -1), freqs.imag.view(1, s, 1, -1)
+    qr = torch.stack((re * cos - im * sin, re * sin + im * cos), -1).flatten(-2).bfloat16().double()
+    kv, pe = kv[:, :t].double(), pe[:, :t].double()
+    out = torch.empty(b, s, h, V, dtype=torch.float64, device=q.device)
+    for i in range(h):
+        k, v = (kv @ w[i, :NOPE].t()).bfloat16().double(), (kv @ w[i, NOPE:].t()).bfloat16().double()
+        sc = q[:, :, i, :NOPE].double() @ k.transpose(1, 2).contiguous() + qr[:, :, i] @ pe.transpose(1, 2).contiguous()
+        sc = sc * scale
+        if mask is not None:
+            sc = sc + mask.double()
+        out[:, :, i] = sc.softmax(-1) @ v
+    return out
+
+
+# one tile and its neighbours in positions (64), wavefronts (32 rows) and workgroups (256 rows); head counts that leave
+# XCDs unequally loaded; more positions than rows (a cached prefix)
+PREFILL = [(1, 32, 32, 1, "causal"), (1, 33, 63, 3, None), (2, 64, 64, 8, "causal"), (1, 65, 65, 9, "causal"),
+           (1, 255, 255, 2, "causal_f32"), (2, 257, 257, 3, "causal"), (1, 40, 500, 4, "causal"), (1, 1, 1, 2, None),
+           (2, 100, 163, 4, "holes"), (1, 1100, 1100, 2, "causal")]
+
+
+@pytest.mark.parametrize("b,s,t,h,kind", PREFILL)
+def test_prefill_attention(b, s, t, h, kind):
+    q, freqs, kv, pe, w8, ws = _inputs(b, s, t, h, s + t)
+    mask = _mask(kind, s, t, 5)
+    scale = 0.08
+    y, ys = torch.ops.dsv3fp8.mla_prefill(q, freqs, kv, pe, w8, ws, mask, t, scale)
+    got = y.float().view(b, s, h, V).double() * ys.double().unsqueeze(-1)
+    ref = _reference(q, freqs, kv, pe, w8, ws, mask, t, scale)
+    if kind == "holes":                                  # softmax over nothing is NaN, in this row only
+        assert torch.isnan(ys[:, 1]).all() and torch.isnan(ref[:, 1]).all()
+        keep = torch.arange(s, device="cuda") != 1
+        got, ref, ys = got[:, keep], ref[:, keep], ys[:, keep]
+    amax = ref.abs().amax(-1)
+    # e4m3 codes: half a step at the top of the range, 16 of 448; in front of them exponentials and result are rounded to
+    # bf16, 2^-9 each of values whose errors average out: 2^-7 of the block's largest value holds them
+    assert ((got - ref).abs() <= amax.unsqueeze(-1) * (16 / 448 + 2.0 ** -7)).all()
+    assert ((ys.double() * 448 - amax).abs() <= 2.0 ** -7 * amax).all()
+
+
+def _layer(M, p, dim, heads, q_rank, max_seq):
+    args = M.ModelArgs(dim=dim, n_heads=heads, q_lora_rank=q_rank, kv_lora_rank=C, qk_nope_head_dim=NOPE,
+                       qk_rope_head_dim=ROPE, v_head_dim=V, max_batch_size=2, max_seq_len=max_seq, original_seq_len=max_seq)
+    with torch.device("cuda"):
+        layer = M.MLA(args)
+    with torch.no_grad():
+        for name in ("wq_a", "wq_b", "wkv_a", "wkv_b", "wo"):
+            getattr(layer, name).weight.copy_(p[name][0].cuda())
+            getattr(layer, name).scale.copy_(p[name][1].cuda())
+        layer.q_norm.weight.copy_(p["q_norm"].cuda())
+        layer.kv_norm.weight.copy_(p["kv_norm"].cuda())
+    return layer
+
+
+def _rel(got, ref):
+    return ((got.float().cpu() - ref.float()).norm() / ref.float().norm()).item()
+
+
+# Two evaluations differ by roundings in front of quantisers; where such a rounding moves an e4m3 code of wo's input the
+# result moves by one step.  Codes carry an error of 2.6 % (rms of the rounding); were every one of them chosen anew the
+# two results would be sqrt(2) * 2.6 % = 3.7 % apart.
+LAYER_TOL = 4e-2
+
+
+def test_layer_prefill_vs_oracle(M):
+    dim, heads, q_rank, s = 256, 4, 128, 70
+    p = small_mla_params(dim, heads, q_rank, C, NOPE, ROPE, V, 31)
+    layer = _layer(M, p, dim, heads, q_rank, 96)
+    assert s >= layer.explicit_min_tokens
+    freqs = _freqs(ROPE, 96)
+    g = torch.Generator().manual_seed(32)
+    x0, x1 = torch.randn(2, s, dim, generator=g).bfloat16(), torch.randn(2, 1, dim, generator=g).bfloat16()
+    mask = torch.full((s, s), float("-inf")).triu_(1)
+    kv, pe = torch.zeros(2, 96, C, dtype=torch.bfloat16), torch.zeros(2, 96, ROPE, dtype=torch.bfloat16)
+    scale = (NOPE + ROPE) ** -0.5
+    ref0 = oracle.mla(x0, 0, freqs[:s], mask, p, kv, pe, heads, NOPE, ROPE, V, C, scale)
+    ref1 = oracle.mla(x1, s, freqs[s:s + 1], None, p, kv, pe, heads, NOPE, ROPE, V, C, scale)
+    with torch.inference_mode():
+        y0 = layer(x0.cuda(), 0, freqs[:s].cuda(), mask.cuda())
+        y1 = layer(x1.cuda(), s, freqs[s:s + 1].cuda(), None)
+    assert _rel(y0, ref0) <= LAYER_TOL and _rel(y1, ref1) <= LAYER_TOL
+    assert _rel(layer.kv_cache, kv) <= 1e-2 and _rel(layer.pe_cache, pe) <= 1e-2
+    # with gradients enabled the layer keeps to differentiable-by-parts tensor operations: same result, other kernels
+    layer.kv_cache.zero_(); layer.pe_cache.zero_()
+    layer.requires_grad_(False)
+    z0 = layer(x0.cuda(), 0, freqs[:s].cuda(), mask.cuda())
+    assert _rel(z0, ref0) <= LAYER_TOL and _rel(y0, z0.cpu()) <= LAYER_TOL
