@@ -1,0 +1,50 @@
+// What the attention kernels of MLA.forward share: bf16 MFMAs of 32 x 32, copies into LDS, masks, the softmax offset.
+#pragma once
+#include "common.hpp"
+
+namespace dsv3 {
+namespace {
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) void* lptr_t;
+
+__device__ __forceinline__ v16f mfma32(v4u a, v4u b, v16f c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ uint32_t lds_addr_of(const void* p) { return (uint32_t)(uintptr_t)(lptr_t)p; }
+// 1 KiB global -> LDS: lane l's 16 bytes at base + lane_off land at lds_addr + 16 l
+__device__ __forceinline__ void copy16(const void* base, uint32_t lane_off, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(lane_off), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+__device__ __forceinline__ void barrier_no_fence() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32); }
+
+template <bool F32> __device__ __forceinline__ float mask_at(const void* m, int64_t i) {
+    return F32 ? ((const float*)m)[i] : u32_as_f32((uint32_t)((const uint16_t*)m)[i] << 16);
+}
+// A mask value in units of the raw scores.  A finite one stays finite: masks of the type's lowest value would otherwise
+// become -inf, and a row that has nothing else NaN instead of equal weights.
+__device__ __forceinline__ float mask_term(float v, float inv_scale) {
+    const float t = v * inv_scale;
+    return t == -__builtin_inff() && v != t ? -__FLT_MAX__ : t;
+}
+// What the exponents fma(S, scale2, -offset) subtract for a row maximum m.  Where the maximum is huge (a row that only
+// finite mask values of such a size reach), the rounding of m * scale2 alone would overflow the exponentials: the maximum
+// is taken off the scores themselves then.
+template <int N> __device__ __forceinline__ float softmax_offset(v16f (&S)[N], float m, float scale2) {
+    float off = m == -__builtin_inff() ? 0.f : m * scale2;
+    const bool huge = __builtin_fabsf(m) > 0x1p20f && m != -__builtin_inff();
+    if (__any(huge)) {
+        const float d = huge ? m : 0.f;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) S[k][e] -= d;
+        off = huge ? 0.f : off;
+    }
+    return off;
+}
+
+}  // namespace
+}  // namespace dsv3

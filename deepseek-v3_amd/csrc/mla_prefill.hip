@@ -15,13 +15,10 @@
 // At 4096 tokens, 128 heads, causal mask: expand 226 us, flags 23 us, attend 915 us (0.75 PFLOP/s of the pairs the mask
 // leaves); the whole layer 1.77 ms where the absorbed form as tensor operations took 20.2 ms (2 x 2.5 ms score products,
 // 1.6 ms value product and 12 ms of passes over the 4.3 GB score matrix).
-#include "common.hpp"
+#include "mla.hpp"
 
 namespace dsv3 {
 namespace {
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) void* lptr_t;
 
 constexpr int kC = 512, kRope = 64, kNope = 128, kV = 128, kQd = kNope + kRope;
 constexpr int kTile = 64;                       // positions per tile
@@ -30,17 +27,6 @@ constexpr int kTile = 64;                       // positions per tile
 constexpr int kKeyBytes = kTile * kNope * 2, kValBytes = kTile * kV * 2, kRopeBytes = kTile * kRope * 2;
 constexpr int kHeadTile = kKeyBytes + kValBytes;
 constexpr int kQTile = 256;                     // query rows per workgroup: 8 wavefronts x 32
-
-__device__ __forceinline__ v16f mfma32(v4u a, v4u b, v16f c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-}
-__device__ __forceinline__ uint32_t lds_addr_of(const void* p) { return (uint32_t)(uintptr_t)(lptr_t)p; }
-// 1 KiB global -> LDS: lane l's 16 bytes at base + lane_off land at lds_addr + 16 l
-__device__ __forceinline__ void copy16(const void* base, uint32_t lane_off, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :: "v"(lane_off), "s"(base), "s"(lds_addr) : "memory", "m0");
-}
-__device__ __forceinline__ void barrier_no_fence() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // ---------------------------------------------------------------------------------------------------------- expand
 
@@ -149,10 +135,6 @@ __global__ __launch_bounds__(512, 2) void mla_expand_kernel(ExpandArgs p) {
 
 enum : uint8_t { kClear = 0, kMixed = 1, kSkip = 2 };
 
-template <bool F32> __device__ __forceinline__ float mask_at(const void* m, int64_t i) {
-    return F32 ? ((const float*)m)[i] : u32_as_f32((uint32_t)((const uint16_t*)m)[i] << 16);
-}
-
 // flags[tile][q / 32]: what the mask does to 32 query rows x 64 positions (all zero, anything, all -inf or no row)
 template <bool F32>
 __global__ __launch_bounds__(512) void mla_mask_flags_kernel(const void* mask, uint8_t* flags, int rows, int positions, int groups) {
@@ -184,8 +166,6 @@ struct AttendArgs {
     int batch, heads, rows, positions, tiles, qtiles, groups;
     float scale, inv_scale;                     // softmax scale and its reciprocal
 };
-
-__device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32); }
 
 // One workgroup: 256 query rows of one head; wavefront w rows 32 w .. 32 w + 31.  Per tile of 64 positions (40 KiB of
 // operands, double-buffered in LDS, copied while the tile before is computed) a wavefront forms S^T = K Q^T (24 MFMAs),
@@ -278,7 +258,7 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         const int pos = t * kTile + 32 * k + 8 * (e >> 2) + 4 * g + (e & 3);
-                        S[k][e] += mask_at<MF32>(p.mask, mrow + min(pos, p.positions - 1)) * p.inv_scale;
+                        S[k][e] += mask_term(mask_at<MF32>(p.mask, mrow + min(pos, p.positions - 1)), p.inv_scale);
                     }
             }
             if ((t + 1) * kTile > p.positions) {            // the last tile may reach past the end
@@ -307,7 +287,7 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
                     for (int e = 0; e < 16; ++e) O[d][e] *= a;
                 m = mn;
             }
-            const float off = m == -__builtin_inff() ? 0.f : m * scale2;
+            const float off = softmax_offset(S, m, scale2);
             float sum = 0.f;
             v4u P[4];
 #pragma unroll

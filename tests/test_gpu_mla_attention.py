@@ -39,6 +39,11 @@ def _mask(kind, s, t, seed):
     if kind.startswith("causal"):
         m = torch.full((s, t), float("-inf")).triu_(1 + t - s)
         return m.cuda() if kind == "causal_f32" else m.bfloat16().cuda()
+    if kind.startswith("lowest"):                       # the type's lowest value for -inf; row 1 has nothing else
+        dtype = torch.float32 if kind == "lowest_f32" else torch.bfloat16
+        m = torch.full((s, t), torch.finfo(dtype).min).triu_(1 + t - s)
+        m[1] = torch.finfo(dtype).min
+        return m.to(dtype).cuda()
     g = torch.Generator().manual_seed(seed)             # finite values and holes; row 1 sees nothing
     m = torch.where(torch.rand(s, t, generator=g) < 0.3, float("-inf"), torch.randn(s, t, generator=g))
     m[1] = float("-inf")
@@ -59,8 +64,8 @@ def _reference(q, freqs, kv, pe, w8, ws, mask, t, scale):
         k, v = (kv @ w[i, :NOPE].t()).bfloat16().double(), (kv @ w[i, NOPE:].t()).bfloat16().double()
         sc = q[:, :, i, :NOPE].double() @ k.transpose(1, 2).contiguous() + qr[:, :, i] @ pe.transpose(1, 2).contiguous()
         sc = sc * scale
-        if mask is not None:
-            sc = sc + mask.double()
+        if mask is not None:                             # added in binary32, as the layer's tensor operations do
+            sc = (sc.float() + mask.float()).double()
         out[:, :, i] = sc.softmax(-1) @ v
     return out
 
@@ -69,7 +74,8 @@ def _reference(q, freqs, kv, pe, w8, ws, mask, t, scale):
 # XCDs unequally loaded; more positions than rows (a cached prefix)
 PREFILL = [(1, 32, 32, 1, "causal"), (1, 33, 63, 3, None), (2, 64, 64, 8, "causal"), (1, 65, 65, 9, "causal"),
            (1, 255, 255, 2, "causal_f32"), (2, 257, 257, 3, "causal"), (1, 40, 500, 4, "causal"), (1, 1, 1, 2, None),
-           (2, 100, 163, 4, "holes"), (1, 1100, 1100, 2, "causal")]
+           (2, 100, 163, 4, "holes"), (1, 1100, 1100, 2, "causal"),
+           (1, 70, 130, 2, "lowest"), (1, 70, 130, 2, "lowest_f32")]
 
 
 @pytest.mark.parametrize("b,s,t,h,kind", PREFILL)
