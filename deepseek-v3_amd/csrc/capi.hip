@@ -378,4 +378,46 @@ int dsv3_mla_prefill(const void* q, const float* freqs, const void* kv_cache, in
                               (hipStream_t)stream);
 }
 
+size_t dsv3_mla_decode_workspace_bytes(int64_t batch, int64_t rows, int64_t positions, int heads) {
+    if (batch <= 0 || rows <= 0 || positions <= 0 || heads <= 0) return 0;
+    return mla_decode_workspace_bytes(batch, rows, positions, heads);
+}
+
+int dsv3_mla_decode(const void* q, const float* freqs, const void* kv_cache, int64_t kv_batch_stride,
+                    const void* pe_cache, int64_t pe_batch_stride, const void* wkv_b, const float* wkv_b_scale,
+                    const void* mask, int mask_dtype, void* y, int64_t batch, int64_t rows, int64_t positions, int heads,
+                    int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale, void* workspace,
+                    size_t workspace_bytes, void* stream) {
+    const int rc = mla_validate(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, mask, mask_dtype, y, batch,
+                                rows, positions, heads, nope_dim, rope_dim, v_dim, kv_rank, softmax_scale);
+    if (rc != DSV3_OK || batch == 0 || rows == 0 || heads == 0) return rc;
+    if (!wkv_b || !wkv_b_scale) return DSV3_ERR_NULL_POINTER;
+    if (!aligned(wkv_b, 16) || !aligned(wkv_b_scale, 4)) return DSV3_ERR_MISALIGNED;
+    if (!workspace || !aligned(workspace, 256) || workspace_bytes < mla_decode_workspace_bytes(batch, rows, positions, heads))
+        return DSV3_ERR_WORKSPACE;
+    return launch_mla_decode(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, wkv_b, wkv_b_scale, mask,
+                             mask_dtype == DSV3_F32, y, batch, rows, positions, heads, softmax_scale, workspace,
+                             (hipStream_t)stream);
+}
+
+int dsv3_mla_latent(const void* a, int64_t a_stride, const void* q_norm, const void* kv_norm, const float* freqs,
+                    void* kv_rows, int64_t kv_batch_stride, void* pe_rows, int64_t pe_batch_stride, void* y, float* s,
+                    int64_t batch, int64_t rows, int64_t q_rank, int64_t kv_rank, int rope_dim, float q_eps, float kv_eps,
+                    void* stream) {
+    if (kv_rank != 512 || rope_dim != 64 || q_rank < 128 || q_rank > 2048 || q_rank % 128 != 0) return DSV3_ERR_BAD_SHAPE;
+    if (batch < 0 || rows < 0 || batch > 65535 || rows > 0x7fffff || batch * rows > 0x7fffffff || a_stride % 8 != 0 ||
+        a_stride < q_rank + kv_rank + rope_dim)
+        return DSV3_ERR_BAD_SHAPE;
+    if (batch > 1 && (kv_batch_stride < rows * kv_rank || pe_batch_stride < rows * rope_dim || kv_batch_stride % 8 != 0 ||
+                      pe_batch_stride % 8 != 0))
+        return DSV3_ERR_BAD_SHAPE;
+    if (batch == 0 || rows == 0) return DSV3_OK;
+    if (!a || !q_norm || !kv_norm || !freqs || !kv_rows || !pe_rows || !y || !s) return DSV3_ERR_NULL_POINTER;
+    if (!aligned(a, 16) || !aligned(q_norm, 16) || !aligned(kv_norm, 16) || !aligned(freqs, 8) || !aligned(kv_rows, 16) ||
+        !aligned(pe_rows, 16) || !aligned(y, 16) || !aligned(s, 4))
+        return DSV3_ERR_MISALIGNED;
+    return launch_mla_latent(a, a_stride, q_norm, kv_norm, freqs, kv_rows, kv_batch_stride, pe_rows, pe_batch_stride, y, s,
+                             batch, rows, (int)q_rank, q_eps, kv_eps, (hipStream_t)stream);
+}
+
 }  // extern "C"

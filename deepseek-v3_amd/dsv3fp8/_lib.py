@@ -60,6 +60,12 @@ EXPORTS = {
     "dsv3_mla_prefill": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
                                  c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int,
                                  c_int64, c_float, c_void_p, c_size_t, c_void_p]),
+    "dsv3_mla_decode_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int]),
+    "dsv3_mla_decode": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
+                                c_void_p, c_int, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int,
+                                c_int64, c_float, c_void_p, c_size_t, c_void_p]),
+    "dsv3_mla_latent": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
+                                c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int, c_float, c_float, c_void_p]),
 }
 
 

@@ -210,6 +210,11 @@ def apply_rotary_emb(x: torch.Tensor, freqs_cis: torch.Tensor) -> torch.Tensor:
     return torch.stack((re * cos - im * sin, re * sin + im * cos), dim=-1).flatten(-2).to(x.dtype)
 
 
+def _plain(module: nn.Module, cls: type) -> bool:
+    """Whether calling ``module`` does no more than ``cls.forward``, so that a fused kernel may take its place."""
+    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks)
+
+
 class MLA(nn.Module):
     """Host of the two ``wkv_b`` products of the absorbed multi-head latent attention (model.py:395-497).
 
@@ -236,7 +241,7 @@ class MLA(nn.Module):
     fused: bool = True
     stacked_a: bool = True
     # from this many new tokens per sequence on, keys and values are formed per head instead of being folded into the
-    # query and the output (csrc/mla_prefill.hip)
+    # query and the output (csrc/mla_prefill.hip; with fewer csrc/mla_decode.hip)
     explicit_min_tokens: int = 32
 
     def __init__(self, args: ModelArgs):
@@ -318,36 +323,58 @@ class MLA(nn.Module):
             w = weight_dequant(w, self.wkv_b.scale, block_size)
         return w.view(self.n_local_heads, -1, self.kv_lora_rank)
 
-    def _attention_kernels_ok(self, x, q, positions: int, freqs_cis, mask) -> bool:
-        """Whether the attention between the query projection and ``wo`` can run on the fused kernels: their head
-        dimensions, FP8 weights on both sides, no gradients (the kernels have no backward), a mask of one value per
-        (query, position) pair as the reference builds it (model.py:738-740)."""
+    def _kernels_ok(self, x, start_pos: int, freqs_cis) -> bool:
+        """What the fused kernels of this layer ask for in common: their head dimensions and dtypes, FP8 weights, no
+        gradients (the kernels have no backward), new rows that fit the caches."""
         b, s = x.size(0), x.size(1)
-        return (not torch.is_grad_enabled() and gemm_impl == "fp8" and block_size == 128 and world_size == 1
-                and torch.get_default_dtype() == torch.bfloat16 and q.dtype == torch.bfloat16 and q.is_contiguous()
+        return (not torch.is_grad_enabled() and gemm_impl == "fp8" and block_size == 128 and world_size == 1 and self.fused
+                and x.is_cuda and x.dtype == torch.bfloat16 and torch.get_default_dtype() == torch.bfloat16
+                and self.attn_impl == "absorb"
                 and (self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim, self.kv_lora_rank) == (128, 64, 128, 512)
                 and self.kv_cache.dtype == torch.bfloat16 and self.kv_cache.is_contiguous() and self.pe_cache.is_contiguous()
-                and b <= self.kv_cache.size(0) and s >= 1 and positions <= self.kv_cache.size(1)
-                and self.wo.weight.element_size() == 1 and self.wo.bias is None and self.wkv_b.bias is None
+                and 1 <= b <= self.kv_cache.size(0) and s >= 1 and start_pos >= 0 and start_pos + s <= self.kv_cache.size(1)
+                and self.wkv_b.weight.element_size() == 1 and self.wkv_b.bias is None
                 and freqs_cis.is_cuda and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous()
-                and freqs_cis.shape == (s, self.qk_rope_head_dim // 2)
-                and (mask is None or (mask.is_cuda and mask.shape == (s, positions) and mask.is_contiguous()
+                and freqs_cis.shape == (s, self.qk_rope_head_dim // 2))
+
+    def _latent_kernel_ok(self) -> bool:
+        """Whether both norms, the cache rows and the quantisation in front of ``wq_b`` can be one launch; modules that
+        were exchanged or carry hooks are called as such."""
+        return (self.q_lora_rank % block_size == 0 and 0 < self.q_lora_rank <= 2048 and self.stacked_a
+                and _plain(self.q_norm, RMSNorm) and _plain(self.kv_norm, RMSNorm) and _plain(self.wq_b, ColumnParallelLinear)
+                and self.q_norm.weight.dtype == torch.bfloat16 and self.kv_norm.weight.dtype == torch.bfloat16
+                and self.wq_b.weight.element_size() == 1 and self.wq_b.bias is None and self.stack_a())
+
+    def _attention_kernels_ok(self, q, positions: int, mask) -> bool:
+        """Whether the attention behind the query projection can run on the fused kernels: a mask of one value per
+        (query, position) pair as the reference builds it (model.py:738-740)."""
+        return (q.dtype == torch.bfloat16 and q.is_contiguous()
+                and (mask is None or (mask.is_cuda and mask.shape == (q.size(1), positions) and mask.is_contiguous()
                                       and mask.dtype in (torch.bfloat16, torch.float32))))
 
     def forward(self, x: torch.Tensor, start_pos: int, freqs_cis: torch.Tensor, mask: Optional[torch.Tensor]):
         b, s = x.size(0), x.size(1)
         t = start_pos + s
-        q, kva = self._project(x)
-        if self.attn_impl == "naive":
-            return self._forward_naive(x, q, kva, start_pos, freqs_cis, mask)
+        kernels = self._kernels_ok(x, start_pos, freqs_cis)
+        if kernels and self._latent_kernel_ok():
+            qq, qs = torch.ops.dsv3fp8.mla_latent(linear(x, self._wa, None, self.wq_a.scale_fmt), self.q_norm.weight,
+                                                  self.kv_norm.weight, freqs_cis, self.kv_cache, self.pe_cache, start_pos,
+                                                  self.q_norm.eps, self.kv_norm.eps)
+            q = fp8_gemm(qq, qs, self.wq_b.weight, self.wq_b.weight.scale).unflatten(-1, (self.n_local_heads, self.qk_head_dim))
+        else:
+            q, kva = self._project(x)
+            if self.attn_impl == "naive":
+                return self._forward_naive(x, q, kva, start_pos, freqs_cis, mask)
+            # this step's rows of the two caches
+            self.kv_cache[:b, start_pos:t] = self.kv_norm(kva[..., :self.kv_lora_rank])
+            self.pe_cache[:b, start_pos:t] = apply_rotary_emb(kva[..., self.kv_lora_rank:].unsqueeze(2), freqs_cis).squeeze(2)
+        if kernels and self._attention_kernels_ok(q, t, mask):
+            args = (q, freqs_cis, self.kv_cache, self.pe_cache, self.wkv_b.weight, self.wkv_b.scale, mask, t, self.softmax_scale)
+            if s < self.explicit_min_tokens:
+                return self.wo(torch.ops.dsv3fp8.mla_decode(*args))
+            if self.wo.weight.element_size() == 1 and self.wo.bias is None and _plain(self.wo, RowParallelLinear):
+                return fp8_gemm(*torch.ops.dsv3fp8.mla_prefill(*args), self.wo.weight, self.wo.weight.scale)
         wkv_b = self._dequantised_wkv_b(x)
-        # this step's rows of the two caches
-        self.kv_cache[:b, start_pos:t] = self.kv_norm(kva[..., :self.kv_lora_rank])
-        self.pe_cache[:b, start_pos:t] = apply_rotary_emb(kva[..., self.kv_lora_rank:].unsqueeze(2), freqs_cis).squeeze(2)
-        if wkv_b is None and s >= self.explicit_min_tokens and self._attention_kernels_ok(x, q, t, freqs_cis, mask):
-            y = torch.ops.dsv3fp8.mla_prefill(q, freqs_cis, self.kv_cache, self.pe_cache, self.wkv_b.weight, self.wkv_b.scale,
-                                              mask, t, self.softmax_scale)
-            return fp8_gemm(*y, self.wo.weight, self.wo.weight.scale)
         latent, rope_keys = self.kv_cache[:b, :t], self.pe_cache[:b, :t]
         # scores over the latent (query folded through wkv_b) plus the rotary part; softmax in binary32
         q_latent = self._absorb(q[..., :self.qk_nope_head_dim], ops._lib.ABSORB_Q, wkv_b)

@@ -40,6 +40,10 @@ _libdef.define("gate_route(Tensor logits, Tensor? bias, int topk, int n_groups, 
                "float route_scale) -> (Tensor, Tensor)")
 _libdef.define("mla_prefill(Tensor q, Tensor freqs, Tensor kv_cache, Tensor pe_cache, Tensor wkv_b, Tensor scale, "
                "Tensor? mask, int positions, float softmax_scale) -> (Tensor, Tensor)")
+_libdef.define("mla_decode(Tensor q, Tensor freqs, Tensor kv_cache, Tensor pe_cache, Tensor wkv_b, Tensor scale, "
+               "Tensor? mask, int positions, float softmax_scale) -> Tensor")
+_libdef.define("mla_latent(Tensor a, Tensor q_norm, Tensor kv_norm, Tensor freqs, Tensor(a!) kv_cache, Tensor(b!) pe_cache, "
+               "int start, float q_eps, float kv_eps) -> (Tensor, Tensor)")
 _libdef.define("wkv_b_absorb(Tensor x, Tensor wkv_b, Tensor scale, int side, int nope_dim, int v_dim) -> Tensor")
 
 
@@ -381,27 +385,28 @@ def _mla_check(q, freqs, kv_cache, pe_cache, mask, positions: int):
                             and mask.dtype in (torch.bfloat16, torch.float32))
 
 
-def _mla_prefill_dev(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions: int, softmax_scale: float):
-    """The attention of q over the first `positions` rows of the caches, quantised for the output projection:
-    (y [b, s, h * v] e4m3, scales [b, s, h]); see dsv3_mla_prefill in include/dsv3_fp8.h."""
+def _mla_call(entry: str, q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions: int, softmax_scale: float, *out):
     _mla_check(q, freqs, kv_cache, pe_cache, mask, positions)
     assert wkv_b.is_contiguous() and scale.is_contiguous() and wkv_b.element_size() == 1
     b, s, h, qd = q.shape
     rope = pe_cache.size(2)
     nope = qd - rope
-    v = wkv_b.size(0) // h - nope
-    y = torch.empty(b, s, h * v, dtype=FP8, device=q.device)
-    ys = torch.empty(b, s, h, dtype=torch.float32, device=q.device)
     with torch.cuda.device(q.device):
-        need = _lib.lib.dsv3_mla_prefill_workspace_bytes(b, s, positions, h)
+        need = getattr(_lib.lib, entry + "_workspace_bytes")(b, s, positions, h)
         ws = torch.empty(need, dtype=torch.uint8, device=q.device)
-        rc = _lib.lib.dsv3_mla_prefill(q.data_ptr(), freqs.data_ptr(), kv_cache.data_ptr(), kv_cache.stride(0),
-                                       pe_cache.data_ptr(), pe_cache.stride(0), wkv_b.data_ptr(), scale.data_ptr(),
-                                       mask.data_ptr() if mask is not None else None,
-                                       dtype_code(mask.dtype) if mask is not None else 0, y.data_ptr(), ys.data_ptr(),
-                                       b, s, positions, h, nope, rope, v, kv_cache.size(2), softmax_scale, ws.data_ptr(),
-                                       need, _stream(q))
-    _lib.check(rc, "dsv3_mla_prefill")
+        rc = getattr(_lib.lib, entry)(
+            q.data_ptr(), freqs.data_ptr(), kv_cache.data_ptr(), kv_cache.stride(0), pe_cache.data_ptr(),
+            pe_cache.stride(0), wkv_b.data_ptr(), scale.data_ptr(), mask.data_ptr() if mask is not None else None,
+            dtype_code(mask.dtype) if mask is not None else 0, *(o.data_ptr() for o in out), b, s, positions, h, nope,
+            rope, wkv_b.size(0) // h - nope, kv_cache.size(2), softmax_scale, ws.data_ptr(), need, _stream(q))
+    _lib.check(rc, entry)
+
+
+def _mla_prefill_dev(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions: int, softmax_scale: float):
+    """The attention of q over the first `positions` rows of the caches, quantised for the output projection:
+    (y [b, s, h * v] e4m3, scales [b, s, h]); see dsv3_mla_prefill in include/dsv3_fp8.h."""
+    y, ys = _mla_prefill_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale)
+    _mla_call("dsv3_mla_prefill", q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale, y, ys)
     return y, ys
 
 
@@ -411,8 +416,49 @@ def _mla_prefill_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, position
     return q.new_empty(b, s, h * v, dtype=FP8), q.new_empty(b, s, h, dtype=torch.float32)
 
 
+def _mla_decode_dev(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions: int, softmax_scale: float):
+    """The same attention for few new tokens: y [b, s, h * v] bf16; see dsv3_mla_decode in include/dsv3_fp8.h."""
+    y = _mla_decode_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale)
+    _mla_call("dsv3_mla_decode", q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale, y)
+    return y
+
+
+def _mla_decode_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale):
+    b, s, h, qd = q.shape
+    return q.new_empty(b, s, wkv_b.size(0) - h * (qd - pe_cache.size(2)))
+
+
+def _mla_latent_dev(a, q_norm, kv_norm, freqs, kv_cache, pe_cache, start: int, q_eps: float, kv_eps: float):
+    """a [b, s, q_rank + kv_rank + rope] -> the normalised query latent, quantised (e4m3, scales per 128), and the caches'
+    rows start .. start + s - 1; see dsv3_mla_latent in include/dsv3_fp8.h."""
+    b, s, width = a.shape
+    c, r = kv_cache.size(2), pe_cache.size(2)
+    assert a.is_contiguous() and a.dtype == torch.bfloat16 and width == q_norm.numel() + c + r and kv_norm.numel() == c
+    assert q_norm.dtype == torch.bfloat16 and kv_norm.dtype == torch.bfloat16
+    assert q_norm.is_contiguous() and kv_norm.is_contiguous()
+    assert freqs.dtype == torch.complex64 and freqs.is_contiguous() and freqs.shape == (s, r // 2)
+    for t in (kv_cache, pe_cache):
+        assert t.dim() == 3 and t.dtype == torch.bfloat16 and t.stride(2) == 1 and t.stride(1) == t.size(2)
+        assert t.size(0) >= b and t.size(1) >= start + s and start >= 0
+    y, ys = _mla_latent_meta(a, q_norm, kv_norm, freqs, kv_cache, pe_cache, start, q_eps, kv_eps)
+    with torch.cuda.device(a.device):
+        rc = _lib.lib.dsv3_mla_latent(a.data_ptr(), width, q_norm.data_ptr(), kv_norm.data_ptr(), freqs.data_ptr(),
+                                      kv_cache.data_ptr() + start * c * 2, kv_cache.stride(0),
+                                      pe_cache.data_ptr() + start * r * 2, pe_cache.stride(0), y.data_ptr(), ys.data_ptr(),
+                                      b, s, q_norm.numel(), c, r, q_eps, kv_eps, _stream(a))
+    _lib.check(rc, "dsv3_mla_latent")
+    return y, ys
+
+
+def _mla_latent_meta(a, q_norm, kv_norm, freqs, kv_cache, pe_cache, start, q_eps, kv_eps):
+    b, s, _ = a.shape
+    return (a.new_empty(b, s, q_norm.numel(), dtype=FP8), a.new_empty(b, s, q_norm.numel() // 128, dtype=torch.float32))
+
+
 _libimpl = torch.library.Library("dsv3fp8", "IMPL")
 for _name, _dev, _meta in (("mla_prefill", _mla_prefill_dev, _mla_prefill_meta),
+                           ("mla_decode", _mla_decode_dev, _mla_decode_meta),
+                           ("mla_latent", _mla_latent_dev, _mla_latent_meta),
                            ("wkv_b_absorb", _wkv_b_absorb_dev, _wkv_b_absorb_meta),
                            ("linear_fp8", _linear_fp8_dev, _linear_fp8_meta),
                            ("gate_route", _gate_route_dev, _gate_route_meta),

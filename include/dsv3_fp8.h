@@ -359,6 +359,31 @@ int dsv3_mla_prefill(const void* q, const float* freqs, const void* kv_cache, in
                      int heads, int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale,
                      void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * The same attention for few new tokens (a decode step), in the absorbed form of inference/model.py:480-497: the query
+ * folded through wkv_b, scores and weighted sums over the latents, the sums folded through wkv_b.  Arguments as
+ * dsv3_mla_prefill; y: bf16 [batch, rows, heads*128], contiguous (the input of the output projection).
+ */
+size_t dsv3_mla_decode_workspace_bytes(int64_t batch, int64_t rows, int64_t positions, int heads);
+int dsv3_mla_decode(const void* q, const float* freqs, const void* kv_cache, int64_t kv_batch_stride,
+                    const void* pe_cache, int64_t pe_batch_stride, const void* wkv_b, const float* wkv_b_scale,
+                    const void* mask, int mask_dtype, void* y, int64_t batch, int64_t rows, int64_t positions, int heads,
+                    int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale, void* workspace,
+                    size_t workspace_bytes, void* stream);
+
+/*
+ * What MLA.forward does between the low-rank projections and the query's up-projection (inference/model.py:457-466 and
+ * :480-483), for rows a[i] = [ query latent (q_rank) | latent (512) | rotary key (64) ] in bf16, a_stride elements apart:
+ *     y, s        = act_quant( bf16( rms_norm(query latent) * q_norm ), 128 )     e4m3 [batch*rows, q_rank] and scales
+ *     kv_rows[i]  = bf16( rms_norm(latent) * kv_norm ),  pe_rows[i] = rotated key
+ * kv_rows / pe_rows point at the caches' rows of the first new position (512 and 64 bf16 per row, the given batch strides
+ * in elements); freqs: binary32 (cos, sin) pairs [rows, 32].  q_rank: a multiple of 128 up to 2048.
+ */
+int dsv3_mla_latent(const void* a, int64_t a_stride, const void* q_norm, const void* kv_norm, const float* freqs,
+                    void* kv_rows, int64_t kv_batch_stride, void* pe_rows, int64_t pe_batch_stride, void* y, float* s,
+                    int64_t batch, int64_t rows, int64_t q_rank, int64_t kv_rank, int rope_dim, float q_eps, float kv_eps,
+                    void* stream);
+
 #ifdef __cplusplus
 }
 #endif

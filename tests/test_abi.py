@@ -307,3 +307,31 @@ def test_mla_prefill_validation(L):
     assert need > 0 and call(ws=None) == 6 and call(wsb=need - 1) == 6 and call(ws=0x1080) == 6
     assert call(b=0, q=None) == 0 and call(rows=0, q=None) == 0
     assert L.lib.dsv3_mla_prefill_workspace_bytes(0, 64, 64, 4) == 0
+
+
+def test_mla_decode_validation(L):
+    def call(q=A16, kv=A16, pe=A16, w=A16, y=A16, mask=None, md=0, b=2, rows=1, pos=64, heads=4, nope=128, rope=64,
+             v=128, c=512, kvs=64 * 512, pes=64 * 64, scale=0.1, ws=0x1000, wsb=1 << 40, freqs=A16):
+        return L.lib.dsv3_mla_decode(q, freqs, kv, kvs, pe, pes, w, A16, mask, md, y, b, rows, pos, heads, nope, rope, v, c,
+                                     scale, ws, wsb, None)
+    for name in ("q", "kv", "pe", "w", "y", "freqs"):
+        assert call(**{name: None}) == 1
+    for bad in ({"nope": 64}, {"c": 256}, {"b": -1}, {"rows": -1}, {"pos": 0}, {"kvs": 64 * 512 - 8}, {"scale": 0.0}):
+        assert call(**bad) == 2, bad
+    for name in ("q", "kv", "pe", "w", "y"):
+        assert call(**{name: A16 + 8}) == 4
+    need = L.lib.dsv3_mla_decode_workspace_bytes(2, 1, 64, 4)
+    assert need > 0 and call(ws=None) == 6 and call(wsb=need - 1) == 6 and call(ws=0x1080) == 6
+    assert call(b=0, q=None) == 0 and L.lib.dsv3_mla_decode_workspace_bytes(2, 0, 64, 4) == 0
+
+
+def test_mla_latent_validation(L):
+    def call(a=A16, stride=2112, qw=A16, kw=A16, f=A16, kv=A16, kvs=512 * 8, pe=A16, pes=64 * 8, y=A16, s=A16, b=2, rows=4,
+             qr=1536, c=512, rope=64):
+        return L.lib.dsv3_mla_latent(a, stride, qw, kw, f, kv, kvs, pe, pes, y, s, b, rows, qr, c, rope, 1e-6, 1e-6, None)
+    for name in ("a", "qw", "kw", "f", "kv", "pe", "y", "s"):
+        assert call(**{name: None}) == 1
+        assert call(**{name: A16 + 2}) == 4
+    for bad in ({"qr": 100}, {"qr": 2176}, {"qr": 0}, {"c": 256}, {"rope": 32}, {"stride": 2104}, {"b": -1}, {"kvs": 2040}):
+        assert call(**bad) == 2, bad
+    assert call(b=0, a=None) == 0 and call(rows=0, a=None) == 0

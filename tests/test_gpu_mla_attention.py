@@ -78,6 +78,84 @@ PREFILL = [(1, 32, 32, 1, "causal"), (1, 33, 63, 3, None), (2, 64, 64, 8, "causa
            (1, 70, 130, 2, "lowest"), (1, 70, 130, 2, "lowest_f32")]
 
 
+# tiles of 32 positions, workgroups of 128 (token, head) rows, wavefronts of 32; one split and many, uneven last ones, more
+# units than compute units
+DECODE = [(1, 1, 1, 1, None), (1, 1, 31, 128, None), (2, 1, 33, 128, None), (1, 1, 700, 128, None), (3, 1, 1000, 16, None),
+          (70, 1, 97, 128, None), (5, 4, 257, 40, "causal"), (1, 31, 95, 16, "causal_f32"), (2, 3, 200, 9, "holes"),
+          (1, 5, 130, 2, "lowest"), (1, 5, 130, 2, "lowest_f32"), (1, 1, 9000, 3, None)]
+
+
+def _decode_reference(q, freqs, kv, pe, w8, ws, mask, t, scale):
+    """Binary64 with the absorbed form's roundings to bf16: weights, rotated and folded query, latent sum."""
+    b, s, h, _ = q.shape
+    w = (w8.float() * ws.repeat_interleave(128, 0).repeat_interleave(128, 1)).bfloat16().double().view(h, NOPE + V, C)
+    pairs = q[..., NOPE:].float().unflatten(-1, (-1, 2))
+    re, im = pairs[..., 0], pairs[..., 1]
+    cos, sin = freqs.real.view(1, s, 1, -1), freqs.imag.view(1, s, 1, -1)
+    qr = torch.stack((re * cos - im * sin, re * sin + im * cos), -1).flatten(-2).bfloat16().double()
+    kv, pe = kv[:, :t].double(), pe[:, :t].double()
+    out = torch.empty(b, s, h, V, dtype=torch.float64, device=q.device)
+    for i in range(h):
+        ql = (q[:, :, i, :NOPE].double() @ w[i, :NOPE]).bfloat16().double()
+        sc = (ql @ kv.transpose(1, 2).contiguous() + qr[:, :, i] @ pe.transpose(1, 2).contiguous()) * scale
+        if mask is not None:
+            sc = (sc.float() + mask.float()).double()
+        out[:, :, i] = (sc.softmax(-1) @ kv).bfloat16().double() @ w[i, NOPE:].t()
+    return out
+
+
+@pytest.mark.parametrize("grow", [False, True])
+@pytest.mark.parametrize("b,s,t,h,kind", DECODE)
+def test_decode_attention(b, s, t, h, kind, grow):
+    q, freqs, kv, pe, w8, ws = _inputs(b, s, t, h, s + t)
+    if grow:                    # scores that grow along the positions by far more than 2^64: the running maximum is raised
+        if kind is not None:
+            pytest.skip("one run per shape without a mask")
+        pe[:, :t] *= torch.linspace(0.01, 400, t, device="cuda").bfloat16().view(1, t, 1)
+    mask = _mask(kind, s, t, 5)
+    scale = 0.08
+    got = torch.ops.dsv3fp8.mla_decode(q, freqs, kv, pe, w8, ws, mask, t, scale).view(b, s, h, V).double()
+    ref = _decode_reference(q, freqs, kv, pe, w8, ws, mask, t, scale)
+    if kind == "holes":
+        assert torch.isnan(got[:, 1]).all() and torch.isnan(ref[:, 1]).all()
+        keep = torch.arange(s, device="cuda") != 1
+        got, ref = got[:, keep], ref[:, keep]
+    # the latent sum and the result round to bf16 (2^-9 each), the exponentials too; in the value product of 512 terms these
+    # errors average out against a result of the same size: 2^-7 of the row's norm
+    assert ((got - ref).norm(dim=-1) <= 2.0 ** -7 * ref.norm(dim=-1)).all()
+
+
+LATENT = [(1, 1, 0, 1536), (3, 1, 7, 1536), (2, 5, 0, 128), (1, 40, 3, 2048), (2, 33, 1, 640)]
+
+
+@pytest.mark.parametrize("b,s,start,q_rank", LATENT)
+def test_latent_rows(b, s, start, q_rank):
+    from dsv3fp8 import kernel
+    import torch.nn.functional as F
+    from dsv3fp8.model import apply_rotary_emb
+    g = torch.Generator().manual_seed(q_rank + s)
+    a = (torch.randn(b, s, q_rank + C + ROPE, generator=g) * 3).bfloat16().cuda()
+    a[0, 0, :q_rank] = 0
+    qw, kw = [(1 + 0.1 * torch.randn(n, generator=g)).bfloat16().cuda() for n in (q_rank, C)]
+    ang = torch.rand(s, ROPE // 2, generator=g) * 6.28
+    freqs = torch.polar(torch.ones_like(ang), ang).cuda()
+    kv, pe = (torch.full((b + 1, start + s + 2, n), 7.0, dtype=torch.bfloat16, device="cuda") for n in (C, ROPE))
+    y, ys = torch.ops.dsv3fp8.mla_latent(a, qw, kw, freqs, kv, pe, start, 1e-6, 1e-6)
+    ref = F.rms_norm(a[..., :q_rank].double(), (q_rank,), qw.double(), 1e-6)
+    got = y.double() * ys.double().repeat_interleave(128, -1)
+    # one rounding to bf16 and one to e4m3 (2^-4 of the value, or half the smallest step of the block)
+    amax = ys.double().repeat_interleave(128, -1) * 448
+    assert ((got - ref).abs() <= ref.abs() * (2.0 ** -4 + 2.0 ** -8) + amax / 448 * 2.0 ** -10).all()
+    q8, s8 = kernel.act_quant(ref.bfloat16().contiguous(), 128)
+    assert (q8.view(torch.uint8) != y.view(torch.uint8)).double().mean() <= 2e-3     # ties of the bf16 rounding only
+    lat = F.rms_norm(a[..., q_rank:q_rank + C].double(), (C,), kw.double(), 1e-6)
+    assert ((kv[:b, start:start + s].double() - lat).abs() <= lat.abs() * 2.0 ** -8).all()
+    assert torch.equal(pe[:b, start:start + s], apply_rotary_emb(a[..., q_rank + C:].unsqueeze(2), freqs).squeeze(2))
+    for t in (kv, pe):                                                               # nothing else is written
+        t[:b, start:start + s] = 7.0
+        assert (t == 7.0).all()
+
+
 @pytest.mark.parametrize("b,s,t,h,kind", PREFILL)
 def test_prefill_attention(b, s, t, h, kind):
     q, freqs, kv, pe, w8, ws = _inputs(b, s, t, h, s + t)
