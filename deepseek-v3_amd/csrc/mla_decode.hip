@@ -20,6 +20,7 @@ constexpr int kTile = 32;                               // positions per tile
 constexpr int kStages = 4;                              // tiles in LDS: one computed, three on their way
 constexpr int kRopeOff = kTile * kC * 2;                // a stage: 32 rows of 1 KiB latents, then 32 rows of 128 B rotary keys
 constexpr int kStage = kRopeOff + kTile * kRope * 2;
+constexpr int kAhead = 6;                               // operands read from LDS ahead of the MFMA that takes them
 constexpr int kRows = 128;                              // rows per workgroup: 4 wavefronts x 32
 constexpr int kPartFloats = kRows * kC;                 // partial sums of a workgroup, in its registers' order
 
@@ -29,7 +30,7 @@ struct DecodeArgs {
     const v2f* freqs;                                   // [tokens][32] (cos, sin)
     const uint16_t* kv; int64_t kv_bs;                  // latent cache, batch stride in elements
     const uint16_t* pe; int64_t pe_bs;
-    const void* mask; int mask_f32;                     // [tokens][positions] or null
+    const void* mask;                                   // [tokens][positions]
     float* part; v2f* ml;                               // [batch][row block][split]: kPartFloats floats; kRows x (maximum, sum)
     uint16_t* out;                                      // bf16 [batch][rows][512]
     int batch, rows, heads, positions, tiles, blocks, splits, per;
@@ -60,6 +61,8 @@ __device__ __forceinline__ void scale_agprs(v16f& v, float a) {
 // values are the same 32 x 512 block: the keys are read as rows, the values through the LDS's transposing reads, four
 // positions of one feature per lane.
 // Bound: per tile 68 MFMAs of 32 cycles and, at 1 KiB of LDS reads per MFMA and wavefront, the same time in the LDS.
+enum { kNoMask, kMaskBf16, kMaskF32 };
+template <int MASK>
 __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -128,16 +131,26 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
         const uint8_t* base = lds + st * kStage;
         v16f T[1] = {};
         v16f& S = T[0];
+        // operands kAhead steps ahead; the barriers keep this order (the scheduler puts each read next to its use and waits)
+        v4u ring[kAhead];
+        auto key = [&](int s) -> v4u {
+            return s < 32 ? *(const v4u*)(base + (kaddr ^ ((s & 7) << 5)) + (s >> 3) * 256) : *(const v4u*)(base + (raddr ^ ((s - 32) << 5)));
+        };
 #pragma unroll
-        for (int s = 0; s < 32; ++s) S = mfma32(*(const v4u*)(base + (kaddr ^ ((s & 7) << 5)) + (s >> 3) * 256), Q[s], S);
+        for (int s = 0; s < kAhead; ++s) ring[s] = key(s);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) S = mfma32(*(const v4u*)(base + (raddr ^ (s << 5))), Q[32 + s], S);
-        if (p.mask) {
+        for (int s = 0; s < 36; ++s) {
+            S = mfma32(ring[s % kAhead], Q[s], S);
+            if (s + kAhead < 36) ring[s % kAhead] = key(s + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (MASK != kNoMask) {
             const int64_t mrow = (int64_t)(row / p.heads) * p.positions;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int64_t at = mrow + min(t * kTile + 8 * (e >> 2) + 4 * g + (e & 3), p.positions - 1);
-                S[e] += mask_term(p.mask_f32 ? mask_at<true>(p.mask, at) : mask_at<false>(p.mask, at), p.inv_scale);
+                S[e] += mask_term(mask_at<MASK == kMaskF32>(p.mask, at), p.inv_scale);
             }
         }
         if ((t + 1) * kTile > p.positions) {            // the last tile may reach past the end
@@ -147,7 +160,7 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
         }
         float mx = S[0];
 #pragma unroll
-        for (int e = 1; e < 16; ++e) mx = fmaxf(mx, S[e]);
+        for (int e = 1; e < 16; ++e) mx = __builtin_elementwise_maximum(mx, S[e]);
         mx = fmaxf(mx, xor32(mx));
         // The maximum is only raised when it grows by more than 2^64: exponentials and sums have room for that in binary32
         // and bf16, and so the 256 multiplications are needed in the rarest of cases.
@@ -164,6 +177,16 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
             }
         }
         const float off = softmax_offset(T, m, scale2);
+        const uint32_t vbase = lds0 + st * kStage + vaddr;      // stages are multiples of 1 KiB: the xors below stay inside a row
+        auto value = [&](int s) -> v4u {                        // positions 16 (s / 16) .. of features 32 (s % 16) ..
+            const uint32_t at = (vbase ^ ((s & 3) << 6)) + (s >> 4) * 16384 + ((s & 15) >> 2) * 256;
+            const v2u lo = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf)(uintptr_t)at));
+            const v2u hi = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf)(uintptr_t)((at ^ 32) + 8192)));
+            return v4u{ lo[0], lo[1], hi[0], hi[1] };
+        };
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) ring[s] = value(s);    // on their way during the exponentials
+        __builtin_amdgcn_sched_barrier(0);
         float sum = 0.f;
         v4u P[2];
 #pragma unroll
@@ -177,16 +200,12 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
                 P[u][q] = pack_bf16(x, y);
             }
         l += sum;
-        const uint32_t vbase = lds0 + st * kStage + vaddr;      // stages are multiples of 1 KiB: the xors below stay inside a row
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int d = 0; d < 16; ++d) {
-                const uint32_t at = (vbase ^ ((d & 3) << 6)) + u * 16384 + (d >> 2) * 256;
-                const v2u lo = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf)(uintptr_t)at));
-                const v2u hi = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf)(uintptr_t)((at ^ 32) + 8192)));
-                O[d] = mfma32(v4u{ lo[0], lo[1], hi[0], hi[1] }, P[u], O[d]);
-            }
+        for (int s = 0; s < 32; ++s) {
+            O[s & 15] = mfma32(ring[s % kAhead], P[s >> 4], O[s & 15]);
+            if (s + kAhead < 32) ring[s % kAhead] = value(s + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         st = (st + 1) % kStages;
     }
 
@@ -372,13 +391,15 @@ int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t 
     a.ml = (v2f*)(a.part + units * kPartFloats);
     a.ql = ql; a.q = (const uint16_t*)q; a.freqs = (const v2f*)freqs;
     a.kv = (const uint16_t*)kv; a.kv_bs = kv_bs; a.pe = (const uint16_t*)pe; a.pe_bs = pe_bs;
-    a.mask = mask; a.mask_f32 = mask_f32; a.heads = heads;
+    a.mask = mask; a.heads = heads;
     a.scale = scale; a.inv_scale = 1.0f / scale;
     int rc = launch_wkv_b_absorb(q, (int64_t)heads * kQd, kQd, w, ws, ql, DSV3_ABSORB_Q, batch * tokens, heads, kNope, kNope, kC, st);
     if (rc != DSV3_OK) return rc;
-    static LdsGrant grant;
-    if (!grant.ensure((const void*)mla_decode_kernel, kStages * kStage)) return DSV3_ERR_LAUNCH;
-    hipLaunchKernelGGL(mla_decode_kernel, dim3(a.splits, (unsigned)batch, a.blocks), dim3(256), kStages * kStage, st, a);
+    const int which = !mask ? kNoMask : mask_f32 ? kMaskF32 : kMaskBf16;
+    void (*const kernel)(DecodeArgs) = !mask ? mla_decode_kernel<kNoMask> : mask_f32 ? mla_decode_kernel<kMaskF32> : mla_decode_kernel<kMaskBf16>;
+    static LdsGrant grant[3];
+    if (!grant[which].ensure((const void*)kernel, kStages * kStage)) return DSV3_ERR_LAUNCH;
+    hipLaunchKernelGGL(kernel, dim3(a.splits, (unsigned)batch, a.blocks), dim3(256), kStages * kStage, st, a);
     hipLaunchKernelGGL(mla_combine_kernel, dim3(64, (unsigned)batch, a.blocks), dim3(256), 0, st, a);
     if ((rc = launch_status()) != DSV3_OK) return rc;
     return launch_wkv_b_absorb(a.out, (int64_t)heads * kC, kC, w, ws, y, DSV3_ABSORB_V, batch * tokens, heads, kNope, kNope, kC, st);
