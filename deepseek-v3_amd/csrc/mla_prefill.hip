@@ -15,6 +15,8 @@
 // At 4096 tokens, 128 heads, causal mask: expand 226 us, flags 23 us, attend 915 us (0.75 PFLOP/s of the pairs the mask
 // leaves); the whole layer 1.77 ms where the absorbed form as tensor operations took 20.2 ms (2 x 2.5 ms score products,
 // 1.6 ms value product and 12 ms of passes over the 4.3 GB score matrix).
+#include <type_traits>
+
 #include "mla.hpp"
 
 namespace dsv3 {
@@ -22,6 +24,7 @@ namespace {
 
 constexpr int kC = 512, kRope = 64, kNope = 128, kV = 128, kQd = kNope + kRope;
 constexpr int kTile = 64;                       // positions per tile
+constexpr int kAhead = 6;                       // operands read from LDS ahead of the MFMA that takes them
 // One tile's operands, bytes.  Keys: [position half][16-wide K step][lane][16]; the same for the rotary keys; values:
 // [32 features][16 positions][lane][16].  A wavefront's operand of one MFMA is 1 KiB, lane l's piece at 16 l.
 constexpr int kKeyBytes = kTile * kNope * 2, kValBytes = kTile * kV * 2, kRopeBytes = kTile * kRope * 2;
@@ -102,7 +105,7 @@ __global__ __launch_bounds__(512, 2) void mla_expand_kernel(ExpandArgs p) {
             W[s] = v4u{ pack_bf16(a.x * k, a.y * k), pack_bf16(b.x * k, b.y * k), pack_bf16(c.x * k, c.y * k), pack_bf16(d.x * k, d.y * k) };
         }
     }
-    const uint32_t frag = i * 1024;
+    const uint32_t frag = i * 1024 + ((g ^ (i & 15)) << 4);        // chunk 2 s + g of row i
     int st = 0;
     for (int sub = s0; sub < s1; ++sub, st ^= 1) {
         if (sub == s0) __builtin_amdgcn_s_waitcnt(0x0f70);          // vmcnt(0)
@@ -110,12 +113,23 @@ __global__ __launch_bounds__(512, 2) void mla_expand_kernel(ExpandArgs p) {
         barrier_no_fence();
         issue(sub + 1, st ^ 1);
         v16f acc = {};
-        const uint8_t* t = lds + st * 32768 + frag;
+        const uint8_t* t = lds + st * 32768;
+        // latents kAhead steps ahead; the barriers keep this order
+        auto chunk = [&](int s) -> v4u { return *(const v4u*)(t + (frag ^ ((s & 7) << 5)) + (s >> 3) * 256); };
+        v4u ring[kAhead];
 #pragma unroll
-        for (int s = 0; s < 32; ++s) {
-            const v4u x = *(const v4u*)(t + (((2 * s + g) ^ (i & 15)) << 4));
-            acc = keys ? mfma32(W[s], x, acc) : mfma32(x, W[s], acc);
-        }
+        for (int s = 0; s < kAhead; ++s) ring[s] = chunk(s);
+        __builtin_amdgcn_sched_barrier(0);
+        auto products = [&](auto is_key) {
+#pragma unroll
+            for (int s = 0; s < 32; ++s) {
+                acc = is_key ? mfma32(W[s], ring[s % kAhead], acc) : mfma32(ring[s % kAhead], W[s], acc);
+                if (s + kAhead < 32) ring[s % kAhead] = chunk(s + kAhead);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        if (keys) products(std::true_type());
+        else products(std::false_type());
         const int b = sub / (p.tiles * 2), sb = sub - b * p.tiles * 2;
         uint8_t* tile = p.img + (((int64_t)b * p.heads + h) * p.tiles + (sb >> 1)) * kHeadTile;
         v4u o[2];
@@ -135,9 +149,10 @@ __global__ __launch_bounds__(512, 2) void mla_expand_kernel(ExpandArgs p) {
 
 enum : uint8_t { kClear = 0, kMixed = 1, kSkip = 2 };
 
-// flags[tile][q / 32]: what the mask does to 32 query rows x 64 positions (all zero, anything, all -inf or no row)
+// flags[q / 256][tile][q / 32 % 8]: what the mask does to 32 query rows x 64 positions (all zero, anything, all -inf or no
+// row).  An attend workgroup's eight flags of a tile are one 64-bit word, its tiles follow one another.
 template <bool F32>
-__global__ __launch_bounds__(512) void mla_mask_flags_kernel(const void* mask, uint8_t* flags, int rows, int positions, int groups) {
+__global__ __launch_bounds__(512) void mla_mask_flags_kernel(const void* mask, uint8_t* flags, int rows, int positions) {
     const int lane = threadIdx.x & 63, q32 = blockIdx.y * 8 + (threadIdx.x >> 6);
     const int pos = blockIdx.x * kTile + lane;
     bool zero = true, ninf = true;
@@ -152,7 +167,7 @@ __global__ __launch_bounds__(512) void mla_mask_flags_kernel(const void* mask, u
             }
         }
     const uint8_t f = __all(ninf) ? kSkip : __all(zero) ? kClear : kMixed;
-    if (lane == 0) flags[(int64_t)blockIdx.x * groups + q32] = f;
+    if (lane == 0) flags[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 8 + (threadIdx.x >> 6)] = f;
 }
 
 // ---------------------------------------------------------------------------------------------------------- attend
@@ -161,9 +176,9 @@ struct AttendArgs {
     const uint16_t* q;                          // [batch][rows][heads][192], rotary part not yet rotated
     const v2f* freqs;                           // [rows][32] (cos, sin)
     const uint8_t* img; const uint8_t* rope;
-    const void* mask; const uint8_t* flags;     // [rows][positions] / [tiles][groups], or null
+    const void* mask; const uint64_t* flags;    // [rows][positions] / [qtiles][tiles], or null
     uint8_t* y; float* ys;                      // fp8 [batch][rows][heads * 128], scales [batch][rows][heads]
-    int batch, heads, rows, positions, tiles, qtiles, groups;
+    int batch, heads, rows, positions, tiles, qtiles;
     float scale, inv_scale;                     // softmax scale and its reciprocal
 };
 
@@ -218,39 +233,63 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
         for (int n = 0; n < 4; ++n) copy16(src + (n * 8 + wave) * 1024, lane16, lds0 + st * kStage + (n * 8 + wave) * 1024);
         copy16(rimg + (int64_t)t * kRopeBytes + wave * 1024, lane16, lds0 + st * kStage + kHeadTile + wave * 1024);
     };
-    // the workgroup's flags of a tile: one byte per wavefront, 2 everywhere = nobody needs the tile
-    auto tile_flags = [&](int t) -> uint64_t {
-        return p.flags ? *(const uint64_t*)(p.flags + (int64_t)t * p.groups + qt * 8) : 0ull;
-    };
+    // Flags of 64 tiles at a time, one word per lane, as three masks: tiles that somebody needs, this wavefront's mixed and
+    // skipped ones.  (A look at memory per tile stood in the way of every tile and of each one behind a causal diagonal.)
     constexpr uint64_t kAllSkip = 0x0202020202020202ull;
-    auto next_tile = [&](int t) {
-        while (t < p.tiles && tile_flags(t) == kAllSkip) ++t;
-        return t;
+    int window = 0;
+    uint64_t act, mix, skip;
+    auto look = [&]() {
+        uint64_t f = kAllSkip;
+        if (window + lane < p.tiles) f = p.flags ? p.flags[(int64_t)qt * p.tiles + window + lane] : 0ull;
+        const uint8_t mine = (uint8_t)(f >> (8 * wave));
+        act = __ballot(f != kAllSkip);
+        mix = __ballot(mine == kMixed);
+        skip = __ballot(mine == kSkip);
+    };
+    auto next_tile = [&](int t, uint8_t& flag) {        // the first tile from t on that somebody needs, and this wavefront's flag
+        for (;;) {
+            if (t >= window + 64) { window += 64; if (window >= p.tiles) return p.tiles; look(); }
+            const uint64_t rest = act >> (t - window);
+            if (rest != 0) {
+                t += __builtin_ctzll(rest);
+                flag = (skip >> (t - window)) & 1 ? kSkip : (mix >> (t - window)) & 1 ? kMixed : kClear;
+                return t;
+            }
+            t = window + 64;
+        }
     };
 
     v16f O[4] = {};
     float m = -__builtin_inff(), l = 0.f;           // running maximum (raw scores), this lane's share of the sum
     const float scale2 = p.scale * 1.44269504088896340736f;
-    int t = next_tile(0), st = 0;
+    look();
+    uint8_t flag = kSkip, flag_next = kSkip;
+    int t = next_tile(0, flag), st = 0;
     if (t < p.tiles) issue(t, 0);
     if (wave >= 4) __builtin_amdgcn_s_setprio(1);
     while (t < p.tiles) {
-        const uint8_t flag = (uint8_t)(tile_flags(t) >> (8 * wave));
-        const int tn = next_tile(t + 1);
+        const int tn = next_tile(t + 1, flag_next);
         __builtin_amdgcn_s_waitcnt(0x0f70);
         barrier_no_fence();
         if (tn < p.tiles) issue(tn, st ^ 1);
         if (flag != kSkip) {
             const uint8_t* base = lds + st * kStage + lane16;
+            // operands are read kAhead steps ahead; the barriers keep this order (left to itself the scheduler reads two ahead
+            // and waits for most of them)
+            v4u ring[kAhead];
+            auto key = [&](int n) -> v4u {              // step n: K step n / 2 of position half n & 1
+                return *(const v4u*)(base + (n < 16 ? (n & 1) * 8 + (n >> 1) : kHeadTile / 1024 + (n & 1) * 4 + (n >> 1) - 8) * 1024);
+            };
             v16f S[2] = {};
 #pragma unroll
-            for (int s = 0; s < 8; ++s)
+            for (int n = 0; n < kAhead; ++n) ring[n] = key(n);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int k = 0; k < 2; ++k) S[k] = mfma32(*(const v4u*)(base + (k * 8 + s) * 1024), Q[s], S[k]);
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int k = 0; k < 2; ++k) S[k] = mfma32(*(const v4u*)(base + kHeadTile + (k * 4 + s) * 1024), Q[8 + s], S[k]);
+            for (int n = 0; n < 24; ++n) {
+                S[n & 1] = mfma32(ring[n % kAhead], Q[n >> 1], S[n & 1]);
+                if (n + kAhead < 24) ring[n % kAhead] = key(n + kAhead);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if (flag == kMixed) {
                 const int64_t mrow = (int64_t)row * p.positions;
 #pragma unroll
@@ -274,7 +313,7 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
 #pragma unroll
             for (int k = 0; k < 2; ++k)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, S[k][e]);
+                for (int e = 0; e < 16; ++e) mx = __builtin_elementwise_maximum(mx, S[k][e]);
             mx = fmaxf(mx, xor32(mx));
             const bool raise = (mx - m) * scale2 > 8.f || (m == -__builtin_inff() && mx > m);
             if (__any(raise)) {
@@ -288,26 +327,34 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
                 m = mn;
             }
             const float off = softmax_offset(S, m, scale2);
+            auto value = [&](int n) -> v4u { return *(const v4u*)(base + kKeyBytes + ((n & 3) * 4 + (n >> 2)) * 1024); };
+#pragma unroll
+            for (int n = 0; n < kAhead; ++n) ring[n] = value(n);
+            __builtin_amdgcn_sched_barrier(0);
             float sum = 0.f;
             v4u P[4];
+            auto expo = [&](int u, int q) {
+                const int e = 8 * (u & 1) + 2 * q;
+                const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(S[u >> 1][e], scale2, -off));
+                const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(S[u >> 1][e + 1], scale2, -off));
+                sum += x + y;
+                P[u][q] = pack_bf16(x, y);
+            };
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int q = 0; q < 4; ++q) expo(0, q);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int e = 8 * (u & 1) + 2 * q;
-                    const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(S[u >> 1][e], scale2, -off));
-                    const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(S[u >> 1][e + 1], scale2, -off));
-                    sum += x + y;
-                    P[u][q] = pack_bf16(x, y);
-                }
+            for (int n = 0; n < 16; ++n) {              // step n: positions 16 (n / 4), features 32 (n & 3); beside it exponentials of the next positions
+                const int u = n >> 2, d = n & 3;
+                O[d] = mfma32(ring[n % kAhead], P[u], O[d]);
+                if (n + kAhead < 16) ring[n % kAhead] = value(n + kAhead);
+                if (u < 3) expo(u + 1, d);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             l += sum;
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int d = 0; d < 4; ++d) O[d] = mfma32(*(const v4u*)(base + kKeyBytes + (d * 4 + u) * 1024), P[u], O[d]);
         }
         st ^= 1;
         t = tn;
+        flag = flag_next;
     }
     __builtin_amdgcn_s_setprio(0);
 
@@ -380,15 +427,15 @@ int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t
 
     AttendArgs a;
     a.q = (const uint16_t*)q; a.freqs = (const v2f*)freqs; a.img = e.img; a.rope = e.rope;
-    a.mask = mask; a.flags = mask ? flags : nullptr;
+    a.mask = mask; a.flags = mask ? (const uint64_t*)flags : nullptr;
     a.y = (uint8_t*)y; a.ys = ys;
     a.batch = (int)batch; a.heads = heads; a.rows = (int)rows; a.positions = (int)positions;
-    a.tiles = (int)tiles; a.qtiles = (int)qtiles; a.groups = (int)(qtiles * 8);
+    a.tiles = (int)tiles; a.qtiles = (int)qtiles;
     a.scale = scale; a.inv_scale = 1.0f / scale;
     if (mask) {
         const dim3 grid((unsigned)tiles, (unsigned)qtiles);
-        if (mask_f32) hipLaunchKernelGGL(mla_mask_flags_kernel<true>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions, a.groups);
-        else hipLaunchKernelGGL(mla_mask_flags_kernel<false>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions, a.groups);
+        if (mask_f32) hipLaunchKernelGGL(mla_mask_flags_kernel<true>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions);
+        else hipLaunchKernelGGL(mla_mask_flags_kernel<false>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions);
     }
     constexpr int bytes = 2 * (kHeadTile + kRopeBytes);
     static LdsGrant grant[2];
