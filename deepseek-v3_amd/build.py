@@ -1,4 +1,5 @@
-"""Builds libdsv3fp8.so (HIP kernels + C ABI) for gfx950 with hipcc, in-tree.
+"""Builds libdsv3fp8.so (HIP kernels + C ABI) for gfx950 with hipcc and libdsv3torch.so (the native part of the torch
+operators, on top of it) with the host compiler, in-tree.
 
     python deepseek-v3_amd/build.py            # build into deepseek-v3_amd/lib/
 """
@@ -15,6 +16,8 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB_DIR = HERE / "lib"
 LIB_PATH = LIB_DIR / "libdsv3fp8.so"
+TORCH_SRC = CSRC / "torch_ops.cpp"
+TORCH_LIB_PATH = LIB_DIR / "libdsv3torch.so"
 
 ARCH = "gfx950"
 # -packed-fp32-ops off: the compiler must not form v_pk_{add,mul,fma}_f32 from scalar float code.
@@ -99,7 +102,27 @@ def build_library(verbose: bool = True) -> Path:
     os.replace(tmp, LIB_PATH)
     if verbose:
         print(f"[build] linked {LIB_PATH}", flush=True)
+    build_torch_library(verbose)
     return LIB_PATH
+
+
+def build_torch_library(verbose: bool = True) -> Path:
+    """csrc/torch_ops.cpp against the installed torch; finds libdsv3fp8.so beside it."""
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(_hipcc()).resolve().parent.parent
+    tmp = TORCH_LIB_PATH.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f"-I{root / 'include'}", f"-I{rocm / 'include'}",
+           "-isystem/opt/rocm/include", str(TORCH_SRC), "-o", str(tmp), f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           f"-L{LIB_DIR}", "-ldsv3fp8", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"building {TORCH_LIB_PATH.name} failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, TORCH_LIB_PATH)
+    if verbose:
+        print(f"[build] linked {TORCH_LIB_PATH}", flush=True)
+    return TORCH_LIB_PATH
 
 
 if __name__ == "__main__":

@@ -1,0 +1,232 @@
+// Device implementations of the torch.ops.dsv3fp8 operators of the linear, cast and attention layers: allocate the results,
+// pass raw pointers and the current stream of the tensors' device to libdsv3fp8.so.
+//
+// Why native: at a few tokens the launches of a layer are shorter than the host's way to them.  The same bodies in Python
+// behind torch.library cost 10 to 14 us an operator (argument boxing, device and stream contexts, two or three ctypes
+// calls); one sequence's decode step of the attention layer (five operators, kernels 72 us) was bound by that at 118 us.
+// Scratch memory comes from the caching allocator on each call: it belongs to the current stream, and under stream capture
+// to the graph's pool.
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/library.h>
+
+#include <tuple>
+
+#include "../../include/dsv3_fp8.h"
+
+namespace {
+
+using at::Tensor;
+using std::tuple;
+typedef c10::optional<Tensor> OptTensor;
+
+constexpr auto kFp8 = at::kFloat8_e4m3fn;
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kBFloat16: return DSV3_BF16;
+        case at::kHalf: return DSV3_F16;
+        case at::kFloat: return DSV3_F32;
+        default: TORCH_CHECK_TYPE(false, "dsv3fp8: unsupported dtype ", t, " (bf16, fp16 and fp32 are implemented)");
+    }
+}
+at::ScalarType dtype_of(int64_t code) {
+    switch (code) {
+        case DSV3_BF16: return at::kBFloat16;
+        case DSV3_F16: return at::kHalf;
+        case DSV3_F32: return at::kFloat;
+        default: TORCH_CHECK_VALUE(false, "dsv3fp8: unknown dtype code ", code);
+    }
+}
+void check(int rc, const char* what) {
+    TORCH_CHECK(rc == DSV3_OK, what, " failed: ", dsv3_status_string(rc), " (dsv3_status ", rc, ")");
+}
+
+// The device of an operator's tensors made current, and its stream.
+struct On {
+    c10::DeviceGuard guard;
+    void* stream;
+    explicit On(const Tensor& t) : guard(t.device()), stream((void*)c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+};
+
+Tensor scratch(const Tensor& like, size_t bytes) {
+    return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
+}
+Tensor with_last(const Tensor& x, int64_t last, at::ScalarType dtype) {
+    auto size = x.sizes().vec();
+    size.back() = last;
+    return at::empty(size, x.options().dtype(dtype));
+}
+
+tuple<Tensor, Tensor> act_quant(const Tensor& x, int64_t block, int64_t fmt) {
+    TORCH_CHECK(block > 0, "act_quant: block_size must be positive");
+    const int64_t last = x.size(-1);
+    const int code = dtype_code(x.scalar_type());
+    Tensor y = at::empty_like(x, x.options().dtype(kFp8)), s = with_last(x, last / block, at::kFloat);
+    On on(x);
+    check(dsv3_act_quant(x.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), x.numel(), last, (int)block, (int)fmt, on.stream),
+          "dsv3_act_quant");
+    return {y, s};
+}
+
+Tensor weight_dequant(const Tensor& x, const Tensor& s, int64_t block, int64_t out) {
+    TORCH_CHECK_VALUE(x.dim() == 2, "weight_dequant: a matrix is needed");
+    Tensor y = at::empty_like(x, x.options().dtype(dtype_of(out)));
+    On on(x);
+    check(dsv3_weight_dequant(x.data_ptr(), (const float*)s.data_ptr(), y.data_ptr(), (int)out, x.size(0), x.size(1), (int)block,
+                              on.stream), "dsv3_weight_dequant");
+    return y;
+}
+
+tuple<Tensor, Tensor> weight_quant(const Tensor& w, int64_t block, int64_t fmt) {
+    TORCH_CHECK_VALUE(w.dim() == 2, "weight_quant: a matrix is needed");
+    TORCH_CHECK(block > 0, "weight_quant: block_size must be positive");
+    const int code = dtype_code(w.scalar_type());
+    const int64_t m = w.size(0), n = w.size(1);
+    Tensor y = at::empty_like(w, w.options().dtype(kFp8));
+    Tensor s = at::empty({(m + block - 1) / block, (n + block - 1) / block}, w.options().dtype(at::kFloat));
+    On on(w);
+    check(dsv3_weight_quant(w.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), m, n, (int)block, (int)fmt, on.stream),
+          "dsv3_weight_quant");
+    return {y, s};
+}
+
+Tensor gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, int64_t out, decltype(dsv3_fp8_gemm)* entry,
+            const char* what) {
+    const int64_t k = a.size(-1), m = k ? a.numel() / k : 0, n = b.size(0);
+    Tensor c = with_last(a, n, dtype_of(out));
+    On on(a);
+    const size_t need = dsv3_fp8_gemm_workspace_bytes(m, n, k);
+    Tensor ws = need ? scratch(a, need) : Tensor();
+    check(entry(a.data_ptr(), (const float*)a_s.data_ptr(), b.data_ptr(), (const float*)b_s.data_ptr(), c.data_ptr(), (int)out,
+                m, n, k, need ? ws.data_ptr() : nullptr, need, on.stream), what);
+    return c;
+}
+Tensor fp8_gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, int64_t out) {
+    return gemm(a, a_s, b, b_s, out, dsv3_fp8_gemm, "dsv3_fp8_gemm");
+}
+Tensor fp8_gemm_pow2(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, int64_t out) {
+    return gemm(a, a_s, b, b_s, out, dsv3_fp8_gemm_pow2, "dsv3_fp8_gemm_pow2");
+}
+
+// act_quant(x, 128, fmt) followed by fp8_gemm, one launch where the library implements it, else two calls
+Tensor linear_fp8(const Tensor& x, const Tensor& b, const Tensor& b_s, int64_t fmt, int64_t out) {
+    const int64_t k = x.size(-1), m = k ? x.numel() / k : 0, n = b.size(0);
+    if (x.scalar_type() != at::kBFloat16 || !dsv3_linear_fp8_fused(m, n, k)) {
+        auto [a, a_s] = act_quant(x, 128, fmt);
+        return fp8_gemm(a, a_s, b, b_s, out);
+    }
+    Tensor c = with_last(x, n, dtype_of(out));
+    On on(x);
+    const size_t need = dsv3_fp8_gemm_workspace_bytes(m, n, k);
+    Tensor ws = need ? scratch(x, need) : Tensor();
+    check(dsv3_linear_fp8(x.data_ptr(), DSV3_BF16, b.data_ptr(), (const float*)b_s.data_ptr(), c.data_ptr(), (int)out, m, n, k,
+                          128, (int)fmt, need ? ws.data_ptr() : nullptr, need, on.stream), "dsv3_linear_fp8");
+    return c;
+}
+
+tuple<Tensor, Tensor> swiglu_quant(const Tensor& h, int64_t block, int64_t fmt) {
+    TORCH_CHECK(h.dim() == 2 && h.is_contiguous() && h.size(1) % 2 == 0, "swiglu_quant: a contiguous matrix of even width is needed");
+    TORCH_CHECK(block > 0, "swiglu_quant: block_size must be positive");
+    const int code = dtype_code(h.scalar_type());
+    const int64_t rows = h.size(0), inter = h.size(1) / 2;
+    Tensor y = at::empty({rows, inter}, h.options().dtype(kFp8)), s = at::empty({rows, inter / block}, h.options().dtype(at::kFloat));
+    On on(h);
+    check(dsv3_swiglu_quant(h.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), rows, inter, (int)block, (int)fmt, on.stream),
+          "dsv3_swiglu_quant");
+    return {y, s};
+}
+
+void check_caches(const Tensor& kv, const Tensor& pe, int64_t batch, int64_t positions) {
+    for (const Tensor* c : {&kv, &pe})
+        TORCH_CHECK(c->dim() == 3 && c->scalar_type() == at::kBFloat16 && c->stride(2) == 1 && c->stride(1) == c->size(2) &&
+                    c->size(0) >= batch && c->size(1) >= positions, "mla: caches must be bf16 [batch, positions, width] with dense rows");
+}
+void check_freqs(const Tensor& f, int64_t rows, int64_t rope) {
+    TORCH_CHECK(f.scalar_type() == at::kComplexFloat && f.is_contiguous() && f.dim() == 2 && f.size(0) == rows && f.size(1) == rope / 2,
+                "mla: freqs must be a contiguous complex64 [rows, rope / 2]");
+}
+
+// What the two attention operators check and pass on alike; `call` gets the shape and the workspace.
+template <class Bytes, class Call>
+void attention(const Tensor& q, const Tensor& freqs, const Tensor& kv, const Tensor& pe, const Tensor& w, const Tensor& ws,
+               const OptTensor& mask, int64_t positions, Bytes bytes, Call call) {
+    TORCH_CHECK(q.dim() == 4 && q.is_contiguous() && q.scalar_type() == at::kBFloat16, "mla: q must be a contiguous bf16 [b, s, h, d]");
+    const int64_t b = q.size(0), s = q.size(1), h = q.size(2);
+    check_caches(kv, pe, b, positions);
+    check_freqs(freqs, s, pe.size(2));
+    TORCH_CHECK(w.dim() == 2 && w.is_contiguous() && ws.is_contiguous() && w.element_size() == 1 && w.size(1) == kv.size(2) &&
+                h > 0 && w.size(0) % h == 0, "mla: wkv_b must be a contiguous fp8 [h * (nope + v), kv_rank]");
+    if (mask)
+        TORCH_CHECK(mask->dim() == 2 && mask->size(0) == s && mask->size(1) == positions && mask->is_contiguous() &&
+                    (mask->scalar_type() == at::kBFloat16 || mask->scalar_type() == at::kFloat),
+                    "mla: mask must be a contiguous bf16 or fp32 [s, positions]");
+    On on(q);
+    const size_t need = bytes(b, s, positions, (int)h);
+    Tensor buf = scratch(q, need);
+    const int rope = (int)pe.size(2), nope = (int)q.size(3) - rope, v = (int)(w.size(0) / h) - nope;
+    call(b, s, (int)h, nope, rope, v, mask ? mask->data_ptr() : nullptr, mask ? dtype_code(mask->scalar_type()) : 0, buf.data_ptr(),
+         need, on.stream);
+}
+
+tuple<Tensor, Tensor> mla_prefill(const Tensor& q, const Tensor& freqs, const Tensor& kv, const Tensor& pe, const Tensor& w,
+                                  const Tensor& ws, const OptTensor& mask, int64_t positions, double scale) {
+    Tensor y, ys;
+    attention(q, freqs, kv, pe, w, ws, mask, positions, dsv3_mla_prefill_workspace_bytes,
+              [&](int64_t b, int64_t s, int h, int nope, int rope, int v, void* m, int md, void* buf, size_t need, void* stream) {
+        y = at::empty({b, s, (int64_t)h * v}, q.options().dtype(kFp8));
+        ys = at::empty({b, s, h}, q.options().dtype(at::kFloat));
+        check(dsv3_mla_prefill(q.data_ptr(), (const float*)freqs.data_ptr(), kv.data_ptr(), kv.stride(0), pe.data_ptr(), pe.stride(0),
+                               w.data_ptr(), (const float*)ws.data_ptr(), m, md, y.data_ptr(), (float*)ys.data_ptr(), b, s, positions,
+                               h, nope, rope, v, kv.size(2), (float)scale, buf, need, stream), "dsv3_mla_prefill");
+    });
+    return {y, ys};
+}
+
+Tensor mla_decode(const Tensor& q, const Tensor& freqs, const Tensor& kv, const Tensor& pe, const Tensor& w, const Tensor& ws,
+                  const OptTensor& mask, int64_t positions, double scale) {
+    Tensor y;
+    attention(q, freqs, kv, pe, w, ws, mask, positions, dsv3_mla_decode_workspace_bytes,
+              [&](int64_t b, int64_t s, int h, int nope, int rope, int v, void* m, int md, void* buf, size_t need, void* stream) {
+        y = at::empty({b, s, (int64_t)h * v}, q.options());
+        check(dsv3_mla_decode(q.data_ptr(), (const float*)freqs.data_ptr(), kv.data_ptr(), kv.stride(0), pe.data_ptr(), pe.stride(0),
+                              w.data_ptr(), (const float*)ws.data_ptr(), m, md, y.data_ptr(), b, s, positions, h, nope, rope, v,
+                              kv.size(2), (float)scale, buf, need, stream), "dsv3_mla_decode");
+    });
+    return y;
+}
+
+// a [b, s, q_rank + kv_rank + rope] -> the normalised query latent, quantised, and the caches' rows start .. start + s - 1
+tuple<Tensor, Tensor> mla_latent(const Tensor& a, const Tensor& qn, const Tensor& kn, const Tensor& freqs, Tensor kv, Tensor pe,
+                                 int64_t start, double q_eps, double kv_eps) {
+    TORCH_CHECK(a.dim() == 3 && a.is_contiguous() && a.scalar_type() == at::kBFloat16 && start >= 0, "mla_latent: a must be a contiguous bf16 [b, s, width]");
+    const int64_t b = a.size(0), s = a.size(1), qr = qn.numel();
+    check_caches(kv, pe, b, start + s);
+    check_freqs(freqs, s, pe.size(2));
+    const int64_t c = kv.size(2), r = pe.size(2);
+    TORCH_CHECK(a.size(2) == qr + c + r && kn.numel() == c && qn.scalar_type() == at::kBFloat16 && kn.scalar_type() == at::kBFloat16 &&
+                qn.is_contiguous() && kn.is_contiguous(), "mla_latent: norm weights do not fit the row");
+    Tensor y = at::empty({b, s, qr}, a.options().dtype(kFp8)), ys = at::empty({b, s, qr / 128}, a.options().dtype(at::kFloat));
+    On on(a);
+    check(dsv3_mla_latent(a.data_ptr(), a.size(2), qn.data_ptr(), kn.data_ptr(), (const float*)freqs.data_ptr(),
+                          (char*)kv.data_ptr() + start * c * 2, kv.stride(0), (char*)pe.data_ptr() + start * r * 2, pe.stride(0),
+                          y.data_ptr(), (float*)ys.data_ptr(), b, s, qr, c, (int)r, (float)q_eps, (float)kv_eps, on.stream),
+          "dsv3_mla_latent");
+    return {y, ys};
+}
+
+}  // namespace
+
+TORCH_LIBRARY_IMPL(dsv3fp8, CUDA, m) {
+    m.impl("act_quant", act_quant);
+    m.impl("weight_dequant", weight_dequant);
+    m.impl("weight_quant", weight_quant);
+    m.impl("fp8_gemm", fp8_gemm);
+    m.impl("fp8_gemm_pow2", fp8_gemm_pow2);
+    m.impl("linear_fp8", linear_fp8);
+    m.impl("swiglu_quant", swiglu_quant);
+    m.impl("mla_prefill", mla_prefill);
+    m.impl("mla_decode", mla_decode);
+    m.impl("mla_latent", mla_latent);
+}

@@ -10,6 +10,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent.parent / "lib" / "libdsv3fp8.so"
+TORCH_LIB_PATH = LIB_PATH.with_name("libdsv3torch.so")      # the operators' native implementations, on top of it
 
 # enum dsv3_dtype / dsv3_scale_fmt / dsv3_status (include/dsv3_fp8.h)
 BF16, F16, F32 = 0, 1, 2
@@ -70,10 +71,11 @@ EXPORTS = {
 
 
 def _load() -> ctypes.CDLL:
-    if not LIB_PATH.exists():
-        raise ImportError(
-            f"{LIB_PATH} is missing: the HIP library has not been built. "
-            f"Run `python {LIB_PATH.parent.parent / 'build.py'}` (needs hipcc); there is no CPU fallback.")
+    for path in (LIB_PATH, TORCH_LIB_PATH):
+        if not path.exists():
+            raise ImportError(
+                f"{path} is missing: the HIP library has not been built. "
+                f"Run `python {LIB_PATH.parent.parent / 'build.py'}` (needs hipcc); there is no CPU fallback.")
     lib = ctypes.CDLL(str(LIB_PATH))
     for name, (res, args) in EXPORTS.items():
         fn = getattr(lib, name)

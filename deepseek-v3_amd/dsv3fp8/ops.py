@@ -2,14 +2,13 @@
 
 ``torch.ops.dsv3fp8.{act_quant, weight_dequant, weight_quant, fp8_gemm}`` and the grouped
 mixture-of-experts ops ``{gate_route, group_tiles, moe_route, fp8_gemm_grouped, swiglu_quant, moe_combine}`` and the
-attention op ``wkv_b_absorb`` take and return torch tensors; the device implementations hand raw device pointers and the
-current HIP stream of the tensors' device to libdsv3fp8.so.  Only a device
+attention ops ``{wkv_b_absorb, mla_latent, mla_decode, mla_prefill}`` take and return torch tensors; the device
+implementations (native in libdsv3torch.so, the mixture-of-experts ones and ``wkv_b_absorb`` below) hand raw device pointers
+and the current HIP stream of the tensors' device to libdsv3fp8.so.  Only a device
 ("CUDA" dispatch key, which is HIP on ROCm) implementation and a shape-only Meta
 implementation are registered: calling an op on CPU tensors raises.
 """
 from __future__ import annotations
-
-from typing import Dict, Tuple
 
 import torch
 
@@ -58,88 +57,18 @@ def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
-# split-K scratch, one buffer per (device, stream): calls on one stream are ordered, so they can share it
-_workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
-
-
-def _workspace(t: torch.Tensor, nbytes: int, stream: int) -> torch.Tensor:
-    # Under stream capture the scratch comes from the graph's own memory pool and lives as long as the graph: the
-    # cached buffer below is replaced when a larger one is needed, which would leave a graph that had captured it
-    # replaying into freed memory.
-    if torch.cuda.is_current_stream_capturing():
-        return torch.empty(nbytes, dtype=torch.uint8, device=t.device)
-    key = (t.device.index, stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1 << 22), dtype=torch.uint8, device=t.device)
-        _workspaces[key] = ws
-    return ws
-
-
-def _act_quant_dev(x: torch.Tensor, block_size: int, scale_fmt: int):
-    y = torch.empty_like(x, dtype=FP8)
-    s = x.new_empty(*x.size()[:-1], x.size(-1) // block_size, dtype=torch.float32)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib.dsv3_act_quant(x.data_ptr(), dtype_code(x.dtype), y.data_ptr(), s.data_ptr(),
-                                     x.numel(), x.size(-1), block_size, scale_fmt, _stream(x))
-    _lib.check(rc, "dsv3_act_quant")
-    return y, s
-
-
 def _act_quant_meta(x, block_size, scale_fmt):
     return (torch.empty_like(x, dtype=FP8),
             x.new_empty(*x.size()[:-1], x.size(-1) // block_size, dtype=torch.float32))
-
-
-def _weight_dequant_dev(x: torch.Tensor, s: torch.Tensor, block_size: int, out_dtype: int):
-    y = torch.empty_like(x, dtype=_CODE_DTYPE[out_dtype])
-    m, n = x.size()
-    with torch.cuda.device(x.device):
-        rc = _lib.lib.dsv3_weight_dequant(x.data_ptr(), s.data_ptr(), y.data_ptr(), out_dtype,
-                                          m, n, block_size, _stream(x))
-    _lib.check(rc, "dsv3_weight_dequant")
-    return y
 
 
 def _weight_dequant_meta(x, s, block_size, out_dtype):
     return torch.empty_like(x, dtype=_CODE_DTYPE[out_dtype])
 
 
-def _weight_quant_dev(w: torch.Tensor, block_size: int, scale_fmt: int):
-    m, n = w.size()
-    y = torch.empty_like(w, dtype=FP8)
-    s = w.new_empty(-(-m // block_size), -(-n // block_size), dtype=torch.float32)
-    with torch.cuda.device(w.device):
-        rc = _lib.lib.dsv3_weight_quant(w.data_ptr(), dtype_code(w.dtype), y.data_ptr(), s.data_ptr(), m, n,
-                                        block_size, scale_fmt, _stream(w))
-    _lib.check(rc, "dsv3_weight_quant")
-    return y, s
-
-
 def _weight_quant_meta(w, block_size, scale_fmt):
     m, n = w.size()
     return torch.empty_like(w, dtype=FP8), w.new_empty(-(-m // block_size), -(-n // block_size), dtype=torch.float32)
-
-
-def _fp8_gemm_dev(a, a_s, b, b_s, out_dtype: int, entry: str = "dsv3_fp8_gemm"):
-    k = a.size(-1)
-    m = a.numel() // k if k else 0
-    n = b.size(0)
-    c = a.new_empty(*a.size()[:-1], n, dtype=_CODE_DTYPE[out_dtype])
-    with torch.cuda.device(a.device):
-        stream = _stream(a)
-        need = _lib.lib.dsv3_fp8_gemm_workspace_bytes(m, n, k)
-        ws = _workspace(a, need, stream) if need else None
-        rc = getattr(_lib.lib, entry)(a.data_ptr(), a_s.data_ptr(), b.data_ptr(), b_s.data_ptr(),
-                                      c.data_ptr(), out_dtype, m, n, k,
-                                      ws.data_ptr() if ws is not None else None,
-                                      ws.numel() if ws is not None else 0, stream)
-    _lib.check(rc, entry)
-    return c
-
-
-def _fp8_gemm_pow2_dev(a, a_s, b, b_s, out_dtype: int):
-    return _fp8_gemm_dev(a, a_s, b, b_s, out_dtype, "dsv3_fp8_gemm_pow2")
 
 
 def _fp8_gemm_meta(a, a_s, b, b_s, out_dtype):
@@ -149,26 +78,6 @@ def _fp8_gemm_meta(a, a_s, b, b_s, out_dtype):
 def linear_fp8_fused(m: int, n: int, k: int) -> bool:
     """Whether act_quant + fp8_gemm of an [m, k] x [n, k] linear run as one launch (dsv3_linear_fp8)."""
     return bool(_lib.lib.dsv3_linear_fp8_fused(m, n, k))
-
-
-def _linear_fp8_dev(x, b, b_s, scale_fmt: int, out_dtype: int):
-    """act_quant(x, 128, scale_fmt) followed by fp8_gemm, fused where the library implements it, else two calls."""
-    k = x.size(-1)
-    m = x.numel() // k if k else 0
-    n = b.size(0)
-    if not (x.dtype == torch.bfloat16 and linear_fp8_fused(m, n, k)):
-        a, a_s = _act_quant_dev(x, 128, scale_fmt)
-        return _fp8_gemm_dev(a, a_s, b, b_s, out_dtype)
-    c = x.new_empty(*x.size()[:-1], n, dtype=_CODE_DTYPE[out_dtype])
-    with torch.cuda.device(x.device):
-        stream = _stream(x)
-        need = _lib.lib.dsv3_fp8_gemm_workspace_bytes(m, n, k)
-        ws = _workspace(x, need, stream) if need else None
-        rc = _lib.lib.dsv3_linear_fp8(x.data_ptr(), _lib.BF16, b.data_ptr(), b_s.data_ptr(), c.data_ptr(), out_dtype,
-                                      m, n, k, 128, scale_fmt, ws.data_ptr() if ws is not None else None,
-                                      ws.numel() if ws is not None else 0, stream)
-    _lib.check(rc, "dsv3_linear_fp8")
-    return c
 
 
 def _linear_fp8_meta(x, b, b_s, scale_fmt, out_dtype):
@@ -270,7 +179,7 @@ def _fp8_gemm_grouped_swiglu_dev(a, a_s, a_rows, b, b_s, rows: int, tile_group, 
     k, inter = a.size(1), b.size(1) // 2
     if not grouped_swiglu_fused(rows, a.size(0), inter, k):
         h = _fp8_gemm_grouped_dev(a, a_s, a_rows, b, b_s, rows, tile_group, tile_row0, tile_rows, _lib.BF16)
-        return _swiglu_quant_dev(h, 128, scale_fmt)
+        return torch.ops.dsv3fp8.swiglu_quant(h, 128, scale_fmt)
     assert a.dim() == 2 and b.dim() == 3 and b_s.dim() == 3 and a.is_contiguous() and b.is_contiguous()
     assert a_s.is_contiguous() and b_s.is_contiguous() and b.size(0) == b_s.size(0) and b.size(2) == k
     for t in (tile_group, tile_row0, tile_rows):
@@ -292,18 +201,6 @@ def _fp8_gemm_grouped_swiglu_dev(a, a_s, a_rows, b, b_s, rows: int, tile_group, 
 def _fp8_gemm_grouped_swiglu_meta(a, a_s, a_rows, b, b_s, rows, tile_group, tile_row0, tile_rows, scale_fmt):
     inter = b.size(1) // 2
     return a.new_empty(rows, inter, dtype=FP8), a.new_empty(rows, inter // 128, dtype=torch.float32)
-
-
-def _swiglu_quant_dev(h: torch.Tensor, block_size: int, scale_fmt: int):
-    assert h.dim() == 2 and h.is_contiguous() and h.size(1) % 2 == 0
-    rows, inter = h.size(0), h.size(1) // 2
-    y = h.new_empty(rows, inter, dtype=FP8)
-    s = h.new_empty(rows, inter // block_size, dtype=torch.float32)
-    with torch.cuda.device(h.device):
-        rc = _lib.lib.dsv3_swiglu_quant(h.data_ptr(), dtype_code(h.dtype), y.data_ptr(), s.data_ptr(),
-                                        rows, inter, block_size, scale_fmt, _stream(h))
-    _lib.check(rc, "dsv3_swiglu_quant")
-    return y, s
 
 
 def _swiglu_quant_meta(h, block_size, scale_fmt):
@@ -373,54 +270,10 @@ def _wkv_b_absorb_meta(x, wkv_b, scale, side, nope_dim, v_dim):
     return x.new_empty(*x.size()[:-1], _absorb_out_dim(wkv_b, side, v_dim))
 
 
-def _mla_check(q, freqs, kv_cache, pe_cache, mask, positions: int):
-    """q [b, s, h, nope + rope] bf16; freqs [s, rope / 2] complex64; caches [>= b, >= positions, width] bf16."""
-    b, s = q.size(0), q.size(1)
-    assert q.dim() == 4 and q.is_contiguous() and q.dtype == torch.bfloat16
-    assert freqs.dtype == torch.complex64 and freqs.is_contiguous() and freqs.shape == (s, pe_cache.size(-1) // 2)
-    for c in (kv_cache, pe_cache):
-        assert c.dim() == 3 and c.dtype == torch.bfloat16 and c.stride(2) == 1 and c.stride(1) == c.size(2)
-        assert c.size(0) >= b and c.size(1) >= positions
-    assert mask is None or (mask.shape == (s, positions) and mask.is_contiguous()
-                            and mask.dtype in (torch.bfloat16, torch.float32))
-
-
-def _mla_call(entry: str, q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions: int, softmax_scale: float, *out):
-    _mla_check(q, freqs, kv_cache, pe_cache, mask, positions)
-    assert wkv_b.is_contiguous() and scale.is_contiguous() and wkv_b.element_size() == 1
-    b, s, h, qd = q.shape
-    rope = pe_cache.size(2)
-    nope = qd - rope
-    with torch.cuda.device(q.device):
-        need = getattr(_lib.lib, entry + "_workspace_bytes")(b, s, positions, h)
-        ws = torch.empty(need, dtype=torch.uint8, device=q.device)
-        rc = getattr(_lib.lib, entry)(
-            q.data_ptr(), freqs.data_ptr(), kv_cache.data_ptr(), kv_cache.stride(0), pe_cache.data_ptr(),
-            pe_cache.stride(0), wkv_b.data_ptr(), scale.data_ptr(), mask.data_ptr() if mask is not None else None,
-            dtype_code(mask.dtype) if mask is not None else 0, *(o.data_ptr() for o in out), b, s, positions, h, nope,
-            rope, wkv_b.size(0) // h - nope, kv_cache.size(2), softmax_scale, ws.data_ptr(), need, _stream(q))
-    _lib.check(rc, entry)
-
-
-def _mla_prefill_dev(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions: int, softmax_scale: float):
-    """The attention of q over the first `positions` rows of the caches, quantised for the output projection:
-    (y [b, s, h * v] e4m3, scales [b, s, h]); see dsv3_mla_prefill in include/dsv3_fp8.h."""
-    y, ys = _mla_prefill_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale)
-    _mla_call("dsv3_mla_prefill", q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale, y, ys)
-    return y, ys
-
-
 def _mla_prefill_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale):
     b, s, h, qd = q.shape
     v = wkv_b.size(0) // h - (qd - pe_cache.size(2))
     return q.new_empty(b, s, h * v, dtype=FP8), q.new_empty(b, s, h, dtype=torch.float32)
-
-
-def _mla_decode_dev(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions: int, softmax_scale: float):
-    """The same attention for few new tokens: y [b, s, h * v] bf16; see dsv3_mla_decode in include/dsv3_fp8.h."""
-    y = _mla_decode_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale)
-    _mla_call("dsv3_mla_decode", q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale, y)
-    return y
 
 
 def _mla_decode_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale):
@@ -428,56 +281,25 @@ def _mla_decode_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions
     return q.new_empty(b, s, wkv_b.size(0) - h * (qd - pe_cache.size(2)))
 
 
-def _mla_latent_dev(a, q_norm, kv_norm, freqs, kv_cache, pe_cache, start: int, q_eps: float, kv_eps: float):
-    """a [b, s, q_rank + kv_rank + rope] -> the normalised query latent, quantised (e4m3, scales per 128), and the caches'
-    rows start .. start + s - 1; see dsv3_mla_latent in include/dsv3_fp8.h."""
-    b, s, width = a.shape
-    c, r = kv_cache.size(2), pe_cache.size(2)
-    assert a.is_contiguous() and a.dtype == torch.bfloat16 and width == q_norm.numel() + c + r and kv_norm.numel() == c
-    assert q_norm.dtype == torch.bfloat16 and kv_norm.dtype == torch.bfloat16
-    assert q_norm.is_contiguous() and kv_norm.is_contiguous()
-    assert freqs.dtype == torch.complex64 and freqs.is_contiguous() and freqs.shape == (s, r // 2)
-    for t in (kv_cache, pe_cache):
-        assert t.dim() == 3 and t.dtype == torch.bfloat16 and t.stride(2) == 1 and t.stride(1) == t.size(2)
-        assert t.size(0) >= b and t.size(1) >= start + s and start >= 0
-    y, ys = _mla_latent_meta(a, q_norm, kv_norm, freqs, kv_cache, pe_cache, start, q_eps, kv_eps)
-    with torch.cuda.device(a.device):
-        rc = _lib.lib.dsv3_mla_latent(a.data_ptr(), width, q_norm.data_ptr(), kv_norm.data_ptr(), freqs.data_ptr(),
-                                      kv_cache.data_ptr() + start * c * 2, kv_cache.stride(0),
-                                      pe_cache.data_ptr() + start * r * 2, pe_cache.stride(0), y.data_ptr(), ys.data_ptr(),
-                                      b, s, q_norm.numel(), c, r, q_eps, kv_eps, _stream(a))
-    _lib.check(rc, "dsv3_mla_latent")
-    return y, ys
-
-
 def _mla_latent_meta(a, q_norm, kv_norm, freqs, kv_cache, pe_cache, start, q_eps, kv_eps):
     b, s, _ = a.shape
     return (a.new_empty(b, s, q_norm.numel(), dtype=FP8), a.new_empty(b, s, q_norm.numel() // 128, dtype=torch.float32))
 
 
+torch.ops.load_library(str(_lib.TORCH_LIB_PATH))       # the device implementations of csrc/torch_ops.cpp
+
 _libimpl = torch.library.Library("dsv3fp8", "IMPL")
-for _name, _dev, _meta in (("mla_prefill", _mla_prefill_dev, _mla_prefill_meta),
-                           ("mla_decode", _mla_decode_dev, _mla_decode_meta),
-                           ("mla_latent", _mla_latent_dev, _mla_latent_meta),
-                           ("wkv_b_absorb", _wkv_b_absorb_dev, _wkv_b_absorb_meta),
-                           ("linear_fp8", _linear_fp8_dev, _linear_fp8_meta),
-                           ("gate_route", _gate_route_dev, _gate_route_meta),
-                           ("group_tiles", _group_tiles_dev, _group_tiles_meta),
-                           ("moe_route", _moe_route_dev, _moe_route_meta),
-                           ("fp8_gemm_grouped", _fp8_gemm_grouped_dev, _fp8_gemm_grouped_meta),
-                           ("fp8_gemm_grouped_pow2", _fp8_gemm_grouped_pow2_dev, _fp8_gemm_grouped_meta),
-                           ("fp8_gemm_grouped_swiglu", _fp8_gemm_grouped_swiglu_dev, _fp8_gemm_grouped_swiglu_meta),
-                           ("swiglu_quant", _swiglu_quant_dev, _swiglu_quant_meta),
-                           ("moe_combine", _moe_combine_dev, _moe_combine_meta)):
+for _name, _dev in (("wkv_b_absorb", _wkv_b_absorb_dev), ("gate_route", _gate_route_dev), ("group_tiles", _group_tiles_dev),
+                    ("moe_route", _moe_route_dev), ("fp8_gemm_grouped", _fp8_gemm_grouped_dev),
+                    ("fp8_gemm_grouped_pow2", _fp8_gemm_grouped_pow2_dev),
+                    ("fp8_gemm_grouped_swiglu", _fp8_gemm_grouped_swiglu_dev), ("moe_combine", _moe_combine_dev)):
     _libimpl.impl(_name, _dev, "CUDA")
+for _name, _meta in (("act_quant", _act_quant_meta), ("weight_dequant", _weight_dequant_meta),
+                     ("weight_quant", _weight_quant_meta), ("fp8_gemm", _fp8_gemm_meta), ("fp8_gemm_pow2", _fp8_gemm_meta),
+                     ("linear_fp8", _linear_fp8_meta), ("swiglu_quant", _swiglu_quant_meta),
+                     ("mla_prefill", _mla_prefill_meta), ("mla_decode", _mla_decode_meta), ("mla_latent", _mla_latent_meta),
+                     ("wkv_b_absorb", _wkv_b_absorb_meta), ("gate_route", _gate_route_meta),
+                     ("group_tiles", _group_tiles_meta), ("moe_route", _moe_route_meta),
+                     ("fp8_gemm_grouped", _fp8_gemm_grouped_meta), ("fp8_gemm_grouped_pow2", _fp8_gemm_grouped_meta),
+                     ("fp8_gemm_grouped_swiglu", _fp8_gemm_grouped_swiglu_meta), ("moe_combine", _moe_combine_meta)):
     _libimpl.impl(_name, _meta, "Meta")
-_libimpl.impl("act_quant", _act_quant_dev, "CUDA")
-_libimpl.impl("weight_dequant", _weight_dequant_dev, "CUDA")
-_libimpl.impl("weight_quant", _weight_quant_dev, "CUDA")
-_libimpl.impl("fp8_gemm", _fp8_gemm_dev, "CUDA")
-_libimpl.impl("fp8_gemm_pow2", _fp8_gemm_pow2_dev, "CUDA")
-_libimpl.impl("act_quant", _act_quant_meta, "Meta")
-_libimpl.impl("weight_dequant", _weight_dequant_meta, "Meta")
-_libimpl.impl("weight_quant", _weight_quant_meta, "Meta")
-_libimpl.impl("fp8_gemm", _fp8_gemm_meta, "Meta")
-_libimpl.impl("fp8_gemm_pow2", _fp8_gemm_meta, "Meta")
