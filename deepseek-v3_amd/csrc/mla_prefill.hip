@@ -12,9 +12,9 @@
 //
 // Three launches: expand (keys and values, and the rotary keys, in the order in which the attention kernel's wavefronts
 // read their operands), flags (which tiles of the mask are all zero or all -inf; only with a mask), attend.
-// At 4096 tokens, 128 heads, causal mask: expand 226 us, flags 23 us, attend 915 us (0.75 PFLOP/s of the pairs the mask
-// leaves); the whole layer 1.77 ms where the absorbed form as tensor operations took 20.2 ms (2 x 2.5 ms score products,
-// 1.6 ms value product and 12 ms of passes over the 4.3 GB score matrix).
+// At 4096 tokens, 128 heads, causal mask: expand 148 us, flags 11 us, attend 850 .. 910 us (0.76 .. 0.81 PFLOP/s of the pairs
+// the mask leaves; the clock falls to 1.8 GHz under it); the layer 1.65 ms where the absorbed form as tensor operations took
+// 20.2 ms (2 x 2.5 ms score products, 1.6 ms value product and 12 ms of passes over the 4.3 GB score matrix).
 #include <type_traits>
 
 #include "mla.hpp"
@@ -49,8 +49,8 @@ struct ExpandArgs {
 // operand order and a store instruction writes 1 KiB of consecutive bytes: MFMA row 8j + 4g + r of a key wavefront is
 // feature 16 (j / 2) + 8 g + 4 (j % 2) + r; a value lane's accumulator registers 8u .. 8u + 7 are, in order, the
 // eight positions that the attention kernel's K step u has in that lane.
-// Bound by the LDS reads of the latents (every wavefront reads the whole sub-tile: 1 KiB per 32-cycle MFMA and SIMD pair,
-// ~0.6 of what the LDS delivers) and the 268 MB of results at 4096 positions.
+// Measured at 4096 positions, 128 heads: 219 us with each LDS read next to its MFMA, 140 .. 148 with six on their way (0.95
+// PFLOP/s; MFMAs 53 % of the cycles, the 268 MB of results alone would take 57 us).
 __global__ __launch_bounds__(512, 2) void mla_expand_kernel(ExpandArgs p) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * 32 * 1024];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -151,21 +151,37 @@ enum : uint8_t { kClear = 0, kMixed = 1, kSkip = 2 };
 
 // flags[q / 256][tile][q / 32 % 8]: what the mask does to 32 query rows x 64 positions (all zero, anything, all -inf or no
 // row).  An attend workgroup's eight flags of a tile are one 64-bit word, its tiles follow one another.
+// A wavefront looks at one such block and requests all of it before it looks at any: 16 bytes per lane where rows are whole
+// 16-byte pieces (`wide`) and the block has all its rows and positions, else one element per lane and row.
 template <bool F32>
-__global__ __launch_bounds__(512) void mla_mask_flags_kernel(const void* mask, uint8_t* flags, int rows, int positions) {
-    const int lane = threadIdx.x & 63, q32 = blockIdx.y * 8 + (threadIdx.x >> 6);
-    const int pos = blockIdx.x * kTile + lane;
+__global__ __launch_bounds__(512) void mla_mask_flags_kernel(const void* mask, uint8_t* flags, int rows, int positions, int wide) {
+    const int lane = threadIdx.x & 63, q32 = blockIdx.y * 8 + (threadIdx.x >> 6), p0 = blockIdx.x * kTile;
     bool zero = true, ninf = true;
-    if (pos < positions)
-#pragma unroll 8
-        for (int r = 0; r < 32; ++r) {
-            const int q = q32 * 32 + r;
-            if (q < rows) {
-                const float v = mask_at<F32>(mask, (int64_t)q * positions + pos);
-                zero = zero && v == 0.f;
-                ninf = ninf && v == -__builtin_inff();
+    if (wide && q32 * 32 + 32 <= rows && p0 + kTile <= positions) {
+        constexpr int kPer = F32 ? 4 : 8, kChunks = kTile / kPer, kRowsAt = 64 / kChunks, kLoads = 32 / kRowsAt;
+        constexpr int kSize = F32 ? 4 : 2;
+        const uint8_t* src = (const uint8_t*)mask + ((int64_t)(q32 * 32 + lane / kChunks) * positions + p0 + lane % kChunks * kPer) * kSize;
+        v4u v[kLoads];
+#pragma unroll
+        for (int n = 0; n < kLoads; ++n) v[n] = *(const v4u*)(src + (int64_t)n * kRowsAt * positions * kSize);
+#pragma unroll
+        for (int n = 0; n < kLoads; ++n)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                zero = zero && (v[n][e] & (F32 ? 0x7fffffffu : 0x7fff7fffu)) == 0u;
+                ninf = ninf && v[n][e] == (F32 ? 0xff800000u : 0xff80ff80u);
             }
-        }
+    } else if (p0 + lane < positions) {
+        float v[32];
+#pragma unroll
+        for (int r = 0; r < 32; ++r) v[r] = mask_at<F32>(mask, (int64_t)min(q32 * 32 + r, rows - 1) * positions + p0 + lane);
+#pragma unroll
+        for (int r = 0; r < 32; ++r)
+            if (q32 * 32 + r < rows) {
+                zero = zero && v[r] == 0.f;
+                ninf = ninf && v[r] == -__builtin_inff();
+            }
+    }
     const uint8_t f = __all(ninf) ? kSkip : __all(zero) ? kClear : kMixed;
     if (lane == 0) flags[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 8 + (threadIdx.x >> 6)] = f;
 }
@@ -178,20 +194,22 @@ struct AttendArgs {
     const uint8_t* img; const uint8_t* rope;
     const void* mask; const uint64_t* flags;    // [rows][positions] / [qtiles][tiles], or null
     uint8_t* y; float* ys;                      // fp8 [batch][rows][heads * 128], scales [batch][rows][heads]
-    int batch, heads, rows, positions, tiles, qtiles;
+    int batch, heads, rows, positions, tiles, qtiles, per_head;     // per_head: workgroups of a head
     float scale, inv_scale;                     // softmax scale and its reciprocal
 };
 
 // One workgroup: 256 query rows of one head; wavefront w rows 32 w .. 32 w + 31.  Per tile of 64 positions (40 KiB of
-// operands, double-buffered in LDS, copied while the tile before is computed) a wavefront forms S^T = K Q^T (24 MFMAs),
+// operands, copied into LDS while the tile before is computed) a wavefront forms S^T = K Q^T (24 MFMAs),
 // exponentials in registers, and O^T += V^T P^T (16 MFMAs).  The transposed products leave a query row in one lane
 // (and the lane 32 further), so maxima and sums need one exchange, the rescale factor is one value per lane, and the
 // accumulator layout of S^T already is the B operand of the second product: position 16 u + 8 a + 4 g + r of a tile sits
 // in register 8 u' + 4 a + r of lane half g, which is slot 4 a + r of K step u, and the values were written in that
 // order.  The running maximum is only raised when it grows by more than 2^8 (exponentials then stay below 2^8, and most
 // tiles skip the 64 multiplications of the rescale).
-// Wavefronts 4-7 run at raised priority: each SIMD holds one wavefront of either group, the two would otherwise do
-// their MFMAs at the same time and their exponentials at the same time.
+// Each SIMD holds one wavefront of either group 0-3 / 4-7.  The first group passes the barrier of tile k (its copies have
+// landed, the copies of the next tile may start) in front of its score product, the second one right behind its score
+// product of tile k - 1: one does matrix products while the other does exponentials.  That takes a third stage.  The
+// second group runs at raised priority.
 template <bool MF32>
 __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
@@ -201,9 +219,17 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
     // heads are dealt over the XCDs (whose L2 then holds a head's keys and values for all its query tiles), the query
     // tiles of a head run last to first: with a causal mask the long ones start first
     const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int bh = xcd + 8 * (idx / p.qtiles), qt = p.qtiles - 1 - idx % p.qtiles;
+    const int bh = xcd + 8 * (idx / p.per_head), part = idx % p.per_head;
     if (bh >= p.batch * p.heads) return;
     const int b = bh / p.heads, h = bh - b * p.heads;
+    const bool late = wave >= 4;
+    const uint8_t* himg = p.img + (int64_t)bh * p.tiles * kHeadTile;
+    const uint8_t* rimg = p.rope + (int64_t)b * p.tiles * kRopeBytes;
+    const uint32_t lds0 = lds_addr_of(lds), lane16 = lane * 16;
+    const float scale2 = p.scale * 1.44269504088896340736f;
+
+#pragma unroll 1
+    for (int qt = p.qtiles - 1 - part;;) {
     const int q0 = qt * kQTile + wave * 32;
     const int row = min(q0 + i, p.rows - 1);
 
@@ -224,9 +250,6 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
             }
     }
 
-    const uint8_t* himg = p.img + (int64_t)bh * p.tiles * kHeadTile;
-    const uint8_t* rimg = p.rope + (int64_t)b * p.tiles * kRopeBytes;
-    const uint32_t lds0 = lds_addr_of(lds), lane16 = lane * 16;
     auto issue = [&](int t, int st) {
         const uint8_t* src = himg + (int64_t)t * kHeadTile;
 #pragma unroll
@@ -261,26 +284,31 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
 
     v16f O[4] = {};
     float m = -__builtin_inff(), l = 0.f;           // running maximum (raw scores), this lane's share of the sum
-    const float scale2 = p.scale * 1.44269504088896340736f;
     look();
-    uint8_t flag = kSkip, flag_next = kSkip;
+    uint8_t flag = kSkip, flag_n = kSkip, flag_nn = kSkip;      // of this tile and the next two
     int t = next_tile(0, flag), st = 0;
+    int tn = t < p.tiles ? next_tile(t + 1, flag_n) : p.tiles;
     if (t < p.tiles) issue(t, 0);
-    if (wave >= 4) __builtin_amdgcn_s_setprio(1);
+    bool first = true;
+    if (late) __builtin_amdgcn_s_setprio(1);
     while (t < p.tiles) {
-        const int tn = next_tile(t + 1, flag_next);
-        __builtin_amdgcn_s_waitcnt(0x0f70);
-        barrier_no_fence();
-        if (tn < p.tiles) issue(tn, st ^ 1);
+        const int tnn = tn < p.tiles ? next_tile(tn + 1, flag_nn) : p.tiles;
+        const int s1 = st == 2 ? 0 : st + 1, s2 = st == 0 ? 2 : st - 1;
+        if (!late || first) {                           // barrier k: tile k has landed
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+            barrier_no_fence();
+            if (tn < p.tiles) issue(tn, s1);
+        }
+        first = false;
+        const uint8_t* base = lds + st * kStage + lane16;
+        v4u ring[kAhead];
+        v16f S[2] = {};
         if (flag != kSkip) {
-            const uint8_t* base = lds + st * kStage + lane16;
             // operands are read kAhead steps ahead; the barriers keep this order (left to itself the scheduler reads two ahead
             // and waits for most of them)
-            v4u ring[kAhead];
             auto key = [&](int n) -> v4u {              // step n: K step n / 2 of position half n & 1
                 return *(const v4u*)(base + (n < 16 ? (n & 1) * 8 + (n >> 1) : kHeadTile / 1024 + (n & 1) * 4 + (n >> 1) - 8) * 1024);
             };
-            v16f S[2] = {};
 #pragma unroll
             for (int n = 0; n < kAhead; ++n) ring[n] = key(n);
             __builtin_amdgcn_sched_barrier(0);
@@ -290,6 +318,13 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
                 if (n + kAhead < 24) ring[n % kAhead] = key(n + kAhead);
                 __builtin_amdgcn_sched_barrier(0);
             }
+        }
+        if (late && tn < p.tiles) {                     // barrier k + 1
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+            barrier_no_fence();
+            if (tnn < p.tiles) issue(tnn, s2);
+        }
+        if (flag != kSkip) {
             if (flag == kMixed) {
                 const int64_t mrow = (int64_t)row * p.positions;
 #pragma unroll
@@ -352,9 +387,9 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
             }
             l += sum;
         }
-        st ^= 1;
-        t = tn;
-        flag = flag_next;
+        st = s1;
+        t = tn; tn = tnn;
+        flag = flag_n; flag_n = flag_nn;
     }
     __builtin_amdgcn_s_setprio(0);
 
@@ -394,6 +429,12 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
             if (live) *(v2u*)(dst + 32 * d + 16 * a + 8 * g) = o;
         }
     if (live && g == 0) p.ys[out] = sc;
+
+    // the head's other query tile, if this workgroup has two
+    if (p.per_head == p.qtiles || qt <= part) return;
+    qt = part;
+    barrier_no_fence();                                 // everybody has read the last tiles
+    }
 }
 
 inline int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
@@ -409,7 +450,12 @@ int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t
                        const void* w, const float* ws, const void* mask, bool mask_f32, void* y, float* ys, int64_t batch,
                        int64_t rows, int64_t positions, int heads, float scale, void* workspace, hipStream_t st) {
     const int64_t tiles = (positions + kTile - 1) / kTile, qtiles = (rows + kQTile - 1) / kQTile;
-    const int64_t wgs = (batch * heads + 7) / 8 * 8 * qtiles;
+    // Two query tiles a workgroup, the j-th last and the j-th first, where that still makes a workgroup per compute unit:
+    // under a causal mask every workgroup then has the same work (4096 rows: 1024 equal ones, four per unit; with one tile
+    // each the units idled 19 % of the time behind the long tiles of the last heads).
+    const int64_t heads8 = (batch * heads + 7) / 8 * 8, pairs = (qtiles + 1) / 2;
+    const int64_t per_head = batch * heads * pairs >= 256 ? pairs : qtiles;
+    const int64_t wgs = heads8 * per_head;
     if (wgs > 0x7fffffff || batch * tiles * 2 > 0x7fffffff || qtiles > 65535) return DSV3_ERR_BAD_SHAPE;
     ExpandArgs e;
     e.kv = (const uint16_t*)kv; e.kv_bs = kv_bs; e.pe = (const uint16_t*)pe; e.pe_bs = pe_bs;
@@ -418,11 +464,11 @@ int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t
     e.rope = e.img + align256(batch * heads * tiles * kHeadTile);
     e.batch = (int)batch; e.heads = heads; e.positions = (int)positions; e.tiles = (int)tiles;
     uint8_t* flags = e.rope + align256(batch * tiles * kRopeBytes);
-    // two workgroups' worth of position ranges per compute unit at 128 heads; each wants a few sub-tiles behind its
-    // weight conversion
+    // one workgroup per compute unit: more ranges of positions would only convert the weights more often (4096 positions
+    // and 128 heads: 2 ranges, against 4 ranges in two rounds)
     const int64_t subs = batch * tiles * 2;
-    int64_t gy = (512 + heads - 1) / heads;
-    gy = gy > (subs + 3) / 4 ? (subs + 3) / 4 : gy;
+    int64_t gy = heads < 256 ? 256 / heads : 1;
+    gy = gy > subs ? subs : gy;
     hipLaunchKernelGGL(mla_expand_kernel, dim3(heads + 1, (unsigned)gy), dim3(512), 0, st, e);
 
     AttendArgs a;
@@ -430,14 +476,15 @@ int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t
     a.mask = mask; a.flags = mask ? (const uint64_t*)flags : nullptr;
     a.y = (uint8_t*)y; a.ys = ys;
     a.batch = (int)batch; a.heads = heads; a.rows = (int)rows; a.positions = (int)positions;
-    a.tiles = (int)tiles; a.qtiles = (int)qtiles;
+    a.tiles = (int)tiles; a.qtiles = (int)qtiles; a.per_head = (int)per_head;
     a.scale = scale; a.inv_scale = 1.0f / scale;
     if (mask) {
         const dim3 grid((unsigned)tiles, (unsigned)qtiles);
-        if (mask_f32) hipLaunchKernelGGL(mla_mask_flags_kernel<true>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions);
-        else hipLaunchKernelGGL(mla_mask_flags_kernel<false>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions);
+        const int wide = (uintptr_t)mask % 16 == 0 && positions * (mask_f32 ? 4 : 2) % 16 == 0;
+        if (mask_f32) hipLaunchKernelGGL(mla_mask_flags_kernel<true>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions, wide);
+        else hipLaunchKernelGGL(mla_mask_flags_kernel<false>, grid, dim3(512), 0, st, mask, flags, (int)rows, (int)positions, wide);
     }
-    constexpr int bytes = 2 * (kHeadTile + kRopeBytes);
+    constexpr int bytes = 3 * (kHeadTile + kRopeBytes);
     static LdsGrant grant[2];
     if (mask && mask_f32) {
         if (!grant[1].ensure((const void*)mla_attend_kernel<true>, bytes)) return DSV3_ERR_LAUNCH;

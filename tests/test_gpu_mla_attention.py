@@ -75,7 +75,8 @@ def _reference(q, freqs, kv, pe, w8, ws, mask, t, scale):
 PREFILL = [(1, 32, 32, 1, "causal"), (1, 33, 63, 3, None), (2, 64, 64, 8, "causal"), (1, 65, 65, 9, "causal"),
            (1, 255, 255, 2, "causal_f32"), (2, 257, 257, 3, "causal"), (1, 40, 500, 4, "causal"), (1, 1, 1, 2, None),
            (2, 100, 163, 4, "holes"), (1, 1100, 1100, 2, "causal"),
-           (1, 70, 130, 2, "lowest"), (1, 70, 130, 2, "lowest_f32")]
+           (1, 70, 130, 2, "lowest"), (1, 70, 130, 2, "lowest_f32"), (1, 256, 320, 2, "causal_f32"),
+           (1, 600, 600, 128, "causal"), (1, 4200, 4200, 16, "causal")]     # two query tiles a workgroup; 66 tiles of flags
 
 
 # tiles of 32 positions, workgroups of 128 (token, head) rows, wavefronts of 32; one split and many, uneven last ones, more
