@@ -14,6 +14,7 @@ variants reduce to plain ``Linear`` and no collective is issued.
 from __future__ import annotations
 
 import math
+import operator
 from dataclasses import dataclass
 from typing import Literal, Optional, Tuple
 
@@ -215,6 +216,11 @@ def _plain(module: nn.Module, cls: type) -> bool:
     return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks)
 
 
+def _offset_aligned(t: torch.Tensor) -> bool:
+    """Whether a tensor starts at a multiple of 16 bytes of its storage, as the kernels' 16-byte accesses need."""
+    return t.storage_offset() * t.element_size() % 16 == 0
+
+
 class MLA(nn.Module):
     """Host of the two ``wkv_b`` products of the absorbed multi-head latent attention (model.py:395-497).
 
@@ -334,8 +340,9 @@ class MLA(nn.Module):
                 and self.kv_cache.dtype == torch.bfloat16 and self.kv_cache.is_contiguous() and self.pe_cache.is_contiguous()
                 and 1 <= b <= self.kv_cache.size(0) and s >= 1 and start_pos >= 0 and start_pos + s <= self.kv_cache.size(1)
                 and self.wkv_b.weight.element_size() == 1 and self.wkv_b.bias is None
+                and all(map(_offset_aligned, (self.kv_cache, self.pe_cache, self.wkv_b.weight)))
                 and freqs_cis.is_cuda and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous()
-                and freqs_cis.shape == (s, self.qk_rope_head_dim // 2))
+                and not freqs_cis.is_conj() and freqs_cis.shape == (s, self.qk_rope_head_dim // 2))
 
     def _latent_kernel_ok(self) -> bool:
         """Whether both norms, the cache rows and the quantisation in front of ``wq_b`` can be one launch; modules that
@@ -343,6 +350,7 @@ class MLA(nn.Module):
         return (self.q_lora_rank % block_size == 0 and 0 < self.q_lora_rank <= 2048 and self.stacked_a
                 and _plain(self.q_norm, RMSNorm) and _plain(self.kv_norm, RMSNorm) and _plain(self.wq_b, ColumnParallelLinear)
                 and self.q_norm.weight.dtype == torch.bfloat16 and self.kv_norm.weight.dtype == torch.bfloat16
+                and _offset_aligned(self.q_norm.weight) and _offset_aligned(self.kv_norm.weight)
                 and self.wq_b.weight.element_size() == 1 and self.wq_b.bias is None and self.stack_a())
 
     def _attention_kernels_ok(self, q, positions: int, mask) -> bool:
@@ -354,6 +362,7 @@ class MLA(nn.Module):
 
     def forward(self, x: torch.Tensor, start_pos: int, freqs_cis: torch.Tensor, mask: Optional[torch.Tensor]):
         b, s = x.size(0), x.size(1)
+        start_pos = operator.index(start_pos)
         t = start_pos + s
         kernels = self._kernels_ok(x, start_pos, freqs_cis)
         if kernels and self._latent_kernel_ok():
