@@ -95,10 +95,11 @@ tuple<Tensor, Tensor> weight_quant(const Tensor& w, int64_t block, int64_t fmt) 
 Tensor gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, int64_t out, decltype(dsv3_fp8_gemm)* entry,
             const char* what) {
     const int64_t k = a.size(-1), m = k ? a.numel() / k : 0, n = b.size(0);
-    Tensor c = with_last(a, n, dtype_of(out));
     On on(a);
+    const at::ScalarType dtype = dtype_of(out);
     const size_t need = dsv3_fp8_gemm_workspace_bytes(m, n, k);
-    Tensor ws = need ? scratch(a, need) : Tensor();
+    Tensor ws = need ? scratch(a, need) : Tensor();     // before the result, which would be cut out of the last call's scratch
+    Tensor c = with_last(a, n, dtype);
     check(entry(a.data_ptr(), (const float*)a_s.data_ptr(), b.data_ptr(), (const float*)b_s.data_ptr(), c.data_ptr(), (int)out,
                 m, n, k, need ? ws.data_ptr() : nullptr, need, on.stream), what);
     return c;
@@ -117,10 +118,11 @@ Tensor linear_fp8(const Tensor& x, const Tensor& b, const Tensor& b_s, int64_t f
         auto [a, a_s] = act_quant(x, 128, fmt);
         return fp8_gemm(a, a_s, b, b_s, out);
     }
-    Tensor c = with_last(x, n, dtype_of(out));
     On on(x);
+    const at::ScalarType dtype = dtype_of(out);
     const size_t need = dsv3_fp8_gemm_workspace_bytes(m, n, k);
     Tensor ws = need ? scratch(x, need) : Tensor();
+    Tensor c = with_last(x, n, dtype);
     check(dsv3_linear_fp8(x.data_ptr(), DSV3_BF16, b.data_ptr(), (const float*)b_s.data_ptr(), c.data_ptr(), (int)out, m, n, k,
                           128, (int)fmt, need ? ws.data_ptr() : nullptr, need, on.stream), "dsv3_linear_fp8");
     return c;

@@ -223,3 +223,31 @@ def test_layer_prefill_vs_oracle(M):
     layer.requires_grad_(False)
     z0 = layer(x0.cuda(), 0, freqs[:s].cuda(), mask.cuda())
     assert _rel(z0, ref0) <= LAYER_TOL and _rel(y0, z0.cpu()) <= LAYER_TOL
+
+
+def test_decode_step_in_a_captured_graph(M):
+    """A captured decode step, replayed on new inputs with eager steps in between, gives the eager step's bits."""
+    dim, heads, q_rank, t = 256, 4, 128, 40
+    layer = _layer(M, small_mla_params(dim, heads, q_rank, C, NOPE, ROPE, V, 31), dim, heads, q_rank, 96)
+    freqs = _freqs(ROPE, 96)[t:t + 1].cuda()
+    g = torch.Generator().manual_seed(33)
+    with torch.inference_mode():
+        layer.kv_cache.copy_(torch.randn(layer.kv_cache.shape, generator=g))
+        layer.pe_cache.copy_(torch.randn(layer.pe_cache.shape, generator=g))
+        x = torch.randn(2, 1, dim, generator=g).bfloat16().cuda()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            layer(x, t, freqs, None)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = layer(x, t, freqs, None)
+        for _ in range(3):
+            new = torch.randn(2, 1, dim, generator=g).bfloat16().cuda()
+            ref = layer(new, t, freqs, None).clone()
+            torch.cuda.synchronize()
+            x.copy_(new)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, ref)
