@@ -11,6 +11,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
+#include <initializer_list>
 #include <tuple>
 
 #include "../../include/dsv3_fp8.h"
@@ -50,6 +51,14 @@ struct On {
     explicit On(const Tensor& t) : guard(t.device()), stream((void*)c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
 };
 
+// The kernels get raw pointers: a tensor of another device or of the host would fault the GPU.  (The dispatcher comes here as
+// soon as one argument is on the GPU.)
+void on_one_gpu(const char* what, const Tensor& x, std::initializer_list<const Tensor*> others) {
+    for (const Tensor* t : others)
+        TORCH_CHECK(t->device() == x.device(), what, ": all tensors must be on one device, got ", x.device(), " and ", t->device());
+    TORCH_CHECK(x.is_cuda(), what, ": tensors must be on the GPU, got ", x.device());
+}
+
 Tensor scratch(const Tensor& like, size_t bytes) {
     return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
 }
@@ -72,6 +81,7 @@ tuple<Tensor, Tensor> act_quant(const Tensor& x, int64_t block, int64_t fmt) {
 
 Tensor weight_dequant(const Tensor& x, const Tensor& s, int64_t block, int64_t out) {
     TORCH_CHECK_VALUE(x.dim() == 2, "weight_dequant: a matrix is needed");
+    on_one_gpu("weight_dequant", x, { &s });
     Tensor y = at::empty_like(x, x.options().dtype(dtype_of(out)));
     On on(x);
     check(dsv3_weight_dequant(x.data_ptr(), (const float*)s.data_ptr(), y.data_ptr(), (int)out, x.size(0), x.size(1), (int)block,
@@ -95,6 +105,7 @@ tuple<Tensor, Tensor> weight_quant(const Tensor& w, int64_t block, int64_t fmt) 
 Tensor gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, int64_t out, decltype(dsv3_fp8_gemm)* entry,
             const char* what) {
     const int64_t k = a.size(-1), m = k ? a.numel() / k : 0, n = b.size(0);
+    on_one_gpu(what, a, { &a_s, &b, &b_s });
     On on(a);
     const at::ScalarType dtype = dtype_of(out);
     const size_t need = dsv3_fp8_gemm_workspace_bytes(m, n, k);
@@ -114,6 +125,7 @@ Tensor fp8_gemm_pow2(const Tensor& a, const Tensor& a_s, const Tensor& b, const 
 // act_quant(x, 128, fmt) followed by fp8_gemm, one launch where the library implements it, else two calls
 Tensor linear_fp8(const Tensor& x, const Tensor& b, const Tensor& b_s, int64_t fmt, int64_t out) {
     const int64_t k = x.size(-1), m = k ? x.numel() / k : 0, n = b.size(0);
+    on_one_gpu("linear_fp8", x, { &b, &b_s });
     if (x.scalar_type() != at::kBFloat16 || !dsv3_linear_fp8_fused(m, n, k)) {
         auto [a, a_s] = act_quant(x, 128, fmt);
         return fp8_gemm(a, a_s, b, b_s, out);
@@ -146,8 +158,8 @@ void check_caches(const Tensor& kv, const Tensor& pe, int64_t batch, int64_t pos
                     c->size(0) >= batch && c->size(1) >= positions, "mla: caches must be bf16 [batch, positions, width] with dense rows");
 }
 void check_freqs(const Tensor& f, int64_t rows, int64_t rope) {
-    TORCH_CHECK(f.scalar_type() == at::kComplexFloat && f.is_contiguous() && f.dim() == 2 && f.size(0) == rows && f.size(1) == rope / 2,
-                "mla: freqs must be a contiguous complex64 [rows, rope / 2]");
+    TORCH_CHECK(f.scalar_type() == at::kComplexFloat && f.is_contiguous() && f.dim() == 2 && f.size(0) == rows && f.size(1) == rope / 2 &&
+                !f.is_conj() && !f.is_neg(), "mla: freqs must be a contiguous complex64 [rows, rope / 2], not lazily conjugated");
 }
 
 // What the two attention operators check and pass on alike; `call` gets the shape and the workspace.
@@ -160,10 +172,13 @@ void attention(const Tensor& q, const Tensor& freqs, const Tensor& kv, const Ten
     check_freqs(freqs, s, pe.size(2));
     TORCH_CHECK(w.dim() == 2 && w.is_contiguous() && ws.is_contiguous() && w.element_size() == 1 && w.size(1) == kv.size(2) &&
                 h > 0 && w.size(0) % h == 0, "mla: wkv_b must be a contiguous fp8 [h * (nope + v), kv_rank]");
+    TORCH_CHECK(ws.scalar_type() == at::kFloat && ws.dim() == 2 && ws.size(0) >= (w.size(0) + 127) / 128 && ws.size(1) == (w.size(1) + 127) / 128,
+                "mla: wkv_b's scales must be fp32, one per block of 128 x 128");
     if (mask)
         TORCH_CHECK(mask->dim() == 2 && mask->size(0) == s && mask->size(1) == positions && mask->is_contiguous() &&
                     (mask->scalar_type() == at::kBFloat16 || mask->scalar_type() == at::kFloat),
                     "mla: mask must be a contiguous bf16 or fp32 [s, positions]");
+    on_one_gpu("mla", q, { &freqs, &kv, &pe, &w, &ws, mask ? &*mask : &q });
     On on(q);
     const size_t need = bytes(b, s, positions, (int)h);
     Tensor buf = scratch(q, need);
@@ -204,11 +219,13 @@ tuple<Tensor, Tensor> mla_latent(const Tensor& a, const Tensor& qn, const Tensor
                                  int64_t start, double q_eps, double kv_eps) {
     TORCH_CHECK(a.dim() == 3 && a.is_contiguous() && a.scalar_type() == at::kBFloat16 && start >= 0, "mla_latent: a must be a contiguous bf16 [b, s, width]");
     const int64_t b = a.size(0), s = a.size(1), qr = qn.numel();
+    TORCH_CHECK(kv.dim() == 3 && start <= kv.size(1), "mla_latent: start lies behind the caches' end");     // start + s cannot overflow
     check_caches(kv, pe, b, start + s);
     check_freqs(freqs, s, pe.size(2));
     const int64_t c = kv.size(2), r = pe.size(2);
     TORCH_CHECK(a.size(2) == qr + c + r && kn.numel() == c && qn.scalar_type() == at::kBFloat16 && kn.scalar_type() == at::kBFloat16 &&
                 qn.is_contiguous() && kn.is_contiguous(), "mla_latent: norm weights do not fit the row");
+    on_one_gpu("mla_latent", a, { &qn, &kn, &freqs, &kv, &pe });
     Tensor y = at::empty({b, s, qr}, a.options().dtype(kFp8)), ys = at::empty({b, s, qr / 128}, a.options().dtype(at::kFloat));
     On on(a);
     check(dsv3_mla_latent(a.data_ptr(), a.size(2), qn.data_ptr(), kn.data_ptr(), (const float*)freqs.data_ptr(),

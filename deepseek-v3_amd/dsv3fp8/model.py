@@ -337,19 +337,22 @@ class MLA(nn.Module):
                 and x.is_cuda and x.dtype == torch.bfloat16 and torch.get_default_dtype() == torch.bfloat16
                 and self.attn_impl == "absorb"
                 and (self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim, self.kv_lora_rank) == (128, 64, 128, 512)
-                and self.kv_cache.dtype == torch.bfloat16 and self.kv_cache.is_contiguous() and self.pe_cache.is_contiguous()
+                and self.kv_cache.dtype == self.pe_cache.dtype == torch.bfloat16
+                and self.kv_cache.is_contiguous() and self.pe_cache.is_contiguous()
+                and self.kv_cache.device == self.pe_cache.device == freqs_cis.device == x.device
                 and 1 <= b <= self.kv_cache.size(0) and s >= 1 and start_pos >= 0 and start_pos + s <= self.kv_cache.size(1)
                 and self.wkv_b.weight.element_size() == 1 and self.wkv_b.bias is None
                 and all(map(_offset_aligned, (self.kv_cache, self.pe_cache, self.wkv_b.weight)))
-                and freqs_cis.is_cuda and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous()
+                and self.wkv_b.weight.device == x.device and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous()
                 and not freqs_cis.is_conj() and freqs_cis.shape == (s, self.qk_rope_head_dim // 2))
 
-    def _latent_kernel_ok(self) -> bool:
+    def _latent_kernel_ok(self, x) -> bool:
         """Whether both norms, the cache rows and the quantisation in front of ``wq_b`` can be one launch; modules that
         were exchanged or carry hooks are called as such."""
         return (self.q_lora_rank % block_size == 0 and 0 < self.q_lora_rank <= 2048 and self.stacked_a
                 and _plain(self.q_norm, RMSNorm) and _plain(self.kv_norm, RMSNorm) and _plain(self.wq_b, ColumnParallelLinear)
                 and self.q_norm.weight.dtype == torch.bfloat16 and self.kv_norm.weight.dtype == torch.bfloat16
+                and self.q_norm.weight.device == self.kv_norm.weight.device == x.device
                 and _offset_aligned(self.q_norm.weight) and _offset_aligned(self.kv_norm.weight)
                 and self.wq_b.weight.element_size() == 1 and self.wq_b.bias is None and self.stack_a())
 
@@ -357,7 +360,7 @@ class MLA(nn.Module):
         """Whether the attention behind the query projection can run on the fused kernels: a mask of one value per
         (query, position) pair as the reference builds it (model.py:738-740)."""
         return (q.dtype == torch.bfloat16 and q.is_contiguous()
-                and (mask is None or (mask.is_cuda and mask.shape == (q.size(1), positions) and mask.is_contiguous()
+                and (mask is None or (mask.device == q.device and mask.shape == (q.size(1), positions) and mask.is_contiguous()
                                       and mask.dtype in (torch.bfloat16, torch.float32))))
 
     def forward(self, x: torch.Tensor, start_pos: int, freqs_cis: torch.Tensor, mask: Optional[torch.Tensor]):
@@ -365,7 +368,7 @@ class MLA(nn.Module):
         start_pos = operator.index(start_pos)
         t = start_pos + s
         kernels = self._kernels_ok(x, start_pos, freqs_cis)
-        if kernels and self._latent_kernel_ok():
+        if kernels and self._latent_kernel_ok(x):
             qq, qs = torch.ops.dsv3fp8.mla_latent(linear(x, self._wa, None, self.wq_a.scale_fmt), self.q_norm.weight,
                                                   self.kv_norm.weight, freqs_cis, self.kv_cache, self.pe_cache, start_pos,
                                                   self.q_norm.eps, self.kv_norm.eps)

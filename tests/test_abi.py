@@ -335,3 +335,58 @@ def test_mla_latent_validation(L):
     for bad in ({"qr": 100}, {"qr": 2176}, {"qr": 0}, {"c": 256}, {"rope": 32}, {"stride": 2104}, {"b": -1}, {"kvs": 2040}):
         assert call(**bad) == 2, bad
     assert call(b=0, a=None) == 0 and call(rows=0, a=None) == 0
+
+
+# The native operator bodies, called on tensors of the host: they must say no before any pointer gets to a kernel (here a
+# body that does not look gets as far as asking for the GPU).
+def _gpu_body(name, *args):
+    from dsv3fp8 import ops  # noqa: F401  (registers torch.ops.dsv3fp8)
+    return getattr(torch.ops.dsv3fp8, name).default.redispatch(torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA), *args)
+
+
+def _operator_args(name):
+    z = torch.zeros
+    fp8, bf16 = torch.float8_e4m3fn, torch.bfloat16
+    if name == "weight_dequant":
+        return [z(128, 128, dtype=fp8), z(1, 1), 128, 0]
+    if name in ("fp8_gemm", "fp8_gemm_pow2"):
+        return [z(2, 128, dtype=fp8), z(2, 1), z(128, 128, dtype=fp8), z(1, 1), 0]
+    if name == "linear_fp8":
+        return [z(2, 128, dtype=bf16), z(128, 128, dtype=fp8), z(1, 1), 0, 0]
+    freqs, kv, pe = z(2, 32, dtype=torch.complex64), z(1, 8, 512, dtype=bf16), z(1, 8, 64, dtype=bf16)
+    if name == "mla_latent":
+        return [z(1, 2, 128 + 576, dtype=bf16), z(128, dtype=bf16), z(512, dtype=bf16), freqs, kv, pe, 3, 1e-6, 1e-6]
+    return [z(1, 2, 4, 192, dtype=bf16), freqs, kv, pe, z(1024, 512, dtype=fp8), z(8, 4), z(2, 8), 8, 0.1]
+
+
+OPERATORS = {"weight_dequant": (0, 1), "fp8_gemm": (0, 1, 2, 3), "fp8_gemm_pow2": (0, 1, 2, 3), "linear_fp8": (0, 1, 2),
+             "mla_prefill": range(7), "mla_decode": range(7), "mla_latent": range(6)}
+
+
+@pytest.mark.parametrize("name", OPERATORS)
+def test_operators_refuse_tensors_of_two_devices(name):
+    with pytest.raises(RuntimeError, match="on the GPU"):
+        _gpu_body(name, *_operator_args(name))
+    for at in OPERATORS[name]:
+        args = _operator_args(name)
+        args[at] = args[at].to("meta")
+        with pytest.raises(RuntimeError, match="one device"):
+            _gpu_body(name, *args)
+
+
+@pytest.mark.parametrize("name", ["mla_prefill", "mla_decode", "mla_latent"])
+def test_attention_operators_refuse_what_their_kernels_cannot_read(name):
+    f = 3 if name == "mla_latent" else 1                # where the phases stand
+    bad = {f: [lambda t: t.conj(), lambda t: t[:1]]}
+    if name == "mla_latent":
+        bad[6] = [lambda t: 7, lambda t: -1, lambda t: 2 ** 63 - 1]
+    else:                                               # scales: too few rows, columns, another type
+        bad[5] = [lambda t: t[:7], lambda t: t[:, :3].contiguous(), lambda t: t.bfloat16(), lambda t: t.flatten()]
+        bad[3] = [lambda t: t.float()]
+        bad[6] = [lambda t: t[:, :7], lambda t: t.half()]
+    for at, changes in bad.items():
+        for change in changes:
+            args = _operator_args(name)
+            args[at] = change(args[at])
+            with pytest.raises(RuntimeError, match="mla.*(must|behind)"):
+                _gpu_body(name, *args)

@@ -251,3 +251,18 @@ def test_decode_step_in_a_captured_graph(M):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, ref)
+
+
+def test_layer_with_parts_on_the_host_raises(M):
+    """A cache, a norm weight or the mask that stayed on the host is refused by the tensor operations; no kernel sees it."""
+    p = small_mla_params(256, 4, 128, C, NOPE, ROPE, V, 31)
+    freqs, x = _freqs(ROPE, 96)[:40].cuda(), torch.ones(2, 40, 256, dtype=torch.bfloat16, device="cuda")
+    mask = torch.full((40, 40), float("-inf")).triu_(1)
+    for part in ("kv_cache", "pe_cache", "q_norm", "mask"):
+        layer = _layer(M, p, 256, 4, 128, 96)
+        if part == "q_norm":
+            layer.q_norm.cpu()
+        elif part != "mask":
+            setattr(layer, part, getattr(layer, part).cpu())
+        with torch.inference_mode(), pytest.raises(RuntimeError, match="device"):
+            layer(x, 0, freqs, mask if part == "mask" else mask.cuda())
