@@ -283,13 +283,17 @@ class MLA(nn.Module):
 
     def stack_a(self) -> bool:
         """wq_a over wkv_a in one buffer (scales likewise); returns whether the layers qualify.  Idempotent; the
-        layers' parameters become views, so in-place weight loading keeps working."""
-        if getattr(self, "_wa", None) is not None:
-            return True
+        layers' parameters become views, so in-place weight loading keeps working.  Parameters that were replaced or
+        moved since (``load_state_dict(assign=True)``, ``.to(device)``) are stacked anew."""
         if self.q_lora_rank == 0 or self.q_lora_rank % block_size or self.wq_a.weight.element_size() != 1 \
                 or self.wkv_a.weight.element_size() != 1 or self.wq_a.scale_fmt != self.wkv_a.scale_fmt:
             return False
         qa, ka = self.wq_a, self.wkv_a
+        wa = getattr(self, "_wa", None)
+        if wa is not None and qa.weight.data_ptr() == wa.data_ptr() and ka.weight.data_ptr() == wa.data_ptr() + qa.weight.numel() \
+                and qa.scale.data_ptr() == wa.scale.data_ptr() \
+                and ka.scale.data_ptr() == wa.scale.data_ptr() + 4 * qa.scale.numel():
+            return True
         with torch.no_grad():
             w = torch.cat([qa.weight.data.view(torch.uint8), ka.weight.data.view(torch.uint8)]).view(qa.weight.dtype)
             sc = torch.cat([qa.scale.data, ka.scale.data])
