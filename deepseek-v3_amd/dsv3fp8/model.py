@@ -21,6 +21,7 @@ from typing import Literal, Optional, Tuple
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules import module as _modules
 
 from . import ops
 from .kernel import act_quant, fp8_gemm, fp8_gemm_pow2, weight_dequant
@@ -212,8 +213,10 @@ def apply_rotary_emb(x: torch.Tensor, freqs_cis: torch.Tensor) -> torch.Tensor:
 
 
 def _plain(module: nn.Module, cls: type) -> bool:
-    """Whether calling ``module`` does no more than ``cls.forward``, so that a fused kernel may take its place."""
-    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks)
+    """Whether calling ``module`` does no more than ``cls.forward``, so that a fused kernel may take its place: neither a
+    module of another type nor one with hooks (its own or those of all modules) or a ``forward`` of its own."""
+    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
+                                        or _modules._global_forward_hooks or _modules._global_forward_pre_hooks)
 
 
 def _offset_aligned(t: torch.Tensor) -> bool:
@@ -282,10 +285,13 @@ class MLA(nn.Module):
             self.register_buffer(name, torch.zeros(args.max_batch_size, args.max_seq_len, *width), persistent=False)
 
     def stack_a(self) -> bool:
-        """wq_a over wkv_a in one buffer (scales likewise); returns whether the layers qualify.  Idempotent; the
+        """wq_a over wkv_a in one buffer (scales likewise); returns whether the layers qualify (FP8 weights without a bias,
+        and nothing but ``Linear.forward`` behind a call of either: exchanged modules and hooks are called).  Idempotent; the
         layers' parameters become views, so in-place weight loading keeps working.  Parameters that were replaced or
         moved since (``load_state_dict(assign=True)``, ``.to(device)``) are stacked anew."""
-        if self.q_lora_rank == 0 or self.q_lora_rank % block_size or self.wq_a.weight.element_size() != 1 \
+        if self.q_lora_rank == 0 or self.q_lora_rank % block_size or not _plain(self.wq_a, Linear) \
+                or not _plain(self.wkv_a, Linear) or self.wq_a.bias is not None or self.wkv_a.bias is not None \
+                or self.wq_a.weight.element_size() != 1 \
                 or self.wkv_a.weight.element_size() != 1 or self.wq_a.scale_fmt != self.wkv_a.scale_fmt:
             return False
         qa, ka = self.wq_a, self.wkv_a
@@ -345,7 +351,7 @@ class MLA(nn.Module):
                 and self.kv_cache.is_contiguous() and self.pe_cache.is_contiguous()
                 and self.kv_cache.device == self.pe_cache.device == freqs_cis.device == x.device
                 and 1 <= b <= self.kv_cache.size(0) and s >= 1 and start_pos >= 0 and start_pos + s <= self.kv_cache.size(1)
-                and self.wkv_b.weight.element_size() == 1 and self.wkv_b.bias is None
+                and self.wkv_b.weight.element_size() == 1
                 and all(map(_offset_aligned, (self.kv_cache, self.pe_cache, self.wkv_b.weight)))
                 and self.wkv_b.weight.device == x.device and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous()
                 and not freqs_cis.is_conj() and freqs_cis.shape == (s, self.qk_rope_head_dim // 2))
@@ -388,7 +394,7 @@ class MLA(nn.Module):
             args = (q, freqs_cis, self.kv_cache, self.pe_cache, self.wkv_b.weight, self.wkv_b.scale, mask, t, self.softmax_scale)
             if s < self.explicit_min_tokens:
                 return self.wo(torch.ops.dsv3fp8.mla_decode(*args))
-            if self.wo.weight.element_size() == 1 and self.wo.bias is None and _plain(self.wo, RowParallelLinear):
+            if _plain(self.wo, RowParallelLinear) and self.wo.weight.element_size() == 1 and self.wo.bias is None:
                 return fp8_gemm(*torch.ops.dsv3fp8.mla_prefill(*args), self.wo.weight, self.wo.weight.scale)
         wkv_b = self._dequantised_wkv_b(x)
         latent, rope_keys = self.kv_cache[:b, :t], self.pe_cache[:b, :t]

@@ -266,3 +266,44 @@ def test_layer_with_parts_on_the_host_raises(M):
             setattr(layer, part, getattr(layer, part).cpu())
         with torch.inference_mode(), pytest.raises(RuntimeError, match="device"):
             layer(x, 0, freqs, mask if part == "mask" else mask.cuda())
+
+
+class _Wrapped(torch.nn.Module):
+    """A module put in a layer's place, with none of its attributes (an adapter, say)."""
+
+    def __init__(self, base):
+        super().__init__()
+        self.base, self.calls = [base], 0
+
+    def forward(self, x):
+        self.calls += 1
+        return self.base[0](x)
+
+
+@pytest.mark.parametrize("s", [1, 40])
+def test_exchanged_modules_and_hooks_are_called(M, s):
+    p = small_mla_params(256, 4, 128, C, NOPE, ROPE, V, 31)
+    freqs = _freqs(ROPE, 96)[:s].cuda()
+    x = torch.randn(2, s, 256, generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
+    mask = torch.full((s, s), float("-inf"), device="cuda").triu_(1)
+    with torch.inference_mode():
+        ref = _layer(M, p, 256, 4, 128, 96)(x, 0, freqs, mask)
+        for name in ("wq_a", "q_norm", "wq_b", "wkv_a", "kv_norm", "wo"):
+            for how in ("module", "hook", "forward"):
+                layer, seen = _layer(M, p, 256, 4, 128, 96), []
+                module = getattr(layer, name)
+                if how == "module":
+                    setattr(layer, name, _Wrapped(module))
+                elif how == "hook":
+                    module.register_forward_hook(lambda *a: seen.append(1))
+                else:
+                    module.forward = lambda x, f=module.forward: (seen.append(1), f(x))[1]
+                assert _rel(layer(x, 0, freqs, mask), ref.cpu()) <= LAYER_TOL
+                assert (getattr(layer, name).calls if how == "module" else len(seen)) == 1, (name, how)
+        seen = []
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *a: seen.append(type(m).__name__))
+        try:
+            _layer(M, p, 256, 4, 128, 96)(x, 0, freqs, mask)
+        finally:
+            handle.remove()
+        assert sorted(seen) == ["ColumnParallelLinear", "Linear", "Linear", "MLA", "RMSNorm", "RMSNorm", "RowParallelLinear"]

@@ -56,3 +56,30 @@ def test_replaced_parameters_are_stacked_anew(layer, name, what):
         lin.weight.data = lin.weight.data.clone()
         lin.scale.data = lin.scale.data.clone()
     _check(layer)
+
+
+@pytest.mark.parametrize("what", ["type", "hook", "pre_hook", "global_hook", "global_pre_hook", "forward"])
+def test_only_plain_modules_are_passed_by(layer, what):
+    from dsv3fp8 import model
+    from torch.nn.modules import module as modules
+    assert layer.stack_a() and model._plain(layer.wkv_a, model.Linear)
+    lin = layer.wkv_a
+    if what == "type":
+        lin.__class__ = type("Other", (model.Linear,), {})
+    elif what == "forward":
+        lin.forward = lambda x: x
+    else:
+        handle = {"hook": lin.register_forward_hook, "pre_hook": lin.register_forward_pre_hook,
+                  "global_hook": modules.register_module_forward_hook,
+                  "global_pre_hook": modules.register_module_forward_pre_hook}[what](lambda *a: None)
+    try:
+        assert not model._plain(lin, model.Linear) and not layer.stack_a()
+    finally:
+        if what.endswith("hook"):
+            handle.remove()
+    assert layer.stack_a() == what.endswith("hook")
+
+
+def test_layers_with_a_bias_are_not_stacked(layer):
+    layer.wq_a.bias = nn.Parameter(torch.ones(128))
+    assert not layer.stack_a()
