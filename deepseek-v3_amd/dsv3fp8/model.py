@@ -363,13 +363,16 @@ class MLA(nn.Module):
                 and _plain(self.q_norm, RMSNorm) and _plain(self.kv_norm, RMSNorm) and _plain(self.wq_b, ColumnParallelLinear)
                 and self.q_norm.weight.dtype == torch.bfloat16 and self.kv_norm.weight.dtype == torch.bfloat16
                 and self.q_norm.weight.device == self.kv_norm.weight.device == x.device
+                and self.q_norm.weight.is_contiguous() and self.kv_norm.weight.is_contiguous()
                 and _offset_aligned(self.q_norm.weight) and _offset_aligned(self.kv_norm.weight)
+                and isinstance(self.q_norm.eps, (int, float)) and isinstance(self.kv_norm.eps, (int, float))
                 and self.wq_b.weight.element_size() == 1 and self.wq_b.bias is None and self.stack_a())
 
     def _attention_kernels_ok(self, q, positions: int, mask) -> bool:
         """Whether the attention behind the query projection can run on the fused kernels: a mask of one value per
-        (query, position) pair as the reference builds it (model.py:738-740)."""
-        return (q.dtype == torch.bfloat16 and q.is_contiguous()
+        (query, position) pair as the reference builds it (model.py:738-740), a positive softmax scale (the kernels work
+        with maxima of unscaled scores) whose reciprocal binary32 holds."""
+        return (isinstance(self.softmax_scale, (int, float)) and 1e-30 < self.softmax_scale < 1e30 and q.dtype == torch.bfloat16 and q.is_contiguous()
                 and (mask is None or (mask.device == q.device and mask.shape == (q.size(1), positions) and mask.is_contiguous()
                                       and mask.dtype in (torch.bfloat16, torch.float32))))
 

@@ -307,3 +307,21 @@ def test_exchanged_modules_and_hooks_are_called(M, s):
         finally:
             handle.remove()
         assert sorted(seen) == ["ColumnParallelLinear", "Linear", "Linear", "MLA", "RMSNorm", "RMSNorm", "RowParallelLinear"]
+
+
+@pytest.mark.parametrize("what", ["scale", "eps", "strided"])
+def test_settings_that_the_kernels_do_not_take_still_run(M, what):
+    """A softmax scale below zero, a norm without an eps or with a strided weight: the layer's tensor operations."""
+    p = small_mla_params(256, 4, 128, C, NOPE, ROPE, V, 31)
+    freqs = _freqs(ROPE, 96)[:5].cuda()
+    x = torch.randn(2, 5, 256, generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
+    layer = _layer(M, p, 256, 4, 128, 96).requires_grad_(False)
+    if what == "scale":
+        layer.softmax_scale = -layer.softmax_scale
+    elif what == "eps":
+        layer.q_norm.eps = layer.kv_norm.eps = None
+    else:
+        layer.kv_norm.weight = torch.nn.Parameter(layer.kv_norm.weight.data.repeat_interleave(2)[::2], requires_grad=False)
+    with torch.inference_mode():
+        y = layer(x, 0, freqs, None)
+    assert torch.isfinite(y).all() and _rel(y, layer(x, 0, freqs, None).cpu()) <= LAYER_TOL    # with gradients: no kernels

@@ -1,0 +1,53 @@
+"""When MLA.forward may take its fused kernels: the conditions, on the host (no kernel runs)."""
+import pytest
+import torch
+from torch import nn
+
+FP8 = torch.float8_e4m3fn
+
+
+@pytest.fixture
+def layer(monkeypatch):
+    from dsv3fp8 import model
+    monkeypatch.setattr(model.Linear, "dtype", FP8)
+    old = torch.get_default_dtype()
+    torch.set_default_dtype(torch.bfloat16)
+    yield model.MLA(model.ModelArgs(dim=256, n_heads=2, q_lora_rank=128, max_batch_size=1, max_seq_len=8))
+    torch.set_default_dtype(old)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.1, 1e-40, float("inf"), float("nan"), torch.tensor(0.1)])
+def test_scales_that_the_attention_kernels_refuse(layer, scale):
+    q = torch.zeros(1, 2, 2, 192, dtype=torch.bfloat16)
+    assert layer._attention_kernels_ok(q, 4, None)
+    layer.softmax_scale = scale
+    assert not layer._attention_kernels_ok(q, 4, None)
+
+
+def _strided(n):
+    return torch.ones(2 * n, dtype=torch.bfloat16)[::2]
+
+
+@pytest.mark.parametrize("name", ["q_norm", "kv_norm"])
+@pytest.mark.parametrize("what", ["eps", "strided", "expanded", "offset", "fp32"])
+def test_norms_that_the_latent_kernel_does_not_take(layer, name, what):
+    x = torch.zeros(1, 2, 256, dtype=torch.bfloat16)
+    assert layer._latent_kernel_ok(x)
+    norm = getattr(layer, name)
+    if what == "eps":
+        norm.eps = None
+    else:
+        n = norm.dim
+        norm.weight = nn.Parameter({"strided": _strided(n), "expanded": torch.ones(1, dtype=torch.bfloat16).expand(n),
+                                    "offset": torch.ones(n + 1, dtype=torch.bfloat16)[1:], "fp32": torch.ones(n, dtype=torch.float32)}[what])
+    assert not layer._latent_kernel_ok(x)
+
+
+def test_masks_that_the_attention_kernels_do_not_take(layer):
+    q = torch.zeros(1, 2, 2, 192, dtype=torch.bfloat16)
+    ones = torch.ones(2, 4)
+    for mask in (ones, ones.bfloat16()):
+        assert layer._attention_kernels_ok(q, 4, mask)
+    for mask in (ones.half(), ones.bool(), ones[:1], torch.ones(4, 2).t(), ones[None], ones.to("meta")):
+        assert not layer._attention_kernels_ok(q, 4, mask)
+    assert not layer._attention_kernels_ok(q.float(), 4, None) and not layer._attention_kernels_ok(q[:, :, :, ::2], 4, None)
