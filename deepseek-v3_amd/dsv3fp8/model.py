@@ -215,7 +215,8 @@ def apply_rotary_emb(x: torch.Tensor, freqs_cis: torch.Tensor) -> torch.Tensor:
 def _plain(module: nn.Module, cls: type) -> bool:
     """Whether calling ``module`` does no more than ``cls.forward``, so that a fused kernel may take its place: neither a
     module of another type nor one with hooks (its own or those of all modules) or a ``forward`` of its own."""
-    return type(module) is cls and not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
+    own = module.__dict__
+    return type(module) is cls and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own
                                         or _modules._global_forward_hooks or _modules._global_forward_pre_hooks)
 
 
@@ -289,22 +290,28 @@ class MLA(nn.Module):
         and nothing but ``Linear.forward`` behind a call of either: exchanged modules and hooks are called).  Idempotent; the
         layers' parameters become views, so in-place weight loading keeps working.  Parameters that were replaced or
         moved since (``load_state_dict(assign=True)``, ``.to(device)``) are stacked anew."""
-        if self.q_lora_rank == 0 or self.q_lora_rank % block_size or not _plain(self.wq_a, Linear) \
-                or not _plain(self.wkv_a, Linear) or self.wq_a.bias is not None or self.wkv_a.bias is not None \
-                or self.wq_a.weight.element_size() != 1 \
-                or self.wkv_a.weight.element_size() != 1 or self.wq_a.scale_fmt != self.wkv_a.scale_fmt:
+        if self.q_lora_rank == 0 or self.q_lora_rank % block_size:
             return False
         qa, ka = self.wq_a, self.wkv_a
-        wa = getattr(self, "_wa", None)
-        if wa is not None and qa.weight.data_ptr() == wa.data_ptr() and ka.weight.data_ptr() == wa.data_ptr() + qa.weight.numel() \
-                and qa.scale.data_ptr() == wa.scale.data_ptr() \
-                and ka.scale.data_ptr() == wa.scale.data_ptr() + 4 * qa.scale.numel():
-            return True
+        if not _plain(qa, Linear) or not _plain(ka, Linear) or qa.scale_fmt != ka.scale_fmt:
+            return False
+        # parameters straight from the modules' dictionaries, here and below: a lookup through nn.Module takes half a
+        # microsecond, and a decode step is bound by the host
+        qp, kp = qa._parameters, ka._parameters
+        qw, kw, qs, ks = qp["weight"], kp["weight"], qp["scale"], kp["scale"]
+        if qw.element_size() != 1 or kw.element_size() != 1 or qp["bias"] is not None or kp["bias"] is not None:
+            return False
+        wa = self.__dict__.get("_wa")
+        if wa is not None:
+            at, scale_at = wa.data_ptr(), wa.scale.data_ptr()
+            if qw.data_ptr() == at and kw.data_ptr() == at + qw.numel() and qs.data_ptr() == scale_at \
+                    and ks.data_ptr() == scale_at + 4 * qs.numel():
+                return True
         with torch.no_grad():
-            w = torch.cat([qa.weight.data.view(torch.uint8), ka.weight.data.view(torch.uint8)]).view(qa.weight.dtype)
-            sc = torch.cat([qa.scale.data, ka.scale.data])
-            qa.weight.data, ka.weight.data = w[:qa.out_features], w[qa.out_features:]
-            qa.scale.data, ka.scale.data = sc[:qa.scale.size(0)], sc[qa.scale.size(0):]
+            w = torch.cat([qw.data.view(torch.uint8), kw.data.view(torch.uint8)]).view(qw.dtype)
+            sc = torch.cat([qs.data, ks.data])
+            qw.data, kw.data = w[:qa.out_features], w[qa.out_features:]
+            qs.data, ks.data = sc[:qs.size(0)], sc[qs.size(0):]
         w.scale = sc
         self._wa = w
         return True
@@ -342,31 +349,35 @@ class MLA(nn.Module):
     def _kernels_ok(self, x, start_pos: int, freqs_cis) -> bool:
         """What the fused kernels of this layer ask for in common: their head dimensions and dtypes, FP8 weights, no
         gradients (the kernels have no backward), new rows that fit the caches."""
-        b, s = x.size(0), x.size(1)
-        return (not torch.is_grad_enabled() and gemm_impl == "fp8" and block_size == 128 and world_size == 1 and self.fused
-                and x.is_cuda and x.dtype == torch.bfloat16 and torch.get_default_dtype() == torch.bfloat16
-                and self.attn_impl == "absorb"
-                and (self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim, self.kv_lora_rank) == (128, 64, 128, 512)
-                and self.kv_cache.dtype == self.pe_cache.dtype == torch.bfloat16
-                and self.kv_cache.is_contiguous() and self.pe_cache.is_contiguous()
-                and self.kv_cache.device == self.pe_cache.device == freqs_cis.device == x.device
-                and 1 <= b <= self.kv_cache.size(0) and s >= 1 and start_pos >= 0 and start_pos + s <= self.kv_cache.size(1)
-                and self.wkv_b.weight.element_size() == 1
-                and all(map(_offset_aligned, (self.kv_cache, self.pe_cache, self.wkv_b.weight)))
-                and self.wkv_b.weight.device == x.device and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous()
-                and not freqs_cis.is_conj() and freqs_cis.shape == (s, self.qk_rope_head_dim // 2))
+        if (torch.is_grad_enabled() or gemm_impl != "fp8" or block_size != 128 or world_size != 1 or not self.fused
+                or self.attn_impl != "absorb" or not x.is_cuda or x.dtype != torch.bfloat16
+                or torch.get_default_dtype() != torch.bfloat16):
+            return False
+        b, s, device = x.size(0), x.size(1), x.device
+        kv, pe, w = self.kv_cache, self.pe_cache, self.wkv_b.weight
+        return ((self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim, self.kv_lora_rank) == (128, 64, 128, 512)
+                and kv.dtype == torch.bfloat16 and pe.dtype == torch.bfloat16 and kv.is_contiguous() and pe.is_contiguous()
+                and 1 <= b <= kv.size(0) and s >= 1 and start_pos >= 0 and start_pos + s <= kv.size(1)
+                and w.element_size() == 1 and _offset_aligned(kv) and _offset_aligned(pe) and _offset_aligned(w)
+                and kv.device == device and pe.device == device and w.device == device and freqs_cis.device == device
+                and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous() and not freqs_cis.is_conj()
+                and freqs_cis.shape == (s, self.qk_rope_head_dim // 2))
 
     def _latent_kernel_ok(self, x) -> bool:
         """Whether both norms, the cache rows and the quantisation in front of ``wq_b`` can be one launch; modules that
         were exchanged or carry hooks are called as such."""
-        return (self.q_lora_rank % block_size == 0 and 0 < self.q_lora_rank <= 2048 and self.stacked_a
-                and _plain(self.q_norm, RMSNorm) and _plain(self.kv_norm, RMSNorm) and _plain(self.wq_b, ColumnParallelLinear)
-                and self.q_norm.weight.dtype == torch.bfloat16 and self.kv_norm.weight.dtype == torch.bfloat16
-                and self.q_norm.weight.device == self.kv_norm.weight.device == x.device
-                and self.q_norm.weight.is_contiguous() and self.kv_norm.weight.is_contiguous()
-                and _offset_aligned(self.q_norm.weight) and _offset_aligned(self.kv_norm.weight)
-                and isinstance(self.q_norm.eps, (int, float)) and isinstance(self.kv_norm.eps, (int, float))
-                and self.wq_b.weight.element_size() == 1 and self.wq_b.bias is None and self.stack_a())
+        if not 0 < self.q_lora_rank <= 2048 or self.q_lora_rank % block_size or not self.stacked_a:
+            return False
+        qn, kn, wq = self.q_norm, self.kv_norm, self.wq_b
+        if not (_plain(qn, RMSNorm) and _plain(kn, RMSNorm) and _plain(wq, ColumnParallelLinear)):
+            return False
+        for norm in (qn, kn):
+            w = norm._parameters["weight"]
+            if w.dtype != torch.bfloat16 or w.device != x.device or not w.is_contiguous() or not _offset_aligned(w) \
+                    or not isinstance(norm.eps, (int, float)):
+                return False
+        wq = wq._parameters
+        return wq["weight"].element_size() == 1 and wq["bias"] is None and self.stack_a()
 
     def _attention_kernels_ok(self, q, positions: int, mask) -> bool:
         """Whether the attention behind the query projection can run on the fused kernels: a mask of one value per
