@@ -23,11 +23,15 @@ __device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32); }
 template <bool F32> __device__ __forceinline__ float mask_at(const void* m, int64_t i) {
     return F32 ? ((const float*)m)[i] : u32_as_f32((uint32_t)((const uint16_t*)m)[i] << 16);
 }
-// A mask value in units of the raw scores.  A finite one stays finite: masks of the type's lowest value would otherwise
-// become -inf, and a row that has nothing else NaN instead of equal weights.
-__device__ __forceinline__ float mask_term(float v, float inv_scale) {
-    const float t = v * inv_scale;
-    return t == -__builtin_inff() && v != t ? -__FLT_MAX__ : t;
+// The unit in which scores are kept beside a mask: the raw ones times the largest power of two that is not above the
+// softmax scale (1 for scales above 1), scale = unit * rest.  The power of two costs no rounding, and a mask value, which
+// counts in units of scale, is divided by a rest of at least 1: every finite one stays finite and keeps its order.  (That
+// quotient is rounded before the score is added: equal mask values of a size that swallows the scores must stay equal.)
+struct ScoreUnit { float unit, rest; };
+inline ScoreUnit score_unit(float scale) {
+    int e;
+    const float m = __builtin_frexpf(scale, &e);        // m * 2^e, m in [1/2, 1)
+    return scale < 1.f ? ScoreUnit{ __builtin_ldexpf(1.f, e - 1), 2.f * m } : ScoreUnit{ 1.f, scale };
 }
 // What the exponents fma(S, scale2, -offset) subtract for a row maximum m.  Where the maximum is huge (a row that only
 // finite mask values of such a size reach), the rounding of m * scale2 alone would overflow the exponentials: the maximum

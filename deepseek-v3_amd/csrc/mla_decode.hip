@@ -34,7 +34,7 @@ struct DecodeArgs {
     float* part; v2f* ml;                               // [batch][row block][split]: kPartFloats floats; kRows x (maximum, sum)
     uint16_t* out;                                      // bf16 [batch][rows][512]
     int batch, rows, heads, positions, tiles, blocks, splits, per;
-    float scale, inv_scale;
+    float unit, scale, inv_scale;                       // score_unit's unit and rest, and the rest's reciprocal; without a mask 1 and the scale
 };
 
 // Chunks of 16 bytes of a latent row r are stored at chunk position c ^ swz(r) (low four bits).  Sixteen rows read at
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
     const uint32_t vaddr = (4 * g + (l15 >> 2)) * 1024 + ((((2 * q2 + ((l15 & 3) >> 1)) ^ g) | ((l15 >> 2) << 2)) << 4) + 8 * (l15 & 1);
 
     v16f O[16] = {};
-    float m = -__builtin_inff(), l = 0.f;               // running maximum (raw scores), this lane's share of the sum
+    float m = -__builtin_inff(), l = 0.f;               // running maximum of the scores, this lane's share of the sum
     const float scale2 = p.scale * 1.44269504088896340736f;
     int st = 0;
     for (int t = t0; t < t1; ++t) {
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int64_t at = mrow + min(t * kTile + 8 * (e >> 2) + 4 * g + (e & 3), p.positions - 1);
-                S[e] += mask_term(mask_at<MASK == kMaskF32>(p.mask, at), p.inv_scale);
+                S[e] = __builtin_fmaf(S[e], p.unit, mask_at<MASK == kMaskF32>(p.mask, at) * p.inv_scale);
             }
         }
         if ((t + 1) * kTile > p.positions) {            // the last tile may reach past the end
@@ -397,7 +397,8 @@ int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t 
     a.ql = ql; a.q = (const uint16_t*)q; a.freqs = (const v2f*)freqs;
     a.kv = (const uint16_t*)kv; a.kv_bs = kv_bs; a.pe = (const uint16_t*)pe; a.pe_bs = pe_bs;
     a.mask = mask; a.heads = heads;
-    a.scale = scale; a.inv_scale = 1.0f / scale;
+    const ScoreUnit u = mask ? score_unit(scale) : ScoreUnit{ 1.f, scale };
+    a.unit = u.unit; a.scale = u.rest; a.inv_scale = 1.0f / u.rest;
     int rc = launch_wkv_b_absorb(q, (int64_t)heads * kQd, kQd, w, ws, ql, DSV3_ABSORB_Q, batch * tokens, heads, kNope, kNope, kC, st);
     if (rc != DSV3_OK) return rc;
     const int which = !mask ? kNoMask : mask_f32 ? kMaskF32 : kMaskBf16;

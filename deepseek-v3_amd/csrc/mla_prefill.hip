@@ -195,7 +195,7 @@ struct AttendArgs {
     const void* mask; const uint64_t* flags;    // [rows][positions] / [qtiles][tiles], or null
     uint8_t* y; float* ys;                      // fp8 [batch][rows][heads * 128], scales [batch][rows][heads]
     int batch, heads, rows, positions, tiles, qtiles, per_head;     // per_head: workgroups of a head
-    float scale, inv_scale;                     // softmax scale and its reciprocal
+    float unit, scale, inv_scale;               // score_unit's unit and rest, and the rest's reciprocal
 };
 
 // One workgroup: 256 query rows of one head; wavefront w rows 32 w .. 32 w + 31.  Per tile of 64 positions (40 KiB of
@@ -233,12 +233,17 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
     const int q0 = qt * kQTile + wave * 32;
     const int row = min(q0 + i, p.rows - 1);
 
-    // query operands: lane (row i, half g) holds elements 16 s + 8 g .. + 7; the last four steps are rotated here
+    // query operands, in the scores' unit: lane (row i, half g) holds elements 16 s + 8 g .. + 7; the last four steps are
+    // rotated here
     v4u Q[12];
     {
         const uint16_t* src = p.q + (((int64_t)b * p.rows + row) * p.heads + h) * kQd + 8 * g;
 #pragma unroll
         for (int s = 0; s < 12; ++s) Q[s] = *(const v4u*)(src + 16 * s);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Q[s][e] = pack_bf16(bf16lo_to_f32(Q[s][e]) * p.unit, bf16hi_to_f32(Q[s][e]) * p.unit);
         const v2f* fr = p.freqs + (int64_t)row * (kRope / 2) + 4 * g;
 #pragma unroll
         for (int s = 0; s < 4; ++s)
@@ -246,7 +251,7 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
             for (int e = 0; e < 4; ++e) {
                 const v2f cs = fr[8 * s + e];
                 const float re = bf16lo_to_f32(Q[8 + s][e]), im = bf16hi_to_f32(Q[8 + s][e]);
-                Q[8 + s][e] = pack_bf16(re * cs.x - im * cs.y, re * cs.y + im * cs.x);
+                Q[8 + s][e] = pack_bf16((re * cs.x - im * cs.y) * p.unit, (re * cs.y + im * cs.x) * p.unit);
             }
     }
 
@@ -283,7 +288,7 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
     };
 
     v16f O[4] = {};
-    float m = -__builtin_inff(), l = 0.f;           // running maximum (raw scores), this lane's share of the sum
+    float m = -__builtin_inff(), l = 0.f;           // running maximum of the scores, this lane's share of the sum
     look();
     uint8_t flag = kSkip, flag_n = kSkip, flag_nn = kSkip;      // of this tile and the next two
     int t = next_tile(0, flag), st = 0;
@@ -332,7 +337,7 @@ __global__ __launch_bounds__(512, 2) void mla_attend_kernel(AttendArgs p) {
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
                         const int pos = t * kTile + 32 * k + 8 * (e >> 2) + 4 * g + (e & 3);
-                        S[k][e] += mask_term(mask_at<MF32>(p.mask, mrow + min(pos, p.positions - 1)), p.inv_scale);
+                        S[k][e] += mask_at<MF32>(p.mask, mrow + min(pos, p.positions - 1)) * p.inv_scale;
                     }
             }
             if ((t + 1) * kTile > p.positions) {            // the last tile may reach past the end
@@ -477,7 +482,8 @@ int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t
     a.y = (uint8_t*)y; a.ys = ys;
     a.batch = (int)batch; a.heads = heads; a.rows = (int)rows; a.positions = (int)positions;
     a.tiles = (int)tiles; a.qtiles = (int)qtiles; a.per_head = (int)per_head;
-    a.scale = scale; a.inv_scale = 1.0f / scale;
+    const ScoreUnit u = score_unit(scale);
+    a.unit = u.unit; a.scale = u.rest; a.inv_scale = 1.0f / u.rest;
     if (mask) {
         const dim3 grid((unsigned)tiles, (unsigned)qtiles);
         const int wide = (uintptr_t)mask % 16 == 0 && positions * (mask_f32 ? 4 : 2) % 16 == 0;

@@ -44,6 +44,13 @@ def _mask(kind, s, t, seed):
         m = torch.full((s, t), torch.finfo(dtype).min).triu_(1 + t - s)
         m[1] = torch.finfo(dtype).min
         return m.to(dtype).cuda()
+    if kind.startswith("ranked"):                       # values near either end of the type's range still have an order
+        m = torch.zeros(s, t)
+        m[0, : t // 2], m[0, t // 2:] = -3e38, -1e38    # the second half gets everything
+        m[1, ::3], m[1, 1::3], m[1, 2::3] = -2e38, -3e38, -2.5e38
+        m[2, 5], m[2, t - 1] = 3e38, 3e38               # these two get everything
+        m[3, : t // 2] = -3e38
+        return m.to(torch.float32 if kind == "ranked_f32" else torch.bfloat16).cuda()
     g = torch.Generator().manual_seed(seed)             # finite values and holes; row 1 sees nothing
     m = torch.where(torch.rand(s, t, generator=g) < 0.3, float("-inf"), torch.randn(s, t, generator=g))
     m[1] = float("-inf")
@@ -75,7 +82,7 @@ def _reference(q, freqs, kv, pe, w8, ws, mask, t, scale):
 PREFILL = [(1, 32, 32, 1, "causal"), (1, 33, 63, 3, None), (2, 64, 64, 8, "causal"), (1, 65, 65, 9, "causal"),
            (1, 255, 255, 2, "causal_f32"), (2, 257, 257, 3, "causal"), (1, 40, 500, 4, "causal"), (1, 1, 1, 2, None),
            (2, 100, 163, 4, "holes"), (1, 1100, 1100, 2, "causal"),
-           (1, 70, 130, 2, "lowest"), (1, 70, 130, 2, "lowest_f32"), (1, 256, 320, 2, "causal_f32"),
+           (1, 70, 130, 2, "lowest"), (1, 70, 130, 2, "lowest_f32"), (1, 70, 130, 2, "ranked"), (1, 40, 300, 2, "ranked_f32"), (1, 256, 320, 2, "causal_f32"),
            (1, 600, 600, 128, "causal"), (1, 4200, 4200, 16, "causal")]     # two query tiles a workgroup; 66 tiles of flags
 
 
@@ -83,7 +90,7 @@ PREFILL = [(1, 32, 32, 1, "causal"), (1, 33, 63, 3, None), (2, 64, 64, 8, "causa
 # units than compute units
 DECODE = [(1, 1, 1, 1, None), (1, 1, 31, 128, None), (2, 1, 33, 128, None), (1, 1, 700, 128, None), (3, 1, 1000, 16, None),
           (70, 1, 97, 128, None), (5, 4, 257, 40, "causal"), (1, 31, 95, 16, "causal_f32"), (2, 3, 200, 9, "holes"),
-          (1, 5, 130, 2, "lowest"), (1, 5, 130, 2, "lowest_f32"), (1, 1, 9000, 3, None)]
+          (1, 5, 130, 2, "lowest"), (1, 5, 130, 2, "lowest_f32"), (1, 5, 130, 2, "ranked"), (2, 4, 300, 2, "ranked_f32"), (1, 1, 9000, 3, None)]
 
 
 def _decode_reference(q, freqs, kv, pe, w8, ws, mask, t, scale):
