@@ -6,7 +6,8 @@
 // folds W_k into the query and W_v into the output, which costs nothing per position but makes every query-key pair
 // a 576-wide and every weighted sum a 512-wide product; here the keys and values are formed first (2 * 512 * 256
 // operations per head and position) and a pair costs 192 + 128.  With as many new tokens as positions that is 3.4 x
-// less work in front of the matrix cores; where few tokens meet many positions the absorbed form wins (mla_decode.hip).
+// less work in front of the matrix cores; where few tokens meet many positions the absorbed form wins (mla_decode.hip;
+// MLA._explicit_pays weighs the two).
 // Roundings: keys and values to bf16 (the absorbed form rounds the folded query and the latent sum instead), exponentials
 // to bf16 in front of the value product, scores and sums in binary32, the result to bf16 and then quantised.
 //

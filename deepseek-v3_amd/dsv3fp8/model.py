@@ -250,8 +250,8 @@ class MLA(nn.Module):
 
     fused: bool = True
     stacked_a: bool = True
-    # from this many new tokens per sequence on, keys and values are formed per head instead of being folded into the
-    # query and the output (csrc/mla_prefill.hip; with fewer csrc/mla_decode.hip)
+    # with fewer new tokens per sequence, wkv_b is always folded into the query and the output (csrc/mla_decode.hip) and
+    # keys and values are never formed per head (csrc/mla_prefill.hip)
     explicit_min_tokens: int = 32
 
     def __init__(self, args: ModelArgs):
@@ -387,6 +387,22 @@ class MLA(nn.Module):
                 and (mask is None or (mask.device == q.device and mask.shape == (q.size(1), positions) and mask.is_contiguous()
                                       and mask.dtype in (torch.bfloat16, torch.float32))))
 
+    def _explicit_pays(self, batch: int, tokens: int, positions: int) -> bool:
+        """Whether forming keys and values of all positions beats folding ``wkv_b`` into queries and outputs, which leaves a
+        pair of 1088 multiply-adds in place of 320 but costs nothing per position.  Both sides in microseconds as the kernels
+        take them, 128 heads: expanding a position 0.048; a round of 256 decode workgroups (128 (token, head) rows x a range
+        of ``per`` 32-position tiles each, one to a compute unit) 5 + 2.65 per tile, a block of rows 0.2 for its partial
+        sums and folded rows.  Over 182 shapes (1 .. 16 sequences, 32 .. 384 new tokens, 64 .. 16384 positions) the form
+        chosen so is at most 4 % slower than the better one; 32 new tokens as the line, whatever the positions, was up to
+        3.7 times slower (8 sequences x 32 tokens at 16384 positions: 6578 us explicit, 1771 absorbed)."""
+        if tokens < self.explicit_min_tokens:
+            return False
+        blocks = batch * -(-tokens * self.n_local_heads // 128)
+        tiles = -(-positions // 32)
+        per = -(-tiles // min(max(256 // blocks, 1), tiles))
+        rounds = -(-blocks * -(-tiles // per) // 256)
+        return rounds * (5 + 2.65 * per) + 0.2 * blocks > 0.048 * batch * positions * self.n_local_heads / 128
+
     def forward(self, x: torch.Tensor, start_pos: int, freqs_cis: torch.Tensor, mask: Optional[torch.Tensor]):
         b, s = x.size(0), x.size(1)
         start_pos = operator.index(start_pos)
@@ -406,7 +422,7 @@ class MLA(nn.Module):
             self.pe_cache[:b, start_pos:t] = apply_rotary_emb(kva[..., self.kv_lora_rank:].unsqueeze(2), freqs_cis).squeeze(2)
         if kernels and self._attention_kernels_ok(q, t, mask):
             args = (q, freqs_cis, self.kv_cache, self.pe_cache, self.wkv_b.weight, self.wkv_b.scale, mask, t, self.softmax_scale)
-            if s < self.explicit_min_tokens:
+            if not self._explicit_pays(b, s, t):
                 return self.wo(torch.ops.dsv3fp8.mla_decode(*args))
             if _plain(self.wo, RowParallelLinear) and self.wo.weight.element_size() == 1 and self.wo.bias is None:
                 return fp8_gemm(*torch.ops.dsv3fp8.mla_prefill(*args), self.wo.weight, self.wo.weight.scale)

@@ -90,6 +90,7 @@ PREFILL = [(1, 32, 32, 1, "causal"), (1, 33, 63, 3, None), (2, 64, 64, 8, "causa
 # units than compute units
 DECODE = [(1, 1, 1, 1, None), (1, 1, 31, 128, None), (2, 1, 33, 128, None), (1, 1, 700, 128, None), (3, 1, 1000, 16, None),
           (70, 1, 97, 128, None), (5, 4, 257, 40, "causal"), (1, 31, 95, 16, "causal_f32"), (2, 3, 200, 9, "holes"),
+          (2, 100, 700, 20, "causal"), (1, 40, 500, 128, "causal_f32"),         # many row blocks a sequence
           (1, 5, 130, 2, "lowest"), (1, 5, 130, 2, "lowest_f32"), (1, 5, 130, 2, "ranked"), (2, 4, 300, 2, "ranked_f32"), (1, 1, 9000, 3, None)]
 
 
@@ -332,3 +333,28 @@ def test_settings_that_the_kernels_do_not_take_still_run(M, what):
     with torch.inference_mode():
         y = layer(x, 0, freqs, None)
     assert torch.isfinite(y).all() and _rel(y, layer(x, 0, freqs, None).cpu()) <= LAYER_TOL    # with gradients: no kernels
+
+
+@pytest.mark.parametrize("s,start,form", [(5, 30, "decode"), (40, 30, "prefill"), (40, 30, "decode"), (1, 0, "decode")])
+def test_layer_on_a_filled_cache_vs_oracle(M, s, start, form):
+    """Several new tokens behind a cached prefix, mask [s, start + s], on either side of the forms' line."""
+    dim, heads, q_rank = 256, 4, 128
+    p = small_mla_params(dim, heads, q_rank, C, NOPE, ROPE, V, 31)
+    layer = _layer(M, p, dim, heads, q_rank, 96)
+    if s >= 32:
+        assert layer._explicit_pays(2, s, start + s)
+    if form == "decode":
+        layer.explicit_min_tokens = 1000
+    freqs = _freqs(ROPE, 96)[start:start + s]
+    g = torch.Generator().manual_seed(35)
+    x = torch.randn(2, s, dim, generator=g).bfloat16()
+    kv, pe = torch.zeros(2, 96, C, dtype=torch.bfloat16), torch.zeros(2, 96, ROPE, dtype=torch.bfloat16)
+    kv[:, :start], pe[:, :start] = torch.randn(2, start, C, generator=g), torch.randn(2, start, ROPE, generator=g)
+    layer.kv_cache.copy_(kv); layer.pe_cache.copy_(pe)
+    mask = torch.full((s, start + s), float("-inf")).triu_(1 + start) if s > 1 else None
+    ref = oracle.mla(x, start, freqs, mask, p, kv, pe, heads, NOPE, ROPE, V, C, (NOPE + ROPE) ** -0.5)
+    with torch.inference_mode():
+        y = layer(x.cuda(), start, freqs.cuda(), mask.cuda() if s > 1 else None)
+    assert _rel(y, ref) <= LAYER_TOL
+    assert _rel(layer.kv_cache, kv) <= 1e-2 and _rel(layer.pe_cache, pe) <= 1e-2
+    assert torch.equal(layer.kv_cache[:, :start].cpu(), kv[:, :start]) and not layer.kv_cache[:, start + s:].any()

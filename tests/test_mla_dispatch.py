@@ -51,3 +51,24 @@ def test_masks_that_the_attention_kernels_do_not_take(layer):
     for mask in (ones.half(), ones.bool(), ones[:1], torch.ones(4, 2).t(), ones[None], ones.to("meta")):
         assert not layer._attention_kernels_ok(q, 4, mask)
     assert not layer._attention_kernels_ok(q.float(), 4, None) and not layer._attention_kernels_ok(q[:, :, :, ::2], 4, None)
+
+
+# (sequences, new tokens, positions, explicit form, absorbed form): the layer's measured microseconds at 128 heads
+MEASURED = [(1, 64, 64, 94, 107), (1, 96, 512, 124, 158), (1, 32, 2048, 188, 131), (1, 192, 2048, 255, 354), (1, 64, 4096, 309, 211),
+            (1, 192, 4096, 382, 552), (1, 64, 16384, 977, 495), (1, 192, 16384, 1122, 1719), (8, 32, 64, 165, 200),
+            (8, 32, 512, 340, 244), (8, 96, 512, 439, 577), (8, 64, 2048, 955, 720), (8, 128, 2048, 1085, 1376),
+            (8, 64, 4096, 1740, 1150), (8, 128, 4096, 1890, 2207), (8, 32, 16384, 6578, 1771), (8, 96, 16384, 6837, 5068),
+            (8, 192, 16384, 7591, 10028), (16, 128, 10000, 8707, 7301), (16, 224, 10000, 9888, 12643)]
+
+
+def test_form_of_the_attention(layer):
+    layer.n_local_heads = 128
+    for b, s, t, explicit, absorbed in MEASURED:
+        assert layer._explicit_pays(b, s, t) == (explicit < absorbed), (b, s, t)
+    for s in range(1, 300):                             # nothing in the caches yet: from 32 tokens on, explicit
+        for b in (1, 3, 8, 64):
+            assert layer._explicit_pays(b, s, s) == (s >= layer.explicit_min_tokens)
+    for heads in (1, 16, 127, 128, 200):                # other head counts
+        layer.n_local_heads = heads
+        for b, t in ((1, 500), (2, 3000), (8, 16384)):
+            assert layer._explicit_pays(b, t, t) and not layer._explicit_pays(b, 31, t)
