@@ -70,12 +70,15 @@ EXPORTS = {
 }
 
 
+def require(path: Path) -> None:
+    if not path.exists():
+        raise ImportError(
+            f"{path} is missing: the HIP library has not been built. "
+            f"Run `python {LIB_PATH.parent.parent / 'build.py'}` (needs hipcc); there is no CPU fallback.")
+
+
 def _load() -> ctypes.CDLL:
-    for path in (LIB_PATH, TORCH_LIB_PATH):
-        if not path.exists():
-            raise ImportError(
-                f"{path} is missing: the HIP library has not been built. "
-                f"Run `python {LIB_PATH.parent.parent / 'build.py'}` (needs hipcc); there is no CPU fallback.")
+    require(LIB_PATH)
     lib = ctypes.CDLL(str(LIB_PATH))
     for name, (res, args) in EXPORTS.items():
         fn = getattr(lib, name)

@@ -286,6 +286,7 @@ def _mla_latent_meta(a, q_norm, kv_norm, freqs, kv_cache, pe_cache, start, q_eps
     return (a.new_empty(b, s, q_norm.numel(), dtype=FP8), a.new_empty(b, s, q_norm.numel() // 128, dtype=torch.float32))
 
 
+_lib.require(_lib.TORCH_LIB_PATH)
 torch.ops.load_library(str(_lib.TORCH_LIB_PATH))       # the device implementations of csrc/torch_ops.cpp
 
 _libimpl = torch.library.Library("dsv3fp8", "IMPL")

@@ -390,3 +390,27 @@ def test_attention_operators_refuse_what_their_kernels_cannot_read(name):
             args[at] = change(args[at])
             with pytest.raises(RuntimeError, match="mla.*(must|behind)"):
                 _gpu_body(name, *args)
+
+
+def test_binding_needs_the_c_library_only():
+    """_lib.py by itself (without the package, which registers the torch operators) loads where libdsv3torch.so is not
+    built; the package says which command builds it."""
+    import subprocess
+    import sys
+    code = """
+import importlib.util, pathlib
+exists = pathlib.Path.exists
+pathlib.Path.exists = lambda path: path.name != "libdsv3torch.so" and exists(path)
+spec = importlib.util.spec_from_file_location("binding", "dsv3fp8/_lib.py")
+binding = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(binding)
+assert binding.lib.dsv3_version() >= 100
+try:
+    import dsv3fp8
+except ImportError as e:
+    assert "libdsv3torch.so" in str(e) and "build.py" in str(e)
+else:
+    raise AssertionError("imported")
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT / "deepseek-v3_amd", capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
