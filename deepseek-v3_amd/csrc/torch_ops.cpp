@@ -44,6 +44,12 @@ void check(int rc, const char* what) {
     TORCH_CHECK(rc == DSV3_OK, what, " failed: ", dsv3_status_string(rc), " (dsv3_status ", rc, ")");
 }
 
+// A block size as the library takes it: one that is cut to 32 bits would not be the one the results are laid out for.
+int checked_block(int64_t block, const char* what) {
+    TORCH_CHECK(block > 0 && block <= 0x7fffffff, what, ": block_size must be positive and fit 32 bits, got ", block);
+    return (int)block;
+}
+
 // The device of an operator's tensors made current, and its stream.
 struct On {
     c10::DeviceGuard guard;
@@ -69,35 +75,36 @@ Tensor with_last(const Tensor& x, int64_t last, at::ScalarType dtype) {
 }
 
 tuple<Tensor, Tensor> act_quant(const Tensor& x, int64_t block, int64_t fmt) {
-    TORCH_CHECK(block > 0, "act_quant: block_size must be positive");
+    const int bs = checked_block(block, "act_quant");
     const int64_t last = x.size(-1);
     const int code = dtype_code(x.scalar_type());
-    Tensor y = at::empty_like(x, x.options().dtype(kFp8)), s = with_last(x, last / block, at::kFloat);
+    Tensor y = at::empty_like(x, x.options().dtype(kFp8)), s = with_last(x, last / bs, at::kFloat);
     On on(x);
-    check(dsv3_act_quant(x.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), x.numel(), last, (int)block, (int)fmt, on.stream),
+    check(dsv3_act_quant(x.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), x.numel(), last, bs, (int)fmt, on.stream),
           "dsv3_act_quant");
     return {y, s};
 }
 
 Tensor weight_dequant(const Tensor& x, const Tensor& s, int64_t block, int64_t out) {
     TORCH_CHECK_VALUE(x.dim() == 2, "weight_dequant: a matrix is needed");
+    const int bs = checked_block(block, "weight_dequant");
     on_one_gpu("weight_dequant", x, { &s });
     Tensor y = at::empty_like(x, x.options().dtype(dtype_of(out)));
     On on(x);
-    check(dsv3_weight_dequant(x.data_ptr(), (const float*)s.data_ptr(), y.data_ptr(), (int)out, x.size(0), x.size(1), (int)block,
+    check(dsv3_weight_dequant(x.data_ptr(), (const float*)s.data_ptr(), y.data_ptr(), (int)out, x.size(0), x.size(1), bs,
                               on.stream), "dsv3_weight_dequant");
     return y;
 }
 
 tuple<Tensor, Tensor> weight_quant(const Tensor& w, int64_t block, int64_t fmt) {
     TORCH_CHECK_VALUE(w.dim() == 2, "weight_quant: a matrix is needed");
-    TORCH_CHECK(block > 0, "weight_quant: block_size must be positive");
+    const int bs = checked_block(block, "weight_quant");
     const int code = dtype_code(w.scalar_type());
     const int64_t m = w.size(0), n = w.size(1);
     Tensor y = at::empty_like(w, w.options().dtype(kFp8));
-    Tensor s = at::empty({(m + block - 1) / block, (n + block - 1) / block}, w.options().dtype(at::kFloat));
+    Tensor s = at::empty({(m + bs - 1) / bs, (n + bs - 1) / bs}, w.options().dtype(at::kFloat));
     On on(w);
-    check(dsv3_weight_quant(w.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), m, n, (int)block, (int)fmt, on.stream),
+    check(dsv3_weight_quant(w.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), m, n, bs, (int)fmt, on.stream),
           "dsv3_weight_quant");
     return {y, s};
 }
@@ -142,12 +149,12 @@ Tensor linear_fp8(const Tensor& x, const Tensor& b, const Tensor& b_s, int64_t f
 
 tuple<Tensor, Tensor> swiglu_quant(const Tensor& h, int64_t block, int64_t fmt) {
     TORCH_CHECK(h.dim() == 2 && h.is_contiguous() && h.size(1) % 2 == 0, "swiglu_quant: a contiguous matrix of even width is needed");
-    TORCH_CHECK(block > 0, "swiglu_quant: block_size must be positive");
+    const int bs = checked_block(block, "swiglu_quant");
     const int code = dtype_code(h.scalar_type());
     const int64_t rows = h.size(0), inter = h.size(1) / 2;
-    Tensor y = at::empty({rows, inter}, h.options().dtype(kFp8)), s = at::empty({rows, inter / block}, h.options().dtype(at::kFloat));
+    Tensor y = at::empty({rows, inter}, h.options().dtype(kFp8)), s = at::empty({rows, inter / bs}, h.options().dtype(at::kFloat));
     On on(h);
-    check(dsv3_swiglu_quant(h.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), rows, inter, (int)block, (int)fmt, on.stream),
+    check(dsv3_swiglu_quant(h.data_ptr(), code, y.data_ptr(), (float*)s.data_ptr(), rows, inter, bs, (int)fmt, on.stream),
           "dsv3_swiglu_quant");
     return {y, s};
 }

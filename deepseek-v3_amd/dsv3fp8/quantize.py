@@ -48,5 +48,7 @@ def weight_quant(w: torch.Tensor, block_size: int = 128,
     from . import _lib, ops  # noqa: F401  (registers torch.ops.dsv3fp8)
     assert w.is_contiguous(), 'Input tensor must be contiguous'
     assert w.dim() == 2, 'Input tensor must have 2 dimensions'
+    if block_size == 0:
+        raise ZeroDivisionError("weight_quant: block_size is 0")
     fmt = _lib.SCALE_FMT_UE8M0 if scale_fmt == "ue8m0" else _lib.SCALE_FMT_NONE
     return torch.ops.dsv3fp8.weight_quant(w, block_size, fmt)

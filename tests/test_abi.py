@@ -414,3 +414,19 @@ else:
 """
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT / "deepseek-v3_amd", capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+@pytest.mark.parametrize("block", [0, -128, 2 ** 32 + 128, 2 ** 31])
+def test_operators_refuse_block_sizes_that_do_not_fit(block):
+    x, w = torch.zeros(2, 256, dtype=torch.bfloat16), torch.zeros(128, 128, dtype=torch.float8_e4m3fn)
+    for name, *args in (("act_quant", x, block, 0), ("weight_quant", x, block, 0), ("swiglu_quant", x, block, 0),
+                        ("weight_dequant", w, torch.zeros(1, 1), block, 0)):
+        with pytest.raises(RuntimeError, match="block_size must"):
+            _gpu_body(name, *args)
+
+
+def test_block_size_zero_divides_by_zero():
+    from dsv3fp8 import act_quant, weight_quant
+    for call in (act_quant, weight_quant):
+        with pytest.raises(ZeroDivisionError):
+            call(torch.zeros(128, 128), 0)
