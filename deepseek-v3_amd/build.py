@@ -35,9 +35,13 @@ HIPCC_FLAGS = [
 # data has landed.  And a kernel that uses scratch at all costs a launch about 3 us more on this hardware (measured:
 # linear() at one row 7.4 -> 10.4 us when a rewrite of the in-kernel quantiser spilled nine registers) -- as much as
 # the whole quantisation such a launch is meant to save.  The build fails if a kernel of these files reports scratch
-# or spills; the one exception is listed with its reason.
-NO_SPILL_SOURCES = {"fp8_gemm_skinny.hip", "fp8_gemm_stream.hip"}
+# or spills; exceptions are listed with their reasons.
+# The attention kernels keep their sums in registers for a whole loop and have none to spare (mla_decode_kernel: 32 x 512
+# sums in the 256 accumulation registers; an ordinary rescale of them spilled 300): a spill there is a copy per tile.
+NO_SPILL_SOURCES = {"fp8_gemm_skinny.hip", "fp8_gemm_stream.hip", "mla_decode.hip", "mla_prefill.hip"}
 SCRATCH_ALLOWED = {
+    # two scalar registers kept in lanes of a vector register: no scratch memory, and outside the tile loop
+    "mla_attend_kernel": 2,
     # the quantising variant with four strips per wavefront (a plan for very wide weights at one or two rows that none
     # of the 671B projections takes): compiler-counted waits, 20 bytes per lane
     "skinny_kernelILi1ELi4ELi2ELb1ELb0E": 24,
@@ -57,7 +61,7 @@ def check_no_spills(name: str, remarks: str) -> None:
             continue
         allowed = max([v for k, v in SCRATCH_ALLOWED.items() if k in kernel], default=0)
         if int(m.group(2)) > allowed:
-            raise RuntimeError(f"{name}: {kernel} reports {m.group(1)} = {m.group(2)} (allowed: {allowed}); the decode "
+            raise RuntimeError(f"{name}: {kernel} reports {m.group(1)} = {m.group(2)} (allowed: {allowed}); these "
                                f"kernels must not spill (lower the kernel's register use or its occupancy target)")
 
 

@@ -430,3 +430,16 @@ def test_block_size_zero_divides_by_zero():
     for call in (act_quant, weight_quant):
         with pytest.raises(ZeroDivisionError):
             call(torch.zeros(128, 128), 0)
+
+
+@pytest.mark.parametrize("source", ["fp8_gemm_skinny.hip", "fp8_gemm_stream.hip", "mla_decode.hip", "mla_prefill.hip"])
+def test_build_refuses_spills(source):
+    import build
+    assert source in build.NO_SPILL_SOURCES and (build.CSRC / source).exists()
+    report = "remark: Function Name: _ZN4dsv317{}EvNS_4ArgsE\nremark:     {}: {}\n"
+    for kernel in ("mla_decode_kernelILi0E", "mla_combine_kernel", "mla_expand_kernel", "mla_attend_kernelILb0E"):
+        build.check_no_spills(source, report.format(kernel, "VGPRs Spill", 0))
+        for what in ("VGPRs Spill", "ScratchSize [bytes/lane]", "SGPRs Spill"):
+            with pytest.raises(RuntimeError, match="must not spill"):
+                build.check_no_spills(source, report.format(kernel, what, 4))
+    build.check_no_spills(source, report.format("mla_attend_kernelILb0E", "SGPRs Spill", 2))
