@@ -233,32 +233,95 @@ def test_layer_prefill_vs_oracle(M):
     assert _rel(z0, ref0) <= LAYER_TOL and _rel(y0, z0.cpu()) <= LAYER_TOL
 
 
-def test_decode_step_in_a_captured_graph(M):
-    """A captured decode step, replayed on new inputs with eager steps in between, gives the eager step's bits."""
+@pytest.mark.parametrize("s", [1, 40])
+def test_step_in_a_captured_graph(M, s):
+    """A captured step, replayed on new inputs with eager steps in between, gives the eager step's bits, in its result and
+    in the cache rows, which hold something else before each replay."""
     dim, heads, q_rank, t = 256, 4, 128, 40
     layer = _layer(M, small_mla_params(dim, heads, q_rank, C, NOPE, ROPE, V, 31), dim, heads, q_rank, 96)
-    freqs = _freqs(ROPE, 96)[t:t + 1].cuda()
+    freqs = _freqs(ROPE, 96)[t:t + s].cuda()
+    mask = torch.full((s, t + s), float("-inf"), device="cuda").triu_(1 + t) if s > 1 else None
     g = torch.Generator().manual_seed(33)
     with torch.inference_mode():
         layer.kv_cache.copy_(torch.randn(layer.kv_cache.shape, generator=g))
         layer.pe_cache.copy_(torch.randn(layer.pe_cache.shape, generator=g))
-        x = torch.randn(2, 1, dim, generator=g).bfloat16().cuda()
+        x = torch.randn(2, s, dim, generator=g).bfloat16().cuda()
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
-            layer(x, t, freqs, None)
+            layer(x, t, freqs, mask)
         torch.cuda.current_stream().wait_stream(side)
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
-            y = layer(x, t, freqs, None)
-        for _ in range(3):
-            new = torch.randn(2, 1, dim, generator=g).bfloat16().cuda()
-            ref = layer(new, t, freqs, None).clone()
+            y = layer(x, t, freqs, mask)
+        for n in range(3):
+            new = torch.randn(2, s, dim, generator=g).bfloat16().cuda()
+            ref, kv, pe = [o.clone() for o in (layer(new, t, freqs, mask), layer.kv_cache, layer.pe_cache)]
+            layer.kv_cache[:, t:t + s] = n
+            layer.pe_cache[:, t:t + s] = n
             torch.cuda.synchronize()
             x.copy_(new)
             graph.replay()
             torch.cuda.synchronize()
-            assert torch.equal(y, ref)
+            assert torch.equal(y, ref) and torch.equal(layer.kv_cache, kv) and torch.equal(layer.pe_cache, pe)
+
+
+@pytest.mark.parametrize("s", [1, 40])
+def test_two_streams_at_once(M, s):
+    """Layers on two streams, several steps without a wait between them: each stream's results are those of a single one."""
+    dim, heads, q_rank = 256, 4, 128
+    freqs = _freqs(ROPE, 96)[:s].cuda()
+    mask = torch.full((s, s), float("-inf"), device="cuda").triu_(1) if s > 1 else None
+    layers = [_layer(M, small_mla_params(dim, heads, q_rank, C, NOPE, ROPE, V, n), dim, heads, q_rank, 96) for n in (31, 32)]
+    g = torch.Generator().manual_seed(36)
+    xs = [torch.randn(2, s, dim, generator=g).bfloat16().cuda() for _ in range(12)]
+    with torch.inference_mode():
+        ref = [[layer(x, 0, freqs, mask).clone() for x in xs] for layer in layers]
+        torch.cuda.synchronize()
+        streams, got = [torch.cuda.Stream(), torch.cuda.Stream()], [[], []]
+        for x in xs:
+            for n, stream in enumerate(streams):
+                with torch.cuda.stream(stream):
+                    got[n].append(layers[n](x, 0, freqs, mask))
+        torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for n in (0, 1) for a, b in zip(got[n], ref[n]))
+
+
+@pytest.mark.parametrize("op", ["prefill", "decode"])
+def test_not_finite_inputs(op):
+    """NaN and infinity in a query, a mask or a cached row make NaN of the rows that the reference makes NaN of."""
+    b, s, t, h, scale = 2, 40, 130, 3, 0.08
+    q, freqs, kv, pe, w8, ws = _inputs(b, s, t, h, 7)
+    mask = torch.zeros(s, t, device="cuda")
+    q[0, 1, 0, 5], q[0, 2, 1, 140], q[0, 3, 2, 60] = float("nan"), float("inf"), float("-inf")
+    mask[5, 7], mask[6, 100] = float("nan"), float("inf")
+    mask[7, 20:] = float("-inf")
+    kv[1, 90, 3] = float("inf")                         # every row of the second sequence
+    args = (q, freqs, kv, pe, w8, ws, mask, t, scale)
+    if op == "prefill":
+        y, ys = torch.ops.dsv3fp8.mla_prefill(*args)
+        got, ref = y.float().view(b, s, h, V).double() * ys.double().unsqueeze(-1), _reference(*args)
+    else:
+        got, ref = torch.ops.dsv3fp8.mla_decode(*args).view(b, s, h, V).double(), _decode_reference(*args)
+    bad = torch.isnan(ref).any(-1)
+    expected = torch.zeros(b, s, h, dtype=torch.bool, device="cuda")
+    expected[1] = True
+    expected[0, 1, 0] = expected[0, 2, 1] = expected[0, 3, 2] = True
+    expected[0, 5:7] = True
+    assert torch.equal(bad, expected) and torch.equal(torch.isnan(got).any(-1), bad)
+    assert ((got - ref).norm(dim=-1) <= 2.0 ** -4 * ref.norm(dim=-1))[~bad].all()       # e4m3 in the prefill's result
+
+
+@pytest.mark.parametrize("op", ["prefill", "decode"])
+def test_caches_of_more_sequences_than_the_call(op):
+    b, s, t, h, scale = 2, 33, 70, 2, 0.08
+    q, freqs, kv, pe, w8, ws = _inputs(b, s, t, h, 9)
+    kv5, pe5 = (torch.full((5, t + 30, c.size(2)), float("nan"), dtype=torch.bfloat16, device="cuda") for c in (kv, pe))
+    kv5[:b, :t], pe5[:b, :t] = kv[:, :t], pe[:, :t]
+    call = getattr(torch.ops.dsv3fp8, "mla_" + op)
+    one, other = call(q, freqs, kv, pe, w8, ws, None, t, scale), call(q, freqs, kv5, pe5, w8, ws, None, t, scale)
+    for a, c in zip(one, other) if op == "prefill" else ((one, other),):
+        assert torch.equal(a.view(torch.uint8), c.view(torch.uint8)) and torch.isfinite(c.float()).all()
 
 
 def test_layer_with_parts_on_the_host_raises(M):
