@@ -65,6 +65,14 @@ void on_one_gpu(const char* what, const Tensor& x, std::initializer_list<const T
     TORCH_CHECK(x.is_cuda(), what, ": tensors must be on the GPU, got ", x.device());
 }
 
+// The library sees no sizes of its operands: what it will read has to be there (nothing, where the result is empty).
+void check_weight(const char* what, const Tensor& b, const Tensor& b_s, int64_t n, int64_t k, int64_t block) {
+    if (n == 0 || k == 0) return;
+    TORCH_CHECK(b.element_size() == 1 && b.is_contiguous() && b.numel() >= n * k, what, ": the weight must be contiguous, one byte an element, [", n, ", ", k, "]");
+    TORCH_CHECK(b_s.scalar_type() == at::kFloat && b_s.is_contiguous() && b_s.numel() >= ((n + block - 1) / block) * ((k + block - 1) / block),
+                what, ": the weight's scales must be contiguous fp32, one per block");
+}
+
 Tensor scratch(const Tensor& like, size_t bytes) {
     return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
 }
@@ -88,6 +96,7 @@ tuple<Tensor, Tensor> act_quant(const Tensor& x, int64_t block, int64_t fmt) {
 Tensor weight_dequant(const Tensor& x, const Tensor& s, int64_t block, int64_t out) {
     TORCH_CHECK_VALUE(x.dim() == 2, "weight_dequant: a matrix is needed");
     const int bs = checked_block(block, "weight_dequant");
+    check_weight("weight_dequant", x, s, x.size(0), x.size(1), bs);
     on_one_gpu("weight_dequant", x, { &s });
     Tensor y = at::empty_like(x, x.options().dtype(dtype_of(out)));
     On on(x);
@@ -127,6 +136,9 @@ Tensor gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b
 Tensor gemm(const Tensor& a, const Tensor& a_s, const Tensor& b, const Tensor& b_s, int64_t out, decltype(dsv3_fp8_gemm)* entry,
             const char* what) {
     const int64_t k = a.size(-1), m = k ? a.numel() / k : 0;
+    TORCH_CHECK(m == 0 || b.size(0) == 0 || (a.element_size() == 1 && a.is_contiguous() && a_s.scalar_type() == at::kFloat && a_s.is_contiguous() &&
+                a_s.numel() >= m * ((k + 127) / 128)), what, ": activations must be contiguous, one byte an element, with fp32 scales per block of 128");
+    check_weight(what, b, b_s, m ? b.size(0) : 0, k, 128);
     on_one_gpu(what, a, { &a_s, &b, &b_s });
     On on(a);
     const Tensor ws = gemm_scratch(a, m, b.size(0), k);
@@ -142,6 +154,8 @@ Tensor fp8_gemm_pow2(const Tensor& a, const Tensor& a_s, const Tensor& b, const 
 // act_quant(x, 128, fmt) followed by fp8_gemm, one launch where the library implements it, else two calls
 Tensor linear_fp8(const Tensor& x, const Tensor& b, const Tensor& b_s, int64_t fmt, int64_t out) {
     const int64_t k = x.size(-1), m = k ? x.numel() / k : 0, n = b.size(0);
+    TORCH_CHECK(x.is_contiguous(), "linear_fp8: x must be contiguous");
+    check_weight("linear_fp8", b, b_s, m ? n : 0, k, 128);
     on_one_gpu("linear_fp8", x, { &b, &b_s });
     On on(x);
     const Tensor ws = gemm_scratch(x, m, n, k);

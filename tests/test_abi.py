@@ -388,7 +388,7 @@ def test_attention_operators_refuse_what_their_kernels_cannot_read(name):
         for change in changes:
             args = _operator_args(name)
             args[at] = change(args[at])
-            with pytest.raises(RuntimeError, match="mla.*(must|behind)"):
+            with pytest.raises(RuntimeError, match=r"mla[^:]*: (?!tensors|all tensors)"):
                 _gpu_body(name, *args)
 
 
@@ -414,6 +414,26 @@ else:
 """
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT / "deepseek-v3_amd", capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+@pytest.mark.parametrize("name", ["fp8_gemm", "fp8_gemm_pow2", "linear_fp8", "weight_dequant"])
+def test_operators_refuse_operands_that_are_too_small(name):
+    """Scales of another type, too few of them, a weight of fewer columns, strided operands: all would be read past their end."""
+    weight = {"linear_fp8": 1, "weight_dequant": 0}.get(name, 2)
+    bad = {weight + 1: [lambda t: t.bfloat16(), lambda t: t[:0]], weight: [lambda t: t.float()]}
+    if name != "weight_dequant":
+        bad[weight].append(lambda t: t[:, :127].contiguous())
+    bad[weight].append(lambda t: torch.zeros(128, 256).to(t.dtype)[:, ::2])
+    if name.startswith("fp8_gemm"):
+        bad[0], bad[1] = [lambda t: t.float()], [lambda t: t.half(), lambda t: t[:1]]
+    elif name == "linear_fp8":
+        bad[0] = [lambda t: torch.zeros(2, 256, dtype=t.dtype)[:, ::2]]
+    for at, changes in bad.items():
+        for change in changes:
+            args = _operator_args(name)
+            args[at] = change(args[at])
+            with pytest.raises(RuntimeError, match="contiguous"):
+                _gpu_body(name, *args)
 
 
 @pytest.mark.parametrize("block", [0, -128, 2 ** 32 + 128, 2 ** 31])
