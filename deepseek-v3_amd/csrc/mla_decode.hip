@@ -61,7 +61,7 @@ __device__ __forceinline__ void scale_agprs(v16f& v, float a) {
 // values are the same 32 x 512 block: the keys are read as rows, the values through the LDS's transposing reads, four
 // positions of one feature per lane.
 // Bound: per tile 68 MFMAs of 32 cycles; with one wavefront per SIMD its exponentials and barriers stand beside them.  32
-// sequences at 4096 positions (16 tiles a workgroup): 57 us, 70 with each LDS read next to its MFMA; 12 us of it are the 67 MB
+// sequences at 4096 positions (16 tiles a workgroup): 53 .. 58 us, 70 with each LDS read next to its MFMA; 12 us of it are the 67 MB
 // of partial sums at the end, and one tile alone (a short context) takes 12 us in all.  The tensor operations in its place
 // took 250 us (58 us in the products, the rest in passes over the scores).
 enum { kNoMask, kMaskBf16, kMaskF32 };

@@ -13,9 +13,10 @@
 //
 // Three launches: expand (keys and values, and the rotary keys, in the order in which the attention kernel's wavefronts
 // read their operands), flags (which tiles of the mask are all zero or all -inf; only with a mask), attend.
-// At 4096 tokens, 128 heads, causal mask: expand 148 us, flags 11 us, attend 850 .. 910 us (0.76 .. 0.81 PFLOP/s of the pairs
-// the mask leaves; the clock falls to 1.8 GHz under it); the layer 1.58 ms where the absorbed form as tensor operations took
-// 20.2 ms (2 x 2.5 ms score products, 1.6 ms value product and 12 ms of passes over the 4.3 GB score matrix).
+// At 4096 tokens, 128 heads, causal mask (kernel trace): expand 136 us, flags 12 us, attend 785 us on a cool card (0.88 PFLOP/s
+// of the pairs the mask leaves) and up to 980 on a warm one, whose clock falls to 1.8 GHz under it; the layer 1.55 ms where the
+// absorbed form as tensor operations took 20.1 ms (2 x 2.5 ms score products, 1.6 ms value product and 12 ms of passes over
+// the 4.3 GB score matrix).
 #include <type_traits>
 
 #include "mla.hpp"
@@ -50,8 +51,8 @@ struct ExpandArgs {
 // operand order and a store instruction writes 1 KiB of consecutive bytes: MFMA row 8j + 4g + r of a key wavefront is
 // feature 16 (j / 2) + 8 g + 4 (j % 2) + r; a value lane's accumulator registers 8u .. 8u + 7 are, in order, the
 // eight positions that the attention kernel's K step u has in that lane.
-// Measured at 4096 positions, 128 heads: 219 us with each LDS read next to its MFMA, 140 .. 148 with six on their way (0.95
-// PFLOP/s; MFMAs 53 % of the cycles, the 268 MB of results alone would take 57 us).
+// Measured at 4096 positions, 128 heads: 219 us with each LDS read next to its MFMA, 136 .. 156 with six on their way (up to 1
+// PFLOP/s; MFMAs 60 % of the cycles, the 268 MB of results alone would take 57 us).
 __global__ __launch_bounds__(512, 2) void mla_expand_kernel(ExpandArgs p) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * 32 * 1024];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

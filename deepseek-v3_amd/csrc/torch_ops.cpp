@@ -3,7 +3,8 @@
 //
 // Why native: at a few tokens the launches of a layer are shorter than the host's way to them.  The same bodies in Python
 // behind torch.library cost 10 to 14 us an operator (argument boxing, device and stream contexts, two or three ctypes
-// calls); one sequence's decode step of the attention layer (five operators, kernels 72 us) was bound by that at 118 us and takes 71 with these.
+// calls); one sequence's decode step of the attention layer (five operators, kernels 72 us) was bound by that at 118 us and
+// takes 71 with these.
 // Scratch memory comes from the caching allocator on each call: it belongs to the current stream, and under stream capture
 // to the graph's pool.
 #include <ATen/ATen.h>

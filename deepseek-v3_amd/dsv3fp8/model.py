@@ -226,7 +226,7 @@ def _offset_aligned(t: torch.Tensor) -> bool:
 
 
 class MLA(nn.Module):
-    """Host of the two ``wkv_b`` products of the absorbed multi-head latent attention (model.py:395-497).
+    """Multi-head latent attention (model.py:395-497).
 
     In the reference's default cache layout (``attn_impl == "absorb"``) the compressed latent
     (``kv_cache`` [b, t, kv_lora_rank]) and the shared rotary key (``pe_cache``) are cached and the up-projection
@@ -238,9 +238,11 @@ class MLA(nn.Module):
     (``k_cache`` [b, t, h, nope + rope], ``v_cache`` [b, t, h, v]): ``wkv_b`` is then an ordinary linear layer on
     the new positions' latents (an FP8 GEMM through ``linear()``), and the scores and the weighted sum are plain
     per-head einsums.
-    ``MLA.fused = False`` selects the dequantise-then-einsum sequence instead.  Everything between the two products
-    (scores, softmax, weighted sum) is bf16 torch arithmetic that never touches FP8 data; it is here so that the
-    products can be tested in place.  Parameter names are the checkpoint's.
+    Without gradients, with FP8 weights and the head dimensions of the 671B configuration, everything between the
+    low-rank projections and ``wo`` runs on kernels (``torch.ops.dsv3fp8.{mla_latent, mla_decode, mla_prefill}``; the
+    conditions are ``_kernels_ok``, ``_latent_kernel_ok`` and ``_attention_kernels_ok``).  Other calls run the scores, the
+    softmax and the weighted sum as bf16 torch operations between the two products; ``MLA.fused = False`` takes
+    the dequantise-then-einsum sequence for the products too.  Parameter names are the checkpoint's.
 
     ``wq_a`` and ``wkv_a`` read the same input.  With FP8 weights (and ``q_lora_rank`` a multiple of the block size,
     so that both keep their own scale blocks) ``stack_a()`` lays them out as one ``[q_lora_rank + kv_lora_rank +
@@ -365,7 +367,7 @@ class MLA(nn.Module):
 
     def _latent_kernel_ok(self, x) -> bool:
         """Whether both norms, the cache rows and the quantisation in front of ``wq_b`` can be one launch; modules that
-        were exchanged or carry hooks are called as such."""
+        were exchanged or carry hooks (``wq_a`` and ``wkv_a`` too, by ``stack_a``) are called as such."""
         if not 0 < self.q_lora_rank <= 2048 or self.q_lora_rank % block_size or not self.stacked_a:
             return False
         qn, kn, wq = self.q_norm, self.kv_norm, self.wq_b
