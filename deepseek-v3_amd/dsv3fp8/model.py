@@ -300,8 +300,9 @@ class MLA(nn.Module):
         # parameters straight from the modules' dictionaries, here and below: a lookup through nn.Module takes half a
         # microsecond, and a decode step is bound by the host
         qp, kp = qa._parameters, ka._parameters
-        qw, kw, qs, ks = qp["weight"], kp["weight"], qp["scale"], kp["scale"]
-        if qw.element_size() != 1 or kw.element_size() != 1 or qp["bias"] is not None or kp["bias"] is not None:
+        qw, kw, qs, ks = qp.get("weight"), kp.get("weight"), qp.get("scale"), kp.get("scale")
+        if qw is None or kw is None or qs is None or ks is None or qw.element_size() != 1 or kw.element_size() != 1 \
+                or qp.get("bias") is not None or kp.get("bias") is not None:
             return False
         wa = self.__dict__.get("_wa")
         if wa is not None:
@@ -374,12 +375,12 @@ class MLA(nn.Module):
         if not (_plain(qn, RMSNorm) and _plain(kn, RMSNorm) and _plain(wq, ColumnParallelLinear)):
             return False
         for norm in (qn, kn):
-            w = norm._parameters["weight"]
-            if w.dtype != torch.bfloat16 or w.device != x.device or not w.is_contiguous() or not _offset_aligned(w) \
+            w = norm._parameters.get("weight")
+            if w is None or w.dtype != torch.bfloat16 or w.device != x.device or not w.is_contiguous() or not _offset_aligned(w) \
                     or not isinstance(norm.eps, (int, float)):
                 return False
-        wq = wq._parameters
-        return wq["weight"].element_size() == 1 and wq["bias"] is None and self.stack_a()
+        w = wq._parameters.get("weight")
+        return w is not None and w.element_size() == 1 and wq._parameters.get("bias") is None and self.stack_a()
 
     def _attention_kernels_ok(self, q, positions: int, mask) -> bool:
         """Whether the attention behind the query projection can run on the fused kernels: a mask of one value per

@@ -43,6 +43,15 @@ def test_norms_that_the_latent_kernel_does_not_take(layer, name, what):
     assert not layer._latent_kernel_ok(x)
 
 
+@pytest.mark.parametrize("name", ["q_norm", "kv_norm", "wq_a", "wkv_a", "wq_b"])
+def test_weights_that_are_not_parameters(layer, name):
+    module = getattr(layer, name)
+    weight = module.weight.detach()
+    del module.weight
+    module.register_buffer("weight", weight)
+    assert not layer._latent_kernel_ok(torch.zeros(1, 2, 256, dtype=torch.bfloat16))
+
+
 def test_masks_that_the_attention_kernels_do_not_take(layer):
     q = torch.zeros(1, 2, 2, 192, dtype=torch.bfloat16)
     ones = torch.ones(2, 4)
