@@ -386,7 +386,8 @@ class MLA(nn.Module):
         """Whether the attention behind the query projection can run on the fused kernels: a mask of one value per
         (query, position) pair as the reference builds it (model.py:738-740), a positive softmax scale (the kernels work
         with maxima of unscaled scores) whose reciprocal binary32 holds."""
-        return (isinstance(self.softmax_scale, (int, float)) and 1e-30 < self.softmax_scale < 1e30 and q.dtype == torch.bfloat16 and q.is_contiguous()
+        return (isinstance(self.softmax_scale, (int, float)) and 1e-30 < self.softmax_scale < 1e30
+                and q.dtype == torch.bfloat16 and q.is_contiguous()
                 and (mask is None or (mask.device == q.device and mask.shape == (q.size(1), positions) and mask.is_contiguous()
                                       and mask.dtype in (torch.bfloat16, torch.float32))))
 
