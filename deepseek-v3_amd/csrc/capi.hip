@@ -383,21 +383,41 @@ size_t dsv3_mla_decode_workspace_bytes(int64_t batch, int64_t rows, int64_t posi
     return mla_decode_workspace_bytes(batch, rows, positions, heads);
 }
 
+static int mla_decode_checked(const void* q, const float* freqs, const void* kv_cache, int64_t kv_batch_stride,
+                              const void* pe_cache, int64_t pe_batch_stride, const void* wkv_b, const float* wkv_b_scale,
+                              const void* mask, int mask_dtype, void* y, float* s, bool quant, int64_t batch, int64_t rows,
+                              int64_t positions, int heads, int nope_dim, int rope_dim, int v_dim, int64_t kv_rank,
+                              float softmax_scale, void* workspace, size_t workspace_bytes, void* stream) {
+    const int rc = mla_validate(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, mask, mask_dtype, y, batch,
+                                rows, positions, heads, nope_dim, rope_dim, v_dim, kv_rank, softmax_scale);
+    if (rc != DSV3_OK || batch == 0 || rows == 0 || heads == 0) return rc;
+    if (!wkv_b || !wkv_b_scale || (quant && !s)) return DSV3_ERR_NULL_POINTER;
+    if (!aligned(wkv_b, 16) || !aligned(wkv_b_scale, 4) || !aligned(s, 4)) return DSV3_ERR_MISALIGNED;
+    if (!workspace || !aligned(workspace, 256) || workspace_bytes < mla_decode_workspace_bytes(batch, rows, positions, heads))
+        return DSV3_ERR_WORKSPACE;
+    return launch_mla_decode(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, wkv_b, wkv_b_scale, mask,
+                             mask_dtype == DSV3_F32, y, s, batch, rows, positions, heads, softmax_scale, workspace,
+                             (hipStream_t)stream);
+}
+
 int dsv3_mla_decode(const void* q, const float* freqs, const void* kv_cache, int64_t kv_batch_stride,
                     const void* pe_cache, int64_t pe_batch_stride, const void* wkv_b, const float* wkv_b_scale,
                     const void* mask, int mask_dtype, void* y, int64_t batch, int64_t rows, int64_t positions, int heads,
                     int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale, void* workspace,
                     size_t workspace_bytes, void* stream) {
-    const int rc = mla_validate(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, mask, mask_dtype, y, batch,
-                                rows, positions, heads, nope_dim, rope_dim, v_dim, kv_rank, softmax_scale);
-    if (rc != DSV3_OK || batch == 0 || rows == 0 || heads == 0) return rc;
-    if (!wkv_b || !wkv_b_scale) return DSV3_ERR_NULL_POINTER;
-    if (!aligned(wkv_b, 16) || !aligned(wkv_b_scale, 4)) return DSV3_ERR_MISALIGNED;
-    if (!workspace || !aligned(workspace, 256) || workspace_bytes < mla_decode_workspace_bytes(batch, rows, positions, heads))
-        return DSV3_ERR_WORKSPACE;
-    return launch_mla_decode(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, wkv_b, wkv_b_scale, mask,
-                             mask_dtype == DSV3_F32, y, batch, rows, positions, heads, softmax_scale, workspace,
-                             (hipStream_t)stream);
+    return mla_decode_checked(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, wkv_b, wkv_b_scale, mask,
+                              mask_dtype, y, nullptr, false, batch, rows, positions, heads, nope_dim, rope_dim, v_dim, kv_rank,
+                              softmax_scale, workspace, workspace_bytes, stream);
+}
+
+int dsv3_mla_decode_quant(const void* q, const float* freqs, const void* kv_cache, int64_t kv_batch_stride,
+                          const void* pe_cache, int64_t pe_batch_stride, const void* wkv_b, const float* wkv_b_scale,
+                          const void* mask, int mask_dtype, void* y, float* s, int64_t batch, int64_t rows, int64_t positions,
+                          int heads, int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale,
+                          void* workspace, size_t workspace_bytes, void* stream) {
+    return mla_decode_checked(q, freqs, kv_cache, kv_batch_stride, pe_cache, pe_batch_stride, wkv_b, wkv_b_scale, mask,
+                              mask_dtype, y, s, true, batch, rows, positions, heads, nope_dim, rope_dim, v_dim, kv_rank,
+                              softmax_scale, workspace, workspace_bytes, stream);
 }
 
 int dsv3_mla_latent(const void* a, int64_t a_stride, const void* q_norm, const void* kv_norm, const float* freqs,

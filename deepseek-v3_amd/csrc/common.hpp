@@ -204,8 +204,8 @@ int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t
                        int64_t rows, int64_t positions, int heads, float scale, void* workspace, hipStream_t st);
 size_t mla_decode_workspace_bytes(int64_t batch, int64_t tokens, int64_t positions, int heads);
 int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
-                      const void* w, const float* ws, const void* mask, bool mask_f32, void* y, int64_t batch, int64_t tokens,
-                      int64_t positions, int heads, float scale, void* workspace, hipStream_t st);
+                      const void* w, const float* ws, const void* mask, bool mask_f32, void* y, float* ys, int64_t batch,
+                      int64_t tokens, int64_t positions, int heads, float scale, void* workspace, hipStream_t st);
 int launch_mla_latent(const void* a, int64_t a_stride, const void* q_w, const void* kv_w, const void* freqs, void* kv,
                       int64_t kv_bs, void* pe, int64_t pe_bs, void* y, float* ys, int64_t batch, int64_t tokens, int q_rank,
                       float q_eps, float kv_eps, hipStream_t st);

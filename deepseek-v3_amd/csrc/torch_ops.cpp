@@ -244,6 +244,20 @@ Tensor mla_decode(const Tensor& q, const Tensor& freqs, const Tensor& kv, const 
     });
     return y;
 }
+// the same, rounded to bf16 and quantised per (token, head): the output projection's input
+tuple<Tensor, Tensor> mla_decode_quant(const Tensor& q, const Tensor& freqs, const Tensor& kv, const Tensor& pe, const Tensor& w,
+                                       const Tensor& ws, const OptTensor& mask, int64_t positions, double scale) {
+    Tensor y, ys;
+    attention(q, freqs, kv, pe, w, ws, mask, positions, dsv3_mla_decode_workspace_bytes,
+              [&](int64_t b, int64_t s, int h, int nope, int rope, int v, void* m, int md, void* buf, size_t need, void* stream) {
+        y = at::empty({b, s, (int64_t)h * v}, q.options().dtype(kFp8));
+        ys = at::empty({b, s, h}, q.options().dtype(at::kFloat));
+        check(dsv3_mla_decode_quant(q.data_ptr(), (const float*)freqs.data_ptr(), kv.data_ptr(), kv.stride(0), pe.data_ptr(), pe.stride(0),
+                                    w.data_ptr(), (const float*)ws.data_ptr(), m, md, y.data_ptr(), (float*)ys.data_ptr(), b, s, positions,
+                                    h, nope, rope, v, kv.size(2), (float)scale, buf, need, stream), "dsv3_mla_decode_quant");
+    });
+    return {y, ys};
+}
 
 // a [b, s, q_rank + kv_rank + rope] -> the normalised query latent, quantised, and the caches' rows start .. start + s - 1
 tuple<Tensor, Tensor> mla_latent(const Tensor& a, const Tensor& qn, const Tensor& kn, const Tensor& freqs, Tensor kv, Tensor pe,
@@ -278,5 +292,6 @@ TORCH_LIBRARY_IMPL(dsv3fp8, CUDA, m) {
     m.impl("swiglu_quant", swiglu_quant);
     m.impl("mla_prefill", mla_prefill);
     m.impl("mla_decode", mla_decode);
+    m.impl("mla_decode_quant", mla_decode_quant);
     m.impl("mla_latent", mla_latent);
 }

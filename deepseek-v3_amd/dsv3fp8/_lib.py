@@ -65,6 +65,9 @@ EXPORTS = {
     "dsv3_mla_decode": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
                                 c_void_p, c_int, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int,
                                 c_int64, c_float, c_void_p, c_size_t, c_void_p]),
+    "dsv3_mla_decode_quant": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p,
+                                 c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int,
+                                 c_int64, c_float, c_void_p, c_size_t, c_void_p]),
     "dsv3_mla_latent": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
                                 c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int, c_float, c_float, c_void_p]),
 }

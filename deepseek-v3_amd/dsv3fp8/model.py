@@ -426,10 +426,13 @@ class MLA(nn.Module):
             self.pe_cache[:b, start_pos:t] = apply_rotary_emb(kva[..., self.kv_lora_rank:].unsqueeze(2), freqs_cis).squeeze(2)
         if kernels and self._attention_kernels_ok(q, t, mask):
             args = (q, freqs_cis, self.kv_cache, self.pe_cache, self.wkv_b.weight, self.wkv_b.scale, mask, t, self.softmax_scale)
-            if not self._explicit_pays(b, s, t):
-                return self.wo(torch.ops.dsv3fp8.mla_decode(*args))
+            explicit = self._explicit_pays(b, s, t)
+            # the attention's last kernel quantises for wo, unless wo was exchanged, carries hooks or is no FP8 layer
             if _plain(self.wo, RowParallelLinear) and self.wo.weight.element_size() == 1 and self.wo.bias is None:
-                return fp8_gemm(*torch.ops.dsv3fp8.mla_prefill(*args), self.wo.weight, self.wo.weight.scale)
+                op = torch.ops.dsv3fp8.mla_prefill if explicit else torch.ops.dsv3fp8.mla_decode_quant
+                return fp8_gemm(*op(*args), self.wo.weight, self.wo.weight.scale)
+            if not explicit:
+                return self.wo(torch.ops.dsv3fp8.mla_decode(*args))
         wkv_b = self._dequantised_wkv_b(x)
         latent, rope_keys = self.kv_cache[:b, :t], self.pe_cache[:b, :t]
         # scores over the latent (query folded through wkv_b) plus the rotary part; softmax in binary32

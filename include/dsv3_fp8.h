@@ -370,6 +370,12 @@ int dsv3_mla_decode(const void* q, const float* freqs, const void* kv_cache, int
                     const void* mask, int mask_dtype, void* y, int64_t batch, int64_t rows, int64_t positions, int heads,
                     int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale, void* workspace,
                     size_t workspace_bytes, void* stream);
+/* dsv3_mla_decode whose result, rounded to bf16, is quantised per (token, head) as dsv3_mla_prefill's: y e4m3, s [batch, rows, heads]. */
+int dsv3_mla_decode_quant(const void* q, const float* freqs, const void* kv_cache, int64_t kv_batch_stride,
+                          const void* pe_cache, int64_t pe_batch_stride, const void* wkv_b, const float* wkv_b_scale,
+                          const void* mask, int mask_dtype, void* y, float* s, int64_t batch, int64_t rows, int64_t positions, int heads,
+                          int nope_dim, int rope_dim, int v_dim, int64_t kv_rank, float softmax_scale, void* workspace,
+                          size_t workspace_bytes, void* stream);
 
 /*
  * What MLA.forward does between the low-rank projections and the query's up-projection (inference/model.py:457-466 and

@@ -134,6 +134,23 @@ def test_decode_attention(b, s, t, h, kind, grow):
     assert ((got - ref).norm(dim=-1) <= 2.0 ** -7 * ref.norm(dim=-1)).all()
 
 
+# tokens in all: 1, 2, 3 .. 4, 5 .. 8 and more share a workgroup's wavefronts differently, 16 are a group; splits below, at and
+# above a wavefront's 64 lanes (256 workgroups over the row blocks, 32 positions a tile)
+@pytest.mark.parametrize("b,s,t,h", [(1, 1, 33, 128), (1, 1, 2080, 128), (1, 1, 8192, 8), (2, 1, 700, 128), (3, 1, 5000, 16),
+                                     (4, 1, 90, 128), (1, 5, 300, 128), (8, 1, 1, 128), (16, 1, 257, 128), (17, 1, 64, 32), (3, 13, 200, 24)])
+def test_decode_attention_quantised_is_the_rounded_result_quantised(b, s, t, h):
+    from dsv3fp8 import kernel
+    q, freqs, kv, pe, w8, ws = _inputs(b, s, t, h, s + t)
+    args = (q, freqs, kv, pe, w8, ws, None, t, 0.08)
+    y = torch.ops.dsv3fp8.mla_decode(*args)
+    ref = _decode_reference(*args)
+    got = y.view(b, s, h, V).double()
+    assert ((got - ref).norm(dim=-1) <= 2.0 ** -7 * ref.norm(dim=-1)).all()         # as in test_decode_attention
+    yq, ys = torch.ops.dsv3fp8.mla_decode_quant(*args)
+    rq, rs = kernel.act_quant(y)
+    assert torch.equal(yq.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(ys, rs)
+
+
 LATENT = [(1, 1, 0, 1536), (3, 1, 7, 1536), (2, 5, 0, 128), (1, 40, 3, 2048), (2, 33, 1, 640)]
 
 
