@@ -28,7 +28,7 @@ constexpr int kRows = 128;                              // rows per workgroup: 4
 constexpr int kPartFloats = kRows * kC;                 // partial sums of a workgroup
 
 struct DecodeArgs {
-    const uint16_t* ql;                                 // folded queries [batch][rows][512], rows = tokens * heads
+    const void* ql;                                     // folded queries [batch][rows][512], rows = tokens * heads, or in operand order
     const uint16_t* q;                                  // queries [batch][rows][192]: their rotary part is read here
     const v2f* freqs;                                   // [tokens][32] (cos, sin)
     const uint16_t* kv; int64_t kv_bs;                  // latent cache, batch stride in elements
@@ -67,8 +67,10 @@ __device__ __forceinline__ void scale_agprs(v16f& v, float a) {
 // sequences at 4096 positions (16 tiles a workgroup): 53 .. 58 us, 70 with each LDS read next to its MFMA; 12 us of it are the 67 MB
 // of partial sums at the end, and one tile alone (a short context) takes 12 us in all.  The tensor operations in its place
 // took 250 us (58 us in the products, the rest in passes over the scores).
+// PACK: the folded queries come in operand order (launch_wkv_b_absorb_q_packed), a KiB of consecutive bytes per load; as rows a
+// load touches 32 of them and takes 64 cycles of the compute unit's load path, 3.8 us for the workgroup's 128.
 enum { kNoMask, kMaskBf16, kMaskF32 };
-template <int MASK>
+template <int MASK, bool PACK>
 __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
     const int split = blockIdx.x, b = blockIdx.y, blk = blockIdx.z;
     const int t0 = split * p.per, t1 = min(p.tiles, t0 + p.per);
     const int row0 = blk * kRows + wave * 32;
-    const int row = min(row0 + i, p.rows - 1);          // rows past the end repeat the last one; combine leaves them out
+    const int row = min(row0 + i, p.rows - 1);          // rows past the end repeat the last one; fold leaves them out
 
     const uint16_t* kvb = p.kv + b * p.kv_bs;
     const uint16_t* peb = p.pe + b * p.pe_bs;
@@ -100,9 +102,10 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
     // lane (row i, half g) holds elements 16 s + 8 g .. + 7; the last four steps are rotated here
     v4u Q[36];
     {
-        const uint16_t* src = p.ql + ((int64_t)b * p.rows + row) * kC + 8 * g;
+        // (packed, a last block's missing rows hold anything; nobody reads their results)
+        const v4u* src = (const v4u*)p.ql + (PACK ? (((int64_t)b * p.blocks + blk) * 4 + wave) * (kC / 16) * 64 + lane : ((int64_t)b * p.rows + row) * (kC / 8) + g);
 #pragma unroll
-        for (int s = 0; s < 32; ++s) Q[s] = *(const v4u*)(src + 16 * s);
+        for (int s = 0; s < 32; ++s) Q[s] = src[s * (PACK ? 64 : 2)];
         const uint16_t* rsrc = p.q + ((int64_t)b * p.rows + row) * kQd + kNope + 8 * g;
         const v2f* fr = p.freqs + (int64_t)(row / p.heads) * (kRope / 2) + 4 * g;
 #pragma unroll
@@ -170,7 +173,8 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
         mx = fmaxf(mx, xor32(mx));
         // The maximum is only raised when it grows by more than 2^64: exponentials and sums have room for that in binary32
         // and bf16, and so the 256 multiplications are needed in the rarest of cases.
-        const bool raise = (mx - m) * scale2 > 64.f || (m == -__builtin_inff() && mx > m);
+        // (Rows past the end, whose queries are whatever the scratch held, do not ask for it: the others' roundings would follow.)
+        const bool raise = row0 + i < p.rows && ((mx - m) * scale2 > 64.f || (m == -__builtin_inff() && mx > m));
         if (__any(raise)) {
             const float mn = fmaxf(m, mx);
             const float a = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f((m - mn) * scale2);
@@ -486,8 +490,6 @@ __global__ __launch_bounds__(320) void mla_latent_kernel(LatentArgs p) {
     }
 }
 
-inline int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
-
 // How the positions of a step are split: one attend workgroup per compute unit (its LDS and registers take a whole one; fewer
 // leave units idle, more write more partial sums), a tile each at least.
 void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) {
@@ -507,7 +509,7 @@ size_t mla_decode_workspace_bytes(int64_t batch, int64_t tokens, int64_t positio
     DecodeArgs a;
     decode_plan(a, batch, tokens * heads, positions);
     const int64_t units = batch * a.blocks * a.splits;
-    return (size_t)(align256(batch * a.rows * kC * 2) + units * (kPartFloats * 4 + kRows * 8));
+    return (size_t)(batch * a.blocks * (kRows * kC * 2) + units * (kPartFloats * 4 + kRows * 8));
 }
 
 int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
@@ -518,22 +520,28 @@ int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t 
     decode_plan(a, batch, tokens * heads, positions);
     if (a.blocks > 65535) return DSV3_ERR_BAD_SHAPE;
     uint8_t* wsp = (uint8_t*)workspace;
-    const int64_t lat = align256(batch * a.rows * kC * 2), units = batch * a.blocks * a.splits;
-    uint16_t* ql = (uint16_t*)wsp;
-    a.part = (float*)(wsp + lat);
+    const int64_t units = batch * a.blocks * a.splits;
+    a.part = (float*)(wsp + batch * a.blocks * (kRows * kC * 2));
     a.ml = (v2f*)(a.part + units * kPartFloats);
-    a.ql = ql; a.q = (const uint16_t*)q; a.freqs = (const v2f*)freqs;
+    a.ql = wsp; a.q = (const uint16_t*)q; a.freqs = (const v2f*)freqs;
     a.kv = (const uint16_t*)kv; a.kv_bs = kv_bs; a.pe = (const uint16_t*)pe; a.pe_bs = pe_bs;
     a.mask = mask; a.heads = heads;
     const ScoreUnit u = mask ? score_unit(scale) : ScoreUnit{ 1.f, scale };
     a.unit = u.unit; a.scale = u.rest; a.inv_scale = 1.0f / u.rest;
-    int rc = launch_wkv_b_absorb(q, (int64_t)heads * kQd, kQd, w, ws, ql, DSV3_ABSORB_Q, batch * tokens, heads, kNope, kNope, kC, st);
+    // Operand order up to 16 tokens in all: the attention gains 2 us (1 at 700: 12.7 -> 10.7, 3 at 200: 12.4 -> 10.3, 8 at 2000: 24.2 ->
+    // 22.2), the fold's scattered stores cost it 0.4.  With more they cost 1 to 1.7 us (32 tokens 5.1 -> 6.1, 64 6.2 -> 7.8), the gain
+    // disappears behind the tiles (32 at 4096: 56.7 -> 56.4, 64 at 1000: 39.7 -> 39.6).
+    const bool pack = batch * tokens <= 16;
+    const int rc = pack ? launch_wkv_b_absorb_q_packed(q, (int64_t)heads * kQd, kQd, w, ws, wsp, batch, tokens, a.blocks, heads, kNope, kNope, st)
+                        : launch_wkv_b_absorb(q, (int64_t)heads * kQd, kQd, w, ws, wsp, DSV3_ABSORB_Q, batch * tokens, heads, kNope, kNope, kC, st);
     if (rc != DSV3_OK) return rc;
-    const int which = !mask ? kNoMask : mask_f32 ? kMaskF32 : kMaskBf16;
-    void (*const kernel)(DecodeArgs) = !mask ? mla_decode_kernel<kNoMask> : mask_f32 ? mla_decode_kernel<kMaskF32> : mla_decode_kernel<kMaskBf16>;
-    static LdsGrant grant[3];
-    if (!grant[which].ensure((const void*)kernel, kStages * kStage)) return DSV3_ERR_LAUNCH;
-    hipLaunchKernelGGL(kernel, dim3(a.splits, (unsigned)batch, a.blocks), dim3(256), kStages * kStage, st, a);
+    const int which = (!mask ? kNoMask : mask_f32 ? kMaskF32 : kMaskBf16) * 2 + pack;
+    static void (*const kernels[6])(DecodeArgs) = { mla_decode_kernel<kNoMask, false>, mla_decode_kernel<kNoMask, true>,
+                                                    mla_decode_kernel<kMaskBf16, false>, mla_decode_kernel<kMaskBf16, true>,
+                                                    mla_decode_kernel<kMaskF32, false>, mla_decode_kernel<kMaskF32, true> };
+    static LdsGrant grant[6];
+    if (!grant[which].ensure((const void*)kernels[which], kStages * kStage)) return DSV3_ERR_LAUNCH;
+    hipLaunchKernelGGL(kernels[which], dim3(a.splits, (unsigned)batch, a.blocks), dim3(256), kStages * kStage, st, a);
     FoldArgs f;
     f.part = a.part; f.ml = a.ml; f.w = (const uint8_t*)w; f.ws = ws; f.y = y; f.ys = ys;
     f.tokens = (int)(batch * tokens); f.per_seq = (int)tokens; f.heads = heads; f.blocks = a.blocks; f.splits = a.splits;

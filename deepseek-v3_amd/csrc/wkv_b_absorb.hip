@@ -50,7 +50,19 @@ struct AbsorbArgs {
     int heads, head_rows, nope, n_out;
     int slabs;              // feature slabs per head (side Q: C/128, side V: v/32)
     int subtiles;           // ceil(tokens / 16)
+    int per_seq, blocks;    // (packed side Q) tokens and 128-row blocks per sequence
 };
+
+// Where the 16-byte piece of features f .. f + 7 of (token, head h) goes on side Q.  PACK: in the order in which the attention
+// over the latents (mla_decode.hip) reads its queries as MFMA operands: [sequence][block of 128 (token, head) rows][32 rows]
+// [K step of 16 features][half of 8][row].
+template <bool PACK>
+__device__ __forceinline__ v4u* q_piece(const AbsorbArgs& p, int64_t tok, int h, int f) {
+    if (!PACK) return (v4u*)(p.y + (tok * p.heads + h) * p.n_out + f);
+    const int t = (int)tok, b = t / p.per_seq, row = (t - b * p.per_seq) * p.heads + h;
+    const int64_t rows32 = ((int64_t)b * p.blocks + (row >> 7)) * 4 + ((row >> 5) & 3);
+    return (v4u*)p.y + (rows32 * (p.n_out / 16) + (f >> 4)) * 64 + ((f >> 3) & 1) * 32 + (row & 31);
+}
 
 // 8 fp8 bytes -> 8 binary32
 __device__ __forceinline__ void cvt8(v2u p, float (&f)[8]) {
@@ -376,11 +388,13 @@ __global__ __launch_bounds__(256) void absorb_v_staged_kernel(AbsorbArgs p) {
 // wavefront reads the whole slab's fragments back and takes every fourth 16-token sub-tile.  An output element is
 // still formed by one wavefront over the whole K range in the same order, so the results are those of the kernels
 // above bit for bit.
-template <int KS, int PF>
+// PACK: the pieces of eight consecutive heads fill a line, so that these heads (a run of heads / 8) are given to one XCD.
+template <int KS, int PF, bool PACK = false>
 __global__ __launch_bounds__(256) void absorb_q_shared_kernel(AbsorbArgs p) {
     __shared__ v4u frag[KS * 8 * 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int slab = blockIdx.y, h = blockIdx.x, i = lane & 15, g = lane >> 4;
+    const int slab = blockIdx.y, i = lane & 15, g = lane >> 4;
+    const int h = PACK && p.heads % 8 == 0 ? (blockIdx.x & 7) * (p.heads >> 3) + (blockIdx.x >> 3) : blockIdx.x;
     const int c0 = slab * 128;
     const int64_t row0 = (int64_t)h * p.head_rows;
     const int stride = gridDim.z * 4;
@@ -449,7 +463,7 @@ __global__ __launch_bounds__(256) void absorb_q_shared_kernel(AbsorbArgs p) {
             v4u o;
 #pragma unroll
             for (int q = 0; q < 4; ++q) o[q] = pack_bf16(acc[2 * q][j], acc[2 * q + 1][j]);
-            *(v4u*)(p.y + (tok * p.heads + h) * p.n_out + c0 + i * 8) = o;
+            *q_piece<PACK>(p, tok, h, c0 + i * 8) = o;
         }
     }
 }
@@ -625,6 +639,20 @@ int launch_wkv_b_absorb(const void* x, int64_t x_ts, int64_t x_hs, const void* w
         else if (kv_rank == 256) hipLaunchKernelGGL(absorb_v_kernel<2>, grid, block, 0, st, p);
         else hipLaunchKernelGGL(absorb_v_kernel<1>, grid, block, 0, st, p);
     }
+    return launch_status();
+}
+
+// Side Q of batch x per_seq <= 16 new tokens, C == 512 and nope == 128, in the attention's operand order (q_piece): y holds
+// batch x blocks x 128 rows of 512, blocks = ceil(per_seq * heads / 128); rows past a sequence's last one are not written.
+int launch_wkv_b_absorb_q_packed(const void* x, int64_t x_ts, int64_t x_hs, const void* w, const float* ws, void* y,
+                                 int64_t batch, int64_t per_seq, int blocks, int heads, int nope, int v, hipStream_t st) {
+    if (nope != 128 || batch * per_seq > 16) return DSV3_ERR_BAD_SHAPE;
+    AbsorbArgs p;
+    p.x = (const uint16_t*)x; p.x_ts = x_ts; p.x_hs = x_hs;
+    p.w = (const uint8_t*)w; p.ws = ws; p.w_cols = 512; p.ws_cols = 4;
+    p.y = (uint16_t*)y; p.tokens = batch * per_seq; p.heads = heads; p.head_rows = nope + v; p.nope = nope;
+    p.subtiles = 1; p.n_out = 512; p.slabs = 4; p.per_seq = (int)per_seq; p.blocks = blocks;
+    hipLaunchKernelGGL((absorb_q_shared_kernel<4, 1, true>), dim3(heads, p.slabs), dim3(256), 0, st, p);
     return launch_status();
 }
 
