@@ -323,11 +323,23 @@ inline Plan make_plan_mt(int64_t m, int64_t n, int64_t k, int mt_min) {
     return p;
 }
 
-inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
+inline Plan search_plan(int64_t m, int64_t n, int64_t k) {
     Plan p = make_plan_mt(m, n, k, 1);
     // 9 .. 16 rows on a K range without one-sub-tile chunks: two sub-tiles, the second one padding
     if (!p.ok && m >= 9 && m <= 16) p = make_plan_mt(m, n, k, 2);
     return p;
+}
+
+// The search prices some hundred candidates, 0.8 us at 7168 -> 576 and 2.4 at 16384 -> 7168, and a linear layer's call wants the
+// plan eight times (the size of its scratch, the choice of the kernel, the launch): 16384 -> 7168 at 32 rows spent 15 of its
+// 24 us on the host there.  Plans depend on the sizes alone; each thread keeps its last ones (not pinned ones: those change).
+inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
+    if (m < 1 || m > 64 || std::getenv("DSV3_STREAM_PLAN")) return search_plan(m, n, k);
+    struct Kept { int64_t m, n, k; Plan p; };
+    static thread_local Kept kept[32];
+    Kept& e = kept[(uint64_t)(m * 7 + (n >> 6) * 5 + (k >> 7)) % 32];
+    if (e.m != m || e.n != n || e.k != k) e = Kept{ m, n, k, search_plan(m, n, k) };
+    return e.p;
 }
 
 template <int MT, int NPF>

@@ -280,6 +280,22 @@ tuple<Tensor, Tensor> mla_latent(const Tensor& a, const Tensor& qn, const Tensor
     return {y, ys};
 }
 
+// The operators above as MLA.forward strings them together, in one call each: a decode step of a few sequences is bound by the
+// host, and an operator's way through Python and the dispatcher takes 3 to 5 us.
+// x [b, s, dim] -> per-head queries [b, s, heads, d]; the caches get the new rows
+Tensor mla_query(const Tensor& x, const Tensor& wa, const Tensor& wa_s, const Tensor& qn, const Tensor& kn, const Tensor& freqs,
+                 Tensor kv, Tensor pe, int64_t start, double q_eps, double kv_eps, const Tensor& wq, const Tensor& wq_s, int64_t heads) {
+    TORCH_CHECK(x.dim() == 3 && heads > 0 && wq.dim() == 2 && wq.size(0) % heads == 0, "mla_query: x must be [b, s, dim], the query's weight [heads * d, q_rank]");
+    const auto [y, ys] = mla_latent(linear_fp8(x, wa, wa_s, DSV3_SCALE_FMT_NONE, DSV3_BF16), qn, kn, freqs, kv, pe, start, q_eps, kv_eps);
+    return fp8_gemm(y, ys, wq, wq_s, DSV3_BF16).view({x.size(0), x.size(1), heads, wq.size(0) / heads});
+}
+// queries and caches -> the layer's output [b, s, dim]
+Tensor mla_output(const Tensor& q, const Tensor& freqs, const Tensor& kv, const Tensor& pe, const Tensor& w, const Tensor& ws,
+                  const OptTensor& mask, int64_t positions, double scale, bool explicit_form, const Tensor& wo, const Tensor& wo_s) {
+    const auto [y, ys] = (explicit_form ? mla_prefill : mla_decode_quant)(q, freqs, kv, pe, w, ws, mask, positions, scale);
+    return fp8_gemm(y, ys, wo, wo_s, DSV3_BF16);
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(dsv3fp8, CUDA, m) {
@@ -294,4 +310,6 @@ TORCH_LIBRARY_IMPL(dsv3fp8, CUDA, m) {
     m.impl("mla_decode", mla_decode);
     m.impl("mla_decode_quant", mla_decode_quant);
     m.impl("mla_latent", mla_latent);
+    m.impl("mla_query", mla_query);
+    m.impl("mla_output", mla_output);
 }

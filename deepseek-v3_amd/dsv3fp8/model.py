@@ -85,6 +85,9 @@ def _scales_are_powers_of_two(weight: torch.Tensor, scale: Optional[torch.Tensor
     return flag
 
 
+_linear_fp8 = torch.ops.dsv3fp8.linear_fp8.default
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
            scale_fmt: Optional[str] = None) -> torch.Tensor:
     """y = x @ weight.T + bias with the reference's three-way dispatch (model.py:153-163): wide weights go to
@@ -103,7 +106,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
             and x.size(-1) % block_size == 0):
         # the same two steps behind one op, which runs them as a single launch for few rows (decode)
         fmt = ops._lib.SCALE_FMT_UE8M0 if scale_fmt == "ue8m0" else ops._lib.SCALE_FMT_NONE
-        y = torch.ops.dsv3fp8.linear_fp8(x, weight, weight.scale, fmt, ops.dtype_code(torch.get_default_dtype()))
+        y = _linear_fp8(x, weight, weight.scale, fmt, ops.dtype_code(torch.get_default_dtype()))
     else:
         xq, xs = act_quant(x, block_size, scale_fmt)
         y = fp8_gemm(xq, xs, weight, weight.scale)
@@ -225,6 +228,10 @@ def _offset_aligned(t: torch.Tensor) -> bool:
     return t.storage_offset() * t.element_size() % 16 == 0
 
 
+_mla_query = torch.ops.dsv3fp8.mla_query.default
+_mla_output = torch.ops.dsv3fp8.mla_output.default
+
+
 class MLA(nn.Module):
     """Multi-head latent attention (model.py:395-497).
 
@@ -239,7 +246,7 @@ class MLA(nn.Module):
     the new positions' latents (an FP8 GEMM through ``linear()``), and the scores and the weighted sum are plain
     per-head einsums.
     Without gradients, with FP8 weights and the head dimensions of the 671B configuration, everything between the
-    low-rank projections and ``wo`` runs on kernels (``torch.ops.dsv3fp8.{mla_latent, mla_decode, mla_prefill}``; the
+    low-rank projections and ``wo`` runs on kernels (``torch.ops.dsv3fp8.{mla_query, mla_output}`` and what these consist of; the
     conditions are ``_kernels_ok``, ``_latent_kernel_ok`` and ``_attention_kernels_ok``).  Other calls run the scores, the
     softmax and the weighted sum as bf16 torch operations between the two products; ``MLA.fused = False`` takes
     the dequantise-then-einsum sequence for the products too.  Parameter names are the checkpoint's.
@@ -413,10 +420,17 @@ class MLA(nn.Module):
         t = start_pos + s
         kernels = self._kernels_ok(x, start_pos, freqs_cis)
         if kernels and self._latent_kernel_ok(x):
-            qq, qs = torch.ops.dsv3fp8.mla_latent(linear(x, self._wa, None, self.wq_a.scale_fmt), self.q_norm.weight,
-                                                  self.kv_norm.weight, freqs_cis, self.kv_cache, self.pe_cache, start_pos,
-                                                  self.q_norm.eps, self.kv_norm.eps)
-            q = fp8_gemm(qq, qs, self.wq_b.weight, self.wq_b.weight.scale).unflatten(-1, (self.n_local_heads, self.qk_head_dim))
+            caches, modules = self._buffers, self._modules
+            wq = modules["wq_b"]._parameters["weight"]
+            if x.is_contiguous() and x.size(-1) % block_size == 0 and wq.is_contiguous() and self.wq_a.scale_fmt != "ue8m0":
+                qn, kn = modules["q_norm"], modules["kv_norm"]
+                q = _mla_query(x, self._wa, self._wa.scale, qn._parameters["weight"], kn._parameters["weight"], freqs_cis,
+                               caches["kv_cache"], caches["pe_cache"], start_pos, qn.eps, kn.eps, wq, wq.scale, self.n_local_heads)
+            else:
+                qq, qs = torch.ops.dsv3fp8.mla_latent(linear(x, self._wa, None, self.wq_a.scale_fmt), self.q_norm.weight,
+                                                      self.kv_norm.weight, freqs_cis, self.kv_cache, self.pe_cache, start_pos,
+                                                      self.q_norm.eps, self.kv_norm.eps)
+                q = fp8_gemm(qq, qs, wq, wq.scale).unflatten(-1, (self.n_local_heads, self.qk_head_dim))
         else:
             q, kva = self._project(x)
             if self.attn_impl == "naive":
@@ -428,9 +442,9 @@ class MLA(nn.Module):
             args = (q, freqs_cis, self.kv_cache, self.pe_cache, self.wkv_b.weight, self.wkv_b.scale, mask, t, self.softmax_scale)
             explicit = self._explicit_pays(b, s, t)
             # the attention's last kernel quantises for wo, unless wo was exchanged, carries hooks or is no FP8 layer
-            if _plain(self.wo, RowParallelLinear) and self.wo.weight.element_size() == 1 and self.wo.bias is None:
-                op = torch.ops.dsv3fp8.mla_prefill if explicit else torch.ops.dsv3fp8.mla_decode_quant
-                return fp8_gemm(*op(*args), self.wo.weight, self.wo.weight.scale)
+            wo = self._modules["wo"]
+            if _plain(wo, RowParallelLinear) and wo.weight.element_size() == 1 and wo.bias is None and wo.weight.is_contiguous():
+                return _mla_output(*args, explicit, wo.weight, wo.weight.scale)
             if not explicit:
                 return self.wo(torch.ops.dsv3fp8.mla_decode(*args))
         wkv_b = self._dequantised_wkv_b(x)

@@ -2,7 +2,7 @@
 
 ``torch.ops.dsv3fp8.{act_quant, weight_dequant, weight_quant, fp8_gemm}`` and the grouped
 mixture-of-experts ops ``{gate_route, group_tiles, moe_route, fp8_gemm_grouped, swiglu_quant, moe_combine}`` and the
-attention ops ``{wkv_b_absorb, mla_latent, mla_decode, mla_decode_quant, mla_prefill}`` take and return torch tensors; the device
+attention ops ``{wkv_b_absorb, mla_latent, mla_decode, mla_decode_quant, mla_prefill, mla_query, mla_output}`` take and return torch tensors; the device
 implementations (native in libdsv3torch.so, the mixture-of-experts ones and ``wkv_b_absorb`` below) hand raw device pointers
 and the current HIP stream of the tensors' device to libdsv3fp8.so.  Only a device
 ("CUDA" dispatch key, which is HIP on ROCm) implementation and a shape-only Meta
@@ -45,6 +45,10 @@ _libdef.define("mla_decode_quant(Tensor q, Tensor freqs, Tensor kv_cache, Tensor
                "Tensor? mask, int positions, float softmax_scale) -> (Tensor, Tensor)")
 _libdef.define("mla_latent(Tensor a, Tensor q_norm, Tensor kv_norm, Tensor freqs, Tensor(a!) kv_cache, Tensor(b!) pe_cache, "
                "int start, float q_eps, float kv_eps) -> (Tensor, Tensor)")
+_libdef.define("mla_query(Tensor x, Tensor wa, Tensor wa_scale, Tensor q_norm, Tensor kv_norm, Tensor freqs, Tensor(a!) kv_cache, "
+               "Tensor(b!) pe_cache, int start, float q_eps, float kv_eps, Tensor wq_b, Tensor wq_b_scale, int heads) -> Tensor")
+_libdef.define("mla_output(Tensor q, Tensor freqs, Tensor kv_cache, Tensor pe_cache, Tensor wkv_b, Tensor scale, Tensor? mask, "
+               "int positions, float softmax_scale, bool explicit, Tensor wo, Tensor wo_scale) -> Tensor")
 _libdef.define("wkv_b_absorb(Tensor x, Tensor wkv_b, Tensor scale, int side, int nope_dim, int v_dim) -> Tensor")
 
 
@@ -288,6 +292,14 @@ def _mla_latent_meta(a, q_norm, kv_norm, freqs, kv_cache, pe_cache, start, q_eps
     return (a.new_empty(b, s, q_norm.numel(), dtype=FP8), a.new_empty(b, s, q_norm.numel() // 128, dtype=torch.float32))
 
 
+def _mla_query_meta(x, wa, wa_scale, q_norm, kv_norm, freqs, kv_cache, pe_cache, start, q_eps, kv_eps, wq_b, wq_b_scale, heads):
+    return x.new_empty(x.size(0), x.size(1), heads, wq_b.size(0) // heads)
+
+
+def _mla_output_meta(q, freqs, kv_cache, pe_cache, wkv_b, scale, mask, positions, softmax_scale, explicit, wo, wo_scale):
+    return q.new_empty(q.size(0), q.size(1), wo.size(0))
+
+
 _lib.require(_lib.TORCH_LIB_PATH)
 torch.ops.load_library(str(_lib.TORCH_LIB_PATH))       # the device implementations of csrc/torch_ops.cpp
 
@@ -301,6 +313,7 @@ for _name, _meta in (("act_quant", _act_quant_meta), ("weight_dequant", _weight_
                      ("weight_quant", _weight_quant_meta), ("fp8_gemm", _fp8_gemm_meta), ("fp8_gemm_pow2", _fp8_gemm_meta),
                      ("linear_fp8", _linear_fp8_meta), ("swiglu_quant", _swiglu_quant_meta),
                      ("mla_prefill", _mla_prefill_meta), ("mla_decode", _mla_decode_meta), ("mla_decode_quant", _mla_prefill_meta), ("mla_latent", _mla_latent_meta),
+                     ("mla_query", _mla_query_meta), ("mla_output", _mla_output_meta),
                      ("wkv_b_absorb", _wkv_b_absorb_meta), ("gate_route", _gate_route_meta),
                      ("group_tiles", _group_tiles_meta), ("moe_route", _moe_route_meta),
                      ("fp8_gemm_grouped", _fp8_gemm_grouped_meta), ("fp8_gemm_grouped_pow2", _fp8_gemm_grouped_meta),
