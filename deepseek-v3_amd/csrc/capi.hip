@@ -420,10 +420,10 @@ int dsv3_mla_decode_quant(const void* q, const float* freqs, const void* kv_cach
                               softmax_scale, workspace, workspace_bytes, stream);
 }
 
-int dsv3_mla_latent(const void* a, int64_t a_stride, const void* q_norm, const void* kv_norm, const float* freqs,
-                    void* kv_rows, int64_t kv_batch_stride, void* pe_rows, int64_t pe_batch_stride, void* y, float* s,
-                    int64_t batch, int64_t rows, int64_t q_rank, int64_t kv_rank, int rope_dim, float q_eps, float kv_eps,
-                    void* stream) {
+static int mla_latent_validate(const void* a, int64_t a_stride, const void* q_norm, const void* kv_norm, const float* freqs,
+                               const void* kv_rows, int64_t kv_batch_stride, const void* pe_rows, int64_t pe_batch_stride,
+                               const void* y, const float* s, int64_t batch, int64_t rows, int64_t q_rank, int64_t kv_rank,
+                               int rope_dim) {
     if (kv_rank != 512 || rope_dim != 64 || q_rank < 128 || q_rank > 2048 || q_rank % 128 != 0) return DSV3_ERR_BAD_SHAPE;
     if (batch < 0 || rows < 0 || batch > 65535 || rows > 0x7fffff || batch * rows > 0x7fffffff || a_stride % 8 != 0 ||
         a_stride < q_rank + kv_rank + rope_dim)
@@ -436,8 +436,36 @@ int dsv3_mla_latent(const void* a, int64_t a_stride, const void* q_norm, const v
     if (!aligned(a, 16) || !aligned(q_norm, 16) || !aligned(kv_norm, 16) || !aligned(freqs, 8) || !aligned(kv_rows, 16) ||
         !aligned(pe_rows, 16) || !aligned(y, 16) || !aligned(s, 4))
         return DSV3_ERR_MISALIGNED;
-    return launch_mla_latent(a, a_stride, q_norm, kv_norm, freqs, kv_rows, kv_batch_stride, pe_rows, pe_batch_stride, y, s,
-                             batch, rows, (int)q_rank, q_eps, kv_eps, (hipStream_t)stream);
+    return DSV3_OK;
+}
+
+int dsv3_mla_latent(const void* a, int64_t a_stride, const void* q_norm, const void* kv_norm, const float* freqs,
+                    void* kv_rows, int64_t kv_batch_stride, void* pe_rows, int64_t pe_batch_stride, void* y, float* s,
+                    int64_t batch, int64_t rows, int64_t q_rank, int64_t kv_rank, int rope_dim, float q_eps, float kv_eps,
+                    void* stream) {
+    const int rc = mla_latent_validate(a, a_stride, q_norm, kv_norm, freqs, kv_rows, kv_batch_stride, pe_rows, pe_batch_stride, y, s,
+                                       batch, rows, q_rank, kv_rank, rope_dim);
+    if (rc != DSV3_OK || batch == 0 || rows == 0) return rc;
+    return launch_mla_latent(a, a_stride, nullptr, 0, q_norm, kv_norm, freqs, kv_rows, kv_batch_stride, pe_rows, pe_batch_stride, y,
+                             s, batch, rows, (int)q_rank, q_eps, kv_eps, (hipStream_t)stream);
+}
+
+int dsv3_mla_latent_gemm(const void* x, const float* x_s, const void* w, const float* w_s, int64_t k, void* a, const void* q_norm,
+                         const void* kv_norm, const float* freqs, void* kv_rows, int64_t kv_batch_stride, void* pe_rows,
+                         int64_t pe_batch_stride, void* y, float* s, int64_t batch, int64_t rows, int64_t q_rank, int64_t kv_rank,
+                         int rope_dim, float q_eps, float kv_eps, void* workspace, size_t workspace_bytes, void* stream) {
+    const int64_t n = q_rank + kv_rank + rope_dim, m = batch * rows;
+    const int rc = mla_latent_validate(a, n, q_norm, kv_norm, freqs, kv_rows, kv_batch_stride, pe_rows, pe_batch_stride, y, s, batch,
+                                       rows, q_rank, kv_rank, rope_dim);
+    if (rc != DSV3_OK || batch == 0 || rows == 0) return rc;
+    if (k % 128 != 0) return DSV3_ERR_BAD_SHAPE;
+    const int rc_g = fp8_gemm_validate(x, x_s, w, w_s, a, DSV3_BF16, m, n, k, workspace, workspace_bytes);
+    if (rc_g != DSV3_OK) return rc_g;
+    int slabs = 0;
+    const int rc_l = launch_fp8_gemm_slabs(x, x_s, w, w_s, a, m, n, k, workspace, &slabs, (hipStream_t)stream);
+    if (rc_l != DSV3_OK) return rc_l;
+    return launch_mla_latent(a, n, (const float*)workspace, slabs, q_norm, kv_norm, freqs, kv_rows, kv_batch_stride, pe_rows,
+                             pe_batch_stride, y, s, batch, rows, (int)q_rank, q_eps, kv_eps, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -165,7 +165,9 @@ bool linear_fp8_supported(int64_t m, int64_t n, int64_t k);
 size_t prefill_workspace_bytes(int64_t m, int64_t n, int64_t k);
 template <int CD, bool P2 = false>        // P2: every scale is a power of two (they go into the MFMA's scale operands)
 int launch_prefill(const void* a, const float* a_s, const void* b, const float* b_s, void* c,
-                   int64_t m, int64_t n, int64_t k, void* ws, hipStream_t stream);
+                   int64_t m, int64_t n, int64_t k, void* ws, hipStream_t stream, int* slabs = nullptr);
+int launch_fp8_gemm_slabs(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int64_t m, int64_t n,
+                          int64_t k, void* ws, int* slabs, hipStream_t stream);
 int grouped_tile_rows();
 bool grouped_supported(int64_t a_num_rows, int64_t n, int64_t k);
 template <int CD, bool P2 = false>
@@ -208,7 +210,7 @@ size_t mla_decode_workspace_bytes(int64_t batch, int64_t tokens, int64_t positio
 int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
                       const void* w, const float* ws, const void* mask, bool mask_f32, void* y, float* ys, int64_t batch,
                       int64_t tokens, int64_t positions, int heads, float scale, void* workspace, hipStream_t st);
-int launch_mla_latent(const void* a, int64_t a_stride, const void* q_w, const void* kv_w, const void* freqs, void* kv,
+int launch_mla_latent(const void* a, int64_t a_stride, const float* parts, int num_parts, const void* q_w, const void* kv_w, const void* freqs, void* kv,
                       int64_t kv_bs, void* pe, int64_t pe_bs, void* y, float* ys, int64_t batch, int64_t tokens, int q_rank,
                       float q_eps, float kv_eps, hipStream_t st);
 

@@ -1012,10 +1012,10 @@ int launch_persistent(const void* a, const float* a_s, const void* b, const floa
     }
 }
 
-// ws must hold prefill_workspace_bytes(m, n, k) bytes
+// ws must hold prefill_workspace_bytes(m, n, k) bytes; slabs as in launch_typed
 template <int CD, bool P2>
 int launch_prefill(const void* a, const float* a_s, const void* b, const float* b_s, void* c,
-                   int64_t m, int64_t n, int64_t k, void* ws, hipStream_t stream) {
+                   int64_t m, int64_t n, int64_t k, void* ws, hipStream_t stream, int* slabs) {
     const PrefillPlan p = prefill_plan(m, n, k);
     const int64_t tn = (n + prefill::BN - 1) / prefill::BN;
     const int64_t tm = (m + p.tile_rows - 1) / p.tile_rows;
@@ -1053,6 +1053,7 @@ int launch_prefill(const void* a, const float* a_s, const void* b, const float* 
     const int64_t n0 = (int64_t)p.tn_plain * prefill::BN, cols = n - n0;
     const int rc = run(std::integral_constant<int, DSV3_F32>{}, ws, p.tn_plain, tn - p.tn_plain, p.slabs, cols);
     if (rc != DSV3_OK) return rc;
+    if (slabs && cols == n) { *slabs = p.slabs; return DSV3_OK; }
     const int64_t threads = (m * cols + 3) / 4;
     hipLaunchKernelGGL((slab_reduce_kernel<CD>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream,
                        (const float*)ws, (typename OutT<CD>::type*)c, m, (int)cols, n, (int)n0, p.slabs);
@@ -1134,8 +1135,8 @@ int launch_grouped_swiglu(const void* a, const float* a_s, const int* a_rows, co
 }
 
 #define DSV3_INST(CD) \
-    template int launch_prefill<CD, false>(const void*, const float*, const void*, const float*, void*, int64_t, int64_t, int64_t, void*, hipStream_t); \
-    template int launch_prefill<CD, true>(const void*, const float*, const void*, const float*, void*, int64_t, int64_t, int64_t, void*, hipStream_t); \
+    template int launch_prefill<CD, false>(const void*, const float*, const void*, const float*, void*, int64_t, int64_t, int64_t, void*, hipStream_t, int*); \
+    template int launch_prefill<CD, true>(const void*, const float*, const void*, const float*, void*, int64_t, int64_t, int64_t, void*, hipStream_t, int*); \
     template int launch_grouped<CD, false>(const void*, const float*, const int*, const void*, const float*, void*, int64_t, int64_t, int64_t, \
                                     int64_t, const int*, const int*, const int*, int64_t, int64_t, hipStream_t);                     \
     template int launch_grouped<CD, true>(const void*, const float*, const int*, const void*, const float*, void*, int64_t, int64_t, int64_t, \

@@ -351,9 +351,12 @@ bool to_large_m_kernel(int64_t m, int64_t n, int64_t k) {
     return !((n < 8192 || m <= 32) && stream_supported(m, n, k));
 }
 
+// slabs (where not null): a product whose K range is cut for all of its columns stays as that many binary32 slabs [m, n] in ws
+// and c is not written; 0 where c holds the result.
 template <int CD>
 int launch_typed(const void* a, const float* a_s, const void* b, const float* b_s, void* c,
-                 int64_t m, int64_t n, int64_t k, void* ws, hipStream_t st, bool pow2) {
+                 int64_t m, int64_t n, int64_t k, void* ws, hipStream_t st, bool pow2, int* slabs = nullptr) {
+    if (slabs) *slabs = 0;
     if (k == 0) {   // empty sum: c = 0
         const int64_t mn0 = m * n;
         hipLaunchKernelGGL((splitk_reduce_kernel<CD>), dim3(splitk_reduce_grid(mn0)), dim3(256), 0, st,
@@ -375,13 +378,14 @@ int launch_typed(const void* a, const float* a_s, const void* b, const float* b_
         const int rc = use_stream ? launch_stream(a, a_s, b, b_s, c, CD, m, n, k, ws, &splits, st)
                                   : launch_skinny(a, a_s, b, b_s, c, CD, m, n, k, ws, &splits, st);
         if (rc != DSV3_OK || splits == 1) return rc;
+        if (slabs) { *slabs = splits; return DSV3_OK; }
         const int64_t mn = m * n;
         hipLaunchKernelGGL((splitk_reduce_kernel<CD>), dim3(splitk_reduce_grid(mn)), dim3(256), 0, st,
                            (const float*)ws, (typename OutT<CD>::type*)c, mn, splits);
         return launch_status();
     }
-    if (to_prefill) return pow2 ? launch_prefill<CD, true>(a, a_s, b, b_s, c, m, n, k, ws, st)
-                                : launch_prefill<CD, false>(a, a_s, b, b_s, c, m, n, k, ws, st);
+    if (to_prefill) return pow2 ? launch_prefill<CD, true>(a, a_s, b, b_s, c, m, n, k, ws, st, slabs)
+                                : launch_prefill<CD, false>(a, a_s, b, b_s, c, m, n, k, ws, st, slabs);
     const Plan p = make_plan(m, n, k);
     if (p.splits == 1) {
         if (p.bm == 32) return launch_cfg<32, 128, 32, 32, CD>(a, a_s, b, b_s, c, m, n, k, 1, p.kb_per_split, st);
@@ -436,6 +440,11 @@ size_t fp8_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (stream_supported(m, n, k) && stream_workspace_bytes(m, n, k) > need) need = stream_workspace_bytes(m, n, k);
     if (to_large_m_kernel(m, n, k) && prefill_workspace_bytes(m, n, k) > need) need = prefill_workspace_bytes(m, n, k);
     return need;
+}
+
+int launch_fp8_gemm_slabs(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int64_t m, int64_t n,
+                          int64_t k, void* ws, int* slabs, hipStream_t stream) {
+    return launch_typed<DSV3_BF16>(a, a_s, b, b_s, c, m, n, k, ws, stream, false, slabs);
 }
 
 int launch_fp8_gemm(const void* a, const float* a_s, const void* b, const float* b_s,

@@ -406,6 +406,7 @@ __global__ __launch_bounds__(512, 4) void mla_fold_kernel(FoldArgs p) {
 
 struct LatentArgs {
     const uint16_t* a; int64_t a_stride;                // bf16 rows [q_rank | 512 | 64], stride in elements
+    const float* parts; int num_parts; int64_t part;    // or that many binary32 slabs of them, `part` elements each, to be added
     const uint16_t* q_w; const uint16_t* kv_w;          // norm weights
     const v2f* freqs;                                   // [tokens][32]
     uint16_t* kv; int64_t kv_bs;                        // cache rows of the first new token, batch strides in elements
@@ -436,17 +437,53 @@ __device__ __forceinline__ float sum_sq8(const float (&f)[8]) {
 // of the 512 latents, rotation of the 64-wide key).  Eight values per lane, one pass.  Bound by its launch up to some
 // hundred tokens; at 4096 it reads 17 MB and writes 11 MB in 14 us.  In its place stood
 // twelve launches of tensor operations (90 us at 4096 tokens).
+// PARTS: the projections come as the slabs of their K slices, added here in order and rounded to bf16 as the reduction that
+// would stand between the two launches does (4 us of a decode step of 3 to 64 sequences).
+template <bool PARTS>
 __global__ __launch_bounds__(320) void mla_latent_kernel(LatentArgs p) {
     __shared__ float part[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t row = blockIdx.x;
     const int b = (int)(row / p.tokens), tok = (int)(row - (int64_t)b * p.tokens);
     const uint16_t* src = p.a + row * p.a_stride;
+    const float* psrc = p.parts + row * p.a_stride;
+    auto eight = [&](int c) -> v4u {                    // elements c .. c + 7 of the row
+        if constexpr (!PARTS) return *(const v4u*)(src + c);
+        constexpr int U = 8;
+        v4f v[2] = {};
+        for (int s = 0; s < p.num_parts; s += U) {      // slabs past the last are requested again from it and left out
+            v4f t[U][2];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float* at = psrc + (int64_t)min(s + u, p.num_parts - 1) * p.part + c;
+                t[u][0] = *(const v4f*)at;
+                t[u][1] = *(const v4f*)(at + 4);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) v[h] = s + u < p.num_parts ? v[h] + t[u][h] : v[h];
+        }
+        return v4u{ pack_bf16(v[0][0], v[0][1]), pack_bf16(v[0][2], v[0][3]), pack_bf16(v[1][0], v[1][1]), pack_bf16(v[1][2], v[1][3]) };
+    };
+    auto two = [&](int c) -> uint32_t {
+        if constexpr (!PARTS) return *(const uint32_t*)(src + c);
+        constexpr int U = 8;
+        v2f v = {};
+        for (int s = 0; s < p.num_parts; s += U) {
+            v2f t[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) t[u] = *(const v2f*)(psrc + (int64_t)min(s + u, p.num_parts - 1) * p.part + c);
+#pragma unroll
+            for (int u = 0; u < U; ++u) v = s + u < p.num_parts ? v + t[u] : v;
+        }
+        return pack_bf16(v[0], v[1]);
+    };
     float x[8], w[8];
     if (wave == 4) {
-        unpack8(*(const v4u*)(src + p.q_rank + lane * 8), x);
+        const uint32_t key = lane < 32 ? two(p.q_rank + kC + lane * 2) : 0u;
+        unpack8(eight(p.q_rank + lane * 8), x);
         unpack8(*(const v4u*)(p.kv_w + lane * 8), w);
-        const uint32_t key = lane < 32 ? *(const uint32_t*)(src + p.q_rank + kC + lane * 2) : 0u;
         const float r = 1.0f / __builtin_sqrtf(wave_sum(sum_sq8(x)) * (1.0f / kC) + p.kv_eps);
         v4u o;
 #pragma unroll
@@ -461,7 +498,7 @@ __global__ __launch_bounds__(320) void mla_latent_kernel(LatentArgs p) {
         const int c = threadIdx.x * 8;
         const bool live = c < p.q_rank;                 // whole 16-lane groups: q_rank is a multiple of 128
         v4u raw = {}, wr = {};
-        if (live) { raw = *(const v4u*)(src + c); wr = *(const v4u*)(p.q_w + c); }
+        if (live) { raw = eight(c); wr = *(const v4u*)(p.q_w + c); }
         unpack8(raw, x);
         unpack8(wr, w);
         const float sum = wave_sum(sum_sq8(x));
@@ -560,16 +597,19 @@ int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t 
     return launch_status();
 }
 
-int launch_mla_latent(const void* a, int64_t a_stride, const void* q_w, const void* kv_w, const void* freqs, void* kv,
+int launch_mla_latent(const void* a, int64_t a_stride, const float* parts, int num_parts, const void* q_w, const void* kv_w, const void* freqs, void* kv,
                       int64_t kv_bs, void* pe, int64_t pe_bs, void* y, float* ys, int64_t batch, int64_t tokens, int q_rank,
                       float q_eps, float kv_eps, hipStream_t st) {
     LatentArgs p;
     p.a = (const uint16_t*)a; p.a_stride = a_stride;
+    p.parts = parts; p.num_parts = num_parts; p.part = batch * tokens * a_stride;
     p.q_w = (const uint16_t*)q_w; p.kv_w = (const uint16_t*)kv_w; p.freqs = (const v2f*)freqs;
     p.kv = (uint16_t*)kv; p.kv_bs = kv_bs; p.pe = (uint16_t*)pe; p.pe_bs = pe_bs;
     p.y = (uint8_t*)y; p.ys = ys; p.tokens = (int)tokens; p.q_rank = q_rank;
     p.q_eps = q_eps; p.kv_eps = kv_eps;
-    hipLaunchKernelGGL(mla_latent_kernel, dim3((unsigned)(batch * tokens)), dim3(320), 0, st, p);
+    const dim3 grid((unsigned)(batch * tokens));
+    if (num_parts > 0) hipLaunchKernelGGL(mla_latent_kernel<true>, grid, dim3(320), 0, st, p);
+    else hipLaunchKernelGGL(mla_latent_kernel<false>, grid, dim3(320), 0, st, p);
     return launch_status();
 }
 

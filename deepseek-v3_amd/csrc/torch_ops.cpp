@@ -259,18 +259,25 @@ tuple<Tensor, Tensor> mla_decode_quant(const Tensor& q, const Tensor& freqs, con
     return {y, ys};
 }
 
+// What mla_latent and mla_query need of everything but the projected rows
+void check_latent(const Tensor& x, const Tensor& qn, const Tensor& kn, const Tensor& freqs, const Tensor& kv, const Tensor& pe, int64_t start) {
+    const int64_t b = x.size(0), s = x.size(1);
+    TORCH_CHECK(start >= 0 && kv.dim() == 3 && start <= kv.size(1), "mla_latent: start lies behind the caches' end");     // start + s cannot overflow
+    check_caches(kv, pe, b, start + s);
+    check_freqs(freqs, s, pe.size(2));
+    TORCH_CHECK(kn.numel() == kv.size(2) && qn.scalar_type() == at::kBFloat16 && kn.scalar_type() == at::kBFloat16 &&
+                qn.is_contiguous() && kn.is_contiguous(), "mla_latent: norm weights do not fit the row");
+    on_one_gpu("mla_latent", x, { &qn, &kn, &freqs, &kv, &pe });
+}
+
 // a [b, s, q_rank + kv_rank + rope] -> the normalised query latent, quantised, and the caches' rows start .. start + s - 1
 tuple<Tensor, Tensor> mla_latent(const Tensor& a, const Tensor& qn, const Tensor& kn, const Tensor& freqs, Tensor kv, Tensor pe,
                                  int64_t start, double q_eps, double kv_eps) {
     TORCH_CHECK(a.dim() == 3 && a.is_contiguous() && a.scalar_type() == at::kBFloat16 && start >= 0, "mla_latent: a must be a contiguous bf16 [b, s, width]");
     const int64_t b = a.size(0), s = a.size(1), qr = qn.numel();
-    TORCH_CHECK(kv.dim() == 3 && start <= kv.size(1), "mla_latent: start lies behind the caches' end");     // start + s cannot overflow
-    check_caches(kv, pe, b, start + s);
-    check_freqs(freqs, s, pe.size(2));
+    check_latent(a, qn, kn, freqs, kv, pe, start);
     const int64_t c = kv.size(2), r = pe.size(2);
-    TORCH_CHECK(a.size(2) == qr + c + r && kn.numel() == c && qn.scalar_type() == at::kBFloat16 && kn.scalar_type() == at::kBFloat16 &&
-                qn.is_contiguous() && kn.is_contiguous(), "mla_latent: norm weights do not fit the row");
-    on_one_gpu("mla_latent", a, { &qn, &kn, &freqs, &kv, &pe });
+    TORCH_CHECK(a.size(2) == qr + c + r, "mla_latent: norm weights do not fit the row");
     Tensor y = at::empty({b, s, qr}, a.options().dtype(kFp8)), ys = at::empty({b, s, qr / 128}, a.options().dtype(at::kFloat));
     On on(a);
     check(dsv3_mla_latent(a.data_ptr(), a.size(2), qn.data_ptr(), kn.data_ptr(), (const float*)freqs.data_ptr(),
@@ -286,8 +293,30 @@ tuple<Tensor, Tensor> mla_latent(const Tensor& a, const Tensor& qn, const Tensor
 Tensor mla_query(const Tensor& x, const Tensor& wa, const Tensor& wa_s, const Tensor& qn, const Tensor& kn, const Tensor& freqs,
                  Tensor kv, Tensor pe, int64_t start, double q_eps, double kv_eps, const Tensor& wq, const Tensor& wq_s, int64_t heads) {
     TORCH_CHECK(x.dim() == 3 && heads > 0 && wq.dim() == 2 && wq.size(0) % heads == 0, "mla_query: x must be [b, s, dim], the query's weight [heads * d, q_rank]");
-    const auto [y, ys] = mla_latent(linear_fp8(x, wa, wa_s, DSV3_SCALE_FMT_NONE, DSV3_BF16), qn, kn, freqs, kv, pe, start, q_eps, kv_eps);
-    return fp8_gemm(y, ys, wq, wq_s, DSV3_BF16).view({x.size(0), x.size(1), heads, wq.size(0) / heads});
+    const int64_t b = x.size(0), s = x.size(1), k = x.size(2), qr = qn.numel(), m = b * s;
+    const int64_t n = wa.dim() == 2 ? wa.size(0) : 0;
+    Tensor y, ys;
+    if (m == 0 || k == 0 || x.scalar_type() != at::kBFloat16 || dsv3_linear_fp8_fused(m, n, k)) {
+        std::tie(y, ys) = mla_latent(linear_fp8(x, wa, wa_s, DSV3_SCALE_FMT_NONE, DSV3_BF16), qn, kn, freqs, kv, pe, start, q_eps, kv_eps);
+    } else {            // the projection's K slices, if it has any, are added by the kernel behind it
+        check_latent(x, qn, kn, freqs, kv, pe, start);
+        const int64_t c = kv.size(2), r = pe.size(2);
+        TORCH_CHECK(x.is_contiguous() && n == qr + c + r, "mla_query: x must be contiguous, the projections' weight [q_rank + kv_rank + rope, dim]");
+        check_weight("mla_query", wa, wa_s, n, k, 128);
+        on_one_gpu("mla_query", x, { &wa, &wa_s });
+        On on(x);
+        const Tensor scr = gemm_scratch(x, m, n, k);
+        const auto [xq, xs] = act_quant(x, 128, DSV3_SCALE_FMT_NONE);
+        const Tensor a = at::empty({m, n}, x.options());
+        y = at::empty({b, s, qr}, x.options().dtype(kFp8));
+        ys = at::empty({b, s, qr / 128}, x.options().dtype(at::kFloat));
+        check(dsv3_mla_latent_gemm(xq.data_ptr(), (const float*)xs.data_ptr(), wa.data_ptr(), (const float*)wa_s.data_ptr(), k, a.data_ptr(),
+                                   qn.data_ptr(), kn.data_ptr(), (const float*)freqs.data_ptr(), (char*)kv.data_ptr() + start * c * 2,
+                                   kv.stride(0), (char*)pe.data_ptr() + start * r * 2, pe.stride(0), y.data_ptr(), (float*)ys.data_ptr(),
+                                   b, s, qr, c, (int)r, (float)q_eps, (float)kv_eps, scr.defined() ? scr.data_ptr() : nullptr,
+                                   scr.defined() ? (size_t)scr.numel() : 0, on.stream), "dsv3_mla_latent_gemm");
+    }
+    return fp8_gemm(y, ys, wq, wq_s, DSV3_BF16).view({b, s, heads, wq.size(0) / heads});
 }
 // queries and caches -> the layer's output [b, s, dim]
 Tensor mla_output(const Tensor& q, const Tensor& freqs, const Tensor& kv, const Tensor& pe, const Tensor& w, const Tensor& ws,

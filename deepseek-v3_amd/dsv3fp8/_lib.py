@@ -70,6 +70,9 @@ EXPORTS = {
                                  c_int64, c_float, c_void_p, c_size_t, c_void_p]),
     "dsv3_mla_latent": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int64,
                                 c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int, c_float, c_float, c_void_p]),
+    "dsv3_mla_latent_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
+                                     c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64,
+                                     c_int, c_float, c_float, c_void_p, c_size_t, c_void_p]),
 }
 
 

@@ -389,6 +389,16 @@ int dsv3_mla_latent(const void* a, int64_t a_stride, const void* q_norm, const v
                     void* kv_rows, int64_t kv_batch_stride, void* pe_rows, int64_t pe_batch_stride, void* y, float* s,
                     int64_t batch, int64_t rows, int64_t q_rank, int64_t kv_rank, int rope_dim, float q_eps, float kv_eps,
                     void* stream);
+/*
+ * The projection in front of it as well: rows a = x (w * w_s)^T of q_rank + 576 elements from the quantised x (e4m3 [batch*rows, k],
+ * scales [batch*rows, k/128]; k a multiple of 128) as dsv3_fp8_gemm forms them, bit for bit.  Where that product's K range is cut, its
+ * slabs are added by the second kernel and `a` (bf16 [batch*rows, q_rank + 576], scratch) is not written.  workspace:
+ * dsv3_fp8_gemm_workspace_bytes(batch*rows, q_rank + 576, k) bytes, 256-byte aligned.
+ */
+int dsv3_mla_latent_gemm(const void* x, const float* x_s, const void* w, const float* w_s, int64_t k, void* a, const void* q_norm,
+                         const void* kv_norm, const float* freqs, void* kv_rows, int64_t kv_batch_stride, void* pe_rows,
+                         int64_t pe_batch_stride, void* y, float* s, int64_t batch, int64_t rows, int64_t q_rank, int64_t kv_rank,
+                         int rope_dim, float q_eps, float kv_eps, void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -151,6 +151,26 @@ def test_decode_attention_quantised_is_the_rounded_result_quantised(b, s, t, h):
     assert torch.equal(yq.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(ys, rs)
 
 
+# rows whose projection runs as one launch, in K slices of the streaming kernel, in slices of the tile kernel (up to eight), plain
+@pytest.mark.parametrize("b,s", [(1, 1), (3, 1), (17, 1), (1, 64), (5, 13), (1, 200), (2, 400), (1, 3000)])
+def test_query_in_one_call_is_its_three_parts(b, s):
+    from dsv3fp8 import kernel, quantize
+    dim, qr, h, start = 7168, 1536, 2, 3
+    g = torch.Generator().manual_seed(b * 1000 + s)
+    x = torch.randn(b, s, dim, generator=g).bfloat16().cuda()
+    wa, wa_s = quantize.weight_quant((torch.randn(qr + C + ROPE, dim, generator=g) * 0.02).bfloat16().cuda())
+    wq, wq_s = quantize.weight_quant((torch.randn(h * 192, qr, generator=g) * 0.02).bfloat16().cuda())
+    qn, kn = [(1 + 0.1 * torch.randn(n, generator=g)).bfloat16().cuda() for n in (qr, C)]
+    ang = torch.rand(s, ROPE // 2, generator=g) * 6.28
+    freqs = torch.polar(torch.ones_like(ang), ang).cuda()
+    one, three = [[torch.zeros(b, start + s + 2, n, dtype=torch.bfloat16, device="cuda") for n in (C, ROPE)] for _ in range(2)]
+    q = torch.ops.dsv3fp8.mla_query(x, wa, wa_s, qn, kn, freqs, *one, start, 1e-6, 1e-6, wq, wq_s, h)
+    a = torch.ops.dsv3fp8.linear_fp8(x, wa, wa_s, 0, 0)
+    y, ys = torch.ops.dsv3fp8.mla_latent(a, qn, kn, freqs, *three, start, 1e-6, 1e-6)
+    assert torch.equal(q, torch.ops.dsv3fp8.fp8_gemm(y, ys, wq, wq_s, 0).view(b, s, h, 192))
+    assert torch.equal(one[0], three[0]) and torch.equal(one[1], three[1]) and one[0][:, start:start + s].any()
+
+
 LATENT = [(1, 1, 0, 1536), (3, 1, 7, 1536), (2, 5, 0, 128), (1, 40, 3, 2048), (2, 33, 1, 640)]
 
 
