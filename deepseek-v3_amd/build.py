@@ -38,7 +38,7 @@ HIPCC_FLAGS = [
 # or spills; exceptions are listed with their reasons.
 # The attention kernels keep their sums in registers for a whole loop and have none to spare (mla_decode_kernel: 32 x 512
 # sums in the 256 accumulation registers; an ordinary rescale of them spilled 300): a spill there is a copy per tile.
-NO_SPILL_SOURCES = {"fp8_gemm_skinny.hip", "fp8_gemm_stream.hip", "mla_decode.hip", "mla_prefill.hip"}
+NO_SPILL_SOURCES = {"fp8_gemm_skinny.hip", "fp8_gemm_stream.hip", "fp8_gemm_mid.hip", "mla_decode.hip", "mla_prefill.hip"}
 SCRATCH_ALLOWED = {
     # two scalar registers kept in lanes of a vector register: no scratch memory, and outside the tile loop
     "mla_attend_kernel": 2,

@@ -155,6 +155,11 @@ bool stream_supported(int64_t m, int64_t n, int64_t k);
 size_t stream_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int launch_stream(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int c_dtype,
                   int64_t m, int64_t n, int64_t k, void* ws, int* splits_out, hipStream_t st);
+bool mid_supported(int64_t m, int64_t n, int64_t k);
+bool mid_takes_scales(const float* a_s, const float* b_s);
+size_t mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
+int launch_mid(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int c_dtype, int64_t m, int64_t n, int64_t k,
+               void* ws, int* splits_out, hipStream_t st);
 bool skinny_supported(int64_t m, int64_t n, int64_t k);
 size_t skinny_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int launch_skinny(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int c_dtype,

@@ -372,10 +372,12 @@ int launch_typed(const void* a, const float* a_s, const void* b, const float* b_
     if (force == 0 && single_group_stream(m, n, k))
         return launch_skinny_single(a, a_s, b, b_s, c, CD, m, n, k, st);
     const bool to_prefill = force != 1 && !(force == 3 && stream_supported(m, n, k)) && to_large_m_kernel(m, n, k);
+    const bool use_mid = to_prefill && force == 0 && mid_supported(m, n, k) && mid_takes_scales(a_s, b_s);
     const bool use_stream = force != 1 && !to_prefill && !(force == 4 && skinny_supported(m, n, k)) && stream_supported(m, n, k);
-    if (use_stream || (force != 1 && !to_prefill && skinny_supported(m, n, k))) {          // decode shapes: weight-streaming kernels
+    if (use_mid || use_stream || (force != 1 && !to_prefill && skinny_supported(m, n, k))) {       // decode shapes: weight-streaming kernels
         int splits = 1;
-        const int rc = use_stream ? launch_stream(a, a_s, b, b_s, c, CD, m, n, k, ws, &splits, st)
+        const int rc = use_mid ? launch_mid(a, a_s, b, b_s, c, CD, m, n, k, ws, &splits, st)
+                     : use_stream ? launch_stream(a, a_s, b, b_s, c, CD, m, n, k, ws, &splits, st)
                                   : launch_skinny(a, a_s, b, b_s, c, CD, m, n, k, ws, &splits, st);
         if (rc != DSV3_OK || splits == 1) return rc;
         if (slabs) { *slabs = splits; return DSV3_OK; }
@@ -439,6 +441,7 @@ size_t fp8_gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     if (skinny_supported(m, n, k) && skinny_workspace_bytes(m, n, k) > need) need = skinny_workspace_bytes(m, n, k);
     if (stream_supported(m, n, k) && stream_workspace_bytes(m, n, k) > need) need = stream_workspace_bytes(m, n, k);
     if (to_large_m_kernel(m, n, k) && prefill_workspace_bytes(m, n, k) > need) need = prefill_workspace_bytes(m, n, k);
+    if (to_large_m_kernel(m, n, k) && mid_workspace_bytes(m, n, k) > need) need = mid_workspace_bytes(m, n, k);
     return need;
 }
 

@@ -118,6 +118,53 @@ def test_mid_m_split_over_k(K, m, n, k):
         assert _lib.lib.dsv3_fp8_gemm_workspace_bytes(m, n, k) >= 2 * m * n * 4
 
 
+@pytest.mark.parametrize("m,n,k", [
+    # one row tile of 160-column tiles: every height, the edges of its rows, a ragged last column tile
+    (65, 30752, 3584), (96, 30752, 3584), (97, 40960, 2560), (130, 30752, 3584), (161, 30724, 3584), (192, 36864, 3072), (193, 30752, 3584), (224, 30721, 3584),
+    (65, 24576, 1536), (128, 22530, 1536), (100, 32768, 1536),                 # 128-column tiles, a round of them
+    (65, 576, 7168), (64 + 1, 1, 4096), (127, 2304, 4096), (200, 1000, 4608), (448, 1536, 7168), (512, 2048, 4096), (2600, 300, 4096),   # 64 x 128, 7 .. 2 slices
+])
+def test_tiles_that_fill_one_round(K, m, n, k):
+    """The kernel between the large-M kernel's tiles: every configuration, ragged rows, columns and K slices, general and
+    power-of-two scales, sampled columns against binary64 and all of them against the large-M kernel, which takes scales that are
+    not 16-byte aligned.  Both form the same products of 128 terms in the matrix core and add them in binary32, in another order
+    where K is sliced: k / 128 <= 56 additions and scale products of relative error 2^-24, together less than 2^-18 of the sum
+    of the terms' sizes, and they err at random: 2^-21 is a bound with room (2^-22 seen)."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    kb, nb = k // 128, (n + 127) // 128
+    a = (torch.randn(m, k, generator=g, device="cuda") * 40).to(torch.float8_e4m3fn)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 40).to(torch.float8_e4m3fn)
+    a_s = torch.rand(m, kb, generator=g, device="cuda") + 0.5
+    w_s = torch.rand(nb, kb, generator=g, device="cuda") + 0.5
+    cols = torch.unique(torch.cat([torch.randint(0, n, (300,), generator=g, device="cuda"),
+                                   torch.tensor([0, n - 1, n // 2, max(n - 17, 0), min(159, n - 1), min(160, n - 1)], device="cuda")]))
+    for pow2 in (False, True):
+        if pow2:
+            a_s, w_s = 2.0 ** torch.round(torch.log2(a_s) * 6), 2.0 ** torch.round(torch.log2(w_s) * 6)
+        odd = torch.empty(a_s.numel() + 1, device="cuda")[1:].view_as(a_s).copy_(a_s)
+        ref = torch.zeros(m, cols.numel(), dtype=torch.float64, device="cuda")
+        size = torch.zeros_like(ref)
+        for b in range(kb):
+            x, y = a[:, b * 128:(b + 1) * 128].double(), w[:, b * 128:(b + 1) * 128][cols].double()
+            s = a_s[:, b:b + 1].double() * w_s[cols // 128, b].double()
+            ref += x @ y.t().contiguous() * s
+            size += x.abs() @ y.abs().t().contiguous() * s
+        rms = ref.pow(2).mean().sqrt()
+        c32, c16 = _gemm_both(K, a, a_s, w, w_s)
+        other = K.fp8_gemm_f32(a, odd, w, w_s)
+        assert ((c32[:, cols].double() - ref).abs().max() <= TOL * rms)
+        assert ((c32 - other)[:, cols].abs().double() <= 2.0 ** -21 * size).all()
+        assert ((c32 - other).abs().max() <= 2.0 ** -21 * 1.5 * size.max())            # (all columns; sizes differ by far less than half)
+        assert torch.equal(c16, c32.to(torch.bfloat16))
+        if pow2:
+            old = torch.get_default_dtype()
+            torch.set_default_dtype(torch.float32)
+            try:
+                assert torch.equal(K.fp8_gemm_pow2(a, a_s, w, w_s), c32)                # (the same kernel)
+            finally:
+                torch.set_default_dtype(old)
+
+
 @pytest.mark.parametrize("n", [1, 15, 16, 100, 129, 576, 577, 1000])
 def test_ragged_n(K, n):
     from dsv3fp8 import workloads
