@@ -65,7 +65,7 @@ __device__ __forceinline__ void scale_agprs(v16f& v, float a) {
 // positions of one feature per lane.
 // Bound: per tile 68 MFMAs of 32 cycles; with one wavefront per SIMD its exponentials and barriers stand beside them.  32
 // sequences at 4096 positions (16 tiles a workgroup): 53 .. 58 us, 70 with each LDS read next to its MFMA; 12 us of it are the 67 MB
-// of partial sums at the end, and one tile alone (a short context) takes 12 us in all.  The tensor operations in its place
+// of partial sums at the end, and one tile alone (a short context) takes 10.7 us in all, 12.7 without PACK.  The tensor operations in its place
 // took 250 us (58 us in the products, the rest in passes over the scores).
 // PACK: the folded queries come in operand order (launch_wkv_b_absorb_q_packed), a KiB of consecutive bytes per load; as rows a
 // load touches 32 of them and takes 64 cycles of the compute unit's load path, 3.8 us for the workgroup's 128.
