@@ -218,9 +218,11 @@ def apply_rotary_emb(x: torch.Tensor, freqs_cis: torch.Tensor) -> torch.Tensor:
 def _plain(module: nn.Module, cls: type) -> bool:
     """Whether calling ``module`` does no more than ``cls.forward``, so that a fused kernel may take its place: neither a
     module of another type nor one with hooks (its own or those of all modules) or a ``forward`` of its own."""
+    if type(module) is not cls:         # (which may be any callable, without a dictionary too)
+        return False
     own = module.__dict__
-    return type(module) is cls and not (own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own
-                                        or _modules._global_forward_hooks or _modules._global_forward_pre_hooks)
+    return not (own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own
+                or _modules._global_forward_hooks or _modules._global_forward_pre_hooks)
 
 
 def _offset_aligned(t: torch.Tensor) -> bool:
@@ -356,38 +358,46 @@ class MLA(nn.Module):
             w = weight_dequant(w, self.wkv_b.scale, block_size)
         return w.view(self.n_local_heads, -1, self.kv_lora_rank)
 
-    def _kernels_ok(self, x, start_pos: int, freqs_cis) -> bool:
+    def _kernels_ok(self, x, start_pos: int, freqs_cis) -> Optional[Tuple[torch.Tensor, ...]]:
         """What the fused kernels of this layer ask for in common: their head dimensions and dtypes, FP8 weights, no
-        gradients (the kernels have no backward), new rows that fit the caches."""
+        gradients (the kernels have no backward), new rows that fit the caches.  Returns what was looked at and is to be
+        handed to the kernels, (kv_cache, pe_cache, wkv_b's weight), or None: a cache may be a buffer, a parameter or an
+        ordinary attribute (a view of a pool, say), and is looked up as one attribute, once."""
         if (torch.is_grad_enabled() or gemm_impl != "fp8" or block_size != 128 or world_size != 1 or not self.fused
                 or self.attn_impl != "absorb" or not x.is_cuda or x.dtype != torch.bfloat16
                 or torch.get_default_dtype() != torch.bfloat16):
-            return False
+            return None
         b, s, device = x.size(0), x.size(1), x.device
         kv, pe, w = self.kv_cache, self.pe_cache, self.wkv_b.weight
-        return ((self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim, self.kv_lora_rank) == (128, 64, 128, 512)
+        fits = ((self.qk_nope_head_dim, self.qk_rope_head_dim, self.v_head_dim, self.kv_lora_rank) == (128, 64, 128, 512)
                 and kv.dtype == torch.bfloat16 and pe.dtype == torch.bfloat16 and kv.is_contiguous() and pe.is_contiguous()
                 and 1 <= b <= kv.size(0) and s >= 1 and start_pos >= 0 and start_pos + s <= kv.size(1)
                 and w.element_size() == 1 and _offset_aligned(kv) and _offset_aligned(pe) and _offset_aligned(w)
                 and kv.device == device and pe.device == device and w.device == device and freqs_cis.device == device
                 and freqs_cis.dtype == torch.complex64 and freqs_cis.is_contiguous() and not freqs_cis.is_conj()
                 and freqs_cis.shape == (s, self.qk_rope_head_dim // 2))
+        return (kv, pe, w) if fits else None
 
-    def _latent_kernel_ok(self, x) -> bool:
+    def _latent_kernel_ok(self, x) -> Optional[tuple]:
         """Whether both norms, the cache rows and the quantisation in front of ``wq_b`` can be one launch; modules that
-        were exchanged or carry hooks (``wq_a`` and ``wkv_a`` too, by ``stack_a``) are called as such."""
+        were exchanged or carry hooks (``wq_a`` and ``wkv_a`` too, by ``stack_a``) are called as such.  Returns what was
+        looked at, (q_norm's weight, kv_norm's weight, their eps, wq_b's weight), or None."""
         if not 0 < self.q_lora_rank <= 2048 or self.q_lora_rank % block_size or not self.stacked_a:
-            return False
+            return None
         qn, kn, wq = self.q_norm, self.kv_norm, self.wq_b
         if not (_plain(qn, RMSNorm) and _plain(kn, RMSNorm) and _plain(wq, ColumnParallelLinear)):
-            return False
+            return None
+        weights = []
         for norm in (qn, kn):
             w = norm._parameters.get("weight")
             if w is None or w.dtype != torch.bfloat16 or w.device != x.device or not w.is_contiguous() or not _offset_aligned(w) \
                     or not isinstance(norm.eps, (int, float)):
-                return False
+                return None
+            weights.append(w)
         w = wq._parameters.get("weight")
-        return w is not None and w.element_size() == 1 and wq._parameters.get("bias") is None and self.stack_a()
+        if w is None or w.element_size() != 1 or wq._parameters.get("bias") is not None or not self.stack_a():
+            return None
+        return (*weights, qn.eps, kn.eps, w)
 
     def _attention_kernels_ok(self, q, positions: int, mask) -> bool:
         """Whether the attention behind the query projection can run on the fused kernels: a mask of one value per
@@ -419,17 +429,17 @@ class MLA(nn.Module):
         start_pos = operator.index(start_pos)
         t = start_pos + s
         kernels = self._kernels_ok(x, start_pos, freqs_cis)
-        if kernels and self._latent_kernel_ok(x):
-            caches, modules = self._buffers, self._modules
-            wq = modules["wq_b"]._parameters["weight"]
+        latent = self._latent_kernel_ok(x) if kernels else None
+        if latent:
+            kv, pe, _ = kernels
+            q_norm, kv_norm, q_eps, kv_eps, wq = latent
+            wa = self._wa
             if x.is_contiguous() and x.size(-1) % block_size == 0 and wq.is_contiguous() and self.wq_a.scale_fmt != "ue8m0":
-                qn, kn = modules["q_norm"], modules["kv_norm"]
-                q = _mla_query(x, self._wa, self._wa.scale, qn._parameters["weight"], kn._parameters["weight"], freqs_cis,
-                               caches["kv_cache"], caches["pe_cache"], start_pos, qn.eps, kn.eps, wq, wq.scale, self.n_local_heads)
+                q = _mla_query(x, wa, wa.scale, q_norm, kv_norm, freqs_cis, kv, pe, start_pos, q_eps, kv_eps, wq, wq.scale,
+                               self.n_local_heads)
             else:
-                qq, qs = torch.ops.dsv3fp8.mla_latent(linear(x, self._wa, None, self.wq_a.scale_fmt), self.q_norm.weight,
-                                                      self.kv_norm.weight, freqs_cis, self.kv_cache, self.pe_cache, start_pos,
-                                                      self.q_norm.eps, self.kv_norm.eps)
+                qq, qs = torch.ops.dsv3fp8.mla_latent(linear(x, wa, None, self.wq_a.scale_fmt), q_norm, kv_norm, freqs_cis,
+                                                      kv, pe, start_pos, q_eps, kv_eps)
                 q = fp8_gemm(qq, qs, wq, wq.scale).unflatten(-1, (self.n_local_heads, self.qk_head_dim))
         else:
             q, kva = self._project(x)
@@ -439,14 +449,15 @@ class MLA(nn.Module):
             self.kv_cache[:b, start_pos:t] = self.kv_norm(kva[..., :self.kv_lora_rank])
             self.pe_cache[:b, start_pos:t] = apply_rotary_emb(kva[..., self.kv_lora_rank:].unsqueeze(2), freqs_cis).squeeze(2)
         if kernels and self._attention_kernels_ok(q, t, mask):
-            args = (q, freqs_cis, self.kv_cache, self.pe_cache, self.wkv_b.weight, self.wkv_b.scale, mask, t, self.softmax_scale)
+            kv, pe, w = kernels
+            args = (q, freqs_cis, kv, pe, w, self.wkv_b.scale, mask, t, self.softmax_scale)
             explicit = self._explicit_pays(b, s, t)
             # the attention's last kernel quantises for wo, unless wo was exchanged, carries hooks or is no FP8 layer
-            wo = self._modules["wo"]
+            wo = self.wo
             if _plain(wo, RowParallelLinear) and wo.weight.element_size() == 1 and wo.bias is None and wo.weight.is_contiguous():
                 return _mla_output(*args, explicit, wo.weight, wo.weight.scale)
             if not explicit:
-                return self.wo(torch.ops.dsv3fp8.mla_decode(*args))
+                return wo(torch.ops.dsv3fp8.mla_decode(*args))
         wkv_b = self._dequantised_wkv_b(x)
         latent, rope_keys = self.kv_cache[:b, :t], self.pe_cache[:b, :t]
         # scores over the latent (query folded through wkv_b) plus the rotary part; softmax in binary32

@@ -52,6 +52,59 @@ def test_weights_that_are_not_parameters(layer, name):
     assert not layer._latent_kernel_ok(torch.zeros(1, 2, 256, dtype=torch.bfloat16))
 
 
+class _OnGpu(torch.Tensor):
+    """A tensor of the host that says it is on the GPU."""
+    is_cuda = True
+    __torch_function__ = torch._C._disabled_torch_function_impl
+
+
+class _Slots:
+    __slots__ = ()
+
+    def __call__(self, x):
+        return x + 1
+
+
+@pytest.mark.parametrize("what", ["buffers", "parameter", "attribute", "beside", "callable", "no dictionary"])
+def test_parts_are_what_the_attributes_say(layer, monkeypatch, what):
+    """The kernels get the very caches and modules that the conditions looked at, also where these are no buffers or registered
+    modules of the layer: a Parameter, a view of a pool that the program owns, an attribute that hides a buffer; wo may be
+    any callable.  (The operators are stand-ins that note their arguments; nothing runs on a GPU.)"""
+    from dsv3fp8 import model
+    monkeypatch.setattr(model, "gemm_impl", "fp8")
+    layer.qk_nope_head_dim, layer.qk_rope_head_dim, layer.v_head_dim, layer.kv_lora_rank = 128, 64, 128, 512
+    pool = torch.zeros(4, 8, 512, dtype=torch.bfloat16), torch.zeros(4, 8, 64, dtype=torch.bfloat16)
+    for name, cache in zip(("kv_cache", "pe_cache"), pool):
+        if what == "parameter":
+            setattr(layer, name, nn.Parameter(cache[:1]))
+        elif what == "attribute":
+            delattr(layer, name)
+            setattr(layer, name, cache[1:2])
+        elif what == "beside":
+            layer.__dict__[name] = cache[1:2]
+    if what == "beside":
+        for name in ("q_norm", "kv_norm", "wq_b", "wo"):
+            layer.__dict__[name] = type(getattr(layer, name))(*{"q_norm": (128,), "kv_norm": (512,), "wq_b": (128, 384), "wo": (256, 256)}[name])
+    if what in ("callable", "no dictionary"):
+        del layer.wo
+        layer.wo = (lambda x: x + 1) if what == "callable" else _Slots()
+    q, out, calls = torch.zeros(1, 1, 2, 192, dtype=torch.bfloat16), torch.zeros(1, 1, 256, dtype=torch.bfloat16), []
+    monkeypatch.setattr(model, "_mla_query", lambda *a: (calls.append(a), q)[1])
+    monkeypatch.setattr(model, "_mla_output", lambda *a: (calls.append(a), out)[1])
+    monkeypatch.setattr(torch.ops.dsv3fp8, "mla_decode", lambda *a: (calls.append(a), out)[1])
+    x = torch.zeros(1, 1, 256, dtype=torch.bfloat16).as_subclass(_OnGpu)
+    with torch.no_grad():
+        y = layer(x, 3, torch.ones(1, 32, dtype=torch.complex64), None)
+    query, attention = calls
+    assert query[3] is layer.q_norm.weight and query[4] is layer.kv_norm.weight and query[11] is layer.wq_b.weight
+    assert query[6] is layer.kv_cache and query[7] is layer.pe_cache
+    assert attention[2] is layer.kv_cache and attention[3] is layer.pe_cache and attention[4] is layer.wkv_b.weight
+    if what in ("callable", "no dictionary"):
+        assert torch.equal(y, out + 1)
+    else:
+        assert y is out and attention[-2] is layer.wo.weight
+
+
 def test_masks_that_the_attention_kernels_do_not_take(layer):
     q = torch.zeros(1, 2, 2, 192, dtype=torch.bfloat16)
     ones = torch.ones(2, 4)
