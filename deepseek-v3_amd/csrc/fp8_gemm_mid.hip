@@ -253,20 +253,25 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     if (m <= 64 || k % 512 || m * k >= (1ll << 32) || n * k >= (1ll << 32)) return p;
     p.splits = 1;
     p.nkb = (int)kb;
-    // Weights of 96 MiB and more, whose columns in tiles of 160 fill three quarters of the chip or more in one round and one row tile: 65 ..
-    // 224 rows of 7168 -> 36864 (231 tiles).  At 256 rows the operands' ring has two stages only (98 against 103 us, 320 rows: slower), and
-    // two row tiles of 116 for 7168 -> 18432 lose behind the quantisation, 129 .. 224 rows 48.4 -> 53.5 us at 193: that one
-    // 128- or 256-row tile of the large-M kernel reads the weights once.
+    // Weights of 96 MiB and more, of more columns than 128 of the large-M kernel's tiles and at most 256 tiles of 160: one round here, with
+    // one row tile.  65 .. 224 rows of 7168 -> 36864 (231 tiles).  Measured with the quantisation in front over 32769 .. 40960 columns and K
+    // of 2560 .. 16384, (large-M kernel's time) / (time here): 1.05 .. 1.30 up to 192 rows, 1.02 .. 1.23 at 193 and 224.  What is left out:
+    // 32768 columns and fewer, where 128-row tiles of the large-M kernel, two a column tile or in two K slices, are one full round
+    // (7168 -> 31744 at 65 / 160 / 193 rows 0.93 / 0.88 / 0.84); K of 32768 (0.81 .. 1.39, most below 1 at 193 rows); from 193 rows on,
+    // whose ring has three stages, fewer than 212 tiles or 32 K blocks (16384 -> 32769 0.94, 2560 -> 40960 0.98); 225 rows and more, whose
+    // ring would have two; two row tiles of 116 for 7168 -> 18432 (129 .. 224 rows, 48.4 us there, 53.5 here at 193): that one 128- or
+    // 256-row tile of the large-M kernel reads the weights once.
     const int64_t t160 = (n + 159) / 160, rows = (m + 15) / 16;
-    if (n * k >= (96ll << 20) && t160 >= 192 && t160 <= 256 && rows <= 14) {
+    if (n * k >= (96ll << 20) && n > 32768 && t160 <= 256 && kb <= 128 && rows <= (t160 < 212 || kb < 32 ? 12 : 14)) {
         p.wm = 4; p.sn = 5;
         p.mt = rows <= 6 ? 6 : rows <= 8 ? 8 : rows <= 10 ? 10 : rows <= 12 ? 12 : 14;
         return p;
     }
-    // Up to 128 rows of a weight of 176 to 256 tiles of 128 columns, in one round where 256 columns make half a round: 1536 -> 24576 13 .. 27 %
-    // less.  Not below 12 K blocks (512 -> 32768: equal to 12 % more).
+    // Up to 128 rows of a weight of 176 to 256 tiles of 128 columns, in one round where 256 columns make half a round: 1536 -> 24576 13 .. 23 %
+    // less; over 22401 .. 32768 columns and K of 1536 .. 16384, measured as above, 0.99 .. 1.77.  Not below 12 K blocks (512 -> 32768: equal to
+    // 12 % more), nor above 128 (32768 -> 28672 at 128 rows 0.98).
     const int64_t t128 = (n + 127) / 128;
-    if (m <= 128 && t128 >= 176 && t128 <= 256 && kb >= 12) {
+    if (m <= 128 && t128 >= 176 && t128 <= 256 && kb >= 12 && kb <= 128) {
         p.mt = 8; p.wm = 4; p.sn = 4;
         return p;
     }

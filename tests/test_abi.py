@@ -392,6 +392,22 @@ def test_attention_operators_refuse_what_their_kernels_cannot_read(name):
                 _gpu_body(name, *args)
 
 
+# (rows, columns, K, taken): sizes on both sides of each limit; past one the large-M kernel is measured faster
+@pytest.mark.parametrize("m,n,k,taken", [
+    (64, 36864, 7168, False), (65, 36864, 7168, True), (224, 36864, 7168, True), (225, 36864, 7168, False), (65, 36864, 7296, False),
+    (129, 32768, 3072, False), (160, 30752, 3584, False), (193, 31744, 7168, False), (129, 32769, 3072, True), (192, 32769, 16384, True),
+    (193, 32769, 16384, False), (193, 33761, 16384, True), (192, 40960, 2560, True), (193, 40960, 3584, False), (224, 40960, 4096, True),
+    (224, 40961, 4096, False), (65, 36864, 16384, True), (65, 36864, 16896, False), (193, 18432, 7168, False),
+    (128, 32768, 16384, True), (128, 24576, 1536, True), (129, 24576, 1536, False), (128, 24576, 1024, False), (65, 28672, 16896, False),
+    (65, 22400, 1536, False), (65, 22401, 1536, True),
+    (448, 1536, 7168, True), (449, 1536, 7168, False), (320, 2112, 7168, True), (321, 2112, 7168, False), (65, 2305, 7168, False),
+    (8192, 128, 4096, True), (8193, 128, 4096, False), (65, 576, 3584, False)])
+def test_sizes_that_the_tiles_of_one_round_take(L, m, n, k, taken):
+    supported = L.lib["_ZN4dsv313mid_supportedElll"]            # dsv3::mid_supported(rows, columns, K)
+    supported.restype, supported.argtypes = ctypes.c_bool, [ctypes.c_int64] * 3
+    assert supported(m, n, k) == taken
+
+
 def test_binding_needs_the_c_library_only():
     """_lib.py by itself (without the package, which registers the torch operators) loads where libdsv3torch.so is not
     built; the package says which command builds it."""

@@ -120,8 +120,8 @@ def test_mid_m_split_over_k(K, m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [
     # one row tile of 160-column tiles: every height, the edges of its rows, a ragged last column tile
-    (65, 30752, 3584), (96, 30752, 3584), (97, 40960, 2560), (130, 30752, 3584), (161, 30724, 3584), (192, 36864, 3072), (193, 30752, 3584), (224, 30721, 3584),
-    (65, 24576, 1536), (128, 22530, 1536), (100, 32768, 1536),                 # 128-column tiles, a round of them
+    (65, 33792, 3072), (96, 32770, 3072), (97, 40960, 2560), (130, 33792, 3072), (161, 33764, 3072), (192, 36864, 3072), (193, 33792, 4096), (224, 33761, 4096),
+    (65, 24576, 1536), (128, 22530, 1536), (100, 32768, 3584),                 # 128-column tiles, a round of them
     (65, 576, 7168), (64 + 1, 1, 4096), (127, 2304, 4096), (200, 1000, 4608), (448, 1536, 7168), (512, 2048, 4096), (2600, 300, 4096),   # 64 x 128, 7 .. 2 slices
 ])
 def test_tiles_that_fill_one_round(K, m, n, k):
