@@ -20,6 +20,7 @@
 // 71.1 / 82.7 (a 128-row tile takes 1.07 us per K block, 4.4 TB/s of weights; each row adds: its copies and the weights' share the load
 // path); 1536 -> 24576 at 65 / 128 rows 17.2 / 17.6 -> 13.6 / 15.5; the narrow ones at the rule below.
 // Not used elsewhere: with both dimensions in whole rounds of 256 x 256 tiles the two-phase kernel is up to 25 % faster.
+#include <cstdlib>
 #include <type_traits>
 #include "common.hpp"
 
@@ -247,10 +248,19 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
 // Three windows in which the large-M kernel's tiles fit the chip badly.  Power-of-two scales take the same kernel (accumulating in the
 // matrix core was equal to 4 % faster here).
 struct Plan { int mt, wm, sn, splits, nkb; };       // mt == 0: not for this kernel
+// The variables that pin how the large-M kernel runs its dense tiles (one K slice, a tile height, a schedule) pin that kernel too.
+inline bool large_m_pinned() {
+    static const bool v = [] {
+        for (const char* name : { "DSV3_PREFILL_TILE", "DSV3_PREFILL_NOSPLIT", "DSV3_PREFILL_NOPP", "DSV3_PREFILL_NOPP128" })
+            if (std::getenv(name)) return true;
+        return false;
+    }();
+    return v;
+}
 inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     Plan p{};
     const int64_t kb = k / 128;
-    if (m <= 64 || k % 512 || m * k >= (1ll << 32) || n * k >= (1ll << 32)) return p;
+    if (m <= 64 || k % 512 || m * k >= (1ll << 32) || n * k >= (1ll << 32) || large_m_pinned()) return p;
     p.splits = 1;
     p.nkb = (int)kb;
     // Weights of 96 MiB and more, of more columns than 128 of the large-M kernel's tiles and at most 256 tiles of 160: one round here, with

@@ -408,6 +408,29 @@ def test_sizes_that_the_tiles_of_one_round_take(L, m, n, k, taken):
     assert supported(m, n, k) == taken
 
 
+@pytest.mark.parametrize("knob", ["DSV3_PREFILL_NOSPLIT=1", "DSV3_PREFILL_TILE=128", "DSV3_PREFILL_NOPP=1", "DSV3_PREFILL_NOPP128=1", "OTHER=1"])
+def test_knobs_of_the_large_m_kernel_keep_products_there(knob):
+    """A knob that says how the large-M kernel runs its dense tiles holds for every size it had when the knob was made; without K slices no
+    product of more than 64 rows asks for scratch."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import ctypes
+from dsv3fp8 import _lib
+f = _lib.lib["_ZN4dsv313mid_supportedElll"]
+f.restype, f.argtypes = ctypes.c_bool, [ctypes.c_int64] * 3
+sizes = [(65, 36864, 7168), (128, 24576, 1536), (448, 1536, 7168)]
+print([f(*s) for s in sizes], sum(_lib.lib.dsv3_fp8_gemm_workspace_bytes(*s) for s in sizes))
+"""
+    name, value = knob.split("=")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT / "deepseek-v3_amd", capture_output=True, text=True, env={**os.environ, name: value})
+    assert r.returncode == 0, r.stderr
+    taken, scratch = r.stdout.strip().rsplit(" ", 1)
+    assert taken == str([name == "OTHER"] * 3)
+    assert (scratch == "0") == (name == "DSV3_PREFILL_NOSPLIT")
+
+
 def test_binding_needs_the_c_library_only():
     """_lib.py by itself (without the package, which registers the torch operators) loads where libdsv3torch.so is not
     built; the package says which command builds it."""
