@@ -60,9 +60,12 @@ struct On {
 
 // The kernels get raw pointers: a tensor of another device or of the host would fault the GPU.  (The dispatcher comes here as
 // soon as one argument is on the GPU.)
-void on_one_gpu(const char* what, const Tensor& x, std::initializer_list<const Tensor*> others) {
+void on_one_device(const char* what, const Tensor& x, std::initializer_list<const Tensor*> others) {
     for (const Tensor* t : others)
         TORCH_CHECK(t->device() == x.device(), what, ": all tensors must be on one device, got ", x.device(), " and ", t->device());
+}
+void on_one_gpu(const char* what, const Tensor& x, std::initializer_list<const Tensor*> others) {
+    on_one_device(what, x, others);
     TORCH_CHECK(x.is_cuda(), what, ": tensors must be on the GPU, got ", x.device());
 }
 
@@ -295,15 +298,16 @@ Tensor mla_query(const Tensor& x, const Tensor& wa, const Tensor& wa_s, const Te
     TORCH_CHECK(x.dim() == 3 && heads > 0 && wq.dim() == 2 && wq.size(0) % heads == 0, "mla_query: x must be [b, s, dim], the query's weight [heads * d, q_rank]");
     const int64_t b = x.size(0), s = x.size(1), k = x.size(2), qr = qn.numel(), m = b * s;
     const int64_t n = wa.dim() == 2 ? wa.size(0) : 0;
+    on_one_device("mla_query", x, { &wa, &wa_s, &wq, &wq_s });          // before the caches are written
     Tensor y, ys;
     if (m == 0 || k == 0 || x.scalar_type() != at::kBFloat16 || dsv3_linear_fp8_fused(m, n, k)) {
         std::tie(y, ys) = mla_latent(linear_fp8(x, wa, wa_s, DSV3_SCALE_FMT_NONE, DSV3_BF16), qn, kn, freqs, kv, pe, start, q_eps, kv_eps);
     } else {            // the projection's K slices, if it has any, are added by the kernel behind it
+        TORCH_CHECK(x.is_contiguous() && kv.dim() == 3 && pe.dim() == 3 && n == qr + kv.size(2) + pe.size(2),
+                    "mla_query: x must be contiguous, the projections' weight [q_rank + kv_rank + rope, dim]");
+        check_weight("mla_query", wa, wa_s, n, k, 128);
         check_latent(x, qn, kn, freqs, kv, pe, start);
         const int64_t c = kv.size(2), r = pe.size(2);
-        TORCH_CHECK(x.is_contiguous() && n == qr + c + r, "mla_query: x must be contiguous, the projections' weight [q_rank + kv_rank + rope, dim]");
-        check_weight("mla_query", wa, wa_s, n, k, 128);
-        on_one_gpu("mla_query", x, { &wa, &wa_s });
         On on(x);
         const Tensor scr = gemm_scratch(x, m, n, k);
         const auto [xq, xs] = act_quant(x, 128, DSV3_SCALE_FMT_NONE);
@@ -321,6 +325,7 @@ Tensor mla_query(const Tensor& x, const Tensor& wa, const Tensor& wa_s, const Te
 // queries and caches -> the layer's output [b, s, dim]
 Tensor mla_output(const Tensor& q, const Tensor& freqs, const Tensor& kv, const Tensor& pe, const Tensor& w, const Tensor& ws,
                   const OptTensor& mask, int64_t positions, double scale, bool explicit_form, const Tensor& wo, const Tensor& wo_s) {
+    on_one_device("mla_output", q, { &wo, &wo_s });
     const auto [y, ys] = (explicit_form ? mla_prefill : mla_decode_quant)(q, freqs, kv, pe, w, ws, mask, positions, scale);
     return fp8_gemm(y, ys, wo, wo_s, DSV3_BF16);
 }

@@ -325,6 +325,37 @@ def test_mla_decode_validation(L):
     assert call(b=0, q=None) == 0 and L.lib.dsv3_mla_decode_workspace_bytes(2, 0, 64, 4) == 0
 
 
+def test_mla_decode_quant_validation(L):
+    def call(q=A16, kv=A16, pe=A16, w=A16, w_s=A16, y=A16, s=A16, mask=None, md=0, b=2, rows=1, pos=64, heads=4, nope=128, rope=64,
+             v=128, c=512, kvs=64 * 512, pes=64 * 64, scale=0.1, ws=0x1000, wsb=1 << 40, freqs=A16):
+        return L.lib.dsv3_mla_decode_quant(q, freqs, kv, kvs, pe, pes, w, w_s, mask, md, y, s, b, rows, pos, heads, nope, rope, v, c,
+                                           scale, ws, wsb, None)
+    for name in ("q", "kv", "pe", "w", "w_s", "y", "s", "freqs"):
+        assert call(**{name: None}) == 1
+    for bad in ({"nope": 64}, {"v": 64}, {"c": 256}, {"b": -1}, {"rows": -1}, {"pos": 0}, {"kvs": 64 * 512 - 8}, {"scale": 0.0}):
+        assert call(**bad) == 2, bad
+    for name in ("q", "kv", "pe", "w", "y"):
+        assert call(**{name: A16 + 8}) == 4
+    assert call(s=A16 + 2) == 4 and call(w_s=A16 + 2) == 4 and call(mask=A16, md=L.F16) == 5
+    need = L.lib.dsv3_mla_decode_workspace_bytes(2, 1, 64, 4)
+    assert call(ws=None) == 6 and call(wsb=need - 1) == 6 and call(ws=0x1080) == 6
+    assert call(b=0, q=None) == 0 and call(rows=0, q=None) == 0
+
+
+def test_mla_latent_gemm_validation(L):
+    def call(x=A16, x_s=A16, w=A16, w_s=A16, k=7168, a=A16, qw=A16, kw=A16, f=A16, kv=A16, kvs=512 * 8, pe=A16, pes=64 * 8, y=A16, s=A16,
+             b=2, rows=4, qr=1536, c=512, rope=64, ws=0x1000, wsb=1 << 40):
+        return L.lib.dsv3_mla_latent_gemm(x, x_s, w, w_s, k, a, qw, kw, f, kv, kvs, pe, pes, y, s, b, rows, qr, c, rope, 1e-6, 1e-6, ws, wsb, None)
+    for name in ("x", "x_s", "w", "w_s", "a", "qw", "kw", "f", "kv", "pe", "y", "s"):
+        assert call(**{name: None}) == 1
+        assert call(**{name: A16 + 2}) == 4
+    for bad in ({"qr": 100}, {"qr": 2176}, {"c": 256}, {"rope": 32}, {"b": -1}, {"rows": -1}, {"kvs": 2040}, {"k": 7000}, {"k": -128}):
+        assert call(**bad) == 2, bad
+    need = L.lib.dsv3_fp8_gemm_workspace_bytes(8, 2112, 7168)
+    assert need > 0 and call(ws=None) == 6 and call(wsb=need - 1) == 6 and call(ws=0x1080) == 6
+    assert call(b=0, a=None) == 0 and call(rows=0, x=None) == 0
+
+
 def test_mla_latent_validation(L):
     def call(a=A16, stride=2112, qw=A16, kw=A16, f=A16, kv=A16, kvs=512 * 8, pe=A16, pes=64 * 8, y=A16, s=A16, b=2, rows=4,
              qr=1536, c=512, rope=64):
@@ -356,11 +387,16 @@ def _operator_args(name):
     freqs, kv, pe = z(2, 32, dtype=torch.complex64), z(1, 8, 512, dtype=bf16), z(1, 8, 64, dtype=bf16)
     if name == "mla_latent":
         return [z(1, 2, 128 + 576, dtype=bf16), z(128, dtype=bf16), z(512, dtype=bf16), freqs, kv, pe, 3, 1e-6, 1e-6]
-    return [z(1, 2, 4, 192, dtype=bf16), freqs, kv, pe, z(1024, 512, dtype=fp8), z(8, 4), z(2, 8), 8, 0.1]
+    if name == "mla_query":         # 20 rows: the branch with the projection's slabs
+        return [z(1, 20, 256, dtype=bf16), z(128 + 576, 256, dtype=fp8), z(6, 2), z(128, dtype=bf16), z(512, dtype=bf16), z(20, 32, dtype=torch.complex64),
+                z(1, 32, 512, dtype=bf16), z(1, 32, 64, dtype=bf16), 3, 1e-6, 1e-6, z(768, 128, dtype=fp8), z(6, 1), 4]
+    args = [z(1, 2, 4, 192, dtype=bf16), freqs, kv, pe, z(1024, 512, dtype=fp8), z(8, 4), z(2, 8), 8, 0.1]
+    return args + [False, z(256, 512, dtype=fp8), z(2, 4)] if name == "mla_output" else args
 
 
 OPERATORS = {"weight_dequant": (0, 1), "fp8_gemm": (0, 1, 2, 3), "fp8_gemm_pow2": (0, 1, 2, 3), "linear_fp8": (0, 1, 2),
-             "mla_prefill": range(7), "mla_decode": range(7), "mla_latent": range(6)}
+             "mla_prefill": range(7), "mla_decode": range(7), "mla_decode_quant": range(7), "mla_output": (*range(7), 10, 11), "mla_latent": range(6),
+             "mla_query": (*range(8), 11, 12)}
 
 
 @pytest.mark.parametrize("name", OPERATORS)
@@ -374,16 +410,23 @@ def test_operators_refuse_tensors_of_two_devices(name):
             _gpu_body(name, *args)
 
 
-@pytest.mark.parametrize("name", ["mla_prefill", "mla_decode", "mla_latent"])
+@pytest.mark.parametrize("name", ["mla_prefill", "mla_decode", "mla_decode_quant", "mla_output", "mla_latent", "mla_query"])
 def test_attention_operators_refuse_what_their_kernels_cannot_read(name):
-    f = 3 if name == "mla_latent" else 1                # where the phases stand
+    f = {"mla_latent": 3, "mla_query": 5}.get(name, 1)  # where the phases stand
     bad = {f: [lambda t: t.conj(), lambda t: t[:1]]}
-    if name == "mla_latent":
-        bad[6] = [lambda t: 7, lambda t: -1, lambda t: 2 ** 63 - 1]
+    if name in ("mla_latent", "mla_query"):
+        bad[f + 3] = [lambda t: 13 if name == "mla_query" else 7, lambda t: -1, lambda t: 2 ** 63 - 1]
+        bad[f - 1] = [lambda t: t.float(), lambda t: t[:511]]
+        bad[f + 1] = [lambda t: t.float(), lambda t: t[:, ::2]]
     else:                                               # scales: too few rows, columns, another type
         bad[5] = [lambda t: t[:7], lambda t: t[:, :3].contiguous(), lambda t: t.bfloat16(), lambda t: t.flatten()]
         bad[3] = [lambda t: t.float()]
         bad[6] = [lambda t: t[:, :7], lambda t: t.half()]
+    if name == "mla_query":
+        bad[0] = [lambda t: torch.zeros(1, 20, 512, dtype=t.dtype)[:, :, ::2], lambda t: t[0]]
+        bad[1] = [lambda t: t[:703], lambda t: t.bfloat16(), lambda t: t[:, :255], lambda t: t[0]]
+        bad[2] = [lambda t: t[:5], lambda t: t[:, :1], lambda t: t.half()]
+        bad[11] = [lambda t: t[:767], lambda t: t[0]]
     for at, changes in bad.items():
         for change in changes:
             args = _operator_args(name)
@@ -491,12 +534,12 @@ def test_block_size_zero_divides_by_zero():
             call(torch.zeros(128, 128), 0)
 
 
-@pytest.mark.parametrize("source", ["fp8_gemm_skinny.hip", "fp8_gemm_stream.hip", "mla_decode.hip", "mla_prefill.hip"])
+@pytest.mark.parametrize("source", ["fp8_gemm_skinny.hip", "fp8_gemm_stream.hip", "fp8_gemm_mid.hip", "mla_decode.hip", "mla_prefill.hip"])
 def test_build_refuses_spills(source):
     import build
     assert source in build.NO_SPILL_SOURCES and (build.CSRC / source).exists()
     report = "remark: Function Name: _ZN4dsv317{}EvNS_4ArgsE\nremark:     {}: {}\n"
-    for kernel in ("mla_decode_kernelILi0E", "mla_combine_kernel", "mla_expand_kernel", "mla_attend_kernelILb0E"):
+    for kernel in ("mla_decode_kernelILi0E", "mla_fold_kernelILb1E", "fp8_gemm_mid_kernelILi6E", "mla_expand_kernel", "mla_attend_kernelILb0E"):
         build.check_no_spills(source, report.format(kernel, "VGPRs Spill", 0))
         for what in ("VGPRs Spill", "ScratchSize [bytes/lane]", "SGPRs Spill"):
             with pytest.raises(RuntimeError, match="must not spill"):
