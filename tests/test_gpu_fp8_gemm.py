@@ -106,6 +106,7 @@ def test_large_m_tile_heights_and_short_k(K, m, n, k):
     (128, 18432, 7168),   # 72 tiles, 3 slices of 19 + 19 + 18 blocks
     (257, 7168, 18432),   # 84 tiles, 3 slices of 48 blocks
     (65, 1536, 1152),     # 9 K blocks: too short to cut, one slice
+    (100, 577, 7296),     # as the first, which the mid-M tiles take (K in whole groups of 512): 7 slices of 9 and 3 blocks; ragged N
 ])
 def test_mid_m_split_over_k(K, m, n, k):
     """Between 65 and a few hundred rows the large-M kernel cuts the K range into slices run by separate

@@ -134,21 +134,45 @@ def test_decode_attention(b, s, t, h, kind, grow):
     assert ((got - ref).norm(dim=-1) <= 2.0 ** -7 * ref.norm(dim=-1)).all()
 
 
-# tokens in all: 1, 2, 3 .. 4, 5 .. 8 and more share a workgroup's wavefronts differently, 16 are a group; splits below, at and
-# above a wavefront's 64 lanes (256 workgroups over the row blocks, 32 positions a tile)
-@pytest.mark.parametrize("b,s,t,h", [(1, 1, 33, 128), (1, 1, 2080, 128), (1, 1, 8192, 8), (2, 1, 700, 128), (3, 1, 5000, 16),
-                                     (4, 1, 90, 128), (1, 5, 300, 128), (8, 1, 1, 128), (16, 1, 257, 128), (17, 1, 64, 32), (3, 13, 200, 24)])
-def test_decode_attention_quantised_is_the_rounded_result_quantised(b, s, t, h):
+# A workgroup of the fold takes a head and 4, 8 or 16 tokens at a time: 16 heads and fewer 4 here, 128 heads 4 up to 8 tokens in all, 8 up to 16,
+# then 16, and past 128 tokens (1024 / heads groups) several groups, one after another.  One token of a group is shared by eight
+# wavefronts, two by four each, three or four by two each, more have one each.  Splits below, at and above a wavefront's 64 lanes (256
+# workgroups over the row blocks, 32 positions a tile).
+FOLD = [(1, 1, 33, 128, None), (1, 1, 2080, 128, None), (1, 1, 8192, 8, None), (2, 1, 700, 128, None), (3, 1, 5000, 16, None),
+        (4, 1, 90, 128, None), (1, 5, 300, 128, None), (8, 1, 1, 128, None), (16, 1, 257, 128, None), (17, 1, 64, 32, None), (3, 13, 200, 24, None),
+        (32, 1, 100, 128, None), (37, 1, 70, 128, None),            # groups of 16, the last one of 5
+        (131, 1, 40, 128, None),                                    # nine groups over eight workgroups a head: 16 tokens, then 3
+        (8, 32, 64, 128, "causal"), (2, 66, 130, 128, "causal_f32"), (2, 9, 200, 128, "holes"), (1, 6, 90, 5, "lowest")]
+
+
+@pytest.mark.parametrize("b,s,t,h,kind", FOLD)
+def test_decode_attention_quantised_is_the_rounded_result_quantised(b, s, t, h, kind):
     from dsv3fp8 import kernel
     q, freqs, kv, pe, w8, ws = _inputs(b, s, t, h, s + t)
-    args = (q, freqs, kv, pe, w8, ws, None, t, 0.08)
+    args = (q, freqs, kv, pe, w8, ws, _mask(kind, s, t, 5), t, 0.08)
     y = torch.ops.dsv3fp8.mla_decode(*args)
     ref = _decode_reference(*args)
     got = y.view(b, s, h, V).double()
-    assert ((got - ref).norm(dim=-1) <= 2.0 ** -7 * ref.norm(dim=-1)).all()         # as in test_decode_attention
+    nan = torch.isnan(ref).any(-1)                       # (a row that sees nothing)
+    assert torch.equal(nan, torch.isnan(got).any(-1)) and nan.any() == (kind == "holes")
+    assert ((got - ref).norm(dim=-1) <= 2.0 ** -7 * ref.norm(dim=-1))[~nan].all()   # as in test_decode_attention
     yq, ys = torch.ops.dsv3fp8.mla_decode_quant(*args)
     rq, rs = kernel.act_quant(y)
-    assert torch.equal(yq.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(ys, rs)
+    assert torch.equal(yq.view(torch.uint8), rq.view(torch.uint8)) and torch.equal(ys.view(torch.int32), rs.view(torch.int32))
+
+
+@pytest.mark.parametrize("explicit", [False, True])
+@pytest.mark.parametrize("b,s,t,h,kind", [(1, 1, 40, 4, None), (3, 1, 500, 128, None), (2, 40, 130, 8, "causal"), (1, 33, 33, 128, "causal_f32"), (2, 36, 70, 4, "holes")])
+def test_output_in_one_call_is_its_two_parts(b, s, t, h, kind, explicit):
+    """mla_output: the attention in either form, quantised, and the product with wo, bit for bit."""
+    from dsv3fp8 import quantize
+    args = (*_inputs(b, s, t, h, s + t), _mask(kind, s, t, 5), t, 0.08)
+    wo, wo_s = quantize.weight_quant((torch.randn(384, h * V, generator=torch.Generator().manual_seed(h)) * 0.02).bfloat16().cuda())
+    y = torch.ops.dsv3fp8.mla_output(*args, explicit, wo, wo_s)
+    attention = torch.ops.dsv3fp8.mla_prefill if explicit else torch.ops.dsv3fp8.mla_decode_quant
+    ref = torch.ops.dsv3fp8.fp8_gemm(*attention(*args), wo, wo_s, 0)
+    assert y.shape == (b, s, 384) and y.dtype == torch.bfloat16
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16)) and torch.isfinite(y[:, 0]).all()
 
 
 # rows whose projection runs as one launch, in K slices of the streaming kernel, in slices of the tile kernel (up to eight), plain
