@@ -1,4 +1,5 @@
-// fp8_gemm for 65 rows to about a thousand where whole 256-column tiles leave compute units without work
+// fp8_gemm for 65 rows and more where whole 256-column tiles leave compute units without work: up to 224 rows of wide weights, up to
+// a few hundred of narrow ones, 8192 where these have 128 columns or fewer
 // (reference arithmetic: inference/kernel.py:118-172).
 //
 // A tile of 16 MT rows x 16 SN WN columns per workgroup: eight wavefronts, WM along the rows (16-row sub-tiles dealt round-robin) x
@@ -267,7 +268,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     // one row tile.  65 .. 224 rows of 7168 -> 36864 (231 tiles).  Measured with the quantisation in front over 32769 .. 40960 columns and K
     // of 2560 .. 16384, (large-M kernel's time) / (time here): 1.05 .. 1.30 up to 192 rows, 1.02 .. 1.23 at 193 and 224.  What is left out:
     // 32768 columns and fewer, where 128-row tiles of the large-M kernel, two a column tile or in two K slices, are one full round
-    // (7168 -> 31744 at 65 / 160 / 193 rows 0.93 / 0.88 / 0.84); K of 32768 (0.81 .. 1.39, most below 1 at 193 rows); from 193 rows on,
+    // (7168 -> 31744 at 65 / 160 / 193 rows 0.93 / 0.88 / 0.84); K of 32768 (0.81 .. 1.50, 0.92 .. 0.96 at 193 rows); from 193 rows on,
     // whose ring has three stages, fewer than 212 tiles or 32 K blocks (16384 -> 32769 0.94, 2560 -> 40960 0.98); 225 rows and more, whose
     // ring would have two; two row tiles of 116 for 7168 -> 18432 (129 .. 224 rows, 48.4 us there, 53.5 here at 193): that one 128- or
     // 256-row tile of the large-M kernel reads the weights once.
@@ -277,9 +278,9 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
         p.mt = rows <= 6 ? 6 : rows <= 8 ? 8 : rows <= 10 ? 10 : rows <= 12 ? 12 : 14;
         return p;
     }
-    // Up to 128 rows of a weight of 176 to 256 tiles of 128 columns, in one round where 256 columns make half a round: 1536 -> 24576 13 .. 23 %
-    // less; over 22401 .. 32768 columns and K of 1536 .. 16384, measured as above, 0.99 .. 1.77.  Not below 12 K blocks (512 -> 32768: equal to
-    // 12 % more), nor above 128 (32768 -> 28672 at 128 rows 0.98).
+    // Up to 128 rows of a weight of 176 to 256 tiles of 128 columns, in one round where 256 columns make half a round: over 22401 .. 32768
+    // columns and K of 1536 .. 16384, measured as above, 0.98 .. 1.77, 1536 -> 24576 1.23 .. 1.14.  Not below 12 K blocks (512 -> 32768: equal to
+    // 12 % more time), nor above 128 (32768 -> 28672 at 128 rows 0.98).
     const int64_t t128 = (n + 127) / 128;
     if (m <= 128 && t128 >= 176 && t128 <= 256 && kb >= 12 && kb <= 128) {
         p.mt = 8; p.wm = 4; p.sn = 4;
@@ -291,6 +292,8 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     // 8 .. 20 blocks: 7168 -> 1536 at 128 / 256 / 448 rows 19.8 / 23.0 / 23.7 -> 16.3 / 18.9 / 22.7, 7168 -> 576 at 256 / 1024 19.5 / 25.0 ->
     // 16.3 / 23.8, 7168 -> 2112 at 128 / 320 20.3 / 22.7 -> 17.2 / 21.6, 4096 -> 1024 at 900 25.5 -> 20.8; of 28: 7168 -> 1536 at 449 24.0 ->
     // 24.8, 7168 -> 2112 at 321 22.9 -> 24.0; of 44: 16384 -> 2304 at 300 30.8 -> 38.0; of 56: 7168 -> 1536 at 777 29.3 -> 33.7.
+    // Over 1 .. 2304 columns and K of 4096 .. 16384, 65 rows up to the last one taken (1 .. 128 columns: 8192 at K of 4096, 5440 at 7168;
+    // 300: 2688; 576: 1600), measured as above: 0.99 .. 1.51, at the last ones 1.01 .. 1.28.
     const int64_t tiles = (m + 63) / 64 * t128;
     if (n <= 2304 && kb >= 32 && tiles <= 256) {
         int64_t s = 256 / tiles;
