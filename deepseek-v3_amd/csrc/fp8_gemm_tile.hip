@@ -339,11 +339,11 @@ int forced_kernel() {
 }
 
 // Which problems go to the large-M kernel (K range cut into slices when the tiles do not fill the chip): every M
-// above 64, unless the mid-M tiles take it (mid_supported, asked behind this), and M = 33 .. 64 when the weight is large (>= 96 MiB) and has 8192 rows or more (7168 -> 36864 at 64 rows:
-// 65 against 66-76 us).  There it runs at a flat 32-34 us per 117-132 MB from 9 to 64 rows.  Everything else the
-// activation-streaming kernel has a plan for goes there (16384 -> 7168 at 16 / 32 / 64 rows 23.5 / 24.5 / 29.5 against
-// 33 / 31.6 / 34.6 us; 7168 -> 18432 at 16 / 32 rows 22.8 / 25.3 against 36.5 / 30.7 us); for the smaller decode
-// weights the streaming and tile kernels are faster anyway.
+// above 64, unless the mid-M tiles take it (mid_supported, asked behind this), and M = 33 .. 64 when the weight is large
+// (>= 96 MiB) and has 8192 rows or more (7168 -> 36864 at 64 rows: 65 against 66-76 us).  There it runs at a flat 32-34 us
+// per 117-132 MB from 9 to 64 rows.  Everything else the activation-streaming kernel has a plan for goes there (16384 -> 7168
+// at 16 / 32 / 64 rows 23.5 / 24.5 / 29.5 against 33 / 31.6 / 34.6 us; 7168 -> 18432 at 16 / 32 rows 22.8 / 25.3 against
+// 36.5 / 30.7 us); for the smaller decode weights the streaming and tile kernels are faster anyway.
 bool to_large_m_kernel(int64_t m, int64_t n, int64_t k) {
     if (!prefill_supported(m, n, k)) return false;
     if (m > 64) return true;
