@@ -1,5 +1,6 @@
 // What the attention kernels of MLA.forward share: bf16 MFMAs of 32 x 32, copies into LDS, masks, the softmax offset.
 #pragma once
+#include <type_traits>
 #include "common.hpp"
 
 namespace dsv3 {
@@ -17,8 +18,29 @@ __device__ __forceinline__ void copy16(const void* base, uint32_t lane_off, uint
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :: "v"(lane_off), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
+// The same through a buffer descriptor (the range check answers requests past its end with zeros), into LDS at lds_addr + IMM
+__device__ __forceinline__ v4i buffer_of(const void* base, int bytes) {
+    const uintptr_t a = (uintptr_t)base;
+    return v4i{ (int)(uint32_t)a, (int)((uint32_t)(a >> 32) & 0xffffu), bytes, 0x00027000 };
+}
+template <int IMM> __device__ __forceinline__ void copy16_buffer(v4i buffer, uint32_t lane_off, uint32_t lds_addr) {
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                 :: "v"(lane_off), "s"(buffer), "s"(lds_addr), "n"(IMM) : "memory", "m0", "scc");
+}
+// f(integral_constant 0), .., f(integral_constant N - 1)
+template <int N, int I = 0, class F> __device__ __forceinline__ void unrolled(F f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        unrolled<N, I + 1>(f);
+    }
+}
 __device__ __forceinline__ void barrier_no_fence() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ __forceinline__ float xor32(float v) { return __shfl_xor(v, 32); }
+// the values of lanes l and l + 32, in this order, in both
+__device__ __forceinline__ v2f halves32(float v) {
+    const v2u r = __builtin_amdgcn_permlane32_swap(f32_as_u32(v), f32_as_u32(v), false, false);
+    return v2f{ u32_as_f32(r[0]), u32_as_f32(r[1]) };
+}
 
 template <bool F32> __device__ __forceinline__ float mask_at(const void* m, int64_t i) {
     return F32 ? ((const float*)m)[i] : u32_as_f32((uint32_t)((const uint16_t*)m)[i] << 16);

@@ -20,12 +20,11 @@ typedef __attribute__((address_space(3))) v4bf* lds_v4bf;
 
 constexpr int kC = 512, kRope = 64, kNope = 128, kQd = kNope + kRope;
 constexpr int kTile = 32;                               // positions per tile
-constexpr int kStages = 4;                              // tiles in LDS: one computed, three on their way
+constexpr int kStages = 4;                              // tiles in LDS, computed or on their way
 constexpr int kRopeOff = kTile * kC * 2;                // a stage: 32 rows of 1 KiB latents, then 32 rows of 128 B rotary keys
 constexpr int kStage = kRopeOff + kTile * kRope * 2;
 constexpr int kAhead = 6;                               // operands read from LDS ahead of the MFMA that takes them
-constexpr int kRows = 128;                              // rows per workgroup: 4 wavefronts x 32
-constexpr int kPartFloats = kRows * kC;                 // partial sums of a workgroup
+constexpr int kSync = 28;                               // the value step behind which a tile's stage is free and the next tile's keys are read
 
 struct DecodeArgs {
     const void* ql;                                     // folded queries [batch][rows][512], rows = tokens * heads, or in operand order
@@ -36,7 +35,8 @@ struct DecodeArgs {
     const void* mask;                                   // [tokens][positions]
     float* part;                                        // [batch][row block][split][row][512]
     v2f* ml;                                            // [batch][row block][row][split] (maximum, sum)
-    int batch, rows, heads, positions, tiles, blocks, splits, per;
+    int rows, heads, positions, tiles, groups, side, blocks, splits, per;   // groups: of 32 rows, in whole 128s; side: tiles that a workgroup takes side by side (G)
+    uint32_t blocks_magic, splits_magic;                // for quotient()
     float unit, scale, inv_scale;                       // score_unit's unit and rest, and the rest's reciprocal; without a mask 1 and the scale
 };
 
@@ -56,54 +56,102 @@ __device__ __forceinline__ void scale_agprs(v16f& v, float a) {
     }
 }
 
+// mfma32 with its result in ordinary registers: the compiler would put it into accumulation registers, which are all taken, and move 16 sums
+// out and back per tile.  It does not know that these are MFMAs, so what it would keep apart stands here: two wait states in front
+// (an ordinary instruction may have written an operand); behind the last one, before its result is read, scores_ready.
+__device__ __forceinline__ void mfma32_first(v16f& d, v4u a, v4u b) {
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma32_next(v16f& d, v4u a, v4u b) {
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(d) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void scores_ready(v16f& d) { asm volatile("s_nop 15" : "+v"(d)); }
+
+// n / d by a multiplication: magic is 2^32 / d rounded up, exact as long as n d < 2^32, or 0 where that does not hold (a division in front of
+// everything else costs a quarter of a microsecond)
+__device__ __forceinline__ int quotient(int n, int d, uint32_t magic) { return d == 1 ? n : magic ? (int)__umulhi((uint32_t)n, magic) : n / d; }
+inline uint32_t magic_of(int64_t most, int64_t d) { return d > 1 && most * d < (1ll << 32) ? (uint32_t)(((1ll << 32) + d - 1) / d) : 0u; }
+
 // Four wavefronts with all 512 registers of their SIMD lane each: a wavefront holds 32 rows' queries as MFMA operands (144
-// registers) and their 32 x 512 weighted sums (256).  Per tile of 32 positions (36 KiB, copied into
-// LDS three tiles ahead): S^T = K Q^T (36 MFMAs), exponentials in registers, O^T += V^T P^T (32 MFMAs).  The
+// registers) and their 32 x 512 weighted sums (256).  Per tile of 32 positions (36 KiB in LDS): S^T = K Q^T (36 MFMAs), exponentials in
+// registers, O^T += V^T P^T (32 MFMAs).  The
 // transposed products leave a row in one lane (and the lane 32 further), and S^T's accumulators already are P^T's operand
 // (position 16 u + 8 a + 4 g + r of a tile in register 8 u + 4 a + r of lane half g, slot 4 a + r of K step u).  Keys and
 // values are the same 32 x 512 block: the keys are read as rows, the values through the LDS's transposing reads, four
 // positions of one feature per lane.
-// Bound: per tile 68 MFMAs of 32 cycles; with one wavefront per SIMD its exponentials and barriers stand beside them.  32
-// sequences at 4096 positions (16 tiles a workgroup): 53 .. 58 us, 70 with each LDS read next to its MFMA; 12 us of it are the 67 MB
-// of partial sums at the end, and one tile alone (a short context) takes 10.7 us in all, 12.7 without PACK.  The tensor operations in its place
-// took 250 us (58 us in the products, the rest in passes over the scores).
+// G tiles side by side: 4 / G groups of 32 rows share a tile, the G wavefronts of a group take every G-th tile of the range and add their
+// sums in LDS at the end.  The partial sums that leave (2 KiB a row and range) and that fold reads again are a G-th, the latents that the
+// workgroups copy G times as many (from the XCD's L2, the row blocks of a range are neighbours there), and the four stages hold three
+// tiles ahead (G = 1), one (2) or none (4).
+// Bound: per tile 68 MFMAs of 32 cycles (2180), 1250 + 1190 cycles with their operands' reads, 700 of exponentials, of which the second half stand
+// beside the first half's products; a tile takes 3800 in all (4630 with the copies in a row in front and every exponential between the products),
+// of which the clock takes back half (1.97 against 2.07 GHz at 32 x 4096).  What a range costs besides: at 256 workgroups and G = 1 67 MB of partial sums, 12 us
+// to write and as long to read.  Attention with the query's fold and mla_fold_kernel (us, before: G = 1): 8 sequences at 2000 positions 41.9 ->
+// 30.0 (G = 4), 16 at 2000 48.7 -> 34.8 (4), 32 at 1000 50.0 -> 38.3 (4), 64 at 1000 62.6 -> 53.4 (2), 32 at 4096 78.7 -> 68.7 (2), 1 at 700 22.6 -> 22.0.
 // PACK: the folded queries come in operand order (launch_wkv_b_absorb_q_packed), a KiB of consecutive bytes per load; as rows a
 // load touches 32 of them and takes 64 cycles of the compute unit's load path, 3.8 us for the workgroup's 128.
 enum { kNoMask, kMaskBf16, kMaskF32 };
-template <int MASK, bool PACK>
+template <int MASK, bool PACK, int G>
 __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    constexpr int RB = 4 / G, R = kStages / G;          // row groups of a workgroup; steps that the stages hold
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i = lane & 31, g = lane >> 5;
-    const int split = blockIdx.x, b = blockIdx.y, blk = blockIdx.z;
-    const int t0 = split * p.per, t1 = min(p.tiles, t0 + p.per);
-    const int row0 = blk * kRows + wave * 32;
+    const int i = lane & 31, g = lane >> 5, rg = wave % RB, par = wave / RB;
+    // a contiguous run of workgroups per XCD, the row blocks of a range next to each other: its latents are in the XCD's L2
+    int unit = blockIdx.x;
+    {
+        const int T = gridDim.x, q = T / 8, r = T % 8, x = unit % 8;
+        unit = x * q + min(x, r) + unit / 8;
+    }
+    const int range = quotient(unit, p.blocks, p.blocks_magic), blk = unit - range * p.blocks;
+    const int b = quotient(range, p.splits, p.splits_magic), split = range - b * p.splits;
+    const int t0 = split * p.per, t1 = min(p.tiles, t0 + p.per), limit = min(p.positions, t1 * kTile);
+    const int row0 = blk * (RB * 32) + rg * 32;
     const int row = min(row0 + i, p.rows - 1);          // rows past the end repeat the last one; fold leaves them out
 
+    // A tile is a buffer of the positions that it has: rows past the end, and all of a tile past the range, read as zeros without a
+    // request, so that every tile is as many copies, whose outstanding ones can be counted.
+    const uint32_t lds0 = lds_addr_of(lds);
     const uint16_t* kvb = p.kv + b * p.kv_bs;
     const uint16_t* peb = p.pe + b * p.pe_bs;
-    const uint32_t lds0 = lds_addr_of(lds);
-    auto issue = [&](int t, int st) {
-#pragma unroll
-        for (int n = 0; n < 8; ++n) {
-            const int r = wave * 8 + n;
-            const int pos = min(t * kTile + r, p.positions - 1);
-            copy16(kvb + (int64_t)pos * kC, (uint32_t)((lane ^ swz(r)) << 4), lds0 + st * kStage + r * 1024);
-        }
-        // eight rows of 128 bytes; chunk c of row r at c ^ (r / 2 & 7)
-        const int r = wave * 8 + (lane >> 3);
-        const int pos = min(t * kTile + r, p.positions - 1);
-        copy16(peb, (uint32_t)pos * (kRope * 2) + (((lane & 7) ^ ((r >> 1) & 7)) << 4), lds0 + st * kStage + kRopeOff + wave * 1024);
+    struct Source { v4i kv, pe; uint32_t at; };
+    auto source = [&](int t, int st) -> Source {
+        const int rows = t < t1 ? min(p.positions - t * kTile, kTile) : 0;
+        return { buffer_of(kvb + (int64_t)t * (kTile * kC), rows * (kC * 2)), buffer_of(peb + (int64_t)t * (kTile * kRope), rows * (kRope * 2)), lds0 + st * kStage };
     };
-#pragma unroll
-    for (int n = 0; n < kStages - 1; ++n)
-        if (t0 + n < t1) issue(t0 + n, n);
+    // G < 4: all wavefronts copy a tile, nine copies each: rows 4 w .. and 16 + 4 w .. of the latents (whose swizzles differ in constants only)
+    // and eight rotary rows.  G = 4: a wavefront its own tile, 36 copies.
+    const uint32_t kvoff = G < 4 ? wave * 4096 + ((lane ^ wave) << 4) : lane << 4;      // row 0 of the wavefront's; row r has chunk c at c ^ swz(r)
+    const int w2 = G < 4 ? (wave & 1) << 2 : 0;
+    const uint32_t peoff = (G < 4 ? wave * 1024 : 0) + (lane >> 3) * 128 + (((lane & 7) ^ ((lane >> 4) & 3 | w2)) << 4);   // row r has chunk c at c ^ (r / 2 & 7)
+    const uint32_t kv_add = G < 4 ? wave * 4096 : 0, pe_add = kRopeOff + (G < 4 ? wave * 1024 : 0);
+    auto issue = [&](const Source& s, auto which) {
+        constexpr int n = decltype(which)::value;
+        if constexpr (G < 4) {
+            if constexpr (n < 8) copy16_buffer<(n & 3) * 1024 + (n >> 2) * 16384>(s.kv, kvoff ^ ((n & 3) * 0x440 + (n >> 2) * 16384), s.at + kv_add);
+            else copy16_buffer<0>(s.pe, peoff, s.at + pe_add);
+        } else {
+            uint32_t off = n < 32 ? kvoff : peoff;
+            asm volatile("" : "+v"(off));               // (nor for 36 copies' offsets)
+            if constexpr (n < 32) copy16_buffer<n * 1024>(s.kv, off ^ (n * 1024 + (((n & 3) << 2 | (n >> 2 & 3)) << 4)), s.at);
+            else copy16_buffer<(n - 32) * 1024>(s.pe, off ^ ((n - 32) * 1024 + ((n & 1) << 6)), s.at + pe_add);
+        }
+    };
+    if constexpr (G < 4) {
+        for (int n = 0; n < (R - 1) * G && (G > 1 || t0 + n < t1); ++n) {
+            const Source s = source(t0 + n, n);
+            unrolled<9>([&](auto k) { issue(s, k); });
+        }
+    } else if (t0 + par < t1) {
+        const Source s = source(t0 + par, par);
+        unrolled<36>([&](auto k) { issue(s, k); });
+    }
 
     // lane (row i, half g) holds elements 16 s + 8 g .. + 7; the last four steps are rotated here
     v4u Q[36];
     {
         // (packed, a last block's missing rows hold anything; nobody reads their results)
-        const v4u* src = (const v4u*)p.ql + (PACK ? (((int64_t)b * p.blocks + blk) * 4 + wave) * (kC / 16) * 64 + lane : ((int64_t)b * p.rows + row) * (kC / 8) + g);
+        const v4u* src = (const v4u*)p.ql + (PACK ? ((int64_t)b * p.groups + row0 / 32) * (kC / 16) * 64 + lane : ((int64_t)b * p.rows + row) * (kC / 8) + g);
 #pragma unroll
         for (int s = 0; s < 32; ++s) Q[s] = src[s * (PACK ? 64 : 2)];
         const uint16_t* rsrc = p.q + ((int64_t)b * p.rows + row) * kQd + kNope + 8 * g;
@@ -129,48 +177,67 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
     v16f O[16] = {};
     float m = -__builtin_inff(), l = 0.f;               // running maximum of the scores, this lane's share of the sum
     const float scale2 = p.scale * 1.44269504088896340736f;
-    int st = 0;
-    for (int t = t0; t < t1; ++t) {
-        // this wavefront's nine copies of the tile: those of the tiles behind it stay in flight
-        if (t + 2 < t1)      __builtin_amdgcn_s_waitcnt(0x0f70 | (18 & 15) | (18 >> 4) << 14);      // vmcnt(18)
-        else if (t + 1 < t1) __builtin_amdgcn_s_waitcnt(0x0f70 | 9);
-        else                 __builtin_amdgcn_s_waitcnt(0x0f70);
-        barrier_no_fence();                             // everybody's, and the stage of the tile before is free
-        if (t + kStages - 1 < t1) issue(t + kStages - 1, (st + kStages - 1) % kStages);
-        const uint8_t* base = lds + st * kStage;
-        v16f T[1] = {};
-        v16f& S = T[0];
-        // operands kAhead steps ahead; the barriers keep this order (the scheduler puts each read next to its use and waits)
-        v4u ring[kAhead];
-        auto key = [&](int s) -> v4u {
-            return s < 32 ? *(const v4u*)(base + (kaddr ^ ((s & 7) << 5)) + (s >> 3) * 256) : *(const v4u*)(base + (raddr ^ ((s - 32) << 5)));
+    // Operands are read kAhead MFMAs ahead of use; the sched_barriers keep the order that is written here (left alone, the scheduler puts each read
+    // next to its MFMA and waits).  The ring goes from the keys to the values and on to the next tile's keys; as it makes no whole
+    // number of turns in the 32 value steps, the first two keys have registers of their own.
+    v4u ring[kAhead], first[2];
+    auto key = [&](const uint8_t* base, int s) -> v4u {
+        return s < 32 ? *(const v4u*)(base + (kaddr ^ ((s & 7) << 5)) + (s >> 3) * 256) : *(const v4u*)(base + (raddr ^ ((s - 32) << 5)));
+    };
+    auto first_keys = [&](const uint8_t* base) {
+        first[0] = key(base, 0);
+        first[1] = key(base, 1);
+#pragma unroll
+        for (int s = 2; s < kAhead + 2; ++s) ring[s % kAhead] = key(base, s);
+    };
+    // the next step's tiles are there, once this wavefront's copies of them are (G = 1: those of the two behind it stay in flight) and everybody's
+    auto arrived = [&] {
+        constexpr int left = R > 2 ? (R - 2) * 9 * G : 0;
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (left & 15) | (left >> 4) << 14);   // vmcnt
+        barrier_no_fence();
+    };
+
+    // One tile.  qk_copy and pv_copy: copies beside the MFMA just issued.  The last value steps read the next tile's first keys (G < 4).
+    auto tile = [&](int t, const uint8_t* base, const uint8_t* next, auto qk_copy, auto pv_copy) {
+        const uint32_t vbase = lds_addr_of(base) + vaddr;       // stages are multiples of 1 KiB: the xors below stay inside a row
+        auto value = [&](int s) -> v4u {                        // positions 16 (s / 16) .. of features 32 (s % 16) ..
+            const uint32_t at = (vbase ^ ((s & 3) << 6)) + (s >> 4) * 16384 + ((s & 15) >> 2) * 256;
+            const v2u lo = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf)(uintptr_t)at));
+            const v2u hi = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf)(uintptr_t)((at ^ 32) + 8192)));
+            return v4u{ lo[0], lo[1], hi[0], hi[1] };
         };
-#pragma unroll
-        for (int s = 0; s < kAhead; ++s) ring[s] = key(s);
+        v16f T[1];
+        v16f& S = T[0];
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s = 0; s < 36; ++s) {
-            S = mfma32(ring[s % kAhead], Q[s], S);
-            if (s + kAhead < 36) ring[s % kAhead] = key(s + kAhead);
+        unrolled<36>([&](auto step) {
+            constexpr int s = decltype(step)::value;
+            if constexpr (s == 0) mfma32_first(S, first[0], Q[0]);
+            else mfma32_next(S, s < 2 ? first[s] : ring[s % kAhead], Q[s]);
+            if constexpr (s >= 2) ring[s % kAhead] = s + kAhead < 36 ? key(base, s + kAhead) : value(s + kAhead - 36);
+            qk_copy(step);
             __builtin_amdgcn_sched_barrier(0);
-        }
+        });
+        scores_ready(S);
         if constexpr (MASK != kNoMask) {
-            const int64_t mrow = (int64_t)(row / p.heads) * p.positions;
+            int tok = row / p.heads;
+            asm volatile("" : "+v"(tok));               // (the addresses are formed here: there are no registers to keep them in)
+            const int64_t mrow = (int64_t)tok * p.positions;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int64_t at = mrow + min(t * kTile + 8 * (e >> 2) + 4 * g + (e & 3), p.positions - 1);
                 S[e] = __builtin_fmaf(S[e], p.unit, mask_at<MASK == kMaskF32>(p.mask, at) * p.inv_scale);
             }
         }
-        if ((t + 1) * kTile > p.positions) {            // the last tile may reach past the end
+        if ((t + 1) * kTile > limit) {                  // the last tile may reach past the end, a step's tiles past the range
 #pragma unroll
             for (int e = 0; e < 16; ++e)
-                if (t * kTile + 8 * (e >> 2) + 4 * g + (e & 3) >= p.positions) S[e] = -__builtin_inff();
+                if (t * kTile + 8 * (e >> 2) + 4 * g + (e & 3) >= limit) S[e] = -__builtin_inff();
         }
         float mx = S[0];
 #pragma unroll
         for (int e = 1; e < 16; ++e) mx = __builtin_elementwise_maximum(mx, S[e]);
-        mx = fmaxf(mx, xor32(mx));
+        const v2f both = halves32(mx);
+        mx = fmaxf(both.x, both.y);
         // The maximum is only raised when it grows by more than 2^64: exponentials and sums have room for that in binary32
         // and bf16, and so the 256 multiplications are needed in the rarest of cases.
         // (Rows past the end, whose queries are whatever the scratch held, do not ask for it: the others' roundings would follow.)
@@ -180,73 +247,156 @@ __global__ __launch_bounds__(256, 1) void mla_decode_kernel(DecodeArgs p) {
             const float a = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f((m - mn) * scale2);
             l *= a;
             m = mn;
-            if (t > t0) {
+            if (t >= t0 + G) {
 #pragma unroll
                 for (int d = 0; d < 16; ++d) scale_agprs(O[d], a);
                 asm volatile("s_nop 7" ::: "memory");
             }
         }
         const float off = softmax_offset(T, m, scale2);
-        const uint32_t vbase = lds0 + st * kStage + vaddr;      // stages are multiples of 1 KiB: the xors below stay inside a row
-        auto value = [&](int s) -> v4u {                        // positions 16 (s / 16) .. of features 32 (s % 16) ..
-            const uint32_t at = (vbase ^ ((s & 3) << 6)) + (s >> 4) * 16384 + ((s & 15) >> 2) * 256;
-            const v2u lo = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf)(uintptr_t)at));
-            const v2u hi = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf)(uintptr_t)((at ^ 32) + 8192)));
-            return v4u{ lo[0], lo[1], hi[0], hi[1] };
-        };
-#pragma unroll
-        for (int s = 0; s < kAhead; ++s) ring[s] = value(s);    // on their way during the exponentials
-        __builtin_amdgcn_sched_barrier(0);
         float sum = 0.f;
         v4u P[2];
+        auto weights = [&](int u, int q) {              // two positions' exponentials
+            const int e = 8 * u + 2 * q;
+            const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e], scale2, -off));
+            const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e + 1], scale2, -off));
+            sum += x + y;
+            P[u][q] = pack_bf16(x, y);
+        };
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int q = 0; q < 4; ++q) weights(0, q);
+        __builtin_amdgcn_sched_barrier(0);
+        unrolled<32>([&](auto step) {
+            constexpr int s = decltype(step)::value;
+            O[s & 15] = mfma32(ring[s % kAhead], P[s >> 4], O[s & 15]);
+            if constexpr (s + kAhead < 32) ring[s % kAhead] = value(s + kAhead);
+            if constexpr (s < 12 && s % 3 == 2) weights(1, s / 3);      // the second half's, beside the first half's products
+            pv_copy(step);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (G < 4 && s == kSync) {                        // this tile's last operands are in registers: its stage is free behind the barrier
+                arrived();
+                first[0] = key(next, 0);
+                first[1] = key(next, 1);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int e = 8 * u + 2 * q;
-                const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e], scale2, -off));
-                const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(S[e + 1], scale2, -off));
-                sum += x + y;
-                P[u][q] = pack_bf16(x, y);
+                for (int f = 2; f <= kSync - 24; ++f) ring[f] = key(next, f);
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if constexpr (G < 4 && s > kSync) {
+                ring[s % kAhead] = key(next, s - 24);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        });
         l += sum;
 #pragma unroll
-        for (int s = 0; s < 32; ++s) {
-            O[s & 15] = mfma32(ring[s % kAhead], P[s >> 4], O[s & 15]);
-            if (s + kAhead < 32) ring[s % kAhead] = value(s + kAhead);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int d = 0; d < 16; ++d) asm volatile("" : "+a"(O[d]));     // (the sums stay where they are)
+    };
+    auto no_copy = [](auto) {};
+
+    if constexpr (G < 4) {
+        if (t0 + (R - 1) * G > t1) __builtin_amdgcn_s_waitcnt(0x0f70);  // (fewer copies than are counted)
+        arrived();
+        first_keys(lds + par * kStage);
+        int st = 0;
+        for (int t = t0; t < t1; t += G) {
+            const int st_next = (st + 1) % R, st_free = (st + R - 1) % R;
+            // A copy beside every fourth (second) MFMA into the stage of the step before, which is free: the four wavefronts take turns on
+            // the compute unit's load path while the matrix cores are busy; nine in a row keep each of them for a thousand cycles.
+            Source ahead[G];
+#pragma unroll
+            for (int j = 0; j < G; ++j) ahead[j] = source(t + (R - 1) * G + j, st_free * G + j);
+            tile(t + par, lds + (st * G + par) * kStage, lds + (st_next * G + par) * kStage, [&](auto step) {
+                constexpr int s = decltype(step)::value, E = 4 / G;
+                if constexpr (s % E == E - 1) issue(ahead[s / E / 9], std::integral_constant<int, s / E % 9>());
+            }, no_copy);
+            st = st_next;
         }
-        st = (st + 1) % kStages;
+    } else {
+        for (int t = t0 + par; t < t1; t += G) {
+            int at = par * kStage;                      // one stage a wavefront, nobody else's
+            asm volatile("" : "+s"(at));                // (its addresses are formed in the loop: there are no registers to keep them in)
+            const uint8_t* own = lds + at;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            first_keys(own);
+            // the next tile comes where this one's rows have been read: the rotary rows behind the scores, the first 16 positions' beside the
+            // second half's products
+            const Source ahead = source(t + G, par);
+            tile(t, own, own, no_copy, [&](auto step) {
+                constexpr int s = decltype(step)::value;
+                if constexpr (s >= 1 && s <= 4) issue(ahead, std::integral_constant<int, 31 + s>());
+                if constexpr (s >= 16) issue(ahead, std::integral_constant<int, s - 16>());
+            });
+            unrolled<16>([&](auto k) { issue(ahead, std::integral_constant<int, decltype(k)::value + 16>()); });
+        }
     }
 
-    l += xor32(l);
+    const v2f parts = halves32(l);
+    l = parts.x + parts.y;
     const int64_t bb = (int64_t)b * p.blocks + blk;
-    if (g == 0) p.ml[(bb * kRows + wave * 32 + i) * p.splits + split] = v2f{ m, l };
+    __builtin_amdgcn_s_waitcnt(0x0f70);                 // (copies of the tiles past the range still write zeros)
+    barrier_no_fence();
     // The sums leave as rows, which fold reads whole: 64 features of 32 rows at a time through LDS (16-byte chunks xor-ed with
-    // the row), so that a store writes four pieces of 256 bytes; straight from the registers it would be 32 of 32.
-    barrier_no_fence();                                 // everybody has read the last tile
-    uint8_t* stg = lds + wave * 16384;                  // two buffers: the next 64 features are written while these are read
-    float* dst = p.part + (bb * p.splits + split) * kPartFloats + (wave * 32 + (lane >> 4)) * kC + (lane & 15) * 4;
-    auto put = [&](int d2) {
+    // the row), so that a store writes four pieces of 256 bytes; straight from the registers it would be 32 of 32.  The G wavefronts of
+    // a row group first add theirs, each for 32 / G of the rows.
+    v2f* const table = (v2f*)(lds + 65536);             // (maximum, sum) [wavefront][row]
+    constexpr int N = 8 / G;
+    float wt[N][G];
+    if constexpr (G == 1) {
+        if (g == 0) p.ml[(bb * (RB * 32) + rg * 32 + i) * p.splits + split] = v2f{ m, l };
+    } else {
+        if (g == 0) table[wave * 32 + i] = v2f{ m, l };
+        barrier_no_fence();
+        auto weigh = [&](int r, float (&w)[G]) -> v2f { // row r's weights; its maximum and sum
+            v2f x[G];
+            float top = -__builtin_inff(), sum = 0.f;
+#pragma unroll
+            for (int j = 0; j < G; ++j) { x[j] = table[(rg + RB * j) * 32 + r]; top = fmaxf(top, x[j].x); }
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+                w[j] = x[j].x == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f((x[j].x - top) * scale2);
+                sum += x[j].y * w[j];
+            }
+            return v2f{ top, sum };
+        };
+#pragma unroll
+        for (int n = 0; n < N; ++n) weigh(4 * (par * N + n) + (lane >> 4), wt[n]);
+        if (par == 0) {
+            float w[G];
+            const v2f ml = weigh(i, w);
+            if (g == 0) p.ml[(bb * (RB * 32) + rg * 32 + i) * p.splits + split] = ml;
+        }
+    }
+    float* dst = p.part + ((bb * p.splits + split) * (RB * 32) + rg * 32 + par * (4 * N) + (lane >> 4)) * kC + (lane & 15) * 4;
+    auto put = [&](int d2) {                            // two buffers a wavefront: the next 64 features are written while these are read
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             const v16f& o = O[2 * d2 + (c >> 2)];
             const int e = 4 * (c & 3);
-            *(v4f*)(stg + (d2 & 1) * 8192 + i * 256 + (((2 * c + g) ^ (i & 15)) << 4)) = v4f{ o[e], o[e + 1], o[e + 2], o[e + 3] };
+            *(v4f*)(lds + wave * 16384 + (d2 & 1) * 8192 + i * 256 + (((2 * c + g) ^ (i & 15)) << 4)) = v4f{ o[e], o[e + 1], o[e + 2], o[e + 3] };
         }
     };
     put(0);
 #pragma unroll
     for (int d2 = 0; d2 < 8; ++d2) {
-        v4f x[8];
+        if constexpr (G > 1) barrier_no_fence();        // everybody's are there, and the buffers written next have been read
+        v4f x[N][G];
 #pragma unroll
-        for (int n = 0; n < 8; ++n) {
-            const int r = 4 * n + (lane >> 4);
-            x[n] = *(const v4f*)(stg + (d2 & 1) * 8192 + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
-        }
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+                const int r = 4 * (par * N + n) + (lane >> 4);
+                x[n][j] = *(const v4f*)(lds + (rg + RB * j) * 16384 + (d2 & 1) * 8192 + r * 256 + (((lane & 15) ^ (r & 15)) << 4));
+            }
         if (d2 < 7) put(d2 + 1);
 #pragma unroll
-        for (int n = 0; n < 8; ++n) *(v4f*)(dst + n * 4 * kC + d2 * 64) = x[n];
+        for (int n = 0; n < N; ++n) {
+            v4f v = x[n][0];
+            if constexpr (G > 1) {
+                v = v * wt[n][0];
+#pragma unroll
+                for (int j = 1; j < G; ++j) v += x[n][j] * wt[n][j];
+            }
+            *(v4f*)(dst + n * 4 * kC + d2 * 64) = v;
+        }
     }
 }
 
@@ -254,7 +404,7 @@ struct FoldArgs {
     const float* part; const v2f* ml;                   // as DecodeArgs
     const uint8_t* w; const float* ws;                  // wkv_b fp8 [heads * 256, 512] and its block scales
     void* y; float* ys;                                 // bf16 [tokens][heads][128], or e4m3 and scales [tokens][heads]
-    int tokens, per_seq, heads, blocks, splits, group;  // tokens of all sequences and of one; tokens at a time, up to 16
+    int tokens, per_seq, heads, rows, blocks, splits, group;    // tokens of all sequences and of one; rows of an attention workgroup and its blocks; tokens at a time, up to 16
     float scale;
 };
 
@@ -285,9 +435,9 @@ __global__ __launch_bounds__(512, 4) void mla_fold_kernel(FoldArgs p) {
         };
         for (int k = wave / per; k < n; k += 8 / per) {
             const int t = ms + k, b = t / p.per_seq, row = (t - b * p.per_seq) * p.heads + h;
-            const int64_t bb = (int64_t)b * p.blocks + row / kRows;
-            const v2f* ml = p.ml + (bb * kRows + row % kRows) * p.splits;
-            const float* src = p.part + bb * p.splits * kPartFloats + (row % kRows) * kC + lane * 4;
+            const int64_t bb = (int64_t)b * p.blocks + row / p.rows, part = (int64_t)p.rows * kC;
+            const v2f* ml = p.ml + (bb * p.rows + row % p.rows) * p.splits;
+            const float* src = p.part + bb * p.splits * part + (row % p.rows) * kC + lane * 4;
             // a chunk of 64 ranges, a lane each; up to six ranges' sums are requested before the first is added
             const v2f none = { -__builtin_inff(), 0.f };
             v2f x = lane < p.splits ? ml[lane] : none;
@@ -304,9 +454,9 @@ __global__ __launch_bounds__(512, 4) void mla_fold_kernel(FoldArgs p) {
                 auto add = [&](auto count, int s) {     // ranges s, s + per, ..
                     constexpr int U = decltype(count)::value;
                     v4f o[U][2];
-                    const float* at = src + (int64_t)(s0 + s) * kPartFloats;
+                    const float* at = src + (s0 + s) * part;
 #pragma unroll
-                    for (int u = 0; u < U; ++u, at += (int64_t)per * kPartFloats) { o[u][0] = *(const v4f*)at; o[u][1] = *(const v4f*)(at + kC / 2); }
+                    for (int u = 0; u < U; ++u, at += per * part) { o[u][0] = *(const v4f*)at; o[u][1] = *(const v4f*)(at + kC / 2); }
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
                         const float k2 = u32_as_f32((uint32_t)__builtin_amdgcn_readlane((int)f32_as_u32(wt), s + u * per));
@@ -528,16 +678,43 @@ __global__ __launch_bounds__(320) void mla_latent_kernel(LatentArgs p) {
 }
 
 // How the positions of a step are split: one attend workgroup per compute unit (its LDS and registers take a whole one; fewer
-// leave units idle, more write more partial sums), a tile each at least.
+// leave units idle, more write more partial sums), a tile a wavefront each at least; and how many tiles a workgroup takes side by side: what
+// costs least by the measured costs (us) of a wavefront's tiles one after another (2.3; 2.65 and 3.4 where two and four at a time leave less or no room for
+// the next ones), of the partial sums (8 to 12 us for those of 256 workgroups of 128 rows) and of adding the wavefronts' sums.  Over 105 shapes (1 .. 128
+// sequences at 40 .. 4096 positions, 1 .. 31 tokens each) the rule is 1.4 % from the best of the three on average, 1.14 x faster than G = 1 everywhere.
+// A wavefront has the tiles that one of G = 1 has: longer ranges would round more exponentials (a range's largest is exactly one).
 void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) {
-    a.batch = (int)batch; a.rows = (int)rows; a.positions = (int)positions;
+    a.rows = (int)rows; a.positions = (int)positions;
     a.tiles = (int)((positions + kTile - 1) / kTile);
-    a.blocks = (int)((rows + kRows - 1) / kRows);
-    const int64_t base = batch * a.blocks;
-    int64_t splits = 256 / base;
-    splits = splits < 1 ? 1 : splits > a.tiles ? a.tiles : splits;
-    a.per = (int)((a.tiles + splits - 1) / splits);
-    a.splits = (a.tiles + a.per - 1) / a.per;
+    a.groups = (int)((rows + 127) / 128 * 4);
+    double best = 0;
+    for (int side = 1; side <= 4; side *= 2) {
+        const int64_t blocks = (rows + 128 / side - 1) / (128 / side), base = batch * blocks, steps = (a.tiles + side - 1) / side;
+        int64_t splits = 256 / base;
+        splits = splits < 1 ? 1 : splits > steps ? steps : splits;
+        const int64_t n = (steps + splits - 1) / splits;
+        splits = (steps + n - 1) / n;
+        const int64_t units = base * splits, rounds = (units + 255) / 256;
+        const double us = rounds * (2.3 + (n - 1) * (side == 1 ? 2.3 : side == 2 ? 2.65 : 3.4)) + (rounds - 1) * 3 + units * (128 / side) * 0.00049 +
+                          (side == 1 ? 0 : side == 2 ? 0.5 : 1.0);
+        if (side > 1 && us >= best) continue;
+        best = us;
+        a.side = side; a.blocks = (int)blocks; a.per = (int)(n * side); a.splits = (int)splits;
+    }
+}
+size_t decode_bytes(const DecodeArgs& a, int64_t batch) {
+    const int64_t units = batch * a.blocks * a.splits, rows = 128 / a.side;
+    return (size_t)(batch * a.groups * (32 * kC * 2) + units * rows * (kC * 4 + 8));
+}
+
+template <int G> int launch_attend(const DecodeArgs& a, int which, unsigned grid, hipStream_t st) {
+    static void (*const kernels[6])(DecodeArgs) = { mla_decode_kernel<kNoMask, false, G>, mla_decode_kernel<kNoMask, true, G>,
+                                                    mla_decode_kernel<kMaskBf16, false, G>, mla_decode_kernel<kMaskBf16, true, G>,
+                                                    mla_decode_kernel<kMaskF32, false, G>, mla_decode_kernel<kMaskF32, true, G> };
+    static LdsGrant grant[6];
+    if (!grant[which].ensure((const void*)kernels[which], kStages * kStage)) return DSV3_ERR_LAUNCH;
+    hipLaunchKernelGGL(kernels[which], dim3(grid), dim3(256), kStages * kStage, st, a);
+    return DSV3_OK;
 }
 
 }  // namespace
@@ -545,21 +722,22 @@ void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) 
 size_t mla_decode_workspace_bytes(int64_t batch, int64_t tokens, int64_t positions, int heads) {
     DecodeArgs a;
     decode_plan(a, batch, tokens * heads, positions);
-    const int64_t units = batch * a.blocks * a.splits;
-    return (size_t)(batch * a.blocks * (kRows * kC * 2) + units * (kPartFloats * 4 + kRows * 8));
+    return decode_bytes(a, batch);
 }
 
 int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
                       const void* w, const float* ws, const void* mask, bool mask_f32, void* y, float* ys, int64_t batch,
                       int64_t tokens, int64_t positions, int heads, float scale, void* workspace, hipStream_t st) {
     DecodeArgs a;
-    if (tokens * heads > 0x7fffffff / kRows || batch * tokens > 0x7fffffff - 16) return DSV3_ERR_BAD_SHAPE;
+    if (tokens * heads > 0x7fffffff / 128 || batch * tokens > 0x7fffffff - 16) return DSV3_ERR_BAD_SHAPE;
     decode_plan(a, batch, tokens * heads, positions);
-    if (a.blocks > 65535) return DSV3_ERR_BAD_SHAPE;
+    const int64_t rows = 128 / a.side, units = batch * a.blocks * a.splits;
+    if (a.groups / 4 > 65535 || batch > 65535 || units > 0x7fffffff) return DSV3_ERR_BAD_SHAPE;
+    a.blocks_magic = magic_of(units, a.blocks);
+    a.splits_magic = magic_of(units, a.splits);
     uint8_t* wsp = (uint8_t*)workspace;
-    const int64_t units = batch * a.blocks * a.splits;
-    a.part = (float*)(wsp + batch * a.blocks * (kRows * kC * 2));
-    a.ml = (v2f*)(a.part + units * kPartFloats);
+    a.part = (float*)(wsp + batch * a.groups * (32 * kC * 2));
+    a.ml = (v2f*)(a.part + units * rows * kC);
     a.ql = wsp; a.q = (const uint16_t*)q; a.freqs = (const v2f*)freqs;
     a.kv = (const uint16_t*)kv; a.kv_bs = kv_bs; a.pe = (const uint16_t*)pe; a.pe_bs = pe_bs;
     a.mask = mask; a.heads = heads;
@@ -569,19 +747,16 @@ int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t 
     // 22.2), the fold's scattered stores cost it 0.4.  With more they cost 1 to 1.7 us (32 tokens 5.1 -> 6.1, 64 6.2 -> 7.8), the gain
     // disappears behind the tiles (32 at 4096: 56.7 -> 56.4, 64 at 1000: 39.7 -> 39.6).
     const bool pack = batch * tokens <= 16;
-    const int rc = pack ? launch_wkv_b_absorb_q_packed(q, (int64_t)heads * kQd, kQd, w, ws, wsp, batch, tokens, a.blocks, heads, kNope, kNope, st)
+    const int rc = pack ? launch_wkv_b_absorb_q_packed(q, (int64_t)heads * kQd, kQd, w, ws, wsp, batch, tokens, a.groups / 4, heads, kNope, kNope, st)
                         : launch_wkv_b_absorb(q, (int64_t)heads * kQd, kQd, w, ws, wsp, DSV3_ABSORB_Q, batch * tokens, heads, kNope, kNope, kC, st);
     if (rc != DSV3_OK) return rc;
     const int which = (!mask ? kNoMask : mask_f32 ? kMaskF32 : kMaskBf16) * 2 + pack;
-    static void (*const kernels[6])(DecodeArgs) = { mla_decode_kernel<kNoMask, false>, mla_decode_kernel<kNoMask, true>,
-                                                    mla_decode_kernel<kMaskBf16, false>, mla_decode_kernel<kMaskBf16, true>,
-                                                    mla_decode_kernel<kMaskF32, false>, mla_decode_kernel<kMaskF32, true> };
-    static LdsGrant grant[6];
-    if (!grant[which].ensure((const void*)kernels[which], kStages * kStage)) return DSV3_ERR_LAUNCH;
-    hipLaunchKernelGGL(kernels[which], dim3(a.splits, (unsigned)batch, a.blocks), dim3(256), kStages * kStage, st, a);
+    const int launched = a.side == 1 ? launch_attend<1>(a, which, (unsigned)units, st) : a.side == 2 ? launch_attend<2>(a, which, (unsigned)units, st)
+                                                                                                     : launch_attend<4>(a, which, (unsigned)units, st);
+    if (launched != DSV3_OK) return launched;
     FoldArgs f;
     f.part = a.part; f.ml = a.ml; f.w = (const uint8_t*)w; f.ws = ws; f.y = y; f.ys = ys;
-    f.tokens = (int)(batch * tokens); f.per_seq = (int)tokens; f.heads = heads; f.blocks = a.blocks; f.splits = a.splits;
+    f.tokens = (int)(batch * tokens); f.per_seq = (int)tokens; f.heads = heads; f.rows = (int)rows; f.blocks = a.blocks; f.splits = a.splits;
     f.scale = a.scale;
     // A head and four, eight or 16 tokens a workgroup, as few as leave a workgroup a compute unit (8 sequences at
     // 2000 positions: 19.5 us with eight tokens in 128 workgroups, 17.0 with four in 256, 18.3 with two in 512; 32 at 4096: 16.5 with

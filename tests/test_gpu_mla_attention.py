@@ -134,6 +134,19 @@ def test_decode_attention(b, s, t, h, kind, grow):
     assert ((got - ref).norm(dim=-1) <= 2.0 ** -7 * ref.norm(dim=-1)).all()
 
 
+# Tiles side by side in a workgroup (the cost rule of csrc/mla_decode.hip): four, two and one, with a wavefront's second and later tiles, ranges
+# whose last step has fewer tiles than wavefronts, tiles past the end and the range, row blocks with missing rows.
+SIDES = [(8, 1, 2030, 128, None), (1, 9, 900, 30, "causal_f32"), (2, 9, 200, 128, "causal"), (3, 13, 200, 24, "holes"),         # four
+         (12, 2, 900, 128, "holes"), (30, 3, 300, 128, "causal"), (64, 1, 1005, 100, None), (5, 11, 2050, 50, "lowest_f32"),    # two
+         (64, 1, 3650, 100, None), (2, 66, 130, 128, "causal_f32"), (1, 6, 90, 5, "lowest")]                                    # one
+
+
+@pytest.mark.parametrize("grow", [False, True])
+@pytest.mark.parametrize("b,s,t,h,kind", SIDES)
+def test_decode_attention_tiles_side_by_side(b, s, t, h, kind, grow):
+    test_decode_attention(b, s, t, h, kind, grow)
+
+
 # A workgroup of the fold takes a head and 4, 8 or 16 tokens at a time: 16 heads and fewer 4 here, 128 heads 4 up to 8 tokens in all, 8 up to 16,
 # then 16, and past 128 tokens (1024 / heads groups) several groups, one after another.  One token of a group is shared by eight
 # wavefronts, two by four each, three or four by two each, more have one each.  Splits below, at and above a wavefront's 64 lanes (256
