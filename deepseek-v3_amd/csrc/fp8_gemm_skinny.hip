@@ -76,11 +76,12 @@ template <int N> struct WaitFor;
 DSV3_WAITFOR(0) DSV3_WAITFOR(2) DSV3_WAITFOR(4) DSV3_WAITFOR(6) DSV3_WAITFOR(8) DSV3_WAITFOR(10) DSV3_WAITFOR(12) DSV3_WAITFOR(14)
 #undef DSV3_WAITFOR
 
+// HALF: strips of eight rows (see make_plan); the fragments' other eight rows repeat them and are not stored.
 // RING (S == 1, every wavefront's K range a multiple of NPF blocks and at least two of them, n k < 2^32): a ring slot
 // is refilled as soon as its block has been multiplied, so a wavefront keeps NPF blocks of loads in flight until its
 // last NPF blocks.  Without it the range is worked through in batches -- issue NPF, use NPF, issue the next NPF --,
 // a wavefront has nothing in flight while it uses a batch, and all wavefronts of the chip reach that point together.
-template <int MT, int S, int NPF, bool QF, bool RING = false>
+template <int MT, int S, int NPF, bool QF, bool RING = false, bool HALF = false>
 __global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 4))) void fp8_gemm_skinny_kernel(
         const uint8_t* __restrict__ a, const float* __restrict__ a_s,
         const uint8_t* __restrict__ b, const float* __restrict__ b_s,
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_
     const int kb0 = wg_kb0 + wave * per_wave;                 // first K block of the wavefront (global index)
     const int nkb = max(0, min(per_wave, wg_kb0 + wg_nkb - kb0));
 
-    const int n0 = blockIdx.x * (16 * S);
+    const int n0 = blockIdx.x * (HALF ? 8 : 16 * S);
     // Weight loads: an instruction fetches 8 rows x 128 contiguous bytes (lanes with fr < 8 take the first 64
     // bytes of row fr&7, lanes with fr >= 8 the last 64 bytes of the same row); a second one does rows 8..15.
     // The halves that landed in the wrong lane are exchanged between lanes fr and fr^8 with DPP row rotates
@@ -164,10 +165,11 @@ __global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             wlo[p][s] = __builtin_nontemporal_load((const v4i*)(wsrc[s] + k * 128));               // rows 0..7
-            whi[p][s] = __builtin_nontemporal_load((const v4i*)(wsrc[s] + wrow8[s] + k * 128));    // rows 8..15
+            whi[p][s] = HALF ? wlo[p][s] : __builtin_nontemporal_load((const v4i*)(wsrc[s] + wrow8[s] + k * 128));    // rows 8..15
         }
     };
     // RING: lane offsets of its two rows from b (< 2^32) and the wavefront-uniform address of its first K block
+    static_assert(!HALF || (S == 1 && !RING), "eight rows: one strip, in batches");
     static_assert(!RING || (S == 1 && NPF == 8), "the ring variant is written for one strip and eight slots");
     const uint32_t ring_lo = (uint32_t)min(n0 + (fr & 7), N - 1) * (uint32_t)K + (fr >> 3) * 64 + fq * 16;
     const uint32_t ring_hi = (uint32_t)min(n0 + (fr & 7) + 8, N - 1) * (uint32_t)K + (fr >> 3) * 64 + fq * 16;
@@ -185,6 +187,8 @@ __global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_
         // the 8 lanes that hold the chunks of one (row, K block) are consecutive and aligned: amax by DPP
 #pragma unroll
         for (int i = 0; i < kSlabChunks; ++i) {
+            // (uniform) Wavefronts without a chunk go on: 16 of them, four turns each, took 0.6 us more of 7.5 (one row of 7168).
+            if (wave * 64 + i * (int)blockDim.x >= chunks) break;
             // (the 16 values are widened twice, for the maximum and for the quotients, instead of being kept: with the
             // weight ring live this section must stay inside the register budget)
             auto widen = [&](int e) { return (e & 1) ? bf16hi_to_f32(raw[i][e >> 3][(e >> 1) & 3]) : bf16lo_to_f32(raw[i][e >> 3][(e >> 1) & 3]); };
@@ -322,7 +326,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_
         const int s = t / MT, j = t % MT;
         const int m = j * 16 + (l & 15);
         const int n = n0 + s * 16 + (l >> 4) * 4;
-        if (m >= M) continue;
+        if (m >= M || (HALF && l >= 32)) continue;
         const size_t idx = slab + (size_t)m * N + n;
         if (n + 3 < N && (N & 3) == 0) {                      // four results in one store
             if (out_dtype == DSV3_F32) *(v4f*)((float*)out + idx) = v;
@@ -340,7 +344,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_
     }
 }
 
-struct Plan { int mt, s, waves, splits, kb_per_wg; };
+struct Plan { int mt, s, waves, splits, kb_per_wg; bool half; };
 
 // The kernels here run for 5-30 us, so the grid is sized to be resident in ONE round: the workgroups of a
 // second, partly filled round would leave most of the chip idle for half the run.  Within that limit: as many
@@ -381,6 +385,11 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
         if (!have || fits) { best = p; have = true; }
         if (fits) break;
     }
+    // Strips of eight rows where all of them still are one round of as many wavefronts: a load's consecutive lanes lie in different rows, which
+    // takes a compute unit's load path 64 cycles a KiB, so that 16 rows of 7168 -> 576 are 3 us of 36 units' time with the others idle.  With the
+    // quantisation, us, 16 rows / 8: 7168 -> 576 7.0 / 5.6, 1536 7.2 / 6.0, 1536 -> 1536 4.2 / 4.0, 16384 -> 2048 14.3 / 14.2.  Not with
+    // fewer wavefronts a workgroup: 7168 -> 2112 7.3 / 8.0, 4096 8.2 / 8.7.
+    best.half = m <= 2 && best.s == 1 && best.splits == 1 && (n + 7) / 8 * best.waves <= capacity;
     return best;
 }
 
@@ -394,6 +403,11 @@ void launch_cfg(const Plan& p, const void* a, const float* a_s, const void* b, c
     const size_t lds = red_bytes > slab_bytes ? red_bytes : slab_bytes;
     const uint64_t m_magic = (uint64_t)(((1ull << 32) + (uint64_t)m - 1) / (uint64_t)m);
     if constexpr (S == 1) {
+        if (p.half) {
+            hipLaunchKernelGGL((fp8_gemm_skinny_kernel<MT, S, NPF, QF, false, true>), dim3((unsigned)((n + 7) / 8)), dim3(p.waves * kWave), lds, st,
+                               (const uint8_t*)a, a_s, (const uint8_t*)b, b_s, out, out_dtype, m, n, k, p.kb_per_wg, ue8m0, m_magic);
+            return;
+        }
         // every wavefront's K range: the same whole number (>= 2) of ring rounds
         const int kb = k / 128, per_wave = p.kb_per_wg / p.waves;
         static const bool no_ring = getenv("DSV3_SKINNY_NORING") != nullptr;

@@ -212,6 +212,23 @@ def test_ragged_n_equals_prefix_of_padded(K):
     assert torch.equal(full[:, :576], part)
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 127, 129, 576, 2041, 2048])
+@pytest.mark.parametrize("m,k", [(1, 128), (2, 384), (1, 1536), (2, 7168), (1, 7168)])
+def test_strips_of_eight_rows_equal_strips_of_sixteen(K, m, n, k):
+    """One and two rows up to 2048 columns take eight weight rows a workgroup, above that 16 (up to 4096 with as many wavefronts, so that the
+    sums run in one order): the same bits as the first columns of a wider weight, quantised inside the kernel, and near the oracle."""
+    from dsv3fp8 import workloads, ops, _lib
+    x = workloads.activations(m, k, seed=n, outliers=True)
+    w8, ws = workloads.weight(4096, k, seed=k % 89)
+    assert ops.linear_fp8_fused(m, n, k) and ops.linear_fp8_fused(m, 4096, k)
+    wide = torch.ops.dsv3fp8.linear_fp8(x.cuda(), w8.cuda(), ws.cuda(), _lib.SCALE_FMT_NONE, _lib.F32)
+    w8, ws = w8[:n].contiguous(), ws[: (n + 127) // 128].contiguous()
+    got = torch.ops.dsv3fp8.linear_fp8(x.cuda(), w8.cuda(), ws.cuda(), _lib.SCALE_FMT_NONE, _lib.F32)
+    assert torch.equal(got, wide[:, :n])
+    ref = oracle.fp8_gemm_f32(*oracle.act_quant(x), w8, ws)
+    assert (got.cpu() - ref).abs().max().item() <= TOL * wide.pow(2).mean().sqrt().item()
+
+
 def test_leading_dims(K):
     from dsv3fp8 import workloads
     x = workloads.activations(6, 256, seed=1).view(2, 3, 256)
