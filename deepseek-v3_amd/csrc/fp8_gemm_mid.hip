@@ -9,8 +9,8 @@
 // chosen so that one round fills the chip, mostly without slices.
 //
 // K blocks of A and B are copied global -> LDS (1 KiB a copy: 8 rows x 128 bytes, chunks xor-ed with the row), S blocks in a ring.  One
-// barrier per block, two sub-tiles before its end: the operands that the block still needs are in registers then, its stage is refilled,
-// a copy beside each MFMA, and the next block's first operands are read while its last MFMAs run.  Each MFMA is followed by the
+// barrier per block, two sub-tiles before its end: the operands that the block still needs are in registers then, its stage is refilled up to the
+// next barrier, and the next block's first operands are read while its last MFMAs run.  Each MFMA is followed by the
 // FMAs of the one before the last.  Loads and copies are the compiler's own, whose counting sees all of them; it keeps to the
 // counted wait in front of the barrier.
 // Scales: a row's a_s are K / 128 values apart, so that a copy of 64 rows' scales of one K block is 64 lines, which takes a compute unit's
@@ -20,6 +20,10 @@
 // Measured against the large-M kernel (us, weights from HBM): 7168 -> 36864 at 65 / 128 / 160 / 224 rows 68.5 / 79.3 / 86.0 / 97.1 -> 57.8 / 64.6 /
 // 71.1 / 82.7 (a 128-row tile takes 1.07 us per K block, 4.4 TB/s of weights; each row adds: its copies and the weights' share the load
 // path); 1536 -> 24576 at 65 / 128 rows 17.2 / 17.6 -> 13.6 / 15.5; the narrow ones at the rule below.
+// A wavefront whose last sub-tile lies past the rows leaves it out, and every other column group deals from the other end, so that a SIMD's two
+// wavefronts share the rest evenly; copies spread over the whole block.  With the quantisation in front, without / with both: 130 rows 75.5 / 69.5, 160 76.6 /
+// 74.3, 193 89.0 / 82.1, 224 92.5 / 85.8.  What bounds it then: at 128 rows the copies (L2 to LDS 8 TB/s of weights and activations, the arithmetic costs 1 us of
+// 67), at 224 both sides cost 1.2 .. 1.3 us a block of 1.4 by themselves (1.3 without LDS reads, 1.2 without copies).
 // Not used elsewhere: with both dimensions in whole rounds of 256 x 256 tiles the two-phase kernel is up to 25 % faster.
 #include <cstdlib>
 #include <type_traits>
@@ -63,7 +67,8 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
     constexpr bool ONE = 8 % SN == 0;           // a wavefront's columns lie in one 128-column block of weight scales
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int fr = lane & 15, fq = lane >> 4, wm = wave % WM, wn = wave / WM;
+    // (every other column group deals its sub-tiles from the other end: where some wavefronts have one more, they are not on one SIMD)
+    const int fr = lane & 15, fq = lane >> 4, wn = wave / WM, wm = wn & 1 ? WM - 1 - wave % WM : wave % WM;
 
     // a contiguous run of tiles per XCD, the row tiles of a column tile next to each other
     int pid = blockIdx.x;
@@ -108,20 +113,9 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
                                                      16, real ? s_off : s_one, real ? (kb0 + grp * 4) * 4 : 0, 0, 0);
         }
     };
-#pragma unroll
-    for (int p = 0; p < S; ++p)
-#pragma unroll
-        for (int t = 0; t < G::PER; ++t) copy(t, p, p);
-
-    v4f acc[JM][SN];
-#pragma unroll
-    for (int j = 0; j < JM; ++j)
-#pragma unroll
-        for (int s = 0; s < SN; ++s) acc[j][s] = (v4f){0.f, 0.f, 0.f, 0.f};
-
     const int fx = swz(fr);
     const int c0 = fr * 128 + (((2 * fq) ^ fx) * 16), c1 = fr * 128 + (((2 * fq + 1) ^ fx) * 16);
-    // sub-tile j of the wavefront: rows 16 (j WM + wm); past the tile's last one it is repeated and its results dropped
+    // sub-tile j of the wavefront: rows 16 (j WM + wm); one past the tile's last one is repeated and its results dropped
     auto a_sub = [&](int j) { return (j + 1) * WM <= MT ? j * WM + wm : min(j * WM + wm, MT - 1); };
     auto frag_a = [&](int j, int st) {
         const uint8_t* p = lds + st * G::A_STAGE + a_sub(j) * 2048;
@@ -138,9 +132,33 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
     for (int s = 0; s < NB; ++s) bs_at[s] = G::LDS_SC + G::SCW * 1024 + (min(n0 + (wn * SN + s) * 16, N - 1) / 128 - nb0) * 16;
     auto scale_b = [&](int s, int kb) { return *(const float*)(lds + bs_at[s] + ((kb >> 2) & 1) * G::SC_BUF + (kb & 3) * 4); };
 
+    // JA: the wavefront's sub-tiles, JM or, where the rows end, JM - 1
+    auto run = [&](auto ja_tag) {
+    constexpr int JA = decltype(ja_tag)::value, Q = JA * SN, SYNC = JA - 2;
+    // The copies into a freed stage are spread over the MFMAs from one barrier to the next, copy t beside MFMA t Q / PER behind the barrier: a
+    // compute unit's load path takes 20 cycles a copy and the wavefront that issues one waits for it.  So the last copies of block S - 1
+    // are requested in front of the first barrier.
+    auto slot_of = [](int t) { return t * Q / G::PER; };
+    constexpr int LATE = [] {
+        int n = 0;
+        for (int t = 0; t < G::PER; ++t) n += t * Q / G::PER < Q - SYNC * SN;
+        return n;
+    }();
+#pragma unroll
+    for (int p = 0; p < S; ++p)
+#pragma unroll
+        for (int t = 0; t < G::PER; ++t)
+            if (p < S - 1 || t < LATE) copy(t, p, p);
+
+    v4f acc[JA][SN];
+#pragma unroll
+    for (int j = 0; j < JA; ++j)
+#pragma unroll
+        for (int s = 0; s < SN; ++s) acc[j][s] = (v4f){0.f, 0.f, 0.f, 0.f};
+
     v8i bf[SN], af[2];
-    float sa[JM], sa_next[JM], bs[NB], bs_next[NB];
-    constexpr int FIRST = (S - 1) * G::PER;
+    float sa[JA], sa_next[JA], bs[NB], bs_next[NB];
+    constexpr int FIRST = (S - 2) * G::PER + LATE;
     __builtin_amdgcn_s_waitcnt(0x0f70 | (FIRST & 15) | ((FIRST >> 4) << 14));       // vmcnt: block 0 has landed
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
@@ -149,19 +167,18 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
     for (int s = 0; s < SN; ++s) bf[s] = frag_b(s, 0);
     af[0] = frag_a(0, 0); af[1] = frag_a(1, 0);
 #pragma unroll
-    for (int j = 0; j < JM; ++j) sa_next[j] = scale_a(j, 0);
+    for (int j = 0; j < JA; ++j) sa_next[j] = scale_a(j, 0);
     v4f pend[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};         // raw products of the last two MFMAs
     float pend_sc[2] = {0.f, 0.f};
     int st = 0;
-    constexpr int Q = JM * SN, SYNC = JM - 2;
 
     for (int kb = 0; kb < KB; ++kb) {
-        const int st_next = st == S - 1 ? 0 : st + 1;
+        const int st_next = st == S - 1 ? 0 : st + 1, st_prev = st == 0 ? S - 1 : st - 1;
         float prev_sc[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) prev_sc[h] = pend_sc[h];
 #pragma unroll
-        for (int j = 0; j < JM; ++j) sa[j] = ONE ? sa_next[j] * bs_next[0] : sa_next[j];
+        for (int j = 0; j < JA; ++j) sa[j] = ONE ? sa_next[j] * bs_next[0] : sa_next[j];
 #pragma unroll
         for (int s = 0; s < NB; ++s) bs[s] = bs_next[s];
         auto factor = [&](int q) { return ONE ? sa[q / SN] : sa[q / SN] * bs[q % NB]; };
@@ -176,7 +193,7 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
                 for (int s2 = 0; s2 < NB; ++s2) bs_next[s2] = scale_b(s2, kb + 1);
 #pragma unroll
-                for (int j2 = 0; j2 < JM; ++j2) sa_next[j2] = scale_a(j2, kb + 1);
+                for (int j2 = 0; j2 < JA; ++j2) sa_next[j2] = scale_a(j2, kb + 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
             const v4f z = {0.f, 0.f, 0.f, 0.f};
@@ -187,25 +204,25 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[pq / SN][pq % SN][e] = __builtin_fmaf(pend[q & 1][e], f, acc[pq / SN][pq % SN][e]);
             pend[q & 1] = r;
-            if (j == JM - 1) bf[s] = frag_b(s, st_next);
-            if (s == SN - 1) af[j & 1] = j + 2 < JM ? frag_a(j + 2, st) : frag_a(j + 2 - JM, st_next);
+            if (j == JA - 1) bf[s] = frag_b(s, st_next);
+            if (s == SN - 1) af[j & 1] = j + 2 < JA ? frag_a(j + 2, st) : frag_a(j + 2 - JA, st_next);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
             __builtin_amdgcn_sched_barrier(0);
-            // refill of this block's stage, beside the MFMAs behind the barrier
-            constexpr int SLOTS = (JM - SYNC) * SN, EACH = (G::PER + SLOTS - 1) / SLOTS;
-            if (q >= SYNC * SN) {
+            // refill: behind the barrier of this block's stage, in front of it the rest of the stage of the block before
 #pragma unroll
-                for (int t = 0; t < EACH; ++t)
-                    if ((q - SYNC * SN) * EACH + t < G::PER) copy((q - SYNC * SN) * EACH + t, kb + S, st);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            for (int t = 0; t < G::PER; ++t)
+                if (slot_of(t) == (q + Q - SYNC * SN) % Q) {
+                    if (q >= SYNC * SN) copy(t, kb + S, st);
+                    else copy(t, kb - 1 + S, st_prev);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
         }
         // (Q odd: the two results in flight change places)
         if (Q & 1) { const v4f x = pend[0]; pend[0] = pend[1]; pend[1] = x; }
         pend_sc[0] = factor(Q - 2); pend_sc[1] = factor(Q - 1);
-        if (JM & 1) { const v8i x = af[0]; af[0] = af[1]; af[1] = x; }      // (and so do the two fragments read ahead)
+        if (JA & 1) { const v8i x = af[0]; af[0] = af[1]; af[1] = x; }      // (and so do the two fragments read ahead)
         st = st_next;
     }
 #pragma unroll
@@ -220,7 +237,7 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
     // lane holds c[m][n .. n + 3] for every (j, s)
     const size_t slab = (size_t)blockIdx.y * M * N;
 #pragma unroll
-    for (int j = 0; j < JM; ++j) {
+    for (int j = 0; j < JA; ++j) {
         const int r = (j * WM + wm) * 16 + fr;
         if (r >= rows_here) continue;
         const int m = m0 + r;
@@ -243,6 +260,11 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
             }
         }
     }
+    };
+    if constexpr (JM > 2) {
+        if (((JM - 1) * WM + wm) * 16 < rows_here) run(std::integral_constant<int, JM>());
+        else run(std::integral_constant<int, JM - 1>());
+    } else run(std::integral_constant<int, JM>());
 #endif
 }
 
