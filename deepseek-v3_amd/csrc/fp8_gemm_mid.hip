@@ -1,4 +1,4 @@
-// fp8_gemm for 65 rows and more where whole 256-column tiles leave compute units without work: up to 224 rows of wide weights, up to
+// fp8_gemm for 65 rows and more where whole 256-column tiles leave compute units without work: up to 256 rows of wide weights, up to
 // a few hundred of narrow ones, 8192 where these have 128 columns or fewer
 // (reference arithmetic: inference/kernel.py:118-172).
 //
@@ -308,6 +308,22 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
         p.mt = 8; p.wm = 4; p.sn = 4;
         return p;
     }
+    // 129 .. 256 rows of 32 to 128 tiles of 128 columns, in as many K slices as one round takes, where slices and columns fill it (240 of 256 units, 220 with
+    // slices of 24 blocks): the large-M kernel's tile has 128 or 256 rows and two stages, one of these as many rows as there are and three.  Up to
+    // 160 rows, and above on slices of 32 blocks and more (three or four, nearly equal) of a K range up to 18432: 16384 -> 7168 at 129 / 193 / 224 / 256 rows 1.15 / 1.04 / 1.08 / 1.10,
+    // 18432 -> 7168 1.05 / 1.02 / 1.04 / 1.04, 16384 -> 8192 1.06 .. 1.11, 7168 -> 16384 at 129 / 160 1.15 / 1.06 times the speed with the quantisation in front;
+    // over 125 drawn and listed sizes 0.98 .. 1.48, 1.05 on average (power-of-two scales 1.04).  Left out: 7168 -> 12288 (192 units) 0.92 .. 1.01 at 16384, 20480 -> 9216
+    // 0.91, 11264 -> 7168 at 193 rows 0.96 (slices of 24), 7168 -> 7168 at 159 0.96 (of 16).
+    if (m > 128 && m <= 256 && t128 >= 32 && t128 <= 128 && kb <= 144) {
+        const int64_t sl = 256 / t128, nkb = ((kb + sl - 1) / sl + 3) / 4 * 4, splits = (kb + nkb - 1) / nkb, units = t128 * splits;
+        if (nkb >= 8 && (units >= 240 || (units >= 220 && nkb >= 24)) && (m <= 160 || (nkb >= 32 && splits >= 3 && nkb * splits - kb <= 8))) {
+            p.nkb = (int)nkb;
+            p.splits = (int)splits;
+            p.wm = 4; p.sn = 4;
+            p.mt = rows <= 10 ? 10 : rows <= 12 ? 12 : rows <= 14 ? 14 : 16;
+            return p;
+        }
+    }
     // Narrow weights on a long K range: tiles of 64 x 128 as far as they are one round, in as many K slices as that leaves room for (up to
     // seven), while a slice is at most 20 blocks: a tile here takes 0.6 times the time per block that one of the large-M kernel's with four
     // times the columns does, which pays only as long as the round is short.  Behind the quantisation (us, large-M kernel / here), slices of
@@ -370,6 +386,10 @@ int launch_mid(const void* a, const float* a_s, const void* b, const float* b_s,
         case 125: return launch_cfg<12, 4, 5, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         case 145: return launch_cfg<14, 4, 5, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         case 84:  return launch_cfg<8, 4, 4, 4>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
+        case 104: return launch_cfg<10, 4, 4, 4>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
+        case 124: return launch_cfg<12, 4, 4, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
+        case 144: return launch_cfg<14, 4, 4, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
+        case 164: return launch_cfg<16, 4, 4, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         case 42:  return launch_cfg<4, 2, 2, 4>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         default: return DSV3_ERR_BAD_SHAPE;
     }

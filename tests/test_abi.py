@@ -451,6 +451,16 @@ def test_sizes_that_the_tiles_of_one_round_take(L, m, n, k, taken):
     assert supported(m, n, k) == taken
 
 
+# the window of 129 .. 256 rows: rows, tiles of 128 columns, units that slices and columns fill, blocks a slice, K
+@pytest.mark.parametrize("m,n,k,taken", [
+    (129, 7168, 16384, True), (256, 7168, 18432, True), (257, 7168, 16384, False), (128, 7168, 16384, False), (161, 7168, 18944, False),
+    (160, 4096, 11264, True), (161, 4096, 11264, False), (129, 3968, 16384, False), (160, 16384, 2048, True), (161, 16384, 16384, False), (129, 16512, 2048, False),
+    (150, 12288, 16384, False), (150, 7168, 7168, False), (150, 7168, 11264, True), (193, 7168, 11264, False), (205, 7168, 14848, False), (205, 7168, 15360, True),
+    (200, 9216, 16384, False), (200, 10240, 16384, True), (150, 8192, 4096, True), (150, 8192, 4224, False)])
+def test_sizes_that_the_sliced_tiles_take(L, m, n, k, taken):
+    test_sizes_that_the_tiles_of_one_round_take(L, m, n, k, taken)
+
+
 @pytest.mark.parametrize("knob", ["DSV3_PREFILL_NOSPLIT=1", "DSV3_PREFILL_TILE=128", "DSV3_PREFILL_NOPP=1", "DSV3_PREFILL_NOPP128=1", "OTHER=1"])
 def test_knobs_of_the_large_m_kernel_keep_products_there(knob):
     """A knob that says how the large-M kernel runs its dense tiles holds for every size it had when the knob was made; without K slices no

@@ -166,6 +166,36 @@ def test_tiles_that_fill_one_round(K, m, n, k):
                 torch.set_default_dtype(old)
 
 
+@pytest.mark.parametrize("m,n,k", [(129, 4096, 11264), (145, 4090, 8192), (160, 16383, 2048), (161, 7168, 16384), (177, 7041, 16384), (193, 8100, 15360),
+                                   (224, 7168, 18432), (225, 7168, 16384), (256, 10180, 16384)])
+def test_sliced_tiles_of_as_many_rows_as_there_are(K, m, n, k):
+    """129 .. 256 rows in one row tile and K slices: every height and number of live sub-tiles, uneven last slices, ragged columns; sampled columns
+    against binary64 and against the large-M kernel, which takes scales that are not 16-byte aligned.  Both form the same products of 128 terms
+    in the matrix core; a scale product, its product and k / 128 additions round by at most 2^-24 of the terms' sizes each, on either side."""
+    from dsv3fp8 import _lib
+    kb = k // 128
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    a = (torch.randn(m, k, generator=g, device="cuda") * 40).to(torch.float8_e4m3fn)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 40).to(torch.float8_e4m3fn)
+    a_s = torch.rand(m, kb, generator=g, device="cuda") + 0.5
+    w_s = torch.rand((n + 127) // 128, kb, generator=g, device="cuda") + 0.5
+    cols = torch.cat([torch.randint(0, n, (200,), generator=g, device="cuda"), torch.tensor([0, 127, 128, n - 1, n - 128], device="cuda")])
+    ref = torch.zeros(m, cols.numel(), dtype=torch.float64, device="cuda")
+    size = torch.zeros_like(ref)
+    for b in range(kb):
+        x, y = a[:, b * 128:(b + 1) * 128].double(), w[:, b * 128:(b + 1) * 128][cols].double()
+        s = a_s[:, b:b + 1].double() * w_s[cols // 128, b].double()
+        ref += x @ y.t().contiguous() * s
+        size += x.abs() @ y.abs().t().contiguous() * s
+    c32, c16 = _gemm_both(K, a, a_s, w, w_s)
+    other = K.fp8_gemm_f32(a, torch.empty(a_s.numel() + 1, device="cuda")[1:].view_as(a_s).copy_(a_s), w, w_s)
+    assert (c32[:, cols].double() - ref).abs().max() <= TOL * ref.pow(2).mean().sqrt()
+    assert ((c32 - other)[:, cols].double().abs() <= 2 * (kb + 2) * 2.0 ** -24 * size).all()
+    assert torch.equal(c16, c32.to(torch.bfloat16))
+    assert torch.equal(torch.ops.dsv3fp8.fp8_gemm_pow2(a, a_s.mul(0).add(2), w, w_s.mul(0).add(0.5), _lib.F32),
+                       K.fp8_gemm_f32(a, a_s.mul(0).add(2), w, w_s.mul(0).add(0.5)))          # (the same kernel)
+
+
 @pytest.mark.parametrize("n", [1, 15, 16, 100, 129, 576, 577, 1000])
 def test_ragged_n(K, n):
     from dsv3fp8 import workloads
