@@ -40,6 +40,8 @@ HIPCC_FLAGS = [
 # sums in the 256 accumulation registers; an ordinary rescale of them spilled 300): a spill there is a copy per tile.
 NO_SPILL_SOURCES = {"fp8_gemm_skinny.hip", "fp8_gemm_stream.hip", "fp8_gemm_mid.hip", "mla_decode.hip", "mla_prefill.hip"}
 SCRATCH_ALLOWED = {
+    # two scalar registers kept in lanes of a vector register: no scratch memory, and outside the tile loop
+    "mla_attend_kernel": 2,
     # the quantising variant with four strips per wavefront (a plan for very wide weights at one or two rows that none
     # of the 671B projections takes): compiler-counted waits, 20 bytes per lane
     "skinny_kernelILi1ELi4ELi2ELb1ELb0E": 24,
