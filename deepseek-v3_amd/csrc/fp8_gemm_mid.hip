@@ -283,7 +283,7 @@ inline bool large_m_pinned() {
 inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     Plan p{};
     const int64_t kb = k / 128;
-    if (m <= 64 || k % 512 || m * k >= (1ll << 32) || n * k >= (1ll << 32) || large_m_pinned()) return p;
+    if (m <= 32 || k % 512 || m * k >= (1ll << 32) || n * k >= (1ll << 32) || large_m_pinned()) return p;
     p.splits = 1;
     p.nkb = (int)kb;
     // Weights of 96 MiB and more, of more columns than 128 of the large-M kernel's tiles and at most 256 tiles of 160: one round here, with
@@ -292,7 +292,8 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     // 32768 columns and fewer, where 128-row tiles of the large-M kernel, two a column tile or in two K slices, are one full round
     // (7168 -> 31744 at 65 / 160 / 193 rows 0.93 / 0.88 / 0.84); K of 32768 (0.81 .. 1.50, 0.92 .. 0.96 at 193 rows); from 193 rows on,
     // whose ring has three stages, fewer than 212 tiles or 32 K blocks (16384 -> 32769 0.94, 2560 -> 40960 0.98); 225 rows and more, whose
-    // ring would have two; two row tiles of 116 for 7168 -> 18432 (129 .. 224 rows, 48.4 us there, 53.5 here at 193): that one 128- or
+    // ring would have two.  33 .. 64 rows of such weights are the large-M kernel's otherwise, too (fp8_gemm_tile.hip): 7168 -> 36864 at 33 / 64 rows 61.2 /
+    // 66.7 us there, 53.5 / 56.9 here, over 32769 .. 40960 columns and K of 2560 .. 16384 1.05 .. 1.21.  Nor two row tiles of 116 for 7168 -> 18432 (129 .. 224 rows, 48.4 us there, 53.5 here at 193): that one 128- or
     // 256-row tile of the large-M kernel reads the weights once.
     const int64_t t160 = (n + 159) / 160, rows = (m + 15) / 16;
     if (n * k >= (96ll << 20) && n > 32768 && t160 <= 256 && kb <= 128 && rows <= (t160 < 212 || kb < 32 ? 12 : 14)) {
@@ -302,7 +303,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     }
     // Up to 128 rows of a weight of 176 to 256 tiles of 128 columns, in one round where 256 columns make half a round: over 22401 .. 32768
     // columns and K of 1536 .. 16384, measured as above, 0.98 .. 1.77, 1536 -> 24576 1.23 .. 1.14.  Not below 12 K blocks (512 -> 32768: equal to
-    // 12 % more time), nor above 128 (32768 -> 28672 at 128 rows 0.98).
+    // 12 % more time), nor above 128 (32768 -> 28672 at 128 rows 0.98).  33 .. 64 rows 0.99 .. 1.20, 1.06 on average.
     const int64_t t128 = (n + 127) / 128;
     if (m <= 128 && t128 >= 176 && t128 <= 256 && kb >= 12 && kb <= 128) {
         p.mt = 8; p.wm = 4; p.sn = 4;
@@ -333,7 +334,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     // Over 1 .. 2304 columns and K of 4096 .. 16384, 65 rows up to the last one taken (1 .. 128 columns: 8192 at K of 4096, 5440 at 7168;
     // 300: 2688; 576: 1600), measured as above: 0.99 .. 1.51, at the last ones 1.01 .. 1.28.
     const int64_t tiles = (m + 63) / 64 * t128;
-    if (n <= 2304 && kb >= 32 && tiles <= 256) {
+    if (m > 64 && n <= 2304 && kb >= 32 && tiles <= 256) {
         int64_t s = 256 / tiles;
         s = s > 7 ? 7 : s;
         int64_t nkb = ((kb + s - 1) / s + 3) / 4 * 4;
@@ -360,7 +361,8 @@ int launch_cfg(const Plan& p, const void* a, const float* a_s, const void* b, co
 
 }  // namespace mid
 
-bool mid_supported(int64_t m, int64_t n, int64_t k) { return mid::make_plan(m, n, k).mt != 0; }
+bool mid_supported(int64_t m, int64_t n, int64_t k) { return m > 64 && mid::make_plan(m, n, k).mt != 0; }
+bool mid_supported_few(int64_t m, int64_t n, int64_t k) { return m <= 64 && mid::make_plan(m, n, k).mt != 0; }
 
 size_t mid_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     const mid::Plan p = mid::make_plan(m, n, k);

@@ -196,6 +196,27 @@ def test_sliced_tiles_of_as_many_rows_as_there_are(K, m, n, k):
                        K.fp8_gemm_f32(a, a_s.mul(0).add(2), w, w_s.mul(0).add(0.5)))          # (the same kernel)
 
 
+@pytest.mark.parametrize("m,n,k", [(33, 32769, 3072), (48, 36864, 4096), (64, 40960, 3072), (64, 24576, 4096), (49, 22500, 7168), (33, 32768, 3584)])
+def test_33_to_64_rows_of_wide_weights(K, m, n, k):
+    """The tiles of one round below 65 rows: wavefronts without a row, ragged columns; against the large-M kernel, which takes scales
+    that are not 16-byte aligned (bound: test_sliced_tiles_of_as_many_rows_as_there_are), and sampled columns against binary64."""
+    kb = k // 128
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    a = (torch.randn(m, k, generator=g, device="cuda") * 40).to(torch.float8_e4m3fn)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 40).to(torch.float8_e4m3fn)
+    a_s = torch.rand(m, kb, generator=g, device="cuda") + 0.5
+    w_s = torch.rand((n + 127) // 128, kb, generator=g, device="cuda") + 0.5
+    cols = torch.cat([torch.randint(0, n, (200,), generator=g, device="cuda"), torch.tensor([0, 127, 128, n - 1, n - 128], device="cuda")])
+    s = a_s.double().repeat_interleave(128, 1), w_s[cols // 128].double().repeat_interleave(128, 1)
+    ref = (a.double() * s[0]) @ (w[cols].double() * s[1]).t().contiguous()
+    size = (a.double().abs() * s[0]) @ (w[cols].double().abs() * s[1]).t().contiguous()
+    c32, c16 = _gemm_both(K, a, a_s, w, w_s)
+    other = K.fp8_gemm_f32(a, torch.empty(a_s.numel() + 1, device="cuda")[1:].view_as(a_s).copy_(a_s), w, w_s)
+    assert (c32[:, cols].double() - ref).abs().max() <= TOL * ref.pow(2).mean().sqrt()
+    assert ((c32 - other)[:, cols].double().abs() <= 2 * (kb + 2) * 2.0 ** -24 * size).all()
+    assert torch.equal(c16, c32.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("n", [1, 15, 16, 100, 129, 576, 577, 1000])
 def test_ragged_n(K, n):
     from dsv3fp8 import workloads
