@@ -270,7 +270,7 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
 
 // Three windows in which the large-M kernel's tiles fit the chip badly.  Power-of-two scales take the same kernel (accumulating in the
 // matrix core was equal to 4 % faster here).
-struct Plan { int mt, wm, sn, splits, nkb; };       // mt == 0: not for this kernel
+struct Plan { int mt, wm, sn, splits, nkb; bool tall; };       // mt == 0: not for this kernel; tall: more than 256 rows of narrow weights
 // The variables that pin how the large-M kernel runs its dense tiles (one K slice, a tile height, a schedule) pin that kernel too.
 inline bool large_m_pinned() {
     static const bool v = [] {
@@ -339,10 +339,30 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
         s = s > 7 ? 7 : s;
         int64_t nkb = ((kb + s - 1) / s + 3) / 4 * 4;
         nkb = nkb < 8 ? 8 : nkb;
-        if (nkb > 20) return p;
-        p.nkb = (int)nkb;
-        p.splits = (int)((kb + nkb - 1) / nkb);
-        p.mt = 4; p.wm = 2; p.sn = 2;
+        if (nkb <= 20) {
+            p.nkb = (int)nkb;
+            p.splits = (int)((kb + nkb - 1) / nkb);
+            p.mt = 4; p.wm = 2; p.sn = 2;
+            return p;
+        }
+    }
+    // More rows of them: tiles of 128 rows (112 where that pads less) x 128 columns in one round, without slices or in three and more: the large-M kernel has
+    // 256-column tiles in up to eight slices, twice the slabs and more, or fewer tiles than units.  Behind the quantisation (us, large-M kernel / here): 7168 -> 1536 at
+    // 512 / 640 / 777 / 896 rows 26.9 / 28.2 / 31.2 / 32.4 -> 24.6 / 27.4 / 29.7 / 30.9, 7168 -> 2112 at 350 / 640 / 1800 26.0 / 32.1 / 57.9 -> 24.5 / 29.9 / 51.2,
+    // 4096 -> 1986 at 1597 51.4 -> 35.8; over 45 listed and drawn sizes of 300 .. 2300 columns and K of 4096 .. 16384 0.99 .. 1.42.  Left out: two
+    // slices (7168 -> 1536 at 930 / 1280 rows 0.94 / 0.97, 8192 -> 381 at 4757 0.94; 16384 -> 1707 at 1060 would be 1.16) and rounds
+    // with more units idle (7168 -> 2112 at 400, 204 of 256: 0.96).
+    if (m > 256 && n <= 2304 && kb >= 32) {
+        for (int mt : {8, 7}) {
+            const int64_t tm = (m + 16 * mt - 1) / (16 * mt), s = 256 / (tm * t128 > 0 ? tm * t128 : 1);
+            if (s < 1 || (mt == 7 && tm * 112 >= (m + 127) / 128 * 128)) continue;
+            int64_t nkb = ((kb + s - 1) / s + 3) / 4 * 4;
+            nkb = nkb < 8 ? 8 : nkb;
+            const int64_t splits = (kb + nkb - 1) / nkb;
+            if (splits == 2 || tm * t128 * splits < (splits == 1 ? 200 : 216) || (p.mt && nkb > p.nkb)) continue;
+            p.mt = mt; p.wm = 4; p.sn = 4;
+            p.nkb = (int)nkb; p.splits = (int)splits; p.tall = true;
+        }
     }
     return p;
 }
@@ -361,8 +381,11 @@ int launch_cfg(const Plan& p, const void* a, const float* a_s, const void* b, co
 
 }  // namespace mid
 
-bool mid_supported(int64_t m, int64_t n, int64_t k) { return m > 64 && mid::make_plan(m, n, k).mt != 0; }
-bool mid_supported_few(int64_t m, int64_t n, int64_t k) { return m <= 64 && mid::make_plan(m, n, k).mt != 0; }
+bool mid_supported(int64_t m, int64_t n, int64_t k) {
+    const mid::Plan p = mid::make_plan(m, n, k);
+    return m > 64 && p.mt != 0 && !p.tall;
+}
+bool mid_takes(int64_t m, int64_t n, int64_t k) { return mid::make_plan(m, n, k).mt != 0; }
 
 size_t mid_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     const mid::Plan p = mid::make_plan(m, n, k);
@@ -388,6 +411,7 @@ int launch_mid(const void* a, const float* a_s, const void* b, const float* b_s,
         case 125: return launch_cfg<12, 4, 5, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         case 145: return launch_cfg<14, 4, 5, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         case 84:  return launch_cfg<8, 4, 4, 4>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
+        case 74:  return launch_cfg<7, 4, 4, 4>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         case 104: return launch_cfg<10, 4, 4, 4>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         case 124: return launch_cfg<12, 4, 4, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);
         case 144: return launch_cfg<14, 4, 4, 3>(p, a, a_s, b, b_s, out, od, (int)m, (int)n, (int)k, st);

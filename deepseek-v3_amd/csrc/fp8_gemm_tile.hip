@@ -341,7 +341,7 @@ int forced_kernel() {
 // Which problems go to the large-M kernel (K range cut into slices when the tiles do not fill the chip): every M
 // above 64, and M = 33 .. 64 when the weight is large
 // (>= 96 MiB) and has 8192 rows or more (7168 -> 36864 at 64 rows: 65 against 66-76 us), unless the mid-M tiles take it
-// (mid_supported, mid_supported_few, asked behind this: 57 us).  There it runs at a flat 32-34 us
+// (mid_takes, asked behind this: 57 us).  There it runs at a flat 32-34 us
 // per 117-132 MB from 9 to 64 rows.  Everything else the activation-streaming kernel has a plan for goes there (16384 -> 7168
 // at 16 / 32 / 64 rows 23.5 / 24.5 / 29.5 against 33 / 31.6 / 34.6 us; 7168 -> 18432 at 16 / 32 rows 22.8 / 25.3 against
 // 36.5 / 30.7 us); for the smaller decode weights the streaming and tile kernels are faster anyway.
@@ -373,7 +373,7 @@ int launch_typed(const void* a, const float* a_s, const void* b, const float* b_
     if (force == 0 && single_group_stream(m, n, k))
         return launch_skinny_single(a, a_s, b, b_s, c, CD, m, n, k, st);
     const bool to_prefill = force != 1 && !(force == 3 && stream_supported(m, n, k)) && to_large_m_kernel(m, n, k);
-    const bool use_mid = to_prefill && force == 0 && (mid_supported(m, n, k) || mid_supported_few(m, n, k)) && mid_takes_scales(a_s, b_s);
+    const bool use_mid = to_prefill && force == 0 && mid_takes(m, n, k) && mid_takes_scales(a_s, b_s);
     const bool use_stream = force != 1 && !to_prefill && !(force == 4 && skinny_supported(m, n, k)) && stream_supported(m, n, k);
     // mid-M tiles, and the weight-streaming kernels of the decode shapes: one launch, or K slices and a reduction
     if (use_mid || use_stream || (force != 1 && !to_prefill && skinny_supported(m, n, k))) {

@@ -196,6 +196,18 @@ def test_sliced_tiles_of_as_many_rows_as_there_are(K, m, n, k):
                        K.fp8_gemm_f32(a, a_s.mul(0).add(2), w, w_s.mul(0).add(0.5)))          # (the same kernel)
 
 
+@pytest.mark.parametrize("m,n,k", [(450, 1536, 7168), (777, 1535, 7168), (896, 1500, 4096), (321, 2112, 7168), (513, 2049, 8192), (1800, 2112, 4096),
+                                   (1597, 1986, 4096), (1400, 524, 8192)])
+def test_tall_tiles_of_narrow_weights(K, m, n, k):
+    """Tiles of 112 and 128 rows in one to seven slices: last tiles of few rows, ragged columns, uneven slices."""
+    import ctypes
+    from dsv3fp8 import _lib
+    takes = _lib.lib["_ZN4dsv39mid_takesElll"]                  # dsv3::mid_takes(rows, columns, K)
+    takes.restype, takes.argtypes = ctypes.c_bool, [ctypes.c_int64] * 3
+    assert takes(m, n, k) and not takes(930, 1536, 7168) and not takes(1280, 1536, 7168) and not takes(4757, 381, 8192)
+    test_33_to_64_rows_of_wide_weights(K, m, n, k)
+
+
 @pytest.mark.parametrize("m,n,k", [(33, 32769, 3072), (48, 36864, 4096), (64, 40960, 3072), (64, 24576, 4096), (49, 22500, 7168), (33, 32768, 3584)])
 def test_33_to_64_rows_of_wide_weights(K, m, n, k):
     """The tiles of one round below 65 rows: wavefronts without a row, ragged columns; against the large-M kernel, which takes scales
