@@ -351,8 +351,9 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     // 512 / 640 / 777 / 896 rows 26.9 / 28.2 / 31.2 / 32.4 -> 24.6 / 27.4 / 29.7 / 30.9, 7168 -> 2112 at 350 / 640 / 1800 26.0 / 32.1 / 57.9 -> 24.5 / 29.9 / 51.2,
     // 4096 -> 1986 at 1597 51.4 -> 35.8; over 45 listed and drawn sizes of 300 .. 2300 columns and K of 4096 .. 16384 0.99 .. 1.42.  Left out: two
     // slices (7168 -> 1536 at 930 / 1280 rows 0.94 / 0.97, 8192 -> 381 at 4757 0.94; 16384 -> 1707 at 1060 would be 1.16) and rounds
-    // with more units idle (7168 -> 2112 at 400, 204 of 256: 0.96).
-    if (m > 256 && n <= 2304 && kb >= 32) {
+    // with more units idle (7168 -> 2112 at 400, 204 of 256: 0.96), and up to 640 columns on a K range up to 8192 (7168 -> 576 at 1700 .. 2048 0.99 .. 1.06, with
+    // power-of-two scales 0.94 .. 1.00; these are 0.98 .. 1.53 else).
+    if (m > 256 && n <= 2304 && kb >= 32 && (t128 >= 6 || kb > 64)) {
         for (int mt : {8, 7}) {
             const int64_t tm = (m + 16 * mt - 1) / (16 * mt), s = 256 / (tm * t128 > 0 ? tm * t128 : 1);
             if (s < 1 || (mt == 7 && tm * 112 >= (m + 127) / 128 * 128)) continue;
