@@ -13,7 +13,7 @@
 //
 // Two launches: expand (keys and values, and the rotary keys, in the order in which the attention kernel's wavefronts
 // read their operands, and which tiles of the mask are all zero or all -inf) and attend.
-// At 4096 tokens, 128 heads, causal mask (kernel trace): expand 140 us, attend 750 .. 770 us on a cool card (0.9 PFLOP/s
+// At 4096 tokens, 128 heads, causal mask (kernel trace): expand 140 .. 149 us, attend 735 .. 770 us on a cool card (0.9 PFLOP/s
 // of the pairs the mask leaves) and more on a warm one, whose clock falls to 1.8 GHz under it; the layer 1.53 ms where the
 // absorbed form as tensor operations took 20.1 ms (2 x 2.5 ms score products, 1.6 ms value product and 12 ms of passes over
 // the 4.3 GB score matrix).
@@ -235,11 +235,11 @@ struct AttendArgs {
 // tiles skip the 64 multiplications of the rescale).
 // Two workgroups share a compute unit, each with two stages of 40 KiB and one wavefront per SIMD: one does matrix products while the
 // other does exponentials, waits for its queries or writes its results, and nothing makes them wait for each other; the exponentials and
-// the products beside them go first (layer at 800 / 4096: 282 -> 279, 1520 -> 1508 us; with the score product first instead about as much, with all products half).  As one workgroup of 256 rows (eight
-// wavefronts in two groups half a tile apart, three stages) the copies of a tile served twice the rows, but the steps of the
-// causal diagonal, a ragged last tile and each start and end kept the whole unit: us at 200 / 800 / 4096 rows of 128 heads 21.6 / 92 / 785, now
-// 16.3 / 70 / 760; with queries' loads behind the first tile's copies and four mask values a load (each was one of its own: 32 lines a
-// load, 2000 cycles of a unit's load path for every block on the diagonal).
+// the products beside them go first (layer at 800 / 4096: 282 -> 279, 1520 -> 1508 us; with the score product first instead about as much, with
+// all products half).  As one workgroup of 256 rows (eight wavefronts in two groups half a tile apart, three stages) the copies of a tile
+// served twice the rows, but the steps of the causal diagonal, a ragged last tile and each start and end kept the whole unit: us at
+// 200 / 800 / 4096 rows of 128 heads 21.6 / 92 / 785, now 16.5 / 69 / 735; with queries' loads behind the first tile's copies and four
+// mask values a load (each was one of its own: 32 lines a load, 2000 cycles of a unit's load path for every block on the diagonal).
 template <bool MF32>
 __global__ __launch_bounds__(kQTile * 2, 2) void mla_attend_kernel(AttendArgs p) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
