@@ -39,9 +39,12 @@ HIPCC_FLAGS = [
 # The attention kernels keep their sums in registers for a whole loop and have none to spare (mla_decode_kernel: 32 x 512
 # sums in the 256 accumulation registers; an ordinary rescale of them spilled 300): a spill there is a copy per tile.
 NO_SPILL_SOURCES = {"fp8_gemm_skinny.hip", "fp8_gemm_stream.hip", "fp8_gemm_mid.hip", "mla_decode.hip", "mla_prefill.hip"}
-SCRATCH_ALLOWED = {
-    # two scalar registers kept in lanes of a vector register: no scratch memory, and outside the tile loop
+SGPR_SPILLS_ALLOWED = {
+    # Scalars kept in lanes of a vector register are no scratch memory and cost nothing outside the tile loop: the limit for them.  (This build
+    # reports none.)  The kernel takes all 256 vector registers, so a spilled one of these would be a copy per tile: refused.
     "mla_attend_kernel": 2,
+}
+SCRATCH_ALLOWED = {
     # the quantising variant with four strips per wavefront (a plan for very wide weights at one or two rows that none
     # of the 671B projections takes): compiler-counted waits, 20 bytes per lane
     "skinny_kernelILi1ELi4ELi2ELb1ELb0E": 24,
@@ -59,7 +62,8 @@ def check_no_spills(name: str, remarks: str) -> None:
         m = re.search(r"(VGPRs Spill|SGPRs Spill|ScratchSize \[bytes/lane\]): (\d+)", line)
         if not (m and kernel and "_kernel" in kernel):
             continue
-        allowed = max([v for k, v in SCRATCH_ALLOWED.items() if k in kernel], default=0)
+        exceptions = {**SCRATCH_ALLOWED, **(SGPR_SPILLS_ALLOWED if m.group(1) == "SGPRs Spill" else {})}
+        allowed = max([v for k, v in exceptions.items() if k in kernel], default=0)
         if int(m.group(2)) > allowed:
             raise RuntimeError(f"{name}: {kernel} reports {m.group(1)} = {m.group(2)} (allowed: {allowed}); these "
                                f"kernels must not spill (lower the kernel's register use or its occupancy target)")

@@ -555,3 +555,12 @@ def test_build_refuses_spills(source):
             with pytest.raises(RuntimeError, match="must not spill"):
                 build.check_no_spills(source, report.format(kernel, what, 4))
     build.check_no_spills(source, report.format("mla_attend_kernelILb0E", "SGPRs Spill", 2))
+
+
+@pytest.mark.parametrize("spilled", [1, 2, 4])
+@pytest.mark.parametrize("what", ["VGPRs Spill", "ScratchSize [bytes/lane]"])
+def test_attention_kernel_may_keep_scalars_in_lanes_but_spill_no_vector_registers(what, spilled):
+    import build
+    report = f"remark: Function Name: _ZN4dsv317mla_attend_kernelILb1EEvNS_10AttendArgsE\nremark:     {what}: {spilled}\n"
+    with pytest.raises(RuntimeError, match="must not spill"):
+        build.check_no_spills("mla_prefill.hip", report)
