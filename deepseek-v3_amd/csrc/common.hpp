@@ -212,6 +212,7 @@ size_t mla_prefill_workspace_bytes(int64_t batch, int64_t rows, int64_t position
 int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
                        const void* w, const float* ws, const void* mask, bool mask_f32, void* y, float* ys, int64_t batch,
                        int64_t rows, int64_t positions, int heads, float scale, void* workspace, hipStream_t st);
+int mla_decode_side(int64_t batch, int64_t tokens, int64_t positions, int heads);      // tiles that a workgroup takes side by side
 size_t mla_decode_workspace_bytes(int64_t batch, int64_t tokens, int64_t positions, int heads);
 int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
                       const void* w, const float* ws, const void* mask, bool mask_f32, void* y, float* ys, int64_t batch,

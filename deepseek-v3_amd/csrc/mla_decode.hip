@@ -87,7 +87,7 @@ inline uint32_t magic_of(int64_t most, int64_t d) { return d > 1 && most * d < (
 // beside the first half's products; a tile takes 3800 in all (4630 with the copies in a row in front and every exponential between the products),
 // of which the clock takes back half (1.97 against 2.07 GHz at 32 x 4096).  What a range costs besides: at 256 workgroups and G = 1 67 MB of partial sums, 12 us
 // to write and as long to read.  Attention with the query's fold and mla_fold_kernel (us, before: G = 1): 8 sequences at 2000 positions 41.9 ->
-// 30.0 (G = 4), 16 at 2000 48.7 -> 34.8 (4), 32 at 1000 50.0 -> 38.3 (4), 64 at 1000 62.6 -> 53.4 (2), 32 at 4096 78.7 -> 68.7 (2), 1 at 700 22.6 -> 22.0.
+// 30.0 (G = 4), 16 at 2000 48.7 -> 34.8 (4), 32 at 1000 50.0 -> 38.3 (4), 64 at 1000 62.6 -> 53.4 (2), 32 at 4096 78.7 -> 68.7 (2).
 // PACK: the folded queries come in operand order (launch_wkv_b_absorb_q_packed), a KiB of consecutive bytes per load; as rows a
 // load touches 32 of them and takes 64 cycles of the compute unit's load path, 3.8 us for the workgroup's 128.
 enum { kNoMask, kMaskBf16, kMaskF32 };
@@ -679,9 +679,13 @@ __global__ __launch_bounds__(320) void mla_latent_kernel(LatentArgs p) {
 
 // How the positions of a step are split: one attend workgroup per compute unit (its LDS and registers take a whole one; fewer
 // leave units idle, more write more partial sums), a tile a wavefront each at least; and how many tiles a workgroup takes side by side: what
-// costs least by the measured costs (us) of a wavefront's tiles one after another (2.3; 2.65 and 3.4 where two and four at a time leave less or no room for
-// the next ones), of the partial sums (8 to 12 us for those of 256 workgroups of 128 rows) and of adding the wavefronts' sums.  Over 105 shapes (1 .. 128
-// sequences at 40 .. 4096 positions, 1 .. 31 tokens each) the rule is 1.4 % from the best of the three on average, 1.14 x faster than G = 1 everywhere.
+// costs least by the measured costs (us) of a wavefront's tiles one after another (2.3; 2.65 and 3.6 where two and four at a time leave less or no room for
+// the next ones), of the partial sums (8 to 12 us for those of 256 workgroups of 128 rows) and of the wavefronts' copies, barrier and sum in LDS (0.8 for
+// two; 1.4 for four, next to nothing where a context of one or two tiles leaves half of them without any).  Attention with the query's fold and
+// mla_fold_kernel, us for one / two / four: 1 sequence at 300 positions 23.0 / 24.1 / 24.1, at 700 24.7 / 25.0 / 24.7, at 2000 28.6 / 27.8 / 26.9, 8 at 64
+// 24.6 / 25.4 / 24.5, 8 at 2000 45.1 / 36.0 / 34.7, 24 at 1000 47.6 / 41.0 / 43.9, 64 at 4096 125 / 129 / 152.  Over 168 shapes (1 .. 128 sequences at 40 .. 4096 positions,
+// 1 .. 31 tokens each) the rule is 0.3 % from the best of the three on average, 4 % at most, 1.09 x faster than one everywhere and nowhere more than
+// 1 % slower (with 0.5 and 1.0 for the sums in LDS it was up to 3.3 % slower, at one tile a wavefront).
 // A wavefront has the tiles that one of G = 1 has: longer ranges would round more exponentials (a range's largest is exactly one).
 void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) {
     a.rows = (int)rows; a.positions = (int)positions;
@@ -695,8 +699,8 @@ void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) 
         const int64_t n = (steps + splits - 1) / splits;
         splits = (steps + n - 1) / n;
         const int64_t units = base * splits, rounds = (units + 255) / 256;
-        const double us = rounds * (2.3 + (n - 1) * (side == 1 ? 2.3 : side == 2 ? 2.65 : 3.4)) + (rounds - 1) * 3 + units * (128 / side) * 0.00049 +
-                          (side == 1 ? 0 : side == 2 ? 0.5 : 1.0);
+        const double us = rounds * (2.3 + (n - 1) * (side == 1 ? 2.3 : side == 2 ? 2.65 : 3.6)) + (rounds - 1) * 3 + units * (128 / side) * 0.00049 +
+                          (side == 1 ? 0 : side == 2 ? 0.8 : a.tiles <= 2 ? 0.2 : 1.4);
         if (side > 1 && us >= best) continue;
         best = us;
         a.side = side; a.blocks = (int)blocks; a.per = (int)(n * side); a.splits = (int)splits;
@@ -718,6 +722,12 @@ template <int G> int launch_attend(const DecodeArgs& a, int which, unsigned grid
 }
 
 }  // namespace
+
+int mla_decode_side(int64_t batch, int64_t tokens, int64_t positions, int heads) {
+    DecodeArgs a;
+    decode_plan(a, batch, tokens * heads, positions);
+    return a.side;
+}
 
 size_t mla_decode_workspace_bytes(int64_t batch, int64_t tokens, int64_t positions, int heads) {
     DecodeArgs a;

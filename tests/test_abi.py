@@ -564,3 +564,18 @@ def test_attention_kernel_may_keep_scalars_in_lanes_but_spill_no_vector_register
     report = f"remark: Function Name: _ZN4dsv317mla_attend_kernelILb1EEvNS_10AttendArgsE\nremark:     {what}: {spilled}\n"
     with pytest.raises(RuntimeError, match="must not spill"):
         build.check_no_spills("mla_prefill.hip", report)
+
+
+# Which variant of the decode attention (tiles that a workgroup takes side by side) the cost rule picks: the measured fastest, or one within 1 % of it
+# (sequences, tokens, positions, heads); then the sizes that tests/test_gpu_mla_attention.py has for each variant.
+@pytest.mark.parametrize("side,b,s,t,h", [
+    (1, 1, 1, 40, 128), (1, 1, 1, 300, 128), (1, 1, 1, 700, 128), (1, 2, 1, 300, 128), (1, 3, 1, 200, 128), (1, 4, 1, 128, 128), (1, 48, 1, 4096, 128),
+    (1, 64, 1, 4096, 128), (1, 96, 1, 2000, 128), (2, 12, 1, 2000, 128), (2, 24, 1, 1000, 128), (2, 32, 1, 4096, 128), (2, 64, 1, 1000, 128),
+    (2, 20, 5, 300, 128), (4, 8, 1, 40, 128), (4, 16, 1, 64, 128), (4, 1, 1, 2000, 128), (4, 2, 1, 1000, 128), (4, 8, 1, 2000, 128), (4, 32, 1, 200, 128),
+    (4, 1, 5, 700, 128),
+    (4, 8, 1, 2030, 128), (4, 1, 9, 900, 30), (4, 2, 9, 200, 128), (4, 3, 13, 200, 24), (2, 12, 2, 900, 128), (2, 30, 3, 300, 128), (2, 64, 1, 1005, 100),
+    (2, 5, 11, 2050, 50), (1, 64, 1, 3650, 100), (1, 2, 66, 130, 128), (1, 1, 6, 90, 5)])
+def test_tiles_side_by_side_of_the_decode_attention(L, side, b, s, t, h):
+    plan = L.lib["_ZN4dsv315mla_decode_sideEllli"]              # dsv3::mla_decode_side(sequences, tokens, positions, heads)
+    plan.restype, plan.argtypes = ctypes.c_int, [ctypes.c_int64] * 3 + [ctypes.c_int]
+    assert plan(b, s, t, h) == side
