@@ -275,6 +275,23 @@ def test_ragged_n_equals_prefix_of_padded(K):
     assert torch.equal(full[:, :576], part)
 
 
+@pytest.mark.parametrize("m,n,padded,k", [(5, 575, 576, 7168), (5, 574, 576, 7168), (3, 573, 576, 7168), (129, 4095, 4096, 11264), (129, 4094, 4096, 11264),
+                                          (129, 4093, 4096, 11264), (130, 4095, 4096, 11264)])
+def test_sums_of_slabs_that_are_no_whole_fours(K, m, n, padded, k):
+    """K slices whose partial sums (m n values a slab) start on every 4-byte boundary, with the last one to three values by themselves: the same
+    bits as the columns of a product whose slabs are whole fours, in every result type."""
+    from dsv3fp8 import _lib
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    a = (torch.randn(m, k, generator=g, device="cuda") * 40).to(torch.float8_e4m3fn)
+    w = (torch.randn(padded, k, generator=g, device="cuda") * 40).to(torch.float8_e4m3fn)
+    a_s = torch.rand(m, k // 128, generator=g, device="cuda") + 0.5
+    w_s = torch.rand((padded + 127) // 128, k // 128, generator=g, device="cuda") + 0.5
+    assert _lib.lib.dsv3_fp8_gemm_workspace_bytes(m, n, k) >= 2 * m * n * 4
+    for dtype in (_lib.F32, _lib.BF16, _lib.F16):
+        got = torch.ops.dsv3fp8.fp8_gemm(a, a_s, w[:n].contiguous(), w_s, dtype)
+        assert torch.equal(got, torch.ops.dsv3fp8.fp8_gemm(a, a_s, w, w_s, dtype)[:, :n])
+
+
 @pytest.mark.parametrize("n", [1, 7, 8, 9, 127, 129, 576, 2041, 2048])
 @pytest.mark.parametrize("m,k", [(1, 128), (2, 384), (1, 1536), (2, 7168), (1, 7168)])
 def test_strips_of_eight_rows_equal_strips_of_sixteen(K, m, n, k):
