@@ -303,9 +303,11 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     }
     // Up to 128 rows of a weight of 176 to 256 tiles of 128 columns, in one round where 256 columns make half a round: over 22401 .. 32768
     // columns and K of 1536 .. 16384, measured as above, 0.98 .. 1.77, 1536 -> 24576 1.23 .. 1.14.  Not below 12 K blocks (512 -> 32768: equal to
-    // 12 % more time), nor above 128 (32768 -> 28672 at 128 rows 0.98).  33 .. 64 rows 0.99 .. 1.20, 1.06 on average.
+    // 12 % more time), nor above 128 (32768 -> 28672 at 128 rows 0.98).  33 .. 64 rows on 28 to 80 K blocks: 1.00 .. 1.17 over 23 sizes, 1.07 on average;
+    // on fewer 0.99 .. 1.01 (2560 -> 24704 at 48 rows 20.0 / 20.0 us), on more 0.87 .. 1.03 (12288 -> 23424 at 35 rows 73.4 / 84.0 us: two K slices of as many tiles
+    // of the large-M kernel fill the chip as well, and their slabs cost little beside that many blocks).
     const int64_t t128 = (n + 127) / 128;
-    if (m <= 128 && t128 >= 176 && t128 <= 256 && kb >= 12 && kb <= 128) {
+    if (m <= 128 && t128 >= 176 && t128 <= 256 && (m <= 64 ? kb >= 28 && kb <= 80 : kb >= 12 && kb <= 128)) {
         p.mt = 8; p.wm = 4; p.sn = 4;
         return p;
     }

@@ -579,3 +579,16 @@ def test_tiles_side_by_side_of_the_decode_attention(L, side, b, s, t, h):
     plan = L.lib["_ZN4dsv315mla_decode_sideEllli"]              # dsv3::mla_decode_side(sequences, tokens, positions, heads)
     plan.restype, plan.argtypes = ctypes.c_int, [ctypes.c_int64] * 3 + [ctypes.c_int]
     assert plan(b, s, t, h) == side
+
+
+# The sizes that the dispatcher sends to the mid-M tiles: both sides of the limits at 33 .. 64 rows, ...
+WIDE_33_TO_64 = [(32, 36864, 7168, False), (33, 36864, 7168, True), (64, 36864, 7168, True), (64, 32769, 3072, True), (64, 32769, 2560, False),
+                 (33, 24576, 3584, True), (33, 24576, 3072, False), (64, 24576, 10240, True), (64, 24576, 10752, False), (65, 24576, 10752, True),
+                 (65, 24576, 1536, True), (64, 22400, 7168, False), (64, 22401, 7168, True), (32, 24576, 7168, False), (64, 24576, 7296, False)]
+
+
+@pytest.mark.parametrize("m,n,k,taken", WIDE_33_TO_64)
+def test_sizes_that_the_dispatcher_sends_to_the_mid_m_tiles(L, m, n, k, taken):
+    takes = L.lib["_ZN4dsv39mid_takesElll"]                     # dsv3::mid_takes(rows, columns, K)
+    takes.restype, takes.argtypes = ctypes.c_bool, [ctypes.c_int64] * 3
+    assert takes(m, n, k) == taken
