@@ -316,10 +316,12 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     // 160 rows, and above on slices of 32 blocks and more (three or four, nearly equal) of a K range up to 18432: 16384 -> 7168 at 129 / 193 / 224 / 256 rows 1.15 / 1.04 / 1.08 / 1.10,
     // 18432 -> 7168 1.05 / 1.02 / 1.04 / 1.04, 16384 -> 8192 1.06 .. 1.11, 7168 -> 16384 at 129 / 160 1.15 / 1.06 times the speed with the quantisation in front;
     // over 125 drawn and listed sizes 0.98 .. 1.48, 1.05 on average (power-of-two scales 1.04).  Left out: 7168 -> 12288 (192 units) 0.92 .. 1.01 at 16384, 20480 -> 9216
-    // 0.91, 11264 -> 7168 at 193 rows 0.96 (slices of 24), 7168 -> 7168 at 159 0.96 (of 16).
+    // 0.91, 11264 -> 7168 at 193 rows 0.96 (slices of 24), 7168 -> 7168 at 159 0.96 (of 16), and slices of eight blocks with a shorter last one, which are a slab more
+    // than the large-M kernel's for nothing (1536 -> 15488 at 139 rows, one slice there, 19.1 us, two here 24.7; 3584 -> 8064 at 159 25.3 / 26.0, 5632 -> 5376 at 159
+    // equal; 2048 -> 16000 at 147, two even ones, 29.0 / 25.5).
     if (m > 128 && m <= 256 && t128 >= 32 && t128 <= 128 && kb <= 144) {
         const int64_t sl = 256 / t128, nkb = ((kb + sl - 1) / sl + 3) / 4 * 4, splits = (kb + nkb - 1) / nkb, units = t128 * splits;
-        if (nkb >= 8 && (units >= 240 || (units >= 220 && nkb >= 24)) && (m <= 160 || (nkb >= 32 && splits >= 3 && nkb * splits - kb <= 8))) {
+        if ((nkb > 8 || (nkb == 8 && kb % 8 == 0)) && (units >= 240 || (units >= 220 && nkb >= 24)) && (m <= 160 || (nkb >= 32 && splits >= 3 && nkb * splits - kb <= 8))) {
             p.nkb = (int)nkb;
             p.splits = (int)splits;
             p.wm = 4; p.sn = 4;

@@ -585,9 +585,13 @@ def test_tiles_side_by_side_of_the_decode_attention(L, side, b, s, t, h):
 WIDE_33_TO_64 = [(32, 36864, 7168, False), (33, 36864, 7168, True), (64, 36864, 7168, True), (64, 32769, 3072, True), (64, 32769, 2560, False),
                  (33, 24576, 3584, True), (33, 24576, 3072, False), (64, 24576, 10240, True), (64, 24576, 10752, False), (65, 24576, 10752, True),
                  (65, 24576, 1536, True), (64, 22400, 7168, False), (64, 22401, 7168, True), (32, 24576, 7168, False), (64, 24576, 7296, False)]
+# ... at 129 .. 256 rows of slices of eight K blocks, ...
+SLICES_OF_EIGHT = [(139, 15488, 1536, False), (151, 15419, 1536, False), (147, 16000, 2048, True), (159, 8064, 3584, False), (159, 8064, 4096, True),
+                   (145, 10816, 2560, False), (145, 10816, 3072, True), (159, 5376, 5632, False), (159, 5376, 6144, True), (158, 4096, 8192, True),
+                   (160, 6400, 5120, True)]
 
 
-@pytest.mark.parametrize("m,n,k,taken", WIDE_33_TO_64)
+@pytest.mark.parametrize("m,n,k,taken", WIDE_33_TO_64 + SLICES_OF_EIGHT)
 def test_sizes_that_the_dispatcher_sends_to_the_mid_m_tiles(L, m, n, k, taken):
     takes = L.lib["_ZN4dsv39mid_takesElll"]                     # dsv3::mid_takes(rows, columns, K)
     takes.restype, takes.argtypes = ctypes.c_bool, [ctypes.c_int64] * 3
