@@ -352,11 +352,15 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     }
     // More rows of them: tiles of 128 rows (112 where that pads less) x 128 columns in one round, without slices or in three and more: the large-M kernel has
     // 256-column tiles in up to eight slices, twice the slabs and more, or fewer tiles than units.  Behind the quantisation (us, large-M kernel / here): 7168 -> 1536 at
-    // 512 / 640 / 777 / 896 rows 26.9 / 28.2 / 31.2 / 32.4 -> 24.6 / 27.4 / 29.7 / 30.9, 7168 -> 2112 at 350 / 640 / 1800 26.0 / 32.1 / 57.9 -> 24.5 / 29.9 / 51.2,
-    // 4096 -> 1986 at 1597 51.4 -> 35.8; over 45 listed and drawn sizes of 300 .. 2300 columns and K of 4096 .. 16384 0.99 .. 1.42.  Left out: two
-    // slices (7168 -> 1536 at 930 / 1280 rows 0.94 / 0.97, 8192 -> 381 at 4757 0.94; 16384 -> 1707 at 1060 would be 1.16) and rounds
+    // 512 / 640 / 896 rows 27.3 / 29.0 / 33.0 -> 25.5 / 28.0 / 31.8, at 777 30.7 .. 35.4 from process to process -> 31.2 .. 31.7, 7168 -> 2112 at 350 / 640 / 1800 26.1 / 32.7 / 57.8
+    // -> 24.8 / 30.6 / 52.0; power-of-two scales alike.  Over 81 drawn and listed sizes of 256 .. 2304 columns and K of 4096 .. 16384 0.98 .. 1.36, 1.07 on average.
+    // A slice of at most 24 blocks: with 28 and more the large-M kernel's twice as many slices were up to 7 % faster on one card and up to 5 % slower on another (9728 -> 1408 at
+    // 817 rows 34.3 .. 39.6 / 37.0 .. 37.6), 16384 -> 1408 at 398 33.0 / 34.8 on both.  Without slices up to 56 blocks in tiles of 128 rows that fill 216 units: 7168 -> 1536 at 1800 rows
+    // (204) 48.4 / 50.5, at 2400 (228) 56.5 / 54.7, 11776 -> 1792 at 1948 (tiles of 112) 72.8 / 80.5, 16384 -> 1024 at 2886 97.3 / 111.5, 8192 -> 2304 at 1600 56.0 / 57.0.
+    // Both lines only where columns are whole fours: the large-M kernel sums other slabs value by value (4096 -> 1453 at 1844 rows 50.1 / 36.9, 13312 -> 2187 at 423
+    // 53.5 / 48.5).  Left out, too: two slices (7168 -> 1536 at 930 / 1280 rows 0.94 / 0.97, 8192 -> 381 at 4757 0.94; 16384 -> 1707 at 1060 would be 1.16) and rounds
     // with more units idle (7168 -> 2112 at 400, 204 of 256: 0.96), and up to 640 columns on a K range up to 8192 (7168 -> 576 at 1700 .. 2048 0.99 .. 1.06, with
-    // power-of-two scales 0.94 .. 1.00; these are 0.98 .. 1.53 else).
+    // power-of-two scales 0.94 .. 1.00).
     if (m > 256 && n <= 2304 && kb >= 32 && (t128 >= 6 || kb > 64)) {
         for (int mt : {8, 7}) {
             const int64_t tm = (m + 16 * mt - 1) / (16 * mt), s = 256 / (tm * t128 > 0 ? tm * t128 : 1);
@@ -364,7 +368,9 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
             int64_t nkb = ((kb + s - 1) / s + 3) / 4 * 4;
             nkb = nkb < 8 ? 8 : nkb;
             const int64_t splits = (kb + nkb - 1) / nkb;
-            if (splits == 2 || tm * t128 * splits < (splits == 1 ? 200 : 216) || (p.mt && nkb > p.nkb)) continue;
+            const bool whole = n % 4 == 0;
+            if (splits == 2 || tm * t128 * splits < (splits == 1 && !whole ? 200 : 216) || (p.mt && nkb > p.nkb)) continue;
+            if (whole && (splits > 1 ? nkb > 24 : mt == 7 || kb > 56)) continue;
             p.mt = mt; p.wm = 4; p.sn = 4;
             p.nkb = (int)nkb; p.splits = (int)splits; p.tall = true;
         }

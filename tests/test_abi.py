@@ -589,10 +589,36 @@ WIDE_33_TO_64 = [(32, 36864, 7168, False), (33, 36864, 7168, True), (64, 36864, 
 SLICES_OF_EIGHT = [(139, 15488, 1536, False), (151, 15419, 1536, False), (147, 16000, 2048, True), (159, 8064, 3584, False), (159, 8064, 4096, True),
                    (145, 10816, 2560, False), (145, 10816, 3072, True), (159, 5376, 5632, False), (159, 5376, 6144, True), (158, 4096, 8192, True),
                    (160, 6400, 5120, True)]
+# ... and of the tall tiles of narrow weights: rows, columns, K; slices (none, two, more), their blocks, units, rows a tile; columns in whole fours
+TALL = [(256, 2304, 8192, False), (257, 2304, 8192, True), (257, 2305, 8192, False), (449, 1536, 7168, True), (321, 2112, 7168, True), (350, 2112, 7168, True),
+        (777, 1536, 7168, True), (700, 1536, 7168, True), (400, 2112, 7168, False), (930, 1536, 7168, False), (1280, 1536, 7168, False),
+        (1500, 640, 7168, False), (1500, 641, 7168, True), (1500, 640, 8704, True), (398, 1408, 16384, False), (398, 920, 16384, True),
+        (881, 1408, 13312, False), (881, 1407, 13312, True), (423, 2187, 13312, True), (423, 2188, 13312, False),
+        (1800, 2112, 7168, True), (1600, 2112, 7168, True), (1600, 2304, 8192, False), (1800, 1536, 7168, False), (2400, 1536, 7168, True),
+        (1468, 2176, 6656, False), (2886, 1024, 16384, False), (1948, 1792, 11776, False), (2907, 907, 7680, True), (1844, 1453, 4096, True)]
 
 
-@pytest.mark.parametrize("m,n,k,taken", WIDE_33_TO_64 + SLICES_OF_EIGHT)
+@pytest.mark.parametrize("m,n,k,taken", WIDE_33_TO_64 + SLICES_OF_EIGHT + TALL)
 def test_sizes_that_the_dispatcher_sends_to_the_mid_m_tiles(L, m, n, k, taken):
     takes = L.lib["_ZN4dsv39mid_takesElll"]                     # dsv3::mid_takes(rows, columns, K)
     takes.restype, takes.argtypes = ctypes.c_bool, [ctypes.c_int64] * 3
     assert takes(m, n, k) == taken
+
+
+@pytest.mark.parametrize("knob", ["DSV3_PREFILL_NOSPLIT=1", "DSV3_PREFILL_TILE=128", "DSV3_PREFILL_NOPP=1", "DSV3_PREFILL_NOPP128=1", "OTHER=1"])
+def test_knobs_of_the_large_m_kernel_hold_in_every_window_of_the_mid_m_tiles(knob):
+    """33 .. 64 rows, 65 rows and more, slices of one row tile, 64 x 128 tiles, tall tiles: as the dispatcher asks."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import ctypes
+from dsv3fp8 import _lib
+f = _lib.lib["_ZN4dsv39mid_takesElll"]
+f.restype, f.argtypes = ctypes.c_bool, [ctypes.c_int64] * 3
+print([f(*s) for s in [(33, 36864, 7168), (64, 24576, 7168), (65, 36864, 7168), (193, 7168, 16384), (448, 1536, 7168), (777, 1536, 7168), (1800, 2112, 7168)]])
+"""
+    name, value = knob.split("=")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT / "deepseek-v3_amd", capture_output=True, text=True, env={**os.environ, name: value})
+    assert r.returncode == 0, r.stderr
+    assert r.stdout.strip() == str([name == "OTHER"] * 7)
