@@ -162,6 +162,7 @@ size_t mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int launch_mid(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int c_dtype, int64_t m, int64_t n, int64_t k,
                void* ws, int* splits_out, hipStream_t st);
 bool skinny_supported(int64_t m, int64_t n, int64_t k);
+int skinny_strip_rows(int64_t m, int64_t n, int64_t k, int* waves);      // weight rows and wavefronts of a workgroup
 size_t skinny_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int launch_skinny(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int c_dtype,
                   int64_t m, int64_t n, int64_t k, void* ws, int* splits_out, hipStream_t st, int quant_mode = 0);

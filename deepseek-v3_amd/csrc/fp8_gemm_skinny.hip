@@ -385,11 +385,12 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
         if (!have || fits) { best = p; have = true; }
         if (fits) break;
     }
-    // Strips of eight rows where all of them still are one round of as many wavefronts: a load's consecutive lanes lie in different rows, which
-    // takes a compute unit's load path 64 cycles a KiB, so that 16 rows of 7168 -> 576 are 3 us of 36 units' time with the others idle.  With the
-    // quantisation, us, 16 rows / 8: 7168 -> 576 7.0 / 5.6, 1536 7.2 / 6.0, 1536 -> 1536 4.2 / 4.0, 16384 -> 2048 14.3 / 14.2.  Not with
-    // fewer wavefronts a workgroup: 7168 -> 2112 7.3 / 8.0, 4096 8.2 / 8.7.
-    best.half = m <= 2 && best.s == 1 && best.splits == 1 && (n + 7) / 8 * best.waves <= capacity;
+    // Strips of eight rows where each of them has a compute unit to itself: a load's consecutive lanes lie in different rows, which takes a compute
+    // unit's load path 64 cycles a KiB, so that 16 rows of 7168 -> 576 are 3 us of 36 units' time with the others idle.  With the quantisation, a
+    // graph's node, us, 16 rows / 8: 7168 -> 576 7.0 / 5.6, -> 1536 7.2 / 5.9, -> 2048 7.2 / 6.4, 4096 -> 576 5.3 / 4.4, 1536 -> 1536 4.2 / 3.9, 512 -> 1024 3.5 / 3.4.
+    // Where units have two and more, the weights come no faster and the activations are quantised more often: 3072 -> 2112 4.7 / 5.0, 1024 -> 4096
+    // 4.1 / 4.2, 256 -> 32768 4.8 / 5.3.
+    best.half = m <= 2 && best.s == 1 && best.splits == 1 && (n + 7) / 8 <= 256;
     return best;
 }
 
@@ -426,6 +427,12 @@ void launch_cfg(const Plan& p, const void* a, const float* a_s, const void* b, c
 
 bool skinny_supported(int64_t m, int64_t n, int64_t k) {
     return m >= 1 && m <= 16 && k >= 128 && n >= 1 && (n + 15) / 16 <= 0x7fffffff;
+}
+
+int skinny_strip_rows(int64_t m, int64_t n, int64_t k, int* waves) {
+    const skinny::Plan p = skinny::make_plan(m, n, k);
+    if (waves) *waves = p.waves;
+    return p.half ? 8 : 16 * p.s;
 }
 
 size_t skinny_workspace_bytes(int64_t m, int64_t n, int64_t k) {

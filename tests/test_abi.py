@@ -622,3 +622,12 @@ print([f(*s) for s in [(33, 36864, 7168), (64, 24576, 7168), (65, 36864, 7168), 
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT / "deepseek-v3_amd", capture_output=True, text=True, env={**os.environ, name: value})
     assert r.returncode == 0, r.stderr
     assert r.stdout.strip() == str([name == "OTHER"] * 7)
+
+
+@pytest.mark.parametrize("m,n,k,rows", [
+    (1, 576, 7168, 8), (2, 1536, 7168, 8), (1, 2048, 7168, 8), (1, 2049, 7168, 16), (3, 576, 7168, 16), (1, 2048, 512, 8), (2, 2049, 512, 16), (1, 2048, 384, 8),
+    (1, 128, 128, 8), (1, 2056, 128, 16), (1, 2112, 3072, 16), (2, 4096, 1024, 16), (1, 32768, 256, 16), (1, 2048, 16384, 16)])
+def test_weight_rows_of_a_decode_workgroup(L, m, n, k, rows):
+    f = L.lib["_ZN4dsv317skinny_strip_rowsElllPi"]              # dsv3::skinny_strip_rows(rows, columns, K, *wavefronts)
+    f.restype, f.argtypes = ctypes.c_int, [ctypes.c_int64] * 3 + [ctypes.POINTER(ctypes.c_int)]
+    assert f(m, n, k, None) == rows

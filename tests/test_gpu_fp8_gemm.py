@@ -309,6 +309,26 @@ def test_strips_of_eight_rows_equal_strips_of_sixteen(K, m, n, k):
     assert (got.cpu() - ref).abs().max().item() <= TOL * wide.pow(2).mean().sqrt().item()
 
 
+@pytest.mark.parametrize("n", [1, 7, 9, 129, 576, 2041, 2048])
+@pytest.mark.parametrize("m,k", [(1, 128), (2, 384), (1, 512), (2, 640), (1, 1536), (2, 2048), (1, 4096), (2, 7168)])
+def test_strips_of_eight_rows_have_the_bits_of_strips_of_sixteen(K, m, n, k):
+    """Every number of wavefronts that takes strips of eight rows, against the first columns of a weight of 2176, which has strips of 16 and as
+    many wavefronts (asserted), so that the sums run in one order."""
+    import ctypes
+    from dsv3fp8 import workloads, ops, _lib
+    f = _lib.lib["_ZN4dsv317skinny_strip_rowsElllPi"]           # dsv3::skinny_strip_rows(rows, columns, K, *wavefronts)
+    f.restype, f.argtypes = ctypes.c_int, [ctypes.c_int64] * 3 + [ctypes.POINTER(ctypes.c_int)]
+    waves = ctypes.c_int(), ctypes.c_int()
+    assert f(m, n, k, waves[0]) == 8 and f(m, 2176, k, waves[1]) == 16 and waves[0].value == waves[1].value
+    assert ops.linear_fp8_fused(m, n, k) and ops.linear_fp8_fused(m, 2176, k)
+    x = workloads.activations(m, k, seed=n, outliers=True).cuda()
+    w8, ws = (t.cuda() for t in workloads.weight(2176, k, seed=k % 89))
+    for dtype in (_lib.F32, _lib.BF16):
+        wide = torch.ops.dsv3fp8.linear_fp8(x, w8, ws, _lib.SCALE_FMT_NONE, dtype)
+        got = torch.ops.dsv3fp8.linear_fp8(x, w8[:n].contiguous(), ws[: (n + 127) // 128].contiguous(), _lib.SCALE_FMT_NONE, dtype)
+        assert torch.equal(got, wide[:, :n])
+
+
 def test_leading_dims(K):
     from dsv3fp8 import workloads
     x = workloads.activations(6, 256, seed=1).view(2, 3, 256)
