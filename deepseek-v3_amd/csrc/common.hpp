@@ -209,6 +209,7 @@ int launch_wkv_b_absorb(const void* x, int64_t x_ts, int64_t x_hs, const void* w
                         int64_t tokens, int heads, int nope, int v, int64_t kv_rank, hipStream_t st);
 int launch_wkv_b_absorb_q_packed(const void* x, int64_t x_ts, int64_t x_hs, const void* w, const float* ws, void* y,
                                  int64_t batch, int64_t per_seq, int blocks, int heads, int nope, int v, hipStream_t st);
+bool mla_prefill_paired(int64_t batch, int64_t rows, int heads);               // two query tiles a workgroup
 size_t mla_prefill_workspace_bytes(int64_t batch, int64_t rows, int64_t positions, int heads);
 int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t kv_bs, const void* pe, int64_t pe_bs,
                        const void* w, const float* ws, const void* mask, bool mask_f32, void* y, float* ys, int64_t batch,

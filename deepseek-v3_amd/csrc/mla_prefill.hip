@@ -489,6 +489,13 @@ inline int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
 
 }  // namespace
 
+// Two query tiles a workgroup, the j-th last and the j-th first, where that still makes two workgroups per compute unit:
+// under a causal mask every workgroup then has the same work.  Layer, paired against one tile each (us): 800 rows 277 / 282, 1024
+// 338 / 352, 4096 1527 / 1557; below the line 400 rows 188 / 169.
+bool mla_prefill_paired(int64_t batch, int64_t rows, int heads) {
+    return batch * heads * (((rows + kQTile - 1) / kQTile + 1) / 2) >= 512;
+}
+
 size_t mla_prefill_workspace_bytes(int64_t batch, int64_t rows, int64_t positions, int heads) {
     const int64_t tiles = (positions + kTile - 1) / kTile, groups = (rows + kQGroup - 1) / kQGroup * 8;
     return (size_t)(align256(batch * heads * tiles * kHeadTile) + align256(batch * tiles * kRopeBytes) + align256(tiles * groups));
@@ -499,11 +506,8 @@ int launch_mla_prefill(const void* q, const void* freqs, const void* kv, int64_t
                        int64_t rows, int64_t positions, int heads, float scale, void* workspace, hipStream_t st) {
     const int64_t tiles = (positions + kTile - 1) / kTile, qgroups = (rows + kQGroup - 1) / kQGroup;
     const int64_t qtiles = (rows + kQTile - 1) / kQTile;
-    // Two query tiles a workgroup, the j-th last and the j-th first, where that still makes two workgroups per compute unit:
-    // under a causal mask every workgroup then has the same work.  Layer, paired against one tile each (us): 800 rows 277 / 282, 1024
-    // 338 / 352, 4096 1527 / 1557; below the line 400 rows 188 / 169.
-    const int64_t heads8 = (batch * heads + 7) / 8 * 8, pairs = (qtiles + 1) / 2;
-    const int64_t per_head = batch * heads * pairs >= 512 ? pairs : qtiles;
+    const int64_t heads8 = (batch * heads + 7) / 8 * 8;
+    const int64_t per_head = mla_prefill_paired(batch, rows, heads) ? (qtiles + 1) / 2 : qtiles;
     const int64_t wgs = heads8 * per_head;
     if (wgs > 0x7fffffff || batch * tiles * 2 > 0x7fffffff || qgroups > 65535) return DSV3_ERR_BAD_SHAPE;
     ExpandArgs e;

@@ -208,6 +208,17 @@ def test_query_in_one_call_is_its_three_parts(b, s):
     assert torch.equal(one[0], three[0]) and torch.equal(one[1], three[1]) and one[0][:, start:start + s].any()
 
 
+@pytest.mark.parametrize("b,s,slabs", [(1, 321, 5), (1, 350, 5), (2, 320, 3), (1, 384, 5)])
+def test_query_in_one_call_adds_the_slabs_of_the_tall_tiles(b, s, slabs):
+    import ctypes
+    from dsv3fp8 import _lib
+    assert _lib.lib.dsv3_fp8_gemm_workspace_bytes(b * s, 2112, 7168) >= slabs * b * s * 2112 * 4
+    takes = _lib.lib["_ZN4dsv39mid_takesElll"]                  # dsv3::mid_takes(rows, columns, K)
+    takes.restype, takes.argtypes = ctypes.c_bool, [ctypes.c_int64] * 3
+    assert takes(b * s, 2112, 7168)
+    test_query_in_one_call_is_its_three_parts(b, s)
+
+
 LATENT = [(1, 1, 0, 1536), (3, 1, 7, 1536), (2, 5, 0, 128), (1, 40, 3, 2048), (2, 33, 1, 640)]
 
 
@@ -278,6 +289,23 @@ def test_prefill_attention_query_tiles_of_128(b, s, t, h, kind, offset):
     amax = ref.abs().amax(-1)
     assert ((got - ref).abs() <= amax.unsqueeze(-1) * (16 / 448 + 13 / 512)).all()
     assert ((ys.double() * 448 - amax).abs() <= 13 / 512 * amax).all()
+
+
+# Two query tiles of 128 rows a workgroup (512 workgroups of a pair and more): the j-th last and the j-th first, j of 0 .. 4, whose flags are other
+# words and other windows of 64 position tiles; a middle tile by itself, a last tile of few rows, cached prefixes, two sequences.
+PAIRED = [(1, 800, 800, 128, "causal"), (1, 770, 770, 128, "causal_f32"), (1, 800, 4200, 128, "causal"), (2, 513, 640, 128, "holes"),
+          (1, 1030, 1030, 128, None), (1, 900, 903, 128, "causal")]
+
+
+@pytest.mark.parametrize("b,s,t,h,kind", PAIRED)
+def test_prefill_attention_two_query_tiles_a_workgroup(b, s, t, h, kind):
+    import ctypes
+    from dsv3fp8 import _lib
+    paired = _lib.lib["_ZN4dsv318mla_prefill_pairedElli"]       # dsv3::mla_prefill_paired(sequences, rows, heads)
+    paired.restype, paired.argtypes = ctypes.c_bool, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    assert paired(b, s, h) and not paired(1, 600, 128) and not paired(1, 4200, 16)
+    # (bound: that of test_prefill_attention_query_tiles_of_128, which holds for rows of few positions; in rows of many the errors average out)
+    test_prefill_attention_query_tiles_of_128(b, s, t, h, kind, 0)
 
 
 def _layer(M, p, dim, heads, q_rank, max_seq):
