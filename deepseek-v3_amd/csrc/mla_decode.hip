@@ -679,28 +679,31 @@ __global__ __launch_bounds__(320) void mla_latent_kernel(LatentArgs p) {
 
 // How the positions of a step are split: one attend workgroup per compute unit (its LDS and registers take a whole one; fewer
 // leave units idle, more write more partial sums), a tile a wavefront each at least; and how many tiles a workgroup takes side by side: what
-// costs least by the measured costs (us) of a wavefront's tiles one after another (2.3; 2.65 and 3.6 where two and four at a time leave less or no room for
-// the next ones), of the partial sums (8 to 12 us for those of 256 workgroups of 128 rows) and of the wavefronts' copies, barrier and sum in LDS (0.8 for
-// two; 1.4 for four, next to nothing where a context of one or two tiles leaves half of them without any).  Attention with the query's fold and
-// mla_fold_kernel, us for one / two / four: 1 sequence at 300 positions 23.0 / 24.1 / 24.1, at 700 24.7 / 25.0 / 24.7, at 2000 28.6 / 27.8 / 26.9, 8 at 64
-// 24.6 / 25.4 / 24.5, 8 at 2000 45.1 / 36.0 / 34.7, 24 at 1000 47.6 / 41.0 / 43.9, 64 at 4096 125 / 129 / 152.  Over 168 shapes (1 .. 128 sequences at 40 .. 4096 positions,
-// 1 .. 31 tokens each) the rule is 0.3 % from the best of the three on average, 4 % at most, 1.09 x faster than one everywhere and nowhere more than
-// 1 % slower (with 0.5 and 1.0 for the sums in LDS it was up to 3.3 % slower, at one tile a wavefront).
+// costs least by the measured costs (us) of a wavefront's tiles one after another (2.3; 2.65 and 3.4 where two and four at a time leave less or no room for
+// the next ones), of the partial sums (8 to 12 us for those of 256 workgroups of 128 rows) and of adding the wavefronts' sums: 0.5 for two and 1.0 for four;
+// 0.8 and 1.4 where a wavefront has one tile, whose copies, barrier and sum stand beside nothing, and next to nothing for four where a context of one or two
+// tiles leaves half of the wavefronts without any.  Attention with the query's fold and mla_fold_kernel, us for one / two / four: 1 sequence at 300 positions
+// 23.0 / 24.1 / 24.1, at 700 24.7 / 25.0 / 24.7, at 2000 28.6 / 27.8 / 26.9, 8 at 64 24.6 / 25.4 / 24.5, 8 at 2000 45.1 / 36.0 / 34.7, 32 at 4096 84.8 / 80.5 / 93.5,
+// 64 at 4096 125 / 129 / 152.  Over 168 shapes (1 .. 128 sequences at 40 .. 4096 positions, 1 .. 31 tokens each) the rule is 0.6 % from the best of the three on average,
+// 7 % at most, 1.09 x faster than one everywhere and nowhere more than 1 % slower (with 0.5 and
+// 1.0 everywhere up to 3.3 % slower, at one tile a wavefront).
 // A wavefront has the tiles that one of G = 1 has: longer ranges would round more exponentials (a range's largest is exactly one).
 void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) {
     a.rows = (int)rows; a.positions = (int)positions;
     a.tiles = (int)((positions + kTile - 1) / kTile);
     a.groups = (int)((rows + 127) / 128 * 4);
     double best = 0;
+    bool one_tile = false;                              // a wavefront has one tile
     for (int side = 1; side <= 4; side *= 2) {
         const int64_t blocks = (rows + 128 / side - 1) / (128 / side), base = batch * blocks, steps = (a.tiles + side - 1) / side;
         int64_t splits = 256 / base;
         splits = splits < 1 ? 1 : splits > steps ? steps : splits;
         const int64_t n = (steps + splits - 1) / splits;
         splits = (steps + n - 1) / n;
+        if (side == 1) one_tile = n == 1;
         const int64_t units = base * splits, rounds = (units + 255) / 256;
-        const double us = rounds * (2.3 + (n - 1) * (side == 1 ? 2.3 : side == 2 ? 2.65 : 3.6)) + (rounds - 1) * 3 + units * (128 / side) * 0.00049 +
-                          (side == 1 ? 0 : side == 2 ? 0.8 : a.tiles <= 2 ? 0.2 : 1.4);
+        const double add = side == 1 ? 0 : side == 2 ? (one_tile ? 0.8 : 0.5) : !one_tile ? 1.0 : a.tiles <= 2 ? 0.2 : 1.4;
+        const double us = rounds * (2.3 + (n - 1) * (side == 1 ? 2.3 : side == 2 ? 2.65 : 3.4)) + (rounds - 1) * 3 + units * (128 / side) * 0.00049 + add;
         if (side > 1 && us >= best) continue;
         best = us;
         a.side = side; a.blocks = (int)blocks; a.per = (int)(n * side); a.splits = (int)splits;
