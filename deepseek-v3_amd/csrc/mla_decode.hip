@@ -680,13 +680,13 @@ __global__ __launch_bounds__(320) void mla_latent_kernel(LatentArgs p) {
 // How the positions of a step are split: one attend workgroup per compute unit (its LDS and registers take a whole one; fewer
 // leave units idle, more write more partial sums), a tile a wavefront each at least; and how many tiles a workgroup takes side by side: what
 // costs least by the measured costs (us) of a wavefront's tiles one after another (2.3; 2.65 and 3.4 where two and four at a time leave less or no room for
-// the next ones), of the partial sums (8 to 12 us for those of 256 workgroups of 128 rows) and of adding the wavefronts' sums: 0.5 for two and 1.0 for four;
-// 0.8 and 1.4 where a wavefront has one tile, whose copies, barrier and sum stand beside nothing, and next to nothing for four where a context of one or two
-// tiles leaves half of the wavefronts without any.  Attention with the query's fold and mla_fold_kernel, us for one / two / four: 1 sequence at 300 positions
-// 23.0 / 24.1 / 24.1, at 700 24.7 / 25.0 / 24.7, at 2000 28.6 / 27.8 / 26.9, 8 at 64 24.6 / 25.4 / 24.5, 8 at 2000 45.1 / 36.0 / 34.7, 32 at 4096 84.8 / 80.5 / 93.5,
-// 64 at 4096 125 / 129 / 152.  Over 168 shapes (1 .. 128 sequences at 40 .. 4096 positions, 1 .. 31 tokens each) the rule is 0.6 % from the best of the three on average,
-// 7 % at most, 1.09 x faster than one everywhere and nowhere more than 1 % slower (with 0.5 and
-// 1.0 everywhere up to 3.3 % slower, at one tile a wavefront).
+// the next ones), of the partial sums (8 to 12 us for those of 256 workgroups of 128 rows) and of adding the wavefronts' sums (0.5 for two, 1.0 for four).
+// Where a wavefront has one tile, copies, barrier and sum stand beside nothing (0.8 for two, 1.2 for four, 0.3 where a context of one or two tiles leaves half of
+// these without any), and of the partial sums those of rows that there are cost most, with 0.005 for each range that a row has.  Attention with the query's
+// fold and mla_fold_kernel, us for one / two / four: 1 sequence of 128 heads at 300 positions 23.0 / 24.1 / 24.1, at 700 24.7 / 25.0 / 24.7, at 2000 28.6 / 27.8 /
+// 26.9, 8 at 64 24.6 / 25.4 / 24.5, 8 at 2000 45.1 / 36.0 / 34.7, 32 at 4096 84.8 / 80.5 / 93.5, 64 at 4096 125 / 129 / 152; 4 of 16 heads at 64 19.9 / 21.0 / 20.3.
+// Over 759 shapes of one tile a wavefront (8 .. 128 heads, 1 .. 128 sequences, 1 .. 5 tokens, 32 .. 4000 positions) the rule is 0.4 % from the best of the three on
+// average and 1.06 x faster than one everywhere, at worst 2 % slower (with the costs of several tiles 1.3 % from the best, at worst 14 % slower than one).
 // A wavefront has the tiles that one of G = 1 has: longer ranges would round more exponentials (a range's largest is exactly one).
 void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) {
     a.rows = (int)rows; a.positions = (int)positions;
@@ -702,8 +702,9 @@ void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) 
         splits = (steps + n - 1) / n;
         if (side == 1) one_tile = n == 1;
         const int64_t units = base * splits, rounds = (units + 255) / 256;
-        const double add = side == 1 ? 0 : side == 2 ? (one_tile ? 0.8 : 0.5) : !one_tile ? 1.0 : a.tiles <= 2 ? 0.2 : 1.4;
-        const double us = rounds * (2.3 + (n - 1) * (side == 1 ? 2.3 : side == 2 ? 2.65 : 3.4)) + (rounds - 1) * 3 + units * (128 / side) * 0.00049 + add;
+        double us = rounds * (2.3 + (n - 1) * (side == 1 ? 2.3 : side == 2 ? 2.65 : 3.4)) + (rounds - 1) * 3;
+        if (one_tile) us += units * (128 / side) * 0.0001 + batch * rows * splits * 0.0004 + splits * 0.005 + (side == 1 ? 0 : side == 2 ? 0.8 : a.tiles <= 2 ? 0.3 : 1.2);
+        else us += units * (128 / side) * 0.00049 + (side == 1 ? 0 : side == 2 ? 0.5 : 1.0);
         if (side > 1 && us >= best) continue;
         best = us;
         a.side = side; a.blocks = (int)blocks; a.per = (int)(n * side); a.splits = (int)splits;
