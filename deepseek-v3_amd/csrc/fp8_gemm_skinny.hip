@@ -187,8 +187,9 @@ __global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_
         // the 8 lanes that hold the chunks of one (row, K block) are consecutive and aligned: amax by DPP
 #pragma unroll
         for (int i = 0; i < kSlabChunks; ++i) {
-            // (uniform) Wavefronts without a chunk go on: 16 of them, four turns each, took 0.6 us more of 7.5 (one row of 7168).
-            if (wave * 64 + i * (int)blockDim.x >= chunks) break;
+            // (uniform) Wavefronts without a chunk go on: 16 of them, four turns each, took 0.6 us more of 7.5 (one row of 7168).  Not in the ring
+            // variant, whose K ranges are long enough to give everybody chunks at two rows (16384 -> 7168: 25.1 us, 25.6 with the question).
+            if (!RING && wave * 64 + i * (int)blockDim.x >= chunks) break;
             // (the 16 values are widened twice, for the maximum and for the quotients, instead of being kept: with the
             // weight ring live this section must stay inside the register budget)
             auto widen = [&](int e) { return (e & 1) ? bf16hi_to_f32(raw[i][e >> 3][(e >> 1) & 3]) : bf16lo_to_f32(raw[i][e >> 3][(e >> 1) & 3]); };
