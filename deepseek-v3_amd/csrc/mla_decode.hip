@@ -682,11 +682,12 @@ __global__ __launch_bounds__(320) void mla_latent_kernel(LatentArgs p) {
 // costs least by the measured costs (us) of a wavefront's tiles one after another (2.3; 2.65 and 3.4 where two and four at a time leave less or no room for
 // the next ones), of the partial sums (8 to 12 us for those of 256 workgroups of 128 rows) and of adding the wavefronts' sums (0.5 for two, 1.0 for four).
 // Where a wavefront has one tile, copies, barrier and sum stand beside nothing (0.8 for two, 1.2 for four, 0.3 where a context of one or two tiles leaves half of
-// these without any), and of the partial sums those of rows that there are cost most, with 0.005 for each range that a row has.  Attention with the query's
-// fold and mla_fold_kernel, us for one / two / four: 1 sequence of 128 heads at 300 positions 23.0 / 24.1 / 24.1, at 700 24.7 / 25.0 / 24.7, at 2000 28.6 / 27.8 /
-// 26.9, 8 at 64 24.6 / 25.4 / 24.5, 8 at 2000 45.1 / 36.0 / 34.7, 32 at 4096 84.8 / 80.5 / 93.5, 64 at 4096 125 / 129 / 152; 4 of 16 heads at 64 19.9 / 21.0 / 20.3.
-// Over 759 shapes of one tile a wavefront (8 .. 128 heads, 1 .. 128 sequences, 1 .. 5 tokens, 32 .. 4000 positions) the rule is 0.4 % from the best of the three on
-// average and 1.06 x faster than one everywhere, at worst 2 % slower (with the costs of several tiles 1.3 % from the best, at worst 14 % slower than one).
+// these without any), and of the partial sums those of rows that there are cost most, with 0.01 for each range that a row has.  The layer, us for one /
+// two / four, three layers' weights in turn: 1 sequence of 128 heads at 300 positions 65.5 / 66.1 / 66.6, at 700 65.9 / 65.4 / 65.6, at 2000 69.2 / 68.2 / 67.4, 8 at 64
+// 69.8 / 69.5 / 68.7; attention with the query's fold and mla_fold_kernel: 8 at 2000 45.1 / 36.0 / 34.7, 32 at 4096 84.8 / 80.5 / 93.5, 64 at 4096 125 / 129 / 152, 4 of 16
+// heads at 64 19.9 / 21.0 / 20.3.  Over 759 shapes of one tile a wavefront (8 .. 128 heads, 1 .. 128 sequences, 1 .. 5 tokens, 32 .. 4000 positions) the rule is 0.4 %
+// from the best of the three on average and 1.06 x faster than one everywhere, at worst 2 % slower (with the costs of several tiles 1.3 % from the
+// best, at worst 14 % slower than one); in the layer 0.10 us from the best on average over 47 of them, 0.27 before.
 // A wavefront has the tiles that one of G = 1 has: longer ranges would round more exponentials (a range's largest is exactly one).
 void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) {
     a.rows = (int)rows; a.positions = (int)positions;
@@ -703,7 +704,7 @@ void decode_plan(DecodeArgs& a, int64_t batch, int64_t rows, int64_t positions) 
         if (side == 1) one_tile = n == 1;
         const int64_t units = base * splits, rounds = (units + 255) / 256;
         double us = rounds * (2.3 + (n - 1) * (side == 1 ? 2.3 : side == 2 ? 2.65 : 3.4)) + (rounds - 1) * 3;
-        if (one_tile) us += units * (128 / side) * 0.0001 + batch * rows * splits * 0.0004 + splits * 0.005 + (side == 1 ? 0 : side == 2 ? 0.8 : a.tiles <= 2 ? 0.3 : 1.2);
+        if (one_tile) us += units * (128 / side) * 0.0001 + batch * rows * splits * 0.0004 + splits * 0.01 + (side == 1 ? 0 : side == 2 ? 0.8 : a.tiles <= 2 ? 0.3 : 1.2);
         else us += units * (128 / side) * 0.00049 + (side == 1 ? 0 : side == 2 ? 0.5 : 1.0);
         if (side > 1 && us >= best) continue;
         best = us;
@@ -757,9 +758,10 @@ int launch_mla_decode(const void* q, const void* freqs, const void* kv, int64_t 
     a.mask = mask; a.heads = heads;
     const ScoreUnit u = mask ? score_unit(scale) : ScoreUnit{ 1.f, scale };
     a.unit = u.unit; a.scale = u.rest; a.inv_scale = 1.0f / u.rest;
-    // Operand order up to 16 tokens in all: the attention gains 2 us (1 at 700: 12.7 -> 10.7, 3 at 200: 12.4 -> 10.3, 8 at 2000: 24.2 ->
-    // 22.2), the fold's scattered stores cost it 0.4.  With more they cost 1 to 1.7 us (32 tokens 5.1 -> 6.1, 64 6.2 -> 7.8), the gain
-    // disappears behind the tiles (32 at 4096: 56.7 -> 56.4, 64 at 1000: 39.7 -> 39.6).
+    // Operand order up to 16 tokens in all, which is what the kernel that writes it takes (a sub-tile of 16 tokens): query's fold, attention and
+    // mla_fold_kernel of 128 heads at 100 / 700 / 4096 positions, rows against operand order, 1 sequence 25.1 / 27.4 / 31.0 -> 23.1 / 25.8 / 28.4 us, 4 26.8 / 30.2 / 37.0 ->
+    // 25.3 / 28.0 / 34.6, 16 29.6 / 35.5 / 54.7 -> 27.9 / 33.7 / 52.9.  With more tokens, tried with one tile at a time, the fold's scattered stores cost 1 to 1.7 us
+    // (32 tokens 5.1 -> 6.1, 64 6.2 -> 7.8) and the gain disappears behind the tiles.
     const bool pack = batch * tokens <= 16;
     const int rc = pack ? launch_wkv_b_absorb_q_packed(q, (int64_t)heads * kQd, kQd, w, ws, wsp, batch, tokens, a.groups / 4, heads, kNope, kNope, st)
                         : launch_wkv_b_absorb(q, (int64_t)heads * kQd, kQd, w, ws, wsp, DSV3_ABSORB_Q, batch * tokens, heads, kNope, kNope, kC, st);

@@ -413,10 +413,11 @@ class MLA(nn.Module):
         pair of 1088 multiply-adds in place of 320 but costs nothing per position.  Both sides in microseconds as the kernels
         take them, 128 heads: expanding a position 0.048; a round of 256 decode workgroups (128 (token, head) rows x a range
         of ``per`` 32-position tiles each, one to a compute unit) 5 + 2.65 per tile, a block of rows 0.2 for its partial
-        sums and folded rows.  The costs were fitted before the absorbed form's last kernels became one, which takes 5 to 15 %
-        less.  Over 272 shapes (1 .. 16 sequences, 32 .. 384 new tokens, 64 .. 16384 positions) the form chosen so is now at
-        most 9 % slower than the better one, 0.2 % on average; 32 new tokens as the line, whatever the positions, would be
-        up to 4.3 times slower (8 sequences x 32 tokens at 16384 positions: 6572 us explicit, 1520 absorbed)."""
+        sums and folded rows.  The costs were fitted to earlier forms of both kernels; as these are now, over 247 shapes
+        (1 .. 16 sequences, 32 .. 384 new tokens, 64 .. 16384 positions) the form chosen so is at most 8 % slower than the
+        better one (1 x 64 tokens at 700 positions: 58.4 us explicit, 53.9 absorbed), 0.1 % on average; 32 new tokens as the
+        line, whatever the positions, would be up to 3.4 times slower (16 sequences x 32 tokens at 4096 positions: 3091 us
+        explicit, 908 absorbed)."""
         if tokens < self.explicit_min_tokens:
             return False
         blocks = batch * -(-tokens * self.n_local_heads // 128)

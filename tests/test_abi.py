@@ -569,7 +569,7 @@ def test_attention_kernel_may_keep_scalars_in_lanes_but_spill_no_vector_register
 # Which variant of the decode attention (tiles that a workgroup takes side by side) the cost rule picks (sequences, tokens, positions, heads): at one
 # tile a wavefront the measured fastest or one within 1 % of it; then the sizes that tests/test_gpu_mla_attention.py has for each variant.
 @pytest.mark.parametrize("side,b,s,t,h", [
-    (1, 1, 1, 40, 128), (1, 1, 1, 300, 128), (1, 1, 1, 700, 128), (1, 2, 1, 300, 128), (1, 3, 1, 200, 128), (1, 4, 1, 128, 128), (1, 48, 1, 4096, 128),
+    (1, 1, 1, 40, 128), (1, 1, 1, 300, 128), (2, 1, 1, 700, 128), (1, 2, 1, 300, 128), (1, 3, 1, 200, 128), (1, 4, 1, 128, 128), (1, 48, 1, 4096, 128),
     (1, 64, 1, 4096, 128), (1, 96, 1, 2000, 128), (2, 12, 1, 4096, 128), (2, 24, 1, 2000, 128), (2, 32, 1, 4096, 128), (2, 64, 1, 1000, 128),
     (4, 1, 1, 1000, 128), (4, 2, 1, 512, 128),
     (1, 4, 1, 64, 16), (1, 8, 1, 128, 64), (1, 1, 2, 700, 16), (1, 4, 1, 300, 16), (1, 1, 1, 700, 32), (4, 1, 5, 2200, 16), (4, 2, 5, 700, 32), (4, 8, 1, 40, 128), (4, 16, 1, 64, 128), (4, 1, 1, 2000, 128), (4, 2, 1, 1000, 128), (4, 8, 1, 2000, 128), (4, 32, 1, 200, 128),
