@@ -156,7 +156,7 @@ size_t stream_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int launch_stream(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int c_dtype,
                   int64_t m, int64_t n, int64_t k, void* ws, int* splits_out, hipStream_t st);
 bool mid_takes(int64_t m, int64_t n, int64_t k);
-bool mid_supported(int64_t m, int64_t n, int64_t k);          // of these, from 65 rows on and not the tall tiles of narrow weights
+bool mid_supported(int64_t m, int64_t n, int64_t k);          // of these, from 65 rows on and not the tall tiles of narrow weights (no dispatcher asks this)
 bool mid_takes_scales(const float* a_s, const float* b_s);
 size_t mid_workspace_bytes(int64_t m, int64_t n, int64_t k);
 int launch_mid(const void* a, const float* a_s, const void* b, const float* b_s, void* c, int c_dtype, int64_t m, int64_t n, int64_t k,

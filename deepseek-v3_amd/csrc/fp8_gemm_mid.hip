@@ -1,5 +1,5 @@
-// fp8_gemm for 65 rows and more where whole 256-column tiles leave compute units without work: up to 256 rows of wide weights, up to
-// a few hundred of narrow ones, 8192 where these have 128 columns or fewer
+// fp8_gemm for 33 rows and more where whole 256-column tiles leave compute units without work: up to 256 rows of wide weights, up to
+// a few thousand of narrow ones, 8192 where these have 128 columns or fewer
 // (reference arithmetic: inference/kernel.py:118-172).
 //
 // A tile of 16 MT rows x 16 SN WN columns per workgroup: eight wavefronts, WM along the rows (16-row sub-tiles dealt round-robin) x
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(2, 2
 #endif
 }
 
-// Three windows in which the large-M kernel's tiles fit the chip badly.  Power-of-two scales take the same kernel (accumulating in the
+// Five windows in which the large-M kernel's tiles fit the chip badly.  Power-of-two scales take the same kernel (accumulating in the
 // matrix core was equal to 4 % faster here).
 struct Plan { int mt, wm, sn, splits, nkb; bool tall; };       // mt == 0: not for this kernel; tall: more than 256 rows of narrow weights
 // The variables that pin how the large-M kernel runs its dense tiles (one K slice, a tile height, a schedule) pin that kernel too.
@@ -292,7 +292,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k) {
     // 32768 columns and fewer, where 128-row tiles of the large-M kernel, two a column tile or in two K slices, are one full round
     // (7168 -> 31744 at 65 / 160 / 193 rows 0.93 / 0.88 / 0.84); K of 32768 (0.81 .. 1.50, 0.92 .. 0.96 at 193 rows); from 193 rows on,
     // whose ring has three stages, fewer than 212 tiles or 32 K blocks (16384 -> 32769 0.94, 2560 -> 40960 0.98); 225 rows and more, whose
-    // ring would have two.  33 .. 64 rows of such weights are the large-M kernel's otherwise, too (fp8_gemm_tile.hip): 7168 -> 36864 at 33 / 64 rows 61.2 /
+    // ring would have two.  33 .. 64 rows of such weights are the large-M kernel's otherwise, too (fp8_gemm_tile.hip): 7168 -> 36864 at 33 / 64 rows, the product alone, 61.2 /
     // 66.7 us there, 53.5 / 56.9 here, over 32769 .. 40960 columns and K of 2560 .. 16384 1.05 .. 1.21.  Nor two row tiles of 116 for 7168 -> 18432 (129 .. 224 rows, 48.4 us there, 53.5 here at 193): that one 128- or
     // 256-row tile of the large-M kernel reads the weights once.
     const int64_t t160 = (n + 159) / 160, rows = (m + 15) / 16;

@@ -416,8 +416,8 @@ class MLA(nn.Module):
         sums and folded rows.  The costs were fitted to earlier forms of both kernels; as these are now, over 247 shapes
         (1 .. 16 sequences, 32 .. 384 new tokens, 64 .. 16384 positions) the form chosen so is at most 8 % slower than the
         better one (1 x 64 tokens at 700 positions: 58.4 us explicit, 53.9 absorbed), 0.1 % on average; 32 new tokens as the
-        line, whatever the positions, would be up to 3.4 times slower (16 sequences x 32 tokens at 4096 positions: 3091 us
-        explicit, 908 absorbed)."""
+        line, whatever the positions, would be up to 4.2 times slower (1 sequence x 32 tokens at 16384 positions: 921 us explicit,
+        220 absorbed)."""
         if tokens < self.explicit_min_tokens:
             return False
         blocks = batch * -(-tokens * self.n_local_heads // 128)
